@@ -59,28 +59,31 @@ def _stale(obj, src, deps):
 
 
 def build_hip(verbose=True, force=True):
-    """Compile the three translation units (in parallel) and link
-    librtm_hip.so.  force=False recompiles only the units whose source or
-    headers changed since their object in lib/obj was written."""
+    """Compile the translation units (in parallel; the stencil kernels once
+    per half-length) and link librtm_hip.so.  force=False recompiles only the
+    units whose source or headers changed since their object in lib/obj was
+    written."""
     os.makedirs(LIB, exist_ok=True)
     obj_dir = os.path.join(LIB, "obj")
     os.makedirs(obj_dir, exist_ok=True)
     out = os.path.join(LIB, "librtm_hip.so")
-    srcs = [os.path.join(CSRC, f) for f in ("rtm_kernels.hip", "rtm_capi.hip", "rtm_cnn.hip")]
-    objs = [os.path.join(obj_dir, os.path.basename(s) + ".o") for s in srcs]
-    deps = [os.path.join(CSRC, "rtm_kernels.h"), os.path.join(ROOT, "include", "rtm_hip.h"),
-            os.path.join(ROOT, "include", "rtm_cnn.h")]
-    todo = [(s, o) for s, o in zip(srcs, objs) if force or _stale(o, s, deps)]
-    # translation units compile in parallel (hipcc is single-threaded)
+    # the longest half-lengths take longest to compile: first
+    units = [("rtm_stencil.hip", f"stencil_{n}.o", [f"-DRTM_NFD={n}"]) for n in range(12, 0, -1)]
+    units += [(f, f + ".o", []) for f in ("rtm_kernels.hip", "rtm_capi.hip", "rtm_cnn.hip")]
+    units = [(os.path.join(CSRC, f), os.path.join(obj_dir, o), d) for f, o, d in units]
+    deps = [os.path.join(CSRC, "rtm_kernels.h"), os.path.join(CSRC, "rtm_device.h"),
+            os.path.join(ROOT, "include", "rtm_hip.h"), os.path.join(ROOT, "include", "rtm_cnn.h")]
+    todo = [(s, o, d) for s, o, d in units if force or _stale(o, s, deps)]
     from concurrent.futures import ThreadPoolExecutor
-    with ThreadPoolExecutor(max_workers=max(1, len(todo))) as ex:
-        futs = [ex.submit(_run, [HIPCC, *HIP_FLAGS, "-I", os.path.join(ROOT, "include"), "-c", s,
-                                 "-o", o + ".tmp"], verbose) for s, o in todo]
+    jobs = int(os.environ.get("MAX_JOBS", 0)) or min(16, os.cpu_count() or 1)
+    with ThreadPoolExecutor(max_workers=jobs) as ex:
+        futs = [ex.submit(_run, [HIPCC, *HIP_FLAGS, *d, "-I", os.path.join(ROOT, "include"), "-c",
+                                 s, "-o", o + ".tmp"], verbose) for s, o, d in todo]
         for f in futs:
             f.result()
-    for _, o in todo:
+    for _, o, _d in todo:
         os.replace(o + ".tmp", o)
-    _run([HIPCC, *HIP_FLAGS, "-shared", "-o", out + ".tmp", *objs], verbose)
+    _run([HIPCC, *HIP_FLAGS, "-shared", "-o", out + ".tmp", *(o for _, o, _d in units)], verbose)
     os.replace(out + ".tmp", out)
     return out
 

@@ -1,7 +1,7 @@
 // rtm_capi.hip -- the C ABI of librtm_hip.so (declared in include/rtm_hip.h).
 //
 // Owns the device memory of a context and sequences the kernels of
-// rtm_kernels.hip on the context's stream.  Replaces the device-side part of
+// rtm_stencil.hip and rtm_kernels.hip on the context's stream.  Replaces the device-side part of
 // the reference's main(): allocation and uploads (kernel.cu:758-786), the
 // forward time loop (kernel.cu:798-825), the backward loop with imaging
 // (kernel.cu:859-933).  Deliver/Deliver_EFF copies are replaced by rotating

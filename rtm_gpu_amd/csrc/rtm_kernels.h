@@ -1,5 +1,5 @@
 // rtm_kernels.h -- device-side data structures shared by the gfx950 kernels
-// (rtm_kernels.hip) and the C-ABI glue (rtm_capi.hip).  Internal header.
+// (rtm_stencil.hip, rtm_kernels.hip) and the C-ABI glue (rtm_capi.hip).  Internal header.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -134,6 +134,17 @@ struct FrameArgs {
   // (k_strip_restore's work)
   float* rf;
   int rbps;
+};
+
+// Stencil kernels of one compile-time half-length: rtm_stencil.hip is compiled
+// once per NFD and defines these members for it.
+template <int NFD>
+struct StencilOps {
+  static hipError_t interior(int epi, dim3 grid, const IntArgs& a, hipStream_t s);
+  static hipError_t frame(int mode, dim3 grid, const FrameArgs& a, hipStream_t s);
+  static hipError_t frame4(int mode, dim3 grid, const FrameArgs& a, hipStream_t s);
+  static hipError_t step(int epi, dim3 grid, const IntArgs& ia, const FrameArgs& fa, unsigned nint,
+                         unsigned nfr, hipStream_t s);
 };
 
 // Launchers (rtm_kernels.hip).  nfd_inst is the compile-time stencil
