@@ -209,8 +209,8 @@ def run_apertures(a):
 def algorithmic_bytes(kind, d, n2, nfd, nshot, n):
     """Minimum HBM bytes one launch of each kernel must move.  Per interior
     cell and shot: forward / source reconstruction read u1, u0 and write u2
-    (12 B); the receiver step reads q1, q0, u(k), sum u, sum q, I1, I2 and
-    writes q2, sum u, sum q, I1, I2 (48 B).  The velocity model is shared by
+    (12 B), and so does the receiver step; every third one also images.  The
+    velocity model is shared by
     the shots of a launch (4 B per cell per launch)."""
     from rtm_gpu_amd import hip
     nz, nx = d.nz, d.nx
@@ -223,17 +223,14 @@ def algorithmic_bytes(kind, d, n2, nfd, nshot, n):
         return nshot * (nF * 12 + ss * 4) + nF * 4
     if kind == hip.K_STRIP_RESTORE:
         return nshot * ss * 8
-    if kind == hip.K_RCV_INTERIOR:
-        return nshot * (nI * 48 + n * 4) + nI * 4
+    if kind == hip.K_RCV_INTERIOR:  # without imaging
+        return nshot * (nI * 12 + n * 4) + nI * 4
     if kind == hip.K_RCV_FRAME:
         return nshot * (nF * 12 + n * 4) + nF * 4
-    # the split backward step (compensated imaging): the reconstruction also
-    # updates sum u and I2 (12 + 16 B); the receiver step reads q1, q0, sum u,
-    # sum q, I1 and writes q2, sum q, I1 (32 B)
-    if kind == hip.K_SRCI_INTERIOR:
-        return nshot * nI * 28 + nI * 4
+    # imaging three steps: also reads u(k), u(k+1), u(k+2), reads and writes
+    # sum u, sum q, I1, I2 (12 + 12 + 32 B)
     if kind == hip.K_RCVI_INTERIOR:
-        return nshot * (nI * 32 + n * 4) + nI * 4
+        return nshot * (nI * 56 + n * 4) + nI * 4
     # Born: dU1, dU0, u(k), u(k-1), u(k-2) read, dU2 written (24 B) + v, m shared
     if kind == hip.K_BORN_INTERIOR:
         return nshot * nI * 24 + nI * 8
@@ -854,7 +851,8 @@ def main():
     # algorithmic bytes of both.
     fusedk = {} if not a.fuse_frame else {
         hip.K_FWD_INTERIOR: (hip.K_FWD_FRAME, "k_step<EPI_FWD+FR_FWD>"),
-        hip.K_RCVI_INTERIOR: (hip.K_RCV_FRAME, "k_step<EPI_RCVI+FR_RCV>")}
+        hip.K_RCV_INTERIOR: (hip.K_RCV_FRAME, "k_step<EPI_RCV0+FR_RCV>"),
+        hip.K_RCVI_INTERIOR: (hip.K_RCV_FRAME, "k_step<EPI_RCV+FR_RCV>")}
     # Without a checkpoint snapshot (none here) and with separate launches, the
     # receiver frame launch of every backward step also restores the strips of
     # the reconstructed field (k_strip_restore's work and bytes).

@@ -76,6 +76,7 @@ struct rtm_ctx {
   int nshot = 0;
   int f0 = 0, f1 = 1, f2 = 2, q0 = 0, q1 = 1, q2 = 2;
   int kf = -1, kb = -2;  // next forward / backward step; -1/-2 = not begun
+  int img_pend = 0;      // backward steps whose image terms are still to be applied (0..2)
   // least-squares migration operators
   bool born = false;     // the forward pass is a Born pass (records hold dU)
   bool adj = false;      // the backward pass is the adjoint of Born modelling
@@ -228,6 +229,7 @@ void fill_int_args(rtm_ctx* c, IntArgs& a) {
   a.zs = c->zs;
   a.data = c->d_data;
   a.uk = nullptr;
+  a.nimg = 1;
   a.su = c->SU; a.sq = c->SQ; a.i1 = c->I1; a.i2 = c->I2;
   a.icompen = c->p.icompen;
   a.ua = a.ub = a.uc = nullptr;
@@ -350,24 +352,24 @@ int forward_step(rtm_ctx* c, int k) {
   return RTM_OK;
 }
 
-int backward_step(rtm_ctx* c, int k) {
+// Backward step k.  The image terms of a step (Rel_*, kernel.cu:489-517) are
+// applied by the receiver step of every third step for the three steps at once
+// (k_interior<EPI_RCV>): the rotating buffers still hold u(k+2), u(k+1), u(k)
+// and the receiver field's operands are q(k+2), q(k+1).  A checkpoint step's
+// u(k) is in its buffer by then too.  flush: the caller may look at the images
+// after this step, so the terms of every step so far are applied.
+int backward_step(rtm_ctx* c, int k, bool flush) {
   const float wv = (k < c->p.nt2) ? c->wav[k + 1] : 0.0f;  // kernel.cu:889-890
-  // Rel_* (kernel.cu:489-517) is split between the two interior kernels: the
-  // terms of u(k) alone (sum u += u, I2 += u*u) go with its reconstruction,
-  // the rest with the receiver step.  At a checkpoint step the snapshot
-  // replaces u(k) after the reconstruction, and the non-compensated image
-  // (I1 += q*u) needs u(k) in the receiver step anyway: there the receiver
-  // step does all.
-  const bool split = c->snap_slot[k] < 0 && c->p.icompen == 1;
-  const int esrc = split ? EPI_SRCI : EPI_SRC, ercv = split ? EPI_RCVI : EPI_RCV;
+  const bool image = flush || c->img_pend == 2;
+  const int ercv = image ? EPI_RCV : EPI_RCV0;
   {  // BKAdd_EFF (kernel.cu:896): u(k) on the interior
     IntArgs a;
     fill_int_args(c, a);
     a.u1 = c->F[c->f1]; a.u0 = c->F[c->f0]; a.u2 = c->F[c->f2];
     a.wav = wv; a.k = k;
-    Timed t(c, split ? RTM_K_SRCI_INTERIOR : RTM_K_SRC_INTERIOR);
-    a.zs = zs_for(c, esrc);
-    HIPCHK(c, launch_interior(esrc, c->nfd, a, c->nshot, c->stream));
+    Timed t(c, RTM_K_SRC_INTERIOR);
+    a.zs = zs_for(c, EPI_SRC);
+    HIPCHK(c, launch_interior(EPI_SRC, c->nfd, a, c->nshot, c->stream));
   }
   // strips of slot k into the rings of u(k): BKEqual of step k-1 (kernel.cu:892).
   // Nothing in the receiver step reads those rings, so on ordinary steps the
@@ -386,7 +388,8 @@ int backward_step(rtm_ctx* c, int k) {
     IntArgs a;
     fill_int_args(c, a);
     a.u1 = c->Q[c->q1]; a.u0 = c->Q[c->q0]; a.u2 = c->Q[c->q2];
-    a.uk = c->F[c->f1];
+    a.uk = c->F[c->f1]; a.ua = c->F[c->f0]; a.ub = c->F[c->f2];
+    a.nimg = c->img_pend + 1;
     a.wav = 0.f; a.k = k;
     a.zs = zs_for(c, ercv);
     FrameArgs f;
@@ -397,7 +400,7 @@ int backward_step(rtm_ctx* c, int k) {
       f.rf = c->F[c->f1];
       f.rbps = strip_restore_blocks(c->g);
     }
-    const int kind = split ? RTM_K_RCVI_INTERIOR : RTM_K_RCV_INTERIOR;
+    const int kind = image ? RTM_K_RCVI_INTERIOR : RTM_K_RCV_INTERIOR;
     if (fused(c, ercv, FR_RCV)) {
       Timed t(c, kind);  // the fused launch counts as the interior kind
       HIPCHK(c, launch_step(ercv, FR_RCV, c->nfd, a, f, c->nshot, c->ntiles, c->stream));
@@ -410,6 +413,7 @@ int backward_step(rtm_ctx* c, int k) {
       HIPCHK(c, launch_frame_split(c, FR_RCV, f));
     }
   }
+  c->img_pend = image ? 0 : c->img_pend + 1;
   if (watch_due(c, k, 0)) {  // the reconstructed u(k) and the new receiver field
     int rc = watch(c, c->F[c->f1], k);
     if (rc == RTM_OK) rc = watch(c, c->Q[c->q2], k);
@@ -1089,6 +1093,7 @@ int rtm_backward_begin(rtm_ctx* c) {
   // BKEqual of the first backward step (kernel.cu:892, k = NT-3): slot NT-2.
   HIPCHK(c, launch_strip_restore(c->g, c->F[c->f1], c->st, c->d_geo, c->p.nt - 2, c->nshot, c->stream));
   c->kb = c->p.nt - 3;
+  c->img_pend = 0;
   return RTM_OK;
 }
 
@@ -1096,7 +1101,7 @@ int rtm_backward_advance(rtm_ctx* c, int nsteps) {
   if (!c) return RTM_E_ARG;
   if (c->kb < -1) return fail(c, RTM_E_STATE, "rtm_backward_begin first");
   for (int i = 0; i < nsteps && c->kb >= 0; ++i, --c->kb) {
-    int rc = backward_step(c, c->kb);
+    int rc = backward_step(c, c->kb, i == nsteps - 1 || c->kb == 0);
     if (rc != RTM_OK) return rc;
   }
   return watch_read(c, "backward");
@@ -1451,8 +1456,8 @@ int rtm_set_zseg(rtm_ctx* c, const int* zseg) {
     if (zseg[i] < 1 || zseg[i] > 4096) return fail(c, RTM_E_ARG, "rows per wave %d", zseg[i]);
   const int fwd = c->p.ilste ? EPI_FWD64 : EPI_FWD;
   c->zs_epi[fwd] = zseg[0];
-  c->zs_epi[EPI_SRC] = c->zs_epi[EPI_SRCI] = zseg[1];
-  c->zs_epi[EPI_RCV] = c->zs_epi[EPI_RCVI] = zseg[2];
+  c->zs_epi[EPI_SRC] = zseg[1];
+  c->zs_epi[EPI_RCV] = c->zs_epi[EPI_RCV0] = zseg[2];
   c->zs_epi[EPI_BORN] = c->zs_epi[EPI_BORN64] = c->zs_epi[EPI_ADJ] = zseg[2];
   c->zs = zseg[0];
   drop_graph(c);
@@ -1501,18 +1506,18 @@ int rtm_autotune(rtm_ctx* c, int nsteps, int* zseg) {
     rc = launch_fill(c->d_data, (long long)c->nshot * c->p.nt * c->p.n, 0.f, c->stream) == hipSuccess
              ? RTM_OK : fail(c, RTM_E_HIP, "autotune: fill");
   const int fwd = c->p.ilste ? EPI_FWD64 : EPI_FWD;
-  const bool split = c->p.icompen == 1;
-  const int kinds[3] = {fwd, split ? EPI_SRCI : EPI_SRC, split ? EPI_RCVI : EPI_RCV};
-  const int timers[3] = {RTM_K_FWD_INTERIOR, split ? RTM_K_SRCI_INTERIOR : RTM_K_SRC_INTERIOR,
-                         split ? RTM_K_RCVI_INTERIOR : RTM_K_RCV_INTERIOR};
-  for (int ki = 0; ki < 3; ++ki)
+  constexpr int kKinds = 4;
+  const int kinds[kKinds] = {fwd, EPI_SRC, EPI_RCV0, EPI_RCV};
+  const int timers[kKinds] = {RTM_K_FWD_INTERIOR, RTM_K_SRC_INTERIOR, RTM_K_RCV_INTERIOR,
+                              RTM_K_RCVI_INTERIOR};
+  for (int ki = 0; ki < kKinds; ++ki)
     if (c->zs_epi[kinds[ki]] <= 0) c->zs_epi[kinds[ki]] = 32;
   const int nt = c->p.nt;
   int kf = 2, kb = nt - 3;
   auto pairs = [&](int n) -> int {
     for (int i = 0; i < n; ++i) {
       int r = forward_step(c, kf);
-      if (r == RTM_OK) r = backward_step(c, kb);
+      if (r == RTM_OK) r = backward_step(c, kb, false);
       if (r != RTM_OK) return r;
       kf = kf + 1 < nt ? kf + 1 : 2;
       kb = kb > 0 ? kb - 1 : nt - 3;
@@ -1523,7 +1528,8 @@ int rtm_autotune(rtm_ctx* c, int nsteps, int* zseg) {
   // The candidates are measured in kRounds interleaved rounds, alternating in
   // direction, and compared on their summed times, so that drift of the
   // device (clocks, caches, the other kernels) falls on all of them alike.
-  const int per = std::max(2, nsteps / 2);
+  // per covers a whole imaging cycle of three backward steps.
+  const int per = std::max(3, nsteps / 2);
   auto measure = [&](unsigned mask, double* ms) -> int {
     c->timing = 0;
     int r = pairs(1);
@@ -1539,7 +1545,7 @@ int rtm_autotune(rtm_ctx* c, int nsteps, int* zseg) {
       if (mask & (1u << k)) *ms += c->t_n[k] ? c->t_ms[k] / c->t_n[k] : 1e300;
     return RTM_OK;
   };
-  for (int ki = 0; ki < 3 && rc == RTM_OK; ++ki) {
+  for (int ki = 0; ki < kKinds && rc == RTM_OK; ++ki) {
     const int epi = kinds[ki];
     const int ql = interior_queue_rows(epi, c->nfd);
     double tot[kNC] = {0.0};
@@ -1570,7 +1576,7 @@ int rtm_autotune(rtm_ctx* c, int nsteps, int* zseg) {
     // carry them (counted under the interior kinds)
     const unsigned fmask =
         (fused(c, fwd, FR_FWD) ? 1u << RTM_K_FWD_INTERIOR : 1u << RTM_K_FWD_FRAME) |
-        (fused(c, kinds[2], FR_RCV) ? 1u << timers[2] : 1u << RTM_K_RCV_FRAME);
+        (fused(c, EPI_RCV0, FR_RCV) ? 1u << RTM_K_RCV_INTERIOR : 1u << RTM_K_RCV_FRAME);
     for (int which = 0; which < 2 && rc == RTM_OK; ++which) {
       int& run = which == 0 ? c->fseg_tb : c->fseg_side;
       double tot[3] = {0.0, 0.0, 0.0};
@@ -1607,19 +1613,15 @@ int rtm_autotune(rtm_ctx* c, int nsteps, int* zseg) {
   c->timing = saved_timing;
   c->check_every = saved_check;
   for (int i = 0; i < RTM_K_NKINDS; ++i) { c->t_ms[i] = 0.0; c->t_n[i] = 0; }
-  if (split) {  // checkpoint steps run the unsplit kernels of the same shape
-    c->zs_epi[EPI_SRC] = c->zs_epi[EPI_SRCI];
-    c->zs_epi[EPI_RCV] = c->zs_epi[EPI_RCVI];
-  }
-  c->zs_epi[EPI_BORN] = c->zs_epi[EPI_BORN64] = c->zs_epi[EPI_ADJ] = c->zs_epi[kinds[2]];
+  c->zs_epi[EPI_BORN] = c->zs_epi[EPI_BORN64] = c->zs_epi[EPI_ADJ] = c->zs_epi[EPI_RCV];
   c->zs = c->zs_epi[fwd];
   c->kf = -1;
   c->kb = -2;
   drop_graph(c);
   if (zseg) {  // the kernels of an ordinary migration step
     zseg[0] = c->zs_epi[fwd];
-    zseg[1] = c->zs_epi[kinds[1]];
-    zseg[2] = c->zs_epi[kinds[2]];
+    zseg[1] = c->zs_epi[EPI_SRC];
+    zseg[2] = c->zs_epi[EPI_RCV0];
   }
   return rc;
 }

@@ -74,12 +74,11 @@ struct Snaps {
 };
 
 // Interior epilogues: forward (FP32 / FP64 combine), source reconstruction,
-// receiver step + imaging, Born scattered field (FP32 / FP64 combine), the
-// adjoint of Born modelling, and the split imaging of the migration: the
-// reconstruction with the source-side image terms (sum u, I2 += u*u) and the
-// receiver step with the rest (sum q, I1; compensated imaging only).
+// receiver step with the imaging of the last nimg steps, Born scattered field
+// (FP32 / FP64 combine), the adjoint of Born modelling, and the receiver step
+// without imaging.
 enum { EPI_FWD = 0, EPI_SRC = 1, EPI_RCV = 2, EPI_FWD64 = 3, EPI_BORN = 4, EPI_BORN64 = 5,
-       EPI_ADJ = 6, EPI_SRCI = 7, EPI_RCVI = 8, EPI_ADJT = 9 };
+       EPI_ADJ = 6, EPI_RCV0 = 7, EPI_ADJT = 8 };
 enum { FR_FWD = 0, FR_RCV = 1, FR_BORN = 2, FR_ADJ = 3 };
 
 struct IntArgs {
@@ -95,7 +94,8 @@ struct IntArgs {
   int nxt, zs;         // interior x tiles, rows per wave (requested)
   int nshot;           // shots of the launch (the fastest-varying block index)
   const float* data;   // [shot][nt][n] (receiver mode)
-  const float* uk;     // u(k) for imaging (receiver mode)
+  const float* uk;     // u(k) for imaging (receiver mode); u(k+1), u(k+2) in ua, ub
+  int nimg;            // steps k+nimg-1 .. k imaged by this launch (1..3)
   float *su, *sq, *i1, *i2;
   int icompen;
   // Born / adjoint: background fields ua, ub, uc with D2u = (ua - 2ub) + uc
@@ -155,7 +155,7 @@ int interior_queue_rows(int epi, int nfd);
 hipError_t launch_interior(int epi, int nfd_inst, IntArgs a, int nshot, hipStream_t s);
 // One launch of a time step's interior kernel (epi) and frame kernel (mode),
 // their blocks interleaved (k_step); only (EPI_FWD, FR_FWD) and
-// (EPI_RCVI, FR_RCV) are fused (step_fusable).
+// (EPI_RCV0 / EPI_RCV, FR_RCV) are fused (step_fusable).
 bool step_fusable(int epi, int mode);
 hipError_t launch_step(int epi, int mode, int nfd, IntArgs ia, FrameArgs fa, int nshot, int nrec,
                        hipStream_t s);

@@ -400,8 +400,8 @@ __global__ void k_stack_finish(int nI, const float* s1, const float* s2, int nre
 #define RTM_NFD_CASES(X) X(1) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12)
 
 int interior_queue_rows(int epi, int nfd) {
-  const bool pd1 = epi == EPI_RCV || epi == EPI_RCVI || epi == EPI_BORN || epi == EPI_BORN64 ||
-                   epi == EPI_ADJ || epi == EPI_ADJT;
+  const bool pd1 = epi == EPI_RCV || epi == EPI_BORN || epi == EPI_BORN64 || epi == EPI_ADJ ||
+                   epi == EPI_ADJT;
   return 2 * nfd + 1 + (pd1 ? 1 : 2);  // EpiTraits<EPI>::PD
 }
 
@@ -512,10 +512,10 @@ hipError_t launch_frame(int mode, int nfd, FrameArgs a, int nshot, int nrec, hip
 
 // The interior grid of launch_interior (rows per wave rounded to the queue
 // length) and one wave per frame record, in one k_step launch; only the
-// forward and the split receiver step are fused (the other kinds keep two
+// forward and the receiver step are fused (the other kinds keep two
 // launches).
 bool step_fusable(int epi, int mode) {
-  return (epi == EPI_FWD && mode == FR_FWD) || (epi == EPI_RCVI && mode == FR_RCV);
+  return (epi == EPI_FWD && mode == FR_FWD) || ((epi == EPI_RCV || epi == EPI_RCV0) && mode == FR_RCV);
 }
 
 hipError_t launch_step(int epi, int mode, int nfd, IntArgs ia, FrameArgs fa, int nshot, int nrec,

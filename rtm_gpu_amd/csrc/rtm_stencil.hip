@@ -38,25 +38,32 @@ namespace rtm {
 // Software pipeline per row: (a) the coefficient rows of the row are gathered
 // (their byte offsets were fetched PD rows earlier); (b) every stencil operand
 // of row z+PD is fetched (u1 row z+NFD+PD, the halo row, u0, the p and offset
-// rows), and for the receiver step the imaging operands of row z+1; (c) the
+// rows); (c) the
 // LDS exchange and the stencil read only data fetched in earlier iterations
 // or in (a).  The memory counter is in-order, so (a) goes first: the wait on
 // the gathers then leaves the prefetches in flight.  Scheduling barriers keep
 // that order.  A segment is a multiple of the queue length QL, so the row
 // loop is fully unrolled without a remainder; rows past the interior at the
 // end of the last segment are computed from clamped rows and not stored.
+//
+// Imaging.  The sums and images are 32 of the 60 bytes that a backward step
+// moved per cell when every step updated them.  The three rotating buffers of
+// each field still hold steps k+2, k+1 and k when the receiver step k runs, and
+// that step has q(k+2) and q(k+1) in registers as its own operands, so every
+// third receiver step (EPI_RCV, nimg = 3) applies the terms of three steps in
+// their order, bit for bit the same, and the two before it are plain updates
+// (EPI_RCV0): (36 + 24 + 56) / 3 = 38.7 bytes per cell and backward step.
 template <int EPI>
 struct EpiTraits {
   static constexpr bool f64 =
-      EPI == EPI_FWD64 || EPI == EPI_SRC || EPI == EPI_SRCI || EPI == EPI_BORN64;  // "2.0*"
-  static constexpr bool rcv = EPI == EPI_RCV || EPI == EPI_RCVI;  // receiver step + imaging
-  static constexpr bool rcvi = EPI == EPI_RCVI;  // ... without the source-side terms
-  static constexpr bool srci = EPI == EPI_SRCI;  // reconstruction + source-side terms
+      EPI == EPI_FWD64 || EPI == EPI_SRC || EPI == EPI_BORN64;  // "2.0*"
+  static constexpr bool rcv = EPI == EPI_RCV || EPI == EPI_RCV0;  // receiver step
+  static constexpr bool img = EPI == EPI_RCV;  // ... with the imaging of up to three steps
   static constexpr bool born = EPI == EPI_BORN || EPI == EPI_BORN64;
   static constexpr bool adj = EPI == EPI_ADJ || EPI == EPI_ADJT;
   static constexpr bool adjt = EPI == EPI_ADJT;  // transposed stencil (per-cell rows)
   static constexpr bool src = !rcv && !born && !adj;  // injects the source wavelet
-  static constexpr int PD = (rcv || born || adj) ? 1 : 2;  // prefetch distance of the stencil operands
+  static constexpr int PD = (img || born || adj) ? 1 : 2;  // prefetch distance of the stencil operands
 };
 
 // Interior body for block bid (k_interior: bid = blockIdx.x; k_step gives
@@ -165,13 +172,15 @@ __device__ __forceinline__ void interior_body(const IntArgs& a, const unsigned b
       }
     }
   }
-  Rsrc RU, RI1, RI2, RSU, RSQ;
-  unsigned vcs = kDrop, vss = kDrop;
-  if (T::rcv || T::srci) {
-    RU = rsrc(a.uk + so, fb);
+  Rsrc RU, RU1, RU2, RI1, RI2, RSU, RSQ;
+  unsigned vcs = kDrop, vss = kDrop, vu1 = kDrop, vu2 = kDrop;
+  if (T::img) {
+    RU = rsrc(a.uk + so, fb); RU1 = rsrc(a.ua + so, fb); RU2 = rsrc(a.ub + so, fb);
     RI1 = rsrc(a.i1 + so, fb); RI2 = rsrc(a.i2 + so, fb);
     RSU = rsrc(a.su + so, fb); RSQ = rsrc(a.sq + so, fb);
     if (a.icompen) { vcs = vcol; vss = vst; }
+    if (a.nimg >= 2) vu1 = vcol;
+    if (a.nimg >= 3) vu2 = vcol;
   }
   // Born / adjoint operands of the centre row: the background fields and the
   // reflectivity (Born) or the gradient accumulator (adjoint, when imaging)
@@ -195,7 +204,7 @@ __device__ __forceinline__ void interior_body(const IntArgs& a, const unsigned b
     u0b[d] = bld4s(R0, vcol, rowb(zs + d));
     hvb[d] = bld4(R1, vhal, rowb(zs + d));
   }
-  float4 ukb[1] = {}, i1b[1] = {}, i2b[1] = {}, sub[1] = {}, sqb[1] = {};
+  float4 ukb = {}, uk1b = {}, uk2b = {}, i1b = {}, i2b = {}, sub = {}, sqb = {};
   float4 xab[2], xbb[2], xcb[2], xxb[2];
   if (T::born || T::adj) {
     xab[0] = bld4(RA, vxl, rowb(zs));
@@ -226,21 +235,18 @@ __device__ __forceinline__ void interior_body(const IntArgs& a, const unsigned b
         cr[3].load(RC, kb[0].w);
       }
       __builtin_amdgcn_sched_barrier(0);
-      // Receiver step: this row's imaging operands, issued ahead of the
-      // prefetches so that their wait leaves the prefetches in flight (a
-      // row of look-ahead for them would cost 20 VGPRs the kernel needs).
-      if (T::rcv) {
+      // Imaging receiver step: this row's imaging operands, issued ahead of
+      // the prefetches so that their wait leaves the prefetches in flight (a
+      // row of look-ahead for them would cost VGPRs the kernel needs).
+      if (T::img) {
         const unsigned rzz = rowb(zz);
-        if (!T::rcvi) ukb[0] = bld4(RU, vcol, rzz);  // the split step never needs u(k)
-        i1b[0] = bld4s(RI1, vcol, rzz);
-        if (!T::rcvi) i2b[0] = bld4s(RI2, vcol, rzz);
-        sub[0] = bld4s(RSU, vcs, rzz);
-        sqb[0] = bld4s(RSQ, vcs, rzz);
-      }
-      if (T::srci) {  // this row's sum u and I2, for the source-side image terms
-        const unsigned rzz = rowb(zz);
-        i2b[0] = bld4s(RI2, vcol, rzz);
-        sub[0] = bld4s(RSU, vcs, rzz);
+        ukb = bld4(RU, vcol, rzz);
+        uk1b = bld4(RU1, vu1, rzz);
+        uk2b = bld4s(RU2, vu2, rzz);
+        i1b = bld4s(RI1, vcol, rzz);
+        i2b = bld4s(RI2, vcol, rzz);
+        sub = bld4s(RSU, vcs, rzz);
+        sqb = bld4s(RSQ, vcs, rzz);
       }
       // (b) operands of later rows
       q[(j + 2 * NFD + PD) % QL] = bld4(R1, vcol, rowb(zz + NFD + PD));
@@ -313,39 +319,27 @@ __device__ __forceinline__ void interior_body(const IntArgs& a, const unsigned b
         for (int jj = 0; jj < 3; ++jj)
           bst1s_(R2, ((part && colok[jj]) ? vst + 4u * jj : kDrop) | rowdrop, rz, out[jj]);
       }
-      if (T::rcv) {  // imaging (kernel.cu:489-517); frame columns keep their values
-        const float4 ukv = ukb[0], i1 = i1b[0], i2 = i2b[0], su = sub[0], sq = sqb[0];
+      if (T::img) {  // imaging (kernel.cu:489-517) of steps k+nimg-1 .. k, in that order
         float r1o[4], r2o[4], rsu[4], rsq[4];
 #pragma unroll
         for (int jj = 0; jj < 4; ++jj) {
-          const float u = T::rcvi ? 0.0f : compr(ukv, jj);
-          // split form (compensated imaging only): sum u already holds this
-          // step's u(k), which the reconstruction added
-          rsu[jj] = T::rcvi ? compr(su, jj) : (a.icompen ? compr(su, jj) + u : u);
-          rsq[jj] = a.icompen ? compr(sq, jj) + out[jj] : out[jj];
-          r1o[jj] = colok[jj] ? __builtin_fmaf(rsq[jj], rsu[jj], compr(i1, jj)) : compr(i1, jj);
-          if (!T::rcvi) r2o[jj] = colok[jj] ? __builtin_fmaf(u, u, compr(i2, jj)) : compr(i2, jj);
-          rsu[jj] = colok[jj] ? rsu[jj] : compr(su, jj);
-          rsq[jj] = colok[jj] ? rsq[jj] : compr(sq, jj);
+          float x1 = compr(i1b, jj), x2 = compr(i2b, jj), su = compr(sub, jj), sq = compr(sqb, jj);
+          auto image = [&](float u, float q, bool on) {  // frame columns keep their values
+            const float a1 = a.icompen ? su + u : u, b1 = a.icompen ? sq + q : q;
+            x1 = on ? __builtin_fmaf(b1, a1, x1) : x1;
+            x2 = on ? __builtin_fmaf(u, u, x2) : x2;
+            su = on ? a1 : su;
+            sq = on ? b1 : sq;
+          };
+          image(compr(uk2b, jj), compr(u0v, jj), colok[jj] && a.nimg >= 3);
+          image(compr(uk1b, jj), compr(qc, jj), colok[jj] && a.nimg >= 2);
+          image(compr(ukb, jj), out[jj], colok[jj]);
+          r1o[jj] = x1; r2o[jj] = x2; rsu[jj] = su; rsq[jj] = sq;
         }
         bst4s(RI1, vst | rowdrop, rz, r1o[0], r1o[1], r1o[2], r1o[3]);
-        if (!T::rcvi) {
-          bst4s(RI2, vst | rowdrop, rz, r2o[0], r2o[1], r2o[2], r2o[3]);
-          bst4s(RSU, vss | rowdrop, rz, rsu[0], rsu[1], rsu[2], rsu[3]);
-        }
-        bst4s(RSQ, vss | rowdrop, rz, rsq[0], rsq[1], rsq[2], rsq[3]);
-      }
-      if (T::srci) {  // source-side image terms of step k on the u(k) just computed
-        const float4 i2 = i2b[0], su = sub[0];
-        float r2o[4], rsu[4];
-#pragma unroll
-        for (int jj = 0; jj < 4; ++jj) {
-          const float u = out[jj];
-          rsu[jj] = colok[jj] ? compr(su, jj) + u : compr(su, jj);
-          r2o[jj] = colok[jj] ? __builtin_fmaf(u, u, compr(i2, jj)) : compr(i2, jj);
-        }
         bst4s(RI2, vst | rowdrop, rz, r2o[0], r2o[1], r2o[2], r2o[3]);
         bst4s(RSU, vss | rowdrop, rz, rsu[0], rsu[1], rsu[2], rsu[3]);
+        bst4s(RSQ, vss | rowdrop, rz, rsq[0], rsq[1], rsq[2], rsq[3]);
       }
       if (T::adj) {  // G += D2u(k+1) * mu(k+2); mu(k+2) is this update's u0
         float go[4];
@@ -1048,8 +1042,7 @@ hipError_t StencilOps<RTM_NFD>::interior(int epi, dim3 grid, const IntArgs& a, h
   else if (epi == EPI_BORN64) hipLaunchKernelGGL((k_interior<N, EPI_BORN64>), grid, block, 0, s, a);
   else if (epi == EPI_ADJ) hipLaunchKernelGGL((k_interior<N, EPI_ADJ>), grid, block, 0, s, a);
   else if (epi == EPI_ADJT) hipLaunchKernelGGL((k_interior<N, EPI_ADJT>), grid, block, 0, s, a);
-  else if (epi == EPI_SRCI) hipLaunchKernelGGL((k_interior<N, EPI_SRCI>), grid, block, 0, s, a);
-  else if (epi == EPI_RCVI) hipLaunchKernelGGL((k_interior<N, EPI_RCVI>), grid, block, 0, s, a);
+  else if (epi == EPI_RCV0) hipLaunchKernelGGL((k_interior<N, EPI_RCV0>), grid, block, 0, s, a);
   else hipLaunchKernelGGL((k_interior<N, EPI_RCV>), grid, block, 0, s, a);
   return hipGetLastError();
 }
@@ -1086,8 +1079,10 @@ hipError_t StencilOps<RTM_NFD>::step(int epi, dim3 grid, const IntArgs& ia, cons
   const dim3 block(256);
   if (epi == EPI_FWD)
     hipLaunchKernelGGL((k_step<N, EPI_FWD, FR_FWD>), grid, block, 0, s, ia, fa, nint, nfr);
+  else if (epi == EPI_RCV0)
+    hipLaunchKernelGGL((k_step<N, EPI_RCV0, FR_RCV>), grid, block, 0, s, ia, fa, nint, nfr);
   else
-    hipLaunchKernelGGL((k_step<N, EPI_RCVI, FR_RCV>), grid, block, 0, s, ia, fa, nint, nfr);
+    hipLaunchKernelGGL((k_step<N, EPI_RCV, FR_RCV>), grid, block, 0, s, ia, fa, nint, nfr);
   return hipGetLastError();
 }
 

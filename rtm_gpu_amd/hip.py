@@ -20,10 +20,10 @@ DATA_GATHERS, DATA_RECORDS = 0, 1
 KERNEL_NAMES = {
     K_FWD_INTERIOR: "k_interior<EPI_FWD>", K_FWD_FRAME: "k_frame<FR_FWD>",
     K_SRC_INTERIOR: "k_interior<EPI_SRC>", K_STRIP_RESTORE: "k_strip_restore",
-    K_RCV_INTERIOR: "k_interior<EPI_RCV>", K_RCV_FRAME: "k_frame<FR_RCV>",
+    K_RCV_INTERIOR: "k_interior<EPI_RCV0>", K_RCV_FRAME: "k_frame<FR_RCV>",
     K_BORN_INTERIOR: "k_interior<EPI_BORN>", K_BORN_FRAME: "k_frame<FR_BORN>",
     K_ADJ_INTERIOR: "k_interior<EPI_ADJ>", K_ADJ_FRAME: "k_frame<FR_ADJ>",
-    K_SRCI_INTERIOR: "k_interior<EPI_SRCI>", K_RCVI_INTERIOR: "k_interior<EPI_RCVI>",
+    K_SRCI_INTERIOR: "k_interior<EPI_SRCI>", K_RCVI_INTERIOR: "k_interior<EPI_RCV>",
 }
 
 
