@@ -51,7 +51,9 @@ enum {
    * RTM_FIELD_Q holds mu = P*lambda and RTM_FIELD_I1 the accumulator G. */
 };
 
-/* Kernel kinds for rtm_kernel_time().  A frame kind times the frame launches
+/* Kernel kinds for rtm_kernel_time().  Small batches run a whole step in one
+ * launch, which counts under the interior kind of its pass (the receiver kinds
+ * for a backward step).  Otherwise a frame kind times the frame launches
  * of one step together; on migration and adjoint steps without a checkpoint
  * snapshot (and with separate launches) RTM_K_RCV_FRAME / RTM_K_ADJ_FRAME
  * include the strip restore of the reconstructed field, which
@@ -78,7 +80,8 @@ typedef struct rtm_params {
   int max_shots;         /* shots per batch this context can hold */
   int strip_format;      /* RTM_STRIP_F32 (reference), RTM_STRIP_F16, RTM_STRIP_BF16 */
   int record;            /* 1: allocate receiver records for forward modelling */
-  int zseg;              /* rows per wave in the interior kernels (0 = auto) */
+  int zseg;              /* rows per wave in the marching interior kernels (0 = auto, and
+                            small batches run whole steps in one launch instead) */
   int snap_every;        /* checkpoint snapshots (not in the reference; 0 = none): the
                             forward pass keeps the whole field u(j) and u(j+1) for
                             j = m*snap_every, 2 <= j, j+1 <= nt-3, in strip_format with a
@@ -278,8 +281,8 @@ int rtm_data_dot_noalloc(const float* x, const float* y, long long n, long long 
  * that kernel inside forward + backward step pairs of the current batch (the
  * other kernels interleaved, the buffers rotating as in a migration) for row
  * segments of 1, 2, 3, 4, 6 and 9 times its register-queue length, in three
- * interleaved rounds of max(2, nsteps/2) timed pairs per candidate, one
- * kernel at a time, and keeps the fastest per kernel for this context (Born
+ * interleaved rounds of max(3, nsteps/2) timed pairs per candidate, all
+ * kernels in the same pairs, each timed by itself, and keeps the fastest per kernel for this context (Born
  * modelling and the adjoint take the receiver step's); zseg[3], when not
  * NULL, receives the three choices in rows.  Needs
  * model, wavelet and shots; leaves the passes to be begun anew and resets the
@@ -287,7 +290,8 @@ int rtm_data_dot_noalloc(const float* x, const float* y, long long n, long long 
  * (2*NFD rows per segment) against the number of waves in flight.  Then the
  * frame kernels' row runs (rtm_set_frame_runs) are timed the same way, top and
  * bottom bands first, on the sum of both frame kernels' times, and last the
- * frame split (rtm_params.frame_split) on and off. */
+ * frame split (rtm_params.frame_split) on and off, and the tuned kernels
+ * against whole steps in one launch. */
 int rtm_autotune(rtm_ctx* ctx, int nsteps, int* zseg);
 /* The autotuner's three choices set by hand: rows per wave of the forward,
  * the source-reconstruction and the receiver-step kernels (Born and the

@@ -98,6 +98,9 @@ struct rtm_ctx {
   bool capturing = false;       // inside rtm_migrate's graph capture
   bool model_ok = false, wav_ok = false, shots_ok = false, data_ok = false, save_strips = true;
   int zs = 32, nxt = 1;
+  long long cells = 0;     // grid cells of the batch
+  bool march_set = false;  // the caller chose something of the marching kernels
+  int tile_tuned = -1;     // rtm_autotune's choice for the batch: 1 k_tile, 0 the marching kernels
   int zs_epi[16] = {0};  // rows per wave per interior kernel kind (0: zs)
   // captured migration (hipGraph)
   bool graph_on = false;
@@ -286,6 +289,50 @@ int watch_read(rtm_ctx* c, const char* pass) {
   return RTM_OK;
 }
 
+// Whole steps by k_tile instead of the marching kernels.
+//
+// A marching wave spends 0.5 to 1 us on each of its 20 to 30 rows whatever the
+// batch, so a small batch costs the same as one that fills the GPU; k_tile is
+// two memory accesses deep, but it is bound by instruction issue where the
+// marching kernels run at the memory's rate.  Its work per cell grows with the
+// half-length, so the line is drawn on cells times half-length.  Measured
+// (k_tile against marching, forward + backward, ms per 100 steps): half-length
+// 3, 1.4 M cells 3.6 / 10.6, 12 M 19 / 22, 23 M 40 / 35; half-length 10, 0.6 M
+// cells 3.1 / 14.1, 2.5 M 8.9 / 14.9, 5 M 15.8 / 15.6, 10 M 31 / 22.  A Born
+// or adjoint step takes both fields through one launch and shares the
+// coefficient rows: at half-length 4, 11 M cells 29 / 34, 22 M 143 / 164 (250
+// steps), so the line is twice as high there.
+//
+// A caller who sets anything that belongs to the marching kernels (zseg,
+// frame runs, fuse_frame, frame_split) gets them, unless rtm_autotune has timed
+// the two for the batch's migration.
+constexpr long long kTileWork = 50000000;
+bool use_tile(const rtm_ctx* c, int pass) {
+  if (c->march_set) return false;
+  const bool two = pass == TILE_BORN || pass == TILE_ADJ;
+  if (!two && c->tile_tuned >= 0) return c->tile_tuned != 0;
+  return c->cells * c->nfd <= (two ? 2 : 1) * kTileWork;
+}
+hipError_t tile_step(rtm_ctx* c, int pass, const TileArgs& a) {
+  return launch_tile(pass, c->nfd, a, c->nshot, c->cells, c->stream);
+}
+
+void fill_tile_args(rtm_ctx* c, TileArgs& a, float wav, int k) {
+  a = TileArgs{};
+  a.g = c->g;
+  a.m = c->m;
+  a.r = c->r;
+  a.geo = c->d_geo;
+  a.u1 = c->F[c->f1]; a.u0 = c->F[c->f0]; a.u2 = c->F[c->f2];
+  a.q1 = c->Q[c->q1]; a.q0 = c->Q[c->q0]; a.q2 = c->Q[c->q2];
+  a.wav = wav; a.k = k; a.nt = c->p.nt;
+  a.f64comb = c->p.ilste != 0;
+  a.data = c->d_data;
+  a.st = c->st;
+  a.su = c->SU; a.sq = c->SQ; a.i1 = c->I1; a.i2 = c->I2;
+  a.icompen = c->p.icompen;
+}
+
 // Interior and frame of a step in one launch (k_step) when the context asks
 // for it and the pair is one of the fused kinds.
 static bool fused(const rtm_ctx* c, int epi, int mode) {
@@ -309,11 +356,21 @@ hipError_t launch_frame_split(rtm_ctx* c, int mode, FrameArgs f) {
   return launch_frame(mode, c->nfd, f, c->nshot, c->ntiles, c->stream);
 }
 
-int forward_step(rtm_ctx* c, int k) {
+// born: the caller runs a Born pass (born_step), whose scattered field a tile
+// launch advances together with the background.
+int forward_step(rtm_ctx* c, int k, bool born = false) {
   const float wv = (k < c->p.nt2) ? c->wav[k - 1] : 0.0f;  // kernel.cu:812-813
   const bool quant = c->save_strips && c->st.fmt != RTM_STRIP_F32;
   if (quant && k >= 3) HIPCHK(c, launch_strip_finish(c->g, c->st, c->d_geo, k - 1, c->nshot, c->stream));
-  {
+  const bool tile = use_tile(c, born ? TILE_BORN : TILE_FWD);
+  if (tile) {
+    TileArgs a;
+    fill_tile_args(c, a, wv, k);
+    a.save_strips = c->save_strips ? 1 : 0;
+    a.rec = (c->p.record && (born || !c->born)) ? c->d_rec : nullptr;
+    Timed t(c, born ? RTM_K_BORN_INTERIOR : RTM_K_FWD_INTERIOR);  // the whole step
+    HIPCHK(c, tile_step(c, born ? TILE_BORN : TILE_FWD, a));
+  } else {
     // Add (FP32 combine) or Add_Con (FP64 combine) (kernel.cu:46-114) on the
     // interior, Add + Hybrid1/2/3 on the frame (kernel.cu:116-208)
     const int epi = c->p.ilste ? EPI_FWD64 : EPI_FWD;
@@ -342,13 +399,26 @@ int forward_step(rtm_ctx* c, int k) {
   if (quant && k == c->p.nt - 1) HIPCHK(c, launch_strip_finish(c->g, c->st, c->d_geo, k, c->nshot, c->stream));
   if (c->save_strips && c->snap_slot[k] >= 0)  // checkpoint snapshot of u(k)
     HIPCHK(c, launch_snap_save(c->g, c->F[c->f2], c->sn, c->d_geo, c->snap_slot[k], c->nshot, c->stream));
-  if (c->p.record && !c->born)  // receiver recording of u(k)
+  if (c->p.record && !c->born && !tile)  // receiver recording of u(k)
     HIPCHK(c, launch_record(c->g, c->r, c->d_geo, c->F[c->f2], c->d_rec, k, c->p.nt, c->nshot, c->stream));
   if (watch_due(c, k, c->p.nt - 1)) {
     int rc = watch(c, c->F[c->f2], k);
     if (rc != RTM_OK) return rc;
   }
   int t = c->f0; c->f0 = c->f1; c->f1 = c->f2; c->f2 = t;  // Deliver (kernel.cu:820)
+  return RTM_OK;
+}
+
+// The end of backward step k: the finite-value watch and the rotation of the
+// receiver field.
+int backward_done(rtm_ctx* c, int k, bool image) {
+  c->img_pend = image ? 0 : c->img_pend + 1;
+  if (watch_due(c, k, 0)) {  // the reconstructed u(k) and the new receiver field
+    int rc = watch(c, c->F[c->f1], k);
+    if (rc == RTM_OK) rc = watch(c, c->Q[c->q2], k);
+    if (rc != RTM_OK) return rc;
+  }
+  { int t = c->q0; c->q0 = c->q1; c->q1 = c->q2; c->q2 = t; }  // Deliver (kernel.cu:921)
   return RTM_OK;
 }
 
@@ -362,6 +432,15 @@ int backward_step(rtm_ctx* c, int k, bool flush) {
   const float wv = (k < c->p.nt2) ? c->wav[k + 1] : 0.0f;  // kernel.cu:889-890
   const bool image = flush || c->img_pend == 2;
   const int ercv = image ? EPI_RCV : EPI_RCV0;
+  if (use_tile(c, TILE_MIG) && c->snap_slot[k] < 0) {
+    TileArgs a;
+    fill_tile_args(c, a, wv, k);
+    a.nimg = image ? c->img_pend + 1 : 0;
+    Timed t(c, image ? RTM_K_RCVI_INTERIOR : RTM_K_RCV_INTERIOR);  // the whole step
+    HIPCHK(c, tile_step(c, TILE_MIG, a));
+    { int r = c->f0; c->f0 = c->f1; c->f1 = c->f2; c->f2 = r; }
+    return backward_done(c, k, image);
+  }
   {  // BKAdd_EFF (kernel.cu:896): u(k) on the interior
     IntArgs a;
     fill_int_args(c, a);
@@ -413,23 +492,17 @@ int backward_step(rtm_ctx* c, int k, bool flush) {
       HIPCHK(c, launch_frame_split(c, FR_RCV, f));
     }
   }
-  c->img_pend = image ? 0 : c->img_pend + 1;
-  if (watch_due(c, k, 0)) {  // the reconstructed u(k) and the new receiver field
-    int rc = watch(c, c->F[c->f1], k);
-    if (rc == RTM_OK) rc = watch(c, c->Q[c->q2], k);
-    if (rc != RTM_OK) return rc;
-  }
-  { int t = c->q0; c->q0 = c->q1; c->q1 = c->q2; c->q2 = t; }  // Deliver (kernel.cu:921)
-  return RTM_OK;
+  return backward_done(c, k, image);
 }
 
 // Born step k: the background step, then the scattered field from dU(k-1),
 // dU(k-2) and D2u = (u(k) - 2u(k-1)) + u(k-2) (the background rotation
 // leaves u(k), u(k-1), u(k-2) in f1, f0, f2), recorded at the receivers.
 int born_step(rtm_ctx* c, int k) {
-  int rc = forward_step(c, k);
+  const bool tile = use_tile(c, TILE_BORN);
+  int rc = forward_step(c, k, true);
   if (rc != RTM_OK) return rc;
-  {
+  if (!tile) {
     IntArgs a;
     fill_int_args(c, a);
     a.u1 = c->Q[c->q1]; a.u0 = c->Q[c->q0]; a.u2 = c->Q[c->q2];
@@ -439,7 +512,7 @@ int born_step(rtm_ctx* c, int k) {
     a.zs = zs_for(c, c->p.ilste ? EPI_BORN64 : EPI_BORN);
     HIPCHK(c, launch_interior(c->p.ilste ? EPI_BORN64 : EPI_BORN, c->nfd, a, c->nshot, c->stream));
   }
-  {
+  if (!tile) {
     FrameArgs a;
     fill_frame_args(c, a);
     a.u1 = c->Q[c->q1]; a.u0 = c->Q[c->q0]; a.u2 = c->Q[c->q2];
@@ -448,9 +521,18 @@ int born_step(rtm_ctx* c, int k) {
     Timed t(c, RTM_K_BORN_FRAME);
     HIPCHK(c, launch_frame(FR_BORN, c->nfd, a, c->nshot, c->ntiles, c->stream));
   }
-  HIPCHK(c, launch_record(c->g, c->r, c->d_geo, c->Q[c->q2], c->d_rec, k, c->p.nt, c->nshot, c->stream));
+  if (!tile) HIPCHK(c, launch_record(c->g, c->r, c->d_geo, c->Q[c->q2], c->d_rec, k, c->p.nt, c->nshot, c->stream));
   if (watch_due(c, k, c->p.nt - 1)) {
     rc = watch(c, c->Q[c->q2], k);
+    if (rc != RTM_OK) return rc;
+  }
+  int t = c->q0; c->q0 = c->q1; c->q1 = c->q2; c->q2 = t;
+  return RTM_OK;
+}
+
+int adjoint_done(rtm_ctx* c, int k, bool image) {
+  if (image && watch_due(c, k, 0)) {
+    int rc = watch(c, c->Q[c->q2], k);
     if (rc != RTM_OK) return rc;
   }
   int t = c->q0; c->q0 = c->q1; c->q1 = c->q2; c->q2 = t;
@@ -490,18 +572,24 @@ int adjoint_update(rtm_ctx* c, int k, bool image, float* restore = nullptr) {
     Timed t(c, RTM_K_ADJ_FRAME);
     HIPCHK(c, launch_frame(FR_ADJ, c->nfd, a, c->nshot, c->ntiles, c->stream));
   }
-  if (image && watch_due(c, k, 0)) {
-    int rc = watch(c, c->Q[c->q2], k);
-    if (rc != RTM_OK) return rc;
-  }
-  int t = c->q0; c->q0 = c->q1; c->q1 = c->q2; c->q2 = t;
-  return RTM_OK;
+  return adjoint_done(c, k, image);
 }
 
 // Adjoint step k: the background u(k) reconstructed as in backward_step,
 // then the adjoint update with imaging.
 int adjoint_step(rtm_ctx* c, int k) {
   const float wv = (k < c->p.nt2) ? c->wav[k + 1] : 0.0f;
+  if (use_tile(c, TILE_ADJ) && c->snap_slot[k] < 0) {
+    TileArgs a;
+    fill_tile_args(c, a, wv, k);
+    a.adjt = c->p.ilste == 0;
+    {
+      Timed t(c, RTM_K_ADJ_INTERIOR);  // the whole step
+      HIPCHK(c, tile_step(c, TILE_ADJ, a));
+    }
+    { int t = c->f0; c->f0 = c->f1; c->f1 = c->f2; c->f2 = t; }
+    return adjoint_done(c, k, true);
+  }
   {
     IntArgs a;
     fill_int_args(c, a);
@@ -578,6 +666,9 @@ int upload_geometry(rtm_ctx* c) {
   HIPCHK(c, hipMemcpyAsync(c->d_geo, c->geo.data(), ns * sizeof(ShotGeo), hipMemcpyHostToDevice, c->stream));
   int rc = upload_frame_records(c);
   if (rc != RTM_OK) return rc;
+  if (ns != c->nshot) c->tile_tuned = -1;  // tuned for another batch
+  c->cells = 0;
+  for (const ShotGeo& q : c->geo) c->cells += (long long)c->g.nz * q.nx;
   c->nshot = ns;
   choose_zs(c, ns);
   drop_graph(c);
@@ -670,6 +761,7 @@ int rtm_create(const rtm_params* p, rtm_ctx** out) {
   else if (p->snap_every < 0) rc = fail(c, RTM_E_ARG, "snap_every=%d < 0", p->snap_every);
   else if (p->stack_nx < 0) rc = fail(c, RTM_E_ARG, "stack_nx=%d < 0", p->stack_nx);
   c->check_every = p->check_every == 0 ? 100 : p->check_every;
+  c->march_set = p->zseg > 0 || p->fuse_frame || p->frame_split;
   if (rc != RTM_OK) {
     int code = rc;
     delete c;
@@ -1460,6 +1552,7 @@ int rtm_set_zseg(rtm_ctx* c, const int* zseg) {
   c->zs_epi[EPI_RCV] = c->zs_epi[EPI_RCV0] = zseg[2];
   c->zs_epi[EPI_BORN] = c->zs_epi[EPI_BORN64] = c->zs_epi[EPI_ADJ] = zseg[2];
   c->zs = zseg[0];
+  c->march_set = true;
   drop_graph(c);
   return RTM_OK;
 }
@@ -1473,6 +1566,7 @@ int rtm_set_frame_runs(rtm_ctx* c, int rows_tb, int rows_side) {
                 min_tb, g.n2, min_side, g.nz);
   c->fseg_tb = rows_tb;
   c->fseg_side = rows_side;
+  c->march_set = true;
   return c->geo.empty() ? RTM_OK : upload_frame_records(c);
 }
 
@@ -1501,6 +1595,8 @@ int rtm_autotune(rtm_ctx* c, int nsteps, int* zseg) {
   // rtm_kernel_time are reset.
   const int saved_timing = c->timing, saved_check = c->check_every;
   c->check_every = -1;
+  c->tile_tuned = 0;
+  c->march_set = c->p.fuse_frame != 0;
   int rc = rtm_forward_begin(c, 1);
   if (rc == RTM_OK && !c->data_ok)
     rc = launch_fill(c->d_data, (long long)c->nshot * c->p.nt * c->p.n, 0.f, c->stream) == hipSuccess
@@ -1545,22 +1641,29 @@ int rtm_autotune(rtm_ctx* c, int nsteps, int* zseg) {
       if (mask & (1u << k)) *ms += c->t_n[k] ? c->t_ms[k] / c->t_n[k] : 1e300;
     return RTM_OK;
   };
-  for (int ki = 0; ki < kKinds && rc == RTM_OK; ++ki) {
-    const int epi = kinds[ki];
-    const int ql = interior_queue_rows(epi, c->nfd);
-    double tot[kNC] = {0.0};
+  // The interior kinds take their candidates in the same measurements (each is
+  // timed by itself): a sweep of each kind in turn took four times as long and
+  // chose the same heights.
+  {
+    double tot[kKinds][kNC] = {};
+    unsigned mask = 0;
+    for (int ki = 0; ki < kKinds; ++ki) mask |= 1u << timers[ki];
     for (int round = 0; round < kRounds && rc == RTM_OK; ++round)
       for (int i = 0; i < kNC && rc == RTM_OK; ++i) {
         const int ci = (round & 1) ? kNC - 1 - i : i;
-        c->zs_epi[epi] = kMult[ci] * ql;
+        for (int ki = 0; ki < kKinds; ++ki)
+          c->zs_epi[kinds[ki]] = kMult[ci] * interior_queue_rows(kinds[ki], c->nfd);
         double ms = 0.0;
-        rc = measure(1u << timers[ki], &ms);
-        tot[ci] += ms;
+        rc = measure(mask, &ms);
+        for (int ki = 0; ki < kKinds; ++ki)
+          tot[ki][ci] += c->t_n[timers[ki]] ? c->t_ms[timers[ki]] / c->t_n[timers[ki]] : 0.0;
       }
-    int bi = 0;
-    for (int i = 1; i < kNC; ++i)
-      if (tot[i] < tot[bi]) bi = i;
-    c->zs_epi[epi] = kMult[bi] * ql;
+    for (int ki = 0; ki < kKinds; ++ki) {
+      int bi = 0;
+      for (int i = 1; i < kNC; ++i)
+        if (tot[ki][i] < tot[ki][bi]) bi = i;
+      c->zs_epi[kinds[ki]] = kMult[bi] * interior_queue_rows(kinds[ki], c->nfd);
+    }
   }
   // Frame record runs, timed on both frame kernels of the step pair: the top
   // and bottom bands in runs of n2, n2/2 or n2/3 rows (with float4 records:
@@ -1609,6 +1712,26 @@ int rtm_autotune(rtm_ctx* c, int nsteps, int* zseg) {
         }
       c->p.frame_split = tot[1] < tot[0] ? 1 : 0;
     }
+  }
+  // The tuned marching kernels against whole steps by k_tile, on the time of
+  // everything a step pair launches over whole imaging cycles.
+  // Batches far from the line between them (use_tile) are not timed.
+  const long long work = c->cells * c->nfd;
+  if (rc == RTM_OK && !c->p.fuse_frame && work <= 4 * kTileWork) {
+    double tot[2] = {0.0, 0.0};
+    for (int round = 0; round < kRounds && rc == RTM_OK; ++round)
+      for (int i = 0; i < 2 && rc == RTM_OK; ++i) {
+        const int on = (round & 1) ? 1 - i : i;
+        c->tile_tuned = on;
+        c->timing = 0;
+        rc = pairs(3);
+        c->timing = -1;
+        for (int k = 0; k < RTM_K_NKINDS; ++k) { c->t_ms[k] = 0.0; c->t_n[k] = 0; }
+        if (rc == RTM_OK) rc = pairs(3 * ((per + 2) / 3));
+        if (rc == RTM_OK) rc = drain_timing(c);
+        for (int k = 0; k < RTM_K_NKINDS; ++k) tot[on] += c->t_ms[k];
+      }
+    c->tile_tuned = tot[1] < tot[0] ? 1 : 0;
   }
   c->timing = saved_timing;
   c->check_every = saved_check;

@@ -136,6 +136,44 @@ struct FrameArgs {
   int rbps;
 };
 
+// A whole time step in one launch, one cell per thread (rtm_tile.hip).
+enum { TILE_FWD = 0, TILE_MIG = 1, TILE_BORN = 2, TILE_ADJ = 3 };
+#define TILE_CPT2_MAX_NFD 4  // tiles of two cells per thread exist up to this half-length
+constexpr int TILE_ROWS = 8;  // a tile is 64 columns by TILE_ROWS * (cells per thread) rows
+
+struct TileArgs {
+  Grid g;
+  Model m;
+  Rcv r;
+  const ShotGeo* geo;
+  // u: the forward field, or the source field stepped backwards; q: the
+  // scattered, receiver or adjoint field.  Newer, older and written step.
+  const float *u1, *u0;
+  float* u2;
+  const float *q1, *q0;
+  float* q2;
+  float wav;           // source amplitude of u this step
+  int k, nt;
+  int f64comb;         // forward and Born updates: FP64 combine (Add_Con)
+  const float* data;   // [shot][nt][n]: gathers, residuals
+  float* rec;          // receiver records of this step, or null
+  Strips st;
+  int save_strips;
+  float *su, *sq, *i1, *i2;
+  int icompen;
+  int nimg;            // TILE_MIG: steps k+nimg-1 .. k imaged by this launch (0..3)
+  int adjt;            // TILE_ADJ: per-cell rows, the transposed stencil on the interior
+};
+
+// Tile kernels of one compile-time half-length, as StencilOps.
+template <int NFD>
+struct TileOps {
+  static hipError_t tile(int pass, int cpt, dim3 grid, const TileArgs& a, hipStream_t s);
+};
+// cells: grid cells of the launch (all shots), for the tile height.
+hipError_t launch_tile(int pass, int nfd_inst, const TileArgs& a, int nshot, long long cells,
+                       hipStream_t s);
+
 // Stencil kernels of one compile-time half-length: rtm_stencil.hip is compiled
 // once per NFD and defines these members for it.
 template <int NFD>

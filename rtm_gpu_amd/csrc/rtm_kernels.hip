@@ -542,6 +542,25 @@ hipError_t launch_step(int epi, int mode, int nfd, IntArgs ia, FrameArgs fa, int
 #undef CASE
 }
 
+hipError_t launch_tile(int pass, int nfd, const TileArgs& a, int nshot, long long cells,
+                       hipStream_t s) {
+  // Two cells per thread halve a tile's scalar work and share its column reads,
+  // one gives twice the blocks and fewer registers.  Measured (two against
+  // one): Born + adjoint at half-length 4, 22 M cells 143 / 157 ms, 1.4 M cells
+  // 34.9 / 32.2; migration at half-length 2, 32 M cells 159 / 171, at 3 and
+  // 23 M cells 40.5 / 40.0; at half-length 10 always slower (18.4 / 15.8).
+  const long long from = (pass == TILE_BORN || pass == TILE_ADJ) ? 2500000 : 24000000;
+  const int cpt = nfd <= TILE_CPT2_MAX_NFD && cells >= from ? 2 : 1;
+  const int ntz = (a.g.nz + TILE_ROWS * cpt - 1) / (TILE_ROWS * cpt);
+  const dim3 grid((unsigned)nshot, (unsigned)((a.g.nx + 63) / 64), (unsigned)ntz);
+#define CASE(N) case N: return TileOps<N>::tile(pass, cpt, grid, a, s);
+  switch (nfd) {
+    RTM_NFD_CASES(CASE)
+    default: return hipErrorInvalidValue;
+  }
+#undef CASE
+}
+
 static inline unsigned blocks_for(long long n, int per = 256, unsigned cap = 4096) {
   long long b = (n + per - 1) / per;
   if (b < 1) b = 1;

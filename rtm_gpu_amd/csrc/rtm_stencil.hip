@@ -384,37 +384,6 @@ __device__ __forceinline__ void interior_body(const IntArgs& a, const unsigned b
 // row earlier), row operands arrive PD rows ahead and the one-way operands two
 // rows ahead, and each row waits only on loads issued a row or more before.
 // No block-level barrier: the four waves of a block are independent.
-__device__ __forceinline__ float bld1(Rsrc r, unsigned vo, unsigned so) {
-  return __uint_as_float((unsigned)__builtin_amdgcn_raw_buffer_load_b32(r, (int)vo, (int)so, 0));
-}
-__device__ __forceinline__ unsigned bld1u(Rsrc r, unsigned vo, unsigned so) {
-  return (unsigned)__builtin_amdgcn_raw_buffer_load_b32(r, (int)vo, (int)so, 0);
-}
-__device__ __forceinline__ void bst1(Rsrc r, unsigned vo, unsigned so, float v) {
-  __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), r, (int)(vo + so), 0, 0);
-}
-// streaming variants (u0 rows, u(k+1) and strip writes: touched once per step)
-__device__ __forceinline__ float bld1s(Rsrc r, unsigned vo, unsigned so) {
-  return __uint_as_float((unsigned)__builtin_amdgcn_raw_buffer_load_b32(r, (int)vo, (int)so,
-                                                                        RTM_STREAM_POLICY));
-}
-__device__ __forceinline__ void bst1s(Rsrc r, unsigned vo, unsigned so, float v) {
-  __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), r, (int)(vo + so), 0, RTM_STREAM_POLICY);
-}
-
-// Strip element of frame cell (z, x) of a shot nx wide, or -1 (strip_index
-// without branches, in 32 bits: a slot holds fewer than 2^31 elements).
-__device__ __forceinline__ int strip_elem(const Grid& g, int nx, int mnx, int z, int x) {
-  const int a = g.mnz * g.nfd, b = g.nfd * mnx, n2 = g.n2, nfd = g.nfd;
-  const bool zin = z >= n2 && z < g.nz - n2, xin = x >= n2 && x < nx - n2;
-  int e = -1;
-  e = (zin && x >= n2 - nfd && x < n2) ? (z - n2) * nfd + (n2 - 1 - x) : e;
-  e = (zin && x >= nx - n2 && x < nx - n2 + nfd) ? a + (z - n2) * nfd + (x - (nx - n2)) : e;
-  e = (xin && z >= n2 - nfd && z < n2) ? 2 * a + (n2 - 1 - z) * mnx + (x - n2) : e;
-  e = (xin && z >= g.nz - n2 && z < g.nz - n2 + nfd) ? 2 * a + b + (z - (g.nz - n2)) * mnx + (x - n2) : e;
-  return e;
-}
-
 template <int NFD, int MODE>
 __device__ __forceinline__ void frame_body(const FrameArgs& a, const unsigned bid) {
   constexpr int PD = 2;                   // rows of prefetch
