@@ -9,8 +9,8 @@
 //
 // Layouts.  Activations are NHWC in BF16 with the channel count padded to a
 // multiple of 8 (Cp), so the eight consecutive K values a lane feeds the
-// MFMA are one 16-byte load.  Convolution as an implicit GEMM: M = 16
-// consecutive pixels of one row, N = 16 output channels, K = 9 taps x Cp
+// MFMA are one 16-byte load.  Convolution as an implicit GEMM: M = 16 output
+// channels, N = 16 consecutive pixels of one row, K = 9 taps x Cp
 // input channels (k = tap*Cp + ci, padded to a multiple of 32).  The MFMA
 // lane layout: A[m][k] at lane m + 16*(k/8), element k%8; B[k][n] at lane
 // n + 16*(k/8), element k%8; D[m][n] at lane n + 16*(m/4), element m%4.
@@ -19,9 +19,9 @@
 //                the last layer y = z + x0 in FP32
 //   input grad   dz_prev = conv(dz, W flipped and transposed) * (a > 0)
 //   weight grad  dW[tap][co][ci] = sum_pix dz[pix][co] * a[pix + tap][ci]:
-//                M = co, N = ci, K = pixels, staged transposed through LDS;
+//                M = co, N = ci, K = pixels, transposed on the way out of LDS;
 //                each workgroup accumulates a range of rows and writes one
-//                partial, two reduction kernels add the partials in a fixed
+//                partial, a reduction kernel adds the partials in a fixed
 //                order (FP64), so the result does not depend on scheduling.
 // Channel counts above 16 run in blocks of 16 (two blocks of output channels
 // per convolution wave; four 16 x 16 blocks per weight-gradient workgroup).
@@ -43,13 +43,15 @@ namespace {
 typedef __bf16 b8 __attribute__((ext_vector_type(8)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+typedef short s4 __attribute__((ext_vector_type(4)));
 typedef unsigned short bf16;
 
 constexpr int MAXC = 32;                    // channels per layer (two blocks of 16)
 constexpr int MAXL = 16;                    // layers
 constexpr int WG_STRIDE = 9 * MAXC * MAXC + MAXC;  // weight-grad partials per workgroup
 constexpr int WG_GROUPS = 1024;             // most workgroups of one weight-gradient launch
-constexpr int WG_LEVEL1 = 32;               // groups of the first reduction level
+constexpr int WG_LEVEL1 = 32;               // groups of the reduction
 // Byte offsets into an activation (MAX_PIXELS x 32 channels x 2 bytes) stay
 // below 2^31, the range of a buffer load's offset.
 constexpr long long MAX_PIXELS = 1LL << 25;
@@ -85,12 +87,73 @@ struct ConvArgs {
   const bf16* mask;   // NHWC, cout_p channels (mode 2)
   int n, h, w, cin_p, kpad, cout_p, mode;
   int ncob;           // blocks of 16 output channels
+  int ch;             // k_conv_rows: output rows of a strip
   int dil;            // dilation: tap (ky, kx) reads (y + (ky-1)*dil, x + (kx-1)*dil)
 };
 
-// Weight-stationary convolution: a wave holds its B operands (all NK K-steps
-// of NCOB blocks of 16 output channels) in registers and walks 16-pixel row
-// tiles, so a tile costs NK 16-byte input loads per lane and NK * NCOB MFMAs.
+// The weights are the first MFMA operand and the pixels the second, so a lane
+// ends with four consecutive channels of one pixel: D[channel 4 kg + j][pixel
+// lane & 15], stored as 8 bytes (one channel a lane and 2-byte stores bound the
+// convolution before: 94 us a 32 x 32 layer at 256 x 64 x 64).
+template <int NCOB>
+struct ConvOut {
+  float bias[NCOB][4];
+  __device__ __forceinline__ void load(const ConvArgs& a, int kg) {
+#pragma unroll
+    for (int cb = 0; cb < NCOB; ++cb)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) bias[cb][j] = a.mode == 2 ? 0.0f : a.bias[cb * 16 + 4 * kg + j];
+  }
+  // What a tile's epilogue reads besides the accumulators, fetched a tile ahead:
+  // the activations that mask an input gradient, or the residual.
+  struct Extra {
+    u32x2 mk[NCOB];
+    float res;
+  };
+  // px: pixel of the row; p: its index in the batch
+  static __device__ __forceinline__ void fetch(const ConvArgs& a, int kg, bool ok, unsigned p,
+                                               Extra& e) {
+    if (a.mode == 2) {
+#pragma unroll
+      for (int cb = 0; cb < NCOB; ++cb) {
+        const int co = cb * 16 + 4 * kg;
+        if (ok && co < a.cout_p)
+          e.mk[cb] = *reinterpret_cast<const u32x2*>(a.mask + (size_t)p * a.cout_p + co);
+      }
+    } else if (a.mode == 1) {
+      if (ok && kg == 0) e.res = a.resid[p];
+    }
+  }
+  __device__ __forceinline__ void store(const ConvArgs& a, const f4* acc, int kg, int px, unsigned p,
+                                        const Extra& e) const {
+    if (px >= a.w) return;
+    if (a.mode == 1) {
+      if (kg == 0) a.out32[p] = (acc[0][0] + bias[0][0]) + e.res;
+      return;
+    }
+#pragma unroll
+    for (int cb = 0; cb < NCOB; ++cb) {
+      const int co = cb * 16 + 4 * kg;
+      if (co >= a.cout_p) continue;
+      bf16 v[4];
+      if (a.mode == 0) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = to_bf16(fmaxf(acc[cb][j] + bias[cb][j], 0.0f));
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          v[j] = to_bf16(from_bf16((bf16)(e.mk[cb][j >> 1] >> (16 * (j & 1)))) > 0.0f ? acc[cb][j]
+                                                                                     : 0.0f);
+      }
+      *reinterpret_cast<u32x2*>(a.out + (size_t)p * a.cout_p + co) =
+          u32x2{(unsigned)v[0] | ((unsigned)v[1] << 16), (unsigned)v[2] | ((unsigned)v[3] << 16)};
+    }
+  }
+};
+
+// Weight-stationary convolution of narrow inputs (8, 16 or 24 channels): a wave
+// holds its weights (all NK K-steps of NCOB blocks of 16 output channels) in
+// registers and walks 16-pixel row tiles, the next tile's inputs in flight.
 // K-step ks covers k = 32 ks .. 32 ks + 31; lane group kg feeds k = 32 ks +
 // 8 kg .. +7, eight consecutive channels of one tap (cin_p is a multiple of 8).
 template <int NK, int NCOB>
@@ -103,6 +166,8 @@ __global__ __launch_bounds__(256) void k_conv(const ConvArgs a) {
 #pragma unroll
     for (int ks = 0; ks < NK; ++ks)
       wv[cb][ks] = *reinterpret_cast<const b8*>(a.wt + (cb * 16 + m) * a.kpad + ks * 32 + 8 * kg);
+  ConvOut<NCOB> co;
+  co.load(a, kg);
   int tdy[NK], tdx[NK], tci[NK];
   bool tok[NK];
 #pragma unroll
@@ -117,21 +182,28 @@ __global__ __launch_bounds__(256) void k_conv(const ConvArgs a) {
   const Rsrc RI = rsrc(a.in, (unsigned)a.n * hw * (unsigned)a.cin_p * 2u);
   const unsigned segs = (unsigned)(a.w + 15) >> 4;
   const unsigned tiles = (unsigned)(a.n * a.h) * segs;
-  for (unsigned t = blockIdx.x * 4u + (threadIdx.x >> 6); t < tiles; t += gridDim.x * 4u) {
+  const unsigned step = gridDim.x * 4u;
+  auto fetch = [&](unsigned t, b8* av, typename ConvOut<NCOB>::Extra& e) {
     const unsigned row = t / segs, seg = t - row * segs;
-    const int y = (int)(row % (unsigned)a.h);
     const unsigned nn = row / (unsigned)a.h;
-    const int x = (int)seg * 16 + m;
-    b8 av[NK];
+    const int y = (int)(row - nn * (unsigned)a.h), x = (int)seg * 16 + m;
 #pragma unroll
     for (int ks = 0; ks < NK; ++ks) {
       const int yy = y + tdy[ks], xx = x + tdx[ks];
-      const bool ok = tok[ks] && x < a.w && yy >= 0 && yy < a.h && xx >= 0 && xx < a.w;
+      const bool ok = t < tiles && tok[ks] && yy >= 0 && yy < a.h && xx >= 0 && xx < a.w;
       const unsigned vo =
           ok ? ((nn * hw + (unsigned)(yy * a.w + xx)) * (unsigned)a.cin_p + (unsigned)tci[ks]) * 2u
              : kDrop;
       av[ks] = __builtin_bit_cast(b8, bld16(RI, vo));
     }
+    ConvOut<NCOB>::fetch(a, kg, t < tiles && x < a.w, row * (unsigned)a.w + (unsigned)x, e);
+  };
+  unsigned t = blockIdx.x * 4u + (threadIdx.x >> 6);
+  b8 av[NK], nx[NK];
+  typename ConvOut<NCOB>::Extra e{}, en{};
+  fetch(t, av, e);
+  for (; t < tiles; t += step) {
+    fetch(t + step, nx, en);
     f4 acc[NCOB];
 #pragma unroll
     for (int cb = 0; cb < NCOB; ++cb) acc[cb] = f4{0.f, 0.f, 0.f, 0.f};
@@ -139,26 +211,89 @@ __global__ __launch_bounds__(256) void k_conv(const ConvArgs a) {
     for (int ks = 0; ks < NK; ++ks)
 #pragma unroll
       for (int cb = 0; cb < NCOB; ++cb)
-        acc[cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[ks], wv[cb][ks], acc[cb], 0, 0, 0);
-    // D[pixel][channel]: lane & 15 = channel in the block, pixels 4 kg + j
+        acc[cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[cb][ks], av[ks], acc[cb], 0, 0, 0);
+    const unsigned row = t / segs;
+    const int px = (int)(t - row * segs) * 16 + m;
+    co.store(a, acc, kg, px, row * (unsigned)a.w + (unsigned)px, e);
+    e = en;
 #pragma unroll
-    for (int cb = 0; cb < NCOB; ++cb) {
-      const int co = cb * 16 + m;
+    for (int ks = 0; ks < NK; ++ks) av[ks] = nx[ks];
+  }
+}
+
+// Convolution of 32-channel inputs: a tap is one K-step, so the three
+// column-shifted operands of an input row serve the output rows above, on and
+// below it.  A wave marches down a strip of 16 columns and `ch` output rows
+// (rows dil apart), loading three operands a row instead of nine; the rows in
+// use and three rows of look-ahead sit in a circular register buffer.  Bound by
+// memory: at 256 x 64 x 64 and 32 x 32 channels 41 us a launch (104 us with nine
+// loads a tile and 2-byte stores), against 25 us for its 134 MB (37 us for an
+// input gradient, which reads the mask) at the streaming rate.  Three waves per
+// SIMD and two rows of look-ahead measured 42 us, two waves with two rows 53.
+template <int NCOB>
+__global__ __launch_bounds__(256, 2) void k_conv_rows(const ConvArgs a) {
+  constexpr int NB = 6;  // rows i-1, i, i+1 and three in flight
+  const int lane = threadIdx.x & 63;
+  const int m = lane & 15, kg = lane >> 4;
+  const int wvi = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  b8 wv[NCOB][9];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int px = (int)seg * 16 + 4 * kg + j;
-        if (px >= a.w) continue;
-        const long long p = (long long)row * a.w + px;
-        if (a.mode == 0) {
-          if (co < a.cout_p) a.out[p * a.cout_p + co] = to_bf16(fmaxf(acc[cb][j] + a.bias[co], 0.0f));
-        } else if (a.mode == 1) {
-          if (co == 0) a.out32[p] = (acc[cb][j] + a.bias[0]) + a.resid[p];
-        } else {
-          if (co < a.cout_p) {
-            const bool on = from_bf16(a.mask[p * a.cout_p + co]) > 0.0f;
-            a.out[p * a.cout_p + co] = to_bf16(on ? acc[cb][j] : 0.0f);
-          }
-        }
+  for (int cb = 0; cb < NCOB; ++cb)
+#pragma unroll
+    for (int t = 0; t < 9; ++t)
+      wv[cb][t] = *reinterpret_cast<const b8*>(a.wt + (cb * 16 + m) * a.kpad + t * 32 + 8 * kg);
+  ConvOut<NCOB> co;
+  co.load(a, kg);
+  const int d = a.dil, segs = (a.w + 15) >> 4;
+  const int per = (a.h + d - 1) / d, chunks = (per + a.ch - 1) / a.ch;  // rows of a residue class
+  const unsigned hw = (unsigned)(a.h * a.w);
+  const Rsrc RI = rsrc(a.in, (unsigned)a.n * hw * 64u);
+  const unsigned strips = (unsigned)(a.n * d * chunks * segs);
+  for (unsigned s = blockIdx.x * 4u + (unsigned)wvi; s < strips; s += gridDim.x * 4u) {
+    const unsigned q = s / (unsigned)segs, q2 = q / (unsigned)chunks, nn = q2 / (unsigned)d;
+    const int x = (int)(s - q * (unsigned)segs) * 16 + m;
+    const int i0 = (int)(q - q2 * (unsigned)chunks) * a.ch, r = (int)(q2 - nn * (unsigned)d);
+    const int i1 = min(i0 + a.ch, (a.h - r + d - 1) / d);
+    unsigned vo[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const int xx = x + (k - 1) * d;
+      vo[k] = xx >= 0 && xx < a.w ? ((unsigned)xx * 32u + 8u * (unsigned)kg) * 2u : kDrop;
+    }
+    b8 buf[NB][3];
+    auto fetch = [&](int i, b8* row) {  // row r + d*i of image nn, zero outside it
+      const int y = r + d * i;
+      const bool ok = i <= i1 && y >= 0 && y < a.h;
+      const unsigned so = ok ? (nn * hw + (unsigned)(y * a.w)) * 64u : 0u;
+#pragma unroll
+      for (int k = 0; k < 3; ++k)
+        row[k] = __builtin_bit_cast(
+            b8, __builtin_amdgcn_raw_buffer_load_b128(RI, (int)(ok ? vo[k] : kDrop), (int)so, 0));
+    };
+    const auto pix = [&](int i) { return nn * hw + (unsigned)((r + d * i) * a.w + x); };
+    typename ConvOut<NCOB>::Extra e{}, en{};
+    ConvOut<NCOB>::fetch(a, kg, i0 < i1 && x < a.w, pix(i0), e);
+#pragma unroll
+    for (int b = 0; b < NB - 1; ++b) fetch(i0 - 1 + b, buf[b]);
+    for (int base = i0; base < i1; base += NB) {
+#pragma unroll
+      for (int j = 0; j < NB; ++j) {
+        const int i = base + j;
+        if (i >= i1) break;
+        ConvOut<NCOB>::fetch(a, kg, i + 1 < i1 && x < a.w, pix(i + 1), en);
+        fetch(i + NB - 2, buf[(j + NB - 1) % NB]);
+        __builtin_amdgcn_sched_barrier(0);  // the look-ahead is issued before the products
+        f4 acc[NCOB];
+#pragma unroll
+        for (int cb = 0; cb < NCOB; ++cb) acc[cb] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int t = 0; t < 9; ++t)
+#pragma unroll
+          for (int cb = 0; cb < NCOB; ++cb)
+            acc[cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[cb][t], buf[(j + t / 3) % NB][t % 3],
+                                                              acc[cb], 0, 0, 0);
+        co.store(a, acc, kg, x, pix(i), e);
+        e = en;
       }
     }
   }
@@ -171,120 +306,252 @@ struct WgradArgs {
   float* part;      // [groups][WG_STRIDE]
   int n, h, w, dz_p, act_p, dil;
   int rows_per;     // image rows (over n*h) of one workgroup
+  int pw;           // pixels of a staged panel of a row (a multiple of 32)
 };
 
-constexpr int SROW = 40;  // LDS row stride (bf16) of a staged 32-pixel chunk
-
 // dW[tap][co][ci] = sum_pix dz[pix][co] act[pix + tap][ci] as MFMAs with
-// M = co, N = ci, K = 32 pixels of one row.  Per chunk the workgroup stages
-// dz (32 px x dz_p) and the nine tap-shifted act chunks (32 px x act_p)
-// transposed into LDS, so each lane's eight K values are one 16-byte LDS
-// read; wave w takes the 16 x 16 block (co block w & 1, ci block w >> 1) and
-// accumulates over all chunks of its rows in registers.  One partial per
-// workgroup; the reduction adds them in a fixed order.
-__global__ __launch_bounds__(256) void k_wgrad(const WgradArgs a) {
-  __shared__ __attribute__((aligned(16))) bf16 sdz[MAXC * SROW];
-  __shared__ __attribute__((aligned(16))) bf16 sact[9 * MAXC * SROW];
-  const int tid = threadIdx.x, lane = tid & 63, wvi = tid >> 6;
-  const int cob = wvi & 1, cib = wvi >> 1;
+// M = co, N = ci, K = 32 pixels of one row.  Both operands need eight
+// consecutive pixels of one channel per lane where memory holds the channels of
+// a pixel together: rows are staged as they are and read with the transposing
+// LDS load (ds_read_b64_tr_b16: of 16 lanes, lanes 4i .. 4i+3 address the 16
+// channels of pixel i and lane l receives channel l of the four pixels), which
+// serves all nine taps from one copy, each at its own pixel offset.
+//
+// A workgroup takes a range of image rows; per row and 32-pixel chunk every
+// wave multiplies its taps of one block of 16 input channels with all output
+// channels, and the accumulators run over all rows.  With RING (no dilation,
+// rows up to WG_RING_W pixels) each row of the layer input is staged once and
+// stays for the next two; otherwise the three rows of every panel of `pw`
+// pixels are staged.  The next unit's rows are in flight meanwhile.  One
+// partial per workgroup; the reduction adds them in a fixed order.
+//
+// Measured over the six layers of a 32-channel network at 256 x 64 x 64: 43 us
+// a launch (59 with three waves per SIMD, which left a fourth round of the 1024
+// workgroups; 132 when nine tap-shifted copies of each chunk were transposed by
+// 2-byte LDS stores), against 25 us for the 134 MB of a 32 x 32 layer.
+constexpr int WG_RING_W = 128;  // widest row of the ring (50 KB of LDS)
+
+// Byte offset in a staged row of channel block half (16 channels), pixel p: 64
+// bytes a pixel, the halves swapped in every second group of eight pixels so
+// that the lanes of a transposing load, eight pixels apart, meet other banks.
+__device__ __forceinline__ unsigned stage_off(int p, int half) {
+  return (unsigned)(p * 64 + ((half ^ ((p >> 3) & 1)) << 5));
+}
+
+template <bool RING>
+__global__ __launch_bounds__(256, RING ? 4 : 2) void k_wgrad(const WgradArgs a) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+  constexpr int NA = RING ? 3 : 8, NZ = RING ? 2 : 1;  // 16-byte loads per thread and unit
+  constexpr int NACT = RING ? 4 : 6;  // staged act rows: a ring of four, or two sets of three
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wvi = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int m = lane & 15, kg = lane >> 4;
-  const int R = a.n * a.h;
+  const int R = a.n * a.h, d = a.dil;
   const int r0 = blockIdx.x * a.rows_per, r1 = min(R, r0 + a.rows_per);
-  for (int i = tid; i < MAXC * SROW; i += 256) sdz[i] = 0;  // padded channels stay zero
-  for (int i = tid; i < 9 * MAXC * SROW; i += 256) sact[i] = 0;
-  __syncthreads();
-  const bool active = cob * 16 < a.dz_p && cib * 16 < a.act_p;
-  f4 acc[9];
-#pragma unroll
-  for (int t = 0; t < 9; ++t) acc[t] = f4{0.f, 0.f, 0.f, 0.f};
-  float bsum = 0.0f;
+  const int sp = (a.pw + 2 * d + 15) & ~15;  // pixels of a staged act row
+  unsigned char* const sz = lds + NACT * sp * 64;  // two dz rows of pw pixels
   const int cvz = a.dz_p >> 3, cva = a.act_p >> 3;
-  const Rsrc RZ = rsrc(a.dz, (unsigned)R * (unsigned)a.w * (unsigned)a.dz_p * 2u);
-  const Rsrc RA = rsrc(a.act, (unsigned)R * (unsigned)a.w * (unsigned)a.act_p * 2u);
-  for (int r = r0; r < r1; ++r) {
-    const int y = r % a.h, nn = r / a.h;
-    for (int x0 = 0; x0 < a.w; x0 += 32) {
-      for (int i = tid; i < 32 * cvz; i += 256) {
-        const int px = i / cvz, cg = i - px * cvz;
-        const int xx = x0 + px;
-        const unsigned vo = xx < a.w ? ((unsigned)(r * a.w + xx) * (unsigned)a.dz_p + 8u * cg) * 2u
-                                     : kDrop;
-        const u32x4 v = bld16(RZ, vo);
+  const int ncob = (a.dz_p + 15) >> 4, ncib = (a.act_p + 15) >> 4;
+  // the wave's taps [tap0, tap0 + ntap) of input channel block cib
+  const int cib = ncib == 2 ? wvi & 1 : 0;
+  const int tap0 = ncib == 2 ? (wvi >> 1) * 5 : (wvi == 0 ? 0 : 1 + 2 * wvi);
+  const int ntap = ncib == 2 ? 5 - (wvi >> 1) : (wvi == 0 ? 3 : 2);
+  f4 acc[5][2];
 #pragma unroll
-        for (int j = 0; j < 8; ++j)
-          sdz[(8 * cg + j) * SROW + px] = (bf16)(v[j >> 1] >> (16 * (j & 1)));
-      }
-      for (int i = tid; i < 9 * 32 * cva; i += 256) {
-        const int tap = i / (32 * cva), q = i - tap * 32 * cva, px = q / cva, cg = q - px * cva;
-        const int yy = y + (tap / 3 - 1) * a.dil, xx = x0 + px + (tap % 3 - 1) * a.dil;
-        const bool ok = yy >= 0 && yy < a.h && xx >= 0 && xx < a.w;
-        const unsigned vo =
-            ok ? ((unsigned)((nn * a.h + yy) * a.w + xx) * (unsigned)a.act_p + 8u * cg) * 2u : kDrop;
-        const u32x4 v = bld16(RA, vo);
+  for (int t = 0; t < 5; ++t) acc[t][0] = acc[t][1] = f4{0.f, 0.f, 0.f, 0.f};
+  float bsum[2] = {0.f, 0.f};
+
+  const unsigned wz = (unsigned)a.w * (unsigned)a.dz_p * 2u, wa = (unsigned)a.w * (unsigned)a.act_p * 2u;
+  const Rsrc RZ = rsrc(a.dz, (unsigned)R * wz), RA = rsrc(a.act, (unsigned)R * wa);
+  // staging items of the thread, the same for every unit: source offset from
+  // the row's panel, LDS offset, the act row (0 .. 2 with full staging)
+  const int arows = RING ? 1 : 3, apx = a.pw + 2 * d;
+  int apos[NA], arow[NA], zpos[NZ];
+  unsigned alds[NA], zlds[NZ], acg[NA], zcg[NZ];
 #pragma unroll
-        for (int j = 0; j < 8; ++j)
-          sact[(tap * MAXC + 8 * cg + j) * SROW + px] = (bf16)(v[j >> 1] >> (16 * (j & 1)));
-      }
-      __syncthreads();
-      if (active) {
-        const u32x4 araw = *reinterpret_cast<const u32x4*>(&sdz[(cob * 16 + m) * SROW + 8 * kg]);
-        const b8 av = __builtin_bit_cast(b8, araw);
-#pragma unroll
-        for (int t = 0; t < 9; ++t) {
-          const b8 bv = *reinterpret_cast<const b8*>(&sact[(t * MAXC + cib * 16 + m) * SROW + 8 * kg]);
-          acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bv, acc[t], 0, 0, 0);
-        }
-        if (cib == 0)
-#pragma unroll
-          for (int j = 0; j < 4; ++j)
-            bsum += __uint_as_float(araw[j] << 16) + __uint_as_float(araw[j] & 0xffff0000u);
-      }
-      __syncthreads();
-    }
+  for (int i = 0; i < NA; ++i) {
+    const int e = tid + i * 256, q = e / cva, row = q / apx;
+    arow[i] = row < arows ? row : -1;
+    apos[i] = q - row * apx;  // pixel x0 - d + apos
+    const int cg = e - q * cva;
+    acg[i] = (unsigned)cg * 16u;
+    alds[i] = stage_off(apos[i], cg >> 1) + (unsigned)(cg & 1) * 16u;
   }
-  if (!active) return;
+#pragma unroll
+  for (int i = 0; i < NZ; ++i) {
+    const int e = tid + i * 256, q = e / cvz, cg = e - q * cvz;
+    zpos[i] = q < a.pw ? q : -1;
+    zcg[i] = (unsigned)cg * 16u;
+    zlds[i] = stage_off(q, cg >> 1) + (unsigned)(cg & 1) * 16u;
+  }
+  u32x4 la[NA], lz[NZ];
+  const auto load_act = [&](int row, int x0) {  // rows row, row + d, row + 2d (RING: row)
+#pragma unroll
+    for (int i = 0; i < NA; ++i) {
+      const int rr = row + arow[i] * d, x = x0 - d + apos[i];
+      const bool ok = arow[i] >= 0 && rr >= 0 && rr < R && x >= 0 && x < a.w;
+      la[i] = bld16(RA, ok ? (unsigned)rr * wa + (unsigned)(x * a.act_p) * 2u + acg[i] : kDrop);
+    }
+  };
+  const auto load_dz = [&](int row, int x0) {
+#pragma unroll
+    for (int i = 0; i < NZ; ++i) {
+      const int x = x0 + zpos[i];
+      const bool ok = zpos[i] >= 0 && row < r1 && x < a.w;
+      lz[i] = bld16(RZ, ok ? (unsigned)row * wz + (unsigned)(x * a.dz_p) * 2u + zcg[i] : kDrop);
+    }
+  };
+  const auto put_act = [&](int slot) {
+#pragma unroll
+    for (int i = 0; i < NA; ++i)
+      if (arow[i] >= 0)
+        *reinterpret_cast<u32x4*>(lds + (slot + arow[i]) * sp * 64 + alds[i]) = la[i];
+  };
+  const auto put_dz = [&](int slot) {
+#pragma unroll
+    for (int i = 0; i < NZ; ++i)
+      if (zpos[i] >= 0) *reinterpret_cast<u32x4*>(sz + slot * a.pw * 64 + zlds[i]) = lz[i];
+  };
+  const auto tr = [&](const unsigned char* p) {
+    return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s4*)p);
+  };
+  const auto pair = [&](s4 lo, s4 hi) {
+    return __builtin_bit_cast(b8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+  };
+  // lane offsets of the operands' two loads (pixels 8 kg + 0..3 and + 4..7)
+  unsigned oz[2][2], oa[5][2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int p = 8 * kg + 4 * h + (m >> 2);
+    const unsigned c = (unsigned)(m & 3) * 8u;
+    oz[0][h] = stage_off(p, 0) + c;
+    oz[1][h] = stage_off(p, 1) + c;
+#pragma unroll
+    for (int t = 0; t < 5; ++t) oa[t][h] = stage_off(p + ((tap0 + t) % 3) * d, cib) + c;
+  }
+
+  const int panels = (a.w + a.pw - 1) / a.pw;
+  int r = r0, x0 = 0, u = 0;
+  if (RING) {  // rows r0-1 and r0, then r0+1 with the first dz row
+    load_act(r0 - 1, 0);
+    put_act((r0 + 3) & 3);
+    load_act(r0, 0);
+    put_act(r0 & 3);
+    load_act(r0 + 1, 0);
+    put_act((r0 + 1) & 3);
+  } else {
+    load_act(r0 - d, 0);
+    put_act(0);
+  }
+  load_dz(r0, 0);
+  put_dz(0);
+  __syncthreads();
+  while (r < r1) {
+    int rn = r, xn = x0 + a.pw;  // the next unit
+    if (xn >= panels * a.pw) { xn = 0; ++rn; }
+    if (RING) load_act(rn + 1, 0);
+    else load_act(rn - d, xn);
+    load_dz(rn, xn);
+    __builtin_amdgcn_sched_barrier(0);
+    const int y = r % a.h;
+    const int chunks = (min(a.pw, a.w - x0) + 31) >> 5;
+    if (cib < ncib) {
+      for (int c = 0; c < chunks; ++c) {
+        const unsigned char* pz = sz + (u & 1) * a.pw * 64 + c * 2048;
+        s4 zr[2][2];
+        b8 av[2];
+#pragma unroll
+        for (int cob = 0; cob < 2; ++cob) {
+          if (cob < ncob) {
+            zr[cob][0] = tr(pz + oz[cob][0]);
+            zr[cob][1] = tr(pz + oz[cob][1]);
+            av[cob] = pair(zr[cob][0], zr[cob][1]);
+          }
+        }
+#pragma unroll
+        for (int t = 0; t < 5; ++t) {
+          const int ky = (tap0 + t) / 3 - 1, yy = y + ky * d;
+          if (t < ntap && yy >= 0 && yy < a.h) {
+            const int slot = RING ? (r + ky) & 3 : (u & 1) * 3 + ky + 1;
+            const unsigned char* pa = lds + slot * sp * 64 + c * 2048;
+            const b8 bv = pair(tr(pa + oa[t][0]), tr(pa + oa[t][1]));
+            acc[t][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[0], bv, acc[t][0], 0, 0, 0);
+            if (ncob == 2)
+              acc[t][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[1], bv, acc[t][1], 0, 0, 0);
+          }
+        }
+        if (wvi == 0) {
+#pragma unroll
+          for (int cob = 0; cob < 2; ++cob) {
+            if (cob < ncob) {
+              const u32x4 w4 = __builtin_bit_cast(u32x4, av[cob]);
+#pragma unroll
+              for (int j = 0; j < 4; ++j)
+                bsum[cob] += __uint_as_float(w4[j] << 16) + __uint_as_float(w4[j] & 0xffff0000u);
+            }
+          }
+        }
+      }
+    }
+    // the slots written hold no row that this unit reads: RING row r+2 (mod 4),
+    // otherwise the other set
+    ++u;
+    if (RING) put_act((rn + 1) & 3);
+    else put_act((u & 1) * 3);
+    put_dz(u & 1);
+    __syncthreads();
+    r = rn;
+    x0 = xn;
+  }
+  if (cib >= ncib) return;
   float* P = a.part + (long long)blockIdx.x * WG_STRIDE;
   const int ci = cib * 16 + m;
 #pragma unroll
-  for (int t = 0; t < 9; ++t)
+  for (int t = 0; t < 5; ++t)
 #pragma unroll
-    for (int j = 0; j < 4; ++j)  // D[m = co][n = ci]: co = cob*16 + 4 kg + j
-      P[(t * MAXC + cob * 16 + 4 * kg + j) * MAXC + ci] = acc[t][j];
+    for (int cob = 0; cob < 2; ++cob)
+      if (t < ntap && cob < ncob)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)  // D[m = co][n = ci]: co = cob*16 + 4 kg + j
+          P[((tap0 + t) * MAXC + cob * 16 + 4 * kg + j) * MAXC + ci] = acc[t][cob][j];
   // bias: lanes m, m+16, m+32, m+48 hold pixels of channel cob*16 + m
-  bsum += __shfl_xor(bsum, 16);
-  bsum += __shfl_xor(bsum, 32);
-  if (kg == 0 && cib == 0) P[9 * MAXC * MAXC + cob * 16 + m] = bsum;
+#pragma unroll
+  for (int cob = 0; cob < 2; ++cob) {
+    float b = bsum[cob];
+    b += __shfl_xor(b, 16);
+    b += __shfl_xor(b, 32);
+    if (wvi == 0 && kg == 0 && cob < ncob) P[9 * MAXC * MAXC + cob * 16 + m] = b;
+  }
 }
 
 // Deterministic two-level sum of the workgroup partials into the layer's
-// gradient (W[co][ci][ky][kx] then b[co]): level 1 adds group g's share of
-// the partials in order (FP64), level 2 adds the groups in order.
-__device__ __forceinline__ int wgrad_src(int e, int cin, int cout) {
-  const int nw = cout * cin * 9;
-  if (e < nw) {
-    const int co = e / (cin * 9), r = e % (cin * 9), ci = r / 9, t = r % 9;
-    return (t * MAXC + co) * MAXC + ci;
+// gradient (W[co][ci][ky][kx] then b[co]): group g adds its share of the
+// partials in order (FP64), then the groups are added in order.  A block takes
+// the 32 input channels of one tap and output channel (one 128-byte line of
+// every partial), or the 32 biases; thread (g, ci).
+__global__ __launch_bounds__(32 * WG_LEVEL1) void k_wgrad_reduce(const float* part, int P, int cin,
+                                                                 int cout, float* grad) {
+  __shared__ double sh[WG_LEVEL1][32];
+  const int ci = threadIdx.x & 31, g = threadIdx.x >> 5;
+  const int G = min(WG_LEVEL1, P);
+  const int tc = blockIdx.x;  // tap * cout + co; 9 * cout: the biases
+  const bool bias = tc == 9 * cout;
+  const int t = tc / cout, co = tc - t * cout;
+  const int src = bias ? 9 * MAXC * MAXC + ci : (t * MAXC + co) * MAXC + ci;
+  const bool on = bias ? ci < cout : ci < cin;
+  double s = 0.0;
+  if (g < G && on) {
+    const int p0 = (int)((long long)P * g / G), p1 = (int)((long long)P * (g + 1) / G);
+#pragma unroll 8
+    for (int p = p0; p < p1; ++p) s += (double)part[(long long)p * WG_STRIDE + src];
   }
-  return 9 * MAXC * MAXC + (e - nw);
-}
-
-__global__ void k_wgrad_reduce1(const float* part, int P, int G, int cin, int cout, double* part2) {
-  const int ne = cout * cin * 9 + cout;
-  const int e = blockIdx.x * blockDim.x + threadIdx.x, g = blockIdx.y;
-  if (e >= ne) return;
-  const int src = wgrad_src(e, cin, cout);
-  const int p0 = (int)((long long)P * g / G), p1 = (int)((long long)P * (g + 1) / G);
-  double s = 0.0;
-  for (int p = p0; p < p1; ++p) s += (double)part[(long long)p * WG_STRIDE + src];
-  part2[(long long)g * ne + e] = s;
-}
-
-__global__ void k_wgrad_reduce2(const double* part2, int G, int ne, float* grad) {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= ne) return;
-  double s = 0.0;
-  for (int g = 0; g < G; ++g) s += part2[(long long)g * ne + e];
-  grad[e] = (float)s;
+  sh[g][ci] = s;
+  __syncthreads();
+  if (g == 0 && on) {
+    double v = 0.0;
+    for (int i = 0; i < G; ++i) v += sh[i][ci];
+    grad[bias ? cout * cin * 9 + ci : (co * cin + ci) * 9 + t] = (float)v;
+  }
 }
 
 // NCHW FP32 input -> NHWC BF16 (cp channels) and the FP32 residual channel 0.
@@ -404,7 +671,6 @@ struct rtm_cnn {
   bf16* dz[MAXL] = {nullptr};   // dz[l]: gradient at the output of layer l, NHWC cp[l+1]
   float *x32 = nullptr, *resid = nullptr, *y32 = nullptr, *t32 = nullptr, *diff = nullptr;
   float* part = nullptr;    // weight-gradient partials [WG_GROUPS][WG_STRIDE]
-  double* part2 = nullptr;  // first reduction level [WG_LEVEL1][WG_STRIDE]
   double* sq = nullptr;
   int adam_t = 0;
   bool grad_ok = false;
@@ -480,10 +746,26 @@ void conv_go(const ConvArgs& a, unsigned blocks, hipStream_t s) {
   hipLaunchKernelGGL((k_conv<NK, NCOB>), dim3(blocks), dim3(256), 0, s, a);
 }
 
-int launch_conv(rtm_cnn* c, const ConvArgs& a) {
+int launch_conv(rtm_cnn* c, ConvArgs a) {
+  const int nk = a.kpad / 32;
+  if (a.cin_p == 32) {
+    // Strips of sixteen rows (two halo rows each) where that still gives every
+    // SIMD four, shorter ones below; the waves that fit at once (two per SIMD)
+    // take an equal number each.
+    const long long cols = (long long)a.n * a.dil * ((a.w + 15) / 16);
+    const int per = (a.h + a.dil - 1) / a.dil;
+    a.ch = 16;
+    while (a.ch > 1 && cols * ((per + a.ch - 1) / a.ch) < 4096) a.ch /= 2;
+    const long long strips = cols * ((per + a.ch - 1) / a.ch);
+    const long long rounds = (strips + 2047) / 2048, waves = (strips + rounds - 1) / rounds;
+    const dim3 grid((unsigned)((waves + 3) / 4));
+    if (a.ncob == 2) hipLaunchKernelGGL((k_conv_rows<2>), grid, dim3(256), 0, c->stream, a);
+    else hipLaunchKernelGGL((k_conv_rows<1>), grid, dim3(256), 0, c->stream, a);
+    CNNCHK(c, hipGetLastError());
+    return RTM_CNN_OK;
+  }
   const long long tiles = (long long)a.n * a.h * ((a.w + 15) / 16);
   const unsigned blocks = (unsigned)std::min<long long>((tiles + 3) / 4, 2048);
-  const int nk = a.kpad / 32;
   switch (nk * 4 + a.ncob) {
     case 3 * 4 + 1: conv_go<3, 1>(a, blocks, c->stream); break;
     case 3 * 4 + 2: conv_go<3, 2>(a, blocks, c->stream); break;
@@ -491,8 +773,6 @@ int launch_conv(rtm_cnn* c, const ConvArgs& a) {
     case 5 * 4 + 2: conv_go<5, 2>(a, blocks, c->stream); break;
     case 7 * 4 + 1: conv_go<7, 1>(a, blocks, c->stream); break;
     case 7 * 4 + 2: conv_go<7, 2>(a, blocks, c->stream); break;
-    case 9 * 4 + 1: conv_go<9, 1>(a, blocks, c->stream); break;
-    case 9 * 4 + 2: conv_go<9, 2>(a, blocks, c->stream); break;
     default: return cfail(c, RTM_CNN_E_ARG, "no convolution for K %d, %d channel blocks", a.kpad, a.ncob);
   }
   CNNCHK(c, hipGetLastError());
@@ -547,16 +827,22 @@ int loss_grad_dev(rtm_cnn* c, const float* t_dev, int n, int h, int w, double* l
     const int rows = n * h;
     const int rows_per = (rows + WG_GROUPS - 1) / WG_GROUPS;
     const int P = (rows + rows_per - 1) / rows_per;
-    WgradArgs g{c->dz[l], c->act[l], c->part, n, h, w, c->cp[l + 1], c->cp[l], c->dil[l], rows_per};
-    hipLaunchKernelGGL(k_wgrad, dim3((unsigned)P), dim3(256), 0, c->stream, g);
+    const int d = c->dil[l];
+    const bool ring = d == 1 && w <= WG_RING_W;
+    // panel: the whole row in the ring; else 64 pixels, 32 where the halo of the
+    // dilated taps needs the room
+    const int pw = ring ? (w + 31) / 32 * 32 : (d <= 8 ? 64 : 32);
+    WgradArgs g{c->dz[l], c->act[l], c->part, n, h, w, c->cp[l + 1], c->cp[l], d, rows_per, pw};
+    const size_t row = (size_t)((pw + 2 * d + 15) & ~15) * 64;
+    if (ring)
+      hipLaunchKernelGGL((k_wgrad<true>), dim3((unsigned)P), dim3(256), 4 * row + 128 * (size_t)pw,
+                         c->stream, g);
+    else
+      hipLaunchKernelGGL((k_wgrad<false>), dim3((unsigned)P), dim3(256), 6 * row + 128 * (size_t)pw,
+                         c->stream, g);
     CNNCHK(c, hipGetLastError());
-    const int ne = c->c[l + 1] * c->c[l] * 9 + c->c[l + 1];
-    const int G = std::min(WG_LEVEL1, P);
-    hipLaunchKernelGGL(k_wgrad_reduce1, dim3((ne + 255) / 256, G), dim3(256), 0, c->stream, c->part,
-                       P, G, c->c[l], c->c[l + 1], c->part2);
-    CNNCHK(c, hipGetLastError());
-    hipLaunchKernelGGL(k_wgrad_reduce2, dim3((ne + 255) / 256), dim3(256), 0, c->stream, c->part2,
-                       G, ne, c->grad + c->off[l]);
+    hipLaunchKernelGGL(k_wgrad_reduce, dim3((unsigned)(9 * c->c[l + 1] + 1)), dim3(32 * WG_LEVEL1), 0,
+                       c->stream, c->part, P, c->c[l], c->c[l + 1], c->grad + c->off[l]);
     CNNCHK(c, hipGetLastError());
     if (l > 0) {  // dz[l-1] = conv(dz[l], W^T flipped) * (act[l] > 0)
       ConvArgs a{};
@@ -651,7 +937,6 @@ int rtm_cnn_create(int nlayer, const int* channels, const int* dilation, long lo
   if (rc == RTM_CNN_OK) rc = calloc_dev(c, &c->diff, (size_t)max_pixels);
   if (rc == RTM_CNN_OK)
     rc = calloc_dev(c, &c->part, (size_t)std::min<long long>(max_rows, WG_GROUPS) * WG_STRIDE);
-  if (rc == RTM_CNN_OK) rc = calloc_dev(c, &c->part2, (size_t)WG_LEVEL1 * WG_STRIDE);
   if (rc == RTM_CNN_OK) rc = calloc_dev(c, &c->sq, 256);
   if (rc == RTM_CNN_OK) {
     if (hipMemsetAsync(c->am, 0, c->np * sizeof(float), c->stream) != hipSuccess ||

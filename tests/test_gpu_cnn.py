@@ -130,6 +130,25 @@ def test_dilated_forward_and_gradient(dil):
     assert _rel(g, gr) < 5e-3
 
 
+@pytest.mark.parametrize("ch,dil,n,h,w", [
+    ([2, 32, 32, 1], [1, 1, 1], 2, 9, 128),   # the widest row of the weight gradient's ring
+    ([2, 32, 16, 1], [1, 1, 1], 2, 5, 129),   # one pixel wider: panels, the last one pixel wide
+    ([2, 32, 32, 1], [1, 9, 64], 1, 11, 70),  # halos past the image; fewer rows than the dilation
+    ([2, 24, 32, 1], [8, 3, 1], 3, 10, 17),   # panels of 64 on a row of 17, residue classes of rows
+    ([2, 32, 32, 1], [1, 1, 1], 5, 1, 1)])    # a single pixel
+def test_staged_weight_gradient_and_row_convolution(ch, dil, n, h, w):
+    """Edges of the row-marching convolution (32 input channels) and of the
+    staged weight gradient, with the bounds of the deep stacks above."""
+    net, p = _net(ch, seed=7, dil=dil)
+    x, t = _data(n, ch[0], h, w, seed=9)
+    y = net.forward(x)
+    yr, lr, gr = reference(p, ch, x, t, dil)
+    assert _rel(y, yr) < 1e-4
+    loss, g = net.loss_grad(x, t)
+    assert abs(loss - lr) <= 1e-4 * lr
+    assert _rel(g, gr) < 5e-3
+
+
 def test_adam_step():
     ch = [2, 8, 1]
     net, p = _net(ch, seed=2)
