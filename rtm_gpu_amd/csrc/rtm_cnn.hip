@@ -554,15 +554,31 @@ __global__ __launch_bounds__(32 * WG_LEVEL1) void k_wgrad_reduce(const float* pa
   }
 }
 
+// Eight BF16 channels of a pixel as one 16-byte store; get(c): channel c.
+template <typename F>
+__device__ __forceinline__ void put8(bf16* dst, const F& get) {
+  u32x4 v;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) v[k] = (unsigned)get(2 * k) | ((unsigned)get(2 * k + 1) << 16);
+  *reinterpret_cast<u32x4*>(dst) = v;
+}
+
 // NCHW FP32 input -> NHWC BF16 (cp channels) and the FP32 residual channel 0.
+// With an order (training batch from the device-resident set), image i of the
+// batch is set entry order[b0 + i] and its target goes to t32.
 __global__ void k_pack_input(const float* x, long long npix, int hw, int cin, int cp, bf16* act,
-                             float* resid) {
+                             float* resid, const int* order, int b0, const float* t, float* t32) {
   for (long long p = (long long)blockIdx.x * blockDim.x + threadIdx.x; p < npix;
        p += (long long)gridDim.x * blockDim.x) {
-    const long long nn = p / hw, q = p % hw;
-    for (int c = 0; c < cp; ++c)
-      act[p * cp + c] = c < cin ? to_bf16(x[(nn * cin + c) * hw + q]) : (bf16)0;
-    resid[p] = x[nn * cin * hw + q];
+    const long long i = p / hw, q = p - i * hw;
+    const long long nn = order ? order[b0 + i] : i;
+    const float* px = x + nn * cin * hw + q;
+    for (int c = 0; c < cp; c += 8)
+      put8(act + p * cp + c, [&](int k) {
+        return c + k < cin ? to_bf16(px[(long long)(c + k) * hw]) : (bf16)0;
+      });
+    resid[p] = px[0];
+    if (order) t32[p] = t[nn * hw + q];
   }
 }
 
@@ -574,21 +590,8 @@ __global__ void k_loss_grad(const float* y, const float* t, long long npix, int 
        p += (long long)gridDim.x * blockDim.x) {
     const float d = y[p] - t[p];
     diff[p] = d;
-    for (int c = 0; c < cp; ++c) dz[p * cp + c] = c == 0 ? to_bf16(scale * d) : (bf16)0;
-  }
-}
-
-// One training batch from the device-resident set: sample i of the batch is
-// set entry order[b0 + i] (inputs c0 channels, then the target).
-__global__ void k_gather_batch(const float* dsx, const float* dst, const int* order, int b0,
-                               int batch, long long img, int c0, float* x32, float* t32) {
-  const long long per = img * (c0 + 1);
-  for (long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x; e < (long long)batch * per;
-       e += (long long)gridDim.x * blockDim.x) {
-    const long long i = e / per, r = e - i * per;
-    const long long k = order[b0 + i];
-    if (r < img * c0) x32[i * img * c0 + r] = dsx[k * img * c0 + r];
-    else t32[i * img + (r - img * c0)] = dst[k * img + (r - img * c0)];
+    for (int c = 0; c < cp; c += 8)
+      put8(dz + p * cp + c, [&](int k) { return c + k == 0 ? to_bf16(scale * d) : (bf16)0; });
   }
 }
 
@@ -604,25 +607,34 @@ __global__ void k_adam(float* p, const float* g, float* m, float* v, int n, floa
   p[i] = p[i] - lr * (mi * c1) / (sqrtf(vi * c2) + eps);
 }
 
-// FP32 params of one layer -> BF16 forward weights [16][kf] (k = tap*cin_p +
-// ci), backward-data weights [16][kb] (row ci, k = tap'*cout_p + co with the
-// flipped tap 8 - tap) and the padded bias.
-__global__ void k_pack_weights(const float* prm, int cin, int cout, int cin_p, int cout_p, int kf,
-                               int kb, bf16* wf, bf16* wb, float* bias) {
+// FP32 params -> BF16 forward weights [32][kf] (k = tap*cin_p + ci),
+// backward-data weights [32][kb] (row ci, k = tap'*cout_p + co with the flipped
+// tap 8 - tap) and the padded bias, of layer blockIdx.y.
+struct PackLayer {
+  const float* prm;
+  bf16 *wf, *wb;
+  float* bias;
+  int cin, cout, cin_p, cout_p, kf, kb;
+};
+struct PackArgs {
+  PackLayer l[MAXL];
+};
+__global__ void k_pack_weights(const PackArgs a) {
+  const PackLayer& l = a.l[blockIdx.y];
   const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e < MAXC * kf) {
-    const int co = e / kf, k = e % kf, tap = k / cin_p, ci = k % cin_p;
+  if (e < MAXC * l.kf) {
+    const int co = e / l.kf, k = e % l.kf, tap = k / l.cin_p, ci = k % l.cin_p;
     float v = 0.0f;
-    if (co < cout && ci < cin && tap < 9) v = prm[(co * cin + ci) * 9 + tap];
-    wf[e] = to_bf16(v);
+    if (co < l.cout && ci < l.cin && tap < 9) v = l.prm[(co * l.cin + ci) * 9 + tap];
+    l.wf[e] = to_bf16(v);
   }
-  if (e < MAXC * kb) {
-    const int ci = e / kb, k = e % kb, tp = k / cout_p, co = k % cout_p;
+  if (e < MAXC * l.kb) {
+    const int ci = e / l.kb, k = e % l.kb, tp = k / l.cout_p, co = k % l.cout_p;
     float v = 0.0f;
-    if (ci < cin && co < cout && tp < 9) v = prm[(co * cin + ci) * 9 + (8 - tp)];
-    wb[e] = to_bf16(v);
+    if (ci < l.cin && co < l.cout && tp < 9) v = l.prm[(co * l.cin + ci) * 9 + (8 - tp)];
+    l.wb[e] = to_bf16(v);
   }
-  if (e < MAXC) bias[e] = e < cout ? prm[cout * cin * 9 + e] : 0.0f;
+  if (e < MAXC) l.bias[e] = e < l.cout ? l.prm[l.cout * l.cin * 9 + e] : 0.0f;
 }
 
 // FP64 sum of squares (fixed order: block partials, then one block).
@@ -677,6 +689,8 @@ struct rtm_cnn {
   // device-resident training set
   float *ds_x = nullptr, *ds_t = nullptr;
   int* ds_order = nullptr;
+  double* ds_sq = nullptr;  // loss partial sums of the batches of an epoch
+  int ds_nb = 0;
   long long ds_cap = 0;
   int ds_n = 0;
 };
@@ -731,13 +745,16 @@ int check_shape(rtm_cnn* c, int n, int h, int w) {
 }
 
 int pack_weights(rtm_cnn* c) {
+  PackArgs a{};
+  int most = 0;
   for (int l = 0; l < c->L; ++l) {
-    const int ne = MAXC * (c->kf[l] > c->kb[l] ? c->kf[l] : c->kb[l]);
-    hipLaunchKernelGGL(k_pack_weights, dim3(nblk(ne, 256, 1 << 20)), dim3(256), 0, c->stream,
-                       c->prm + c->off[l], c->c[l], c->c[l + 1], c->cp[l], c->cp[l + 1], c->kf[l],
-                       c->kb[l], c->wf[l], c->wb[l], c->bias[l]);
-    CNNCHK(c, hipGetLastError());
+    a.l[l] = PackLayer{c->prm + c->off[l], c->wf[l], c->wb[l], c->bias[l], c->c[l], c->c[l + 1],
+                       c->cp[l], c->cp[l + 1], c->kf[l], c->kb[l]};
+    most = std::max(most, MAXC * std::max(c->kf[l], c->kb[l]));
   }
+  hipLaunchKernelGGL(k_pack_weights, dim3((unsigned)((most + 255) / 256), (unsigned)c->L), dim3(256), 0,
+                     c->stream, a);
+  CNNCHK(c, hipGetLastError());
   return RTM_CNN_OK;
 }
 
@@ -806,16 +823,27 @@ int forward_dev(rtm_cnn* c, int n, int h, int w) {
   return RTM_CNN_OK;
 }
 
-int pack_input(rtm_cnn* c, const float* x_dev, int n, int h, int w) {
+// order: a training batch, images order[b0 ..] of the set x_dev with targets t_dev.
+int pack_input(rtm_cnn* c, const float* x_dev, int n, int h, int w, const int* order = nullptr,
+               int b0 = 0, const float* t_dev = nullptr) {
   const long long npix = (long long)n * h * w;
   hipLaunchKernelGGL(k_pack_input, dim3(nblk(npix)), dim3(256), 0, c->stream, x_dev, npix, h * w,
-                     c->c[0], c->cp[0], c->act[0], c->resid);
+                     c->c[0], c->cp[0], c->act[0], c->resid, order, b0, t_dev, c->t32);
   CNNCHK(c, hipGetLastError());
   return RTM_CNN_OK;
 }
 
-// Loss and gradients for the batch in act[0] / resid with targets t_dev.
-int loss_grad_dev(rtm_cnn* c, const float* t_dev, int n, int h, int w, double* loss) {
+constexpr int SQ_BLOCKS = 256;  // partial sums of a batch's loss
+// The loss of a batch of npix pixels from its partial sums.
+double loss_of(const double* part, long long npix) {
+  double s = 0.0;
+  for (int i = 0; i < SQ_BLOCKS; ++i) s += part[i];
+  return s / (double)npix;
+}
+
+// Gradients for the batch in act[0] / resid with targets t_dev; sq: device
+// room for the partial sums of its loss, or null.
+int loss_grad_dev(rtm_cnn* c, const float* t_dev, int n, int h, int w, double* sq) {
   int rc = forward_dev(c, n, h, w);
   if (rc != RTM_CNN_OK) return rc;
   const long long npix = (long long)n * h * w;
@@ -861,15 +889,9 @@ int loss_grad_dev(rtm_cnn* c, const float* t_dev, int n, int h, int w, double* l
       if (rc != RTM_CNN_OK) return rc;
     }
   }
-  if (loss) {
-    hipLaunchKernelGGL(k_sumsq, dim3(256), dim3(256), 0, c->stream, c->diff, npix, c->sq);
+  if (sq) {
+    hipLaunchKernelGGL(k_sumsq, dim3(SQ_BLOCKS), dim3(256), 0, c->stream, c->diff, npix, sq);
     CNNCHK(c, hipGetLastError());
-    std::vector<double> part(256);
-    CNNCHK(c, hipMemcpyAsync(part.data(), c->sq, 256 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    CNNCHK(c, hipStreamSynchronize(c->stream));
-    double s = 0.0;
-    for (double v : part) s += v;
-    *loss = s / (double)npix;
   }
   c->grad_ok = true;
   return RTM_CNN_OK;
@@ -937,7 +959,7 @@ int rtm_cnn_create(int nlayer, const int* channels, const int* dilation, long lo
   if (rc == RTM_CNN_OK) rc = calloc_dev(c, &c->diff, (size_t)max_pixels);
   if (rc == RTM_CNN_OK)
     rc = calloc_dev(c, &c->part, (size_t)std::min<long long>(max_rows, WG_GROUPS) * WG_STRIDE);
-  if (rc == RTM_CNN_OK) rc = calloc_dev(c, &c->sq, 256);
+  if (rc == RTM_CNN_OK) rc = calloc_dev(c, &c->sq, SQ_BLOCKS);
   if (rc == RTM_CNN_OK) {
     if (hipMemsetAsync(c->am, 0, c->np * sizeof(float), c->stream) != hipSuccess ||
         hipMemsetAsync(c->av, 0, c->np * sizeof(float), c->stream) != hipSuccess ||
@@ -1009,10 +1031,13 @@ int rtm_cnn_loss_grad(rtm_cnn* c, const float* x, const float* t, int n, int h, 
   CNNCHK(c, hipMemcpyAsync(c->x32, x, npix * c->c[0] * sizeof(float), hipMemcpyHostToDevice, c->stream));
   CNNCHK(c, hipMemcpyAsync(c->t32, t, npix * sizeof(float), hipMemcpyHostToDevice, c->stream));
   rc = pack_input(c, c->x32, n, h, w);
-  if (rc == RTM_CNN_OK) rc = loss_grad_dev(c, c->t32, n, h, w, loss);
+  if (rc == RTM_CNN_OK) rc = loss_grad_dev(c, c->t32, n, h, w, loss ? c->sq : nullptr);
   if (rc != RTM_CNN_OK) return rc;
+  double part[SQ_BLOCKS];
+  if (loss) CNNCHK(c, hipMemcpyAsync(part, c->sq, sizeof(part), hipMemcpyDeviceToHost, c->stream));
   if (grad) CNNCHK(c, hipMemcpyAsync(grad, c->grad, c->np * sizeof(float), hipMemcpyDeviceToHost, c->stream));
   CNNCHK(c, hipStreamSynchronize(c->stream));
+  if (loss) *loss = loss_of(part, (long long)npix);
   return RTM_CNN_OK;
 }
 
@@ -1047,6 +1072,16 @@ int rtm_cnn_fit(rtm_cnn* c, const float* x, const float* t, int n, int h, int w,
     c->ds_cap = (long long)need;
     c->ds_n = n;
   }
+  const int batches = n / batch;
+  if (batches > c->ds_nb) {
+    CNNCHK(c, hipStreamSynchronize(c->stream));
+    cfree_dev(c, &c->ds_sq);
+    c->ds_nb = 0;
+    rc = calloc_dev(c, &c->ds_sq, (size_t)batches * SQ_BLOCKS);
+    if (rc != RTM_CNN_OK) return rc;
+    c->ds_nb = batches;
+  }
+  std::vector<double> part((size_t)batches * SQ_BLOCKS);
   CNNCHK(c, hipMemcpyAsync(c->ds_x, x, need * c->c[0] * sizeof(float), hipMemcpyHostToDevice, c->stream));
   CNNCHK(c, hipMemcpyAsync(c->ds_t, t, need * sizeof(float), hipMemcpyHostToDevice, c->stream));
   std::vector<int> order(n);
@@ -1063,21 +1098,21 @@ int rtm_cnn_fit(rtm_cnn* c, const float* x, const float* t, int n, int h, int w,
     }
     // the previous epoch ended with a stream synchronisation (the loss read-back)
     CNNCHK(c, hipMemcpyAsync(c->ds_order, order.data(), n * sizeof(int), hipMemcpyHostToDevice, c->stream));
-    double sum = 0.0;
     int nb = 0;
     for (int b0 = 0; b0 + batch <= n; b0 += batch) {
-      hipLaunchKernelGGL(k_gather_batch, dim3(nblk((long long)batch * img * (c->c[0] + 1))), dim3(256), 0,
-                         c->stream, c->ds_x, c->ds_t, c->ds_order, b0, batch, (long long)img, c->c[0],
-                         c->x32, c->t32);
-      CNNCHK(c, hipGetLastError());
-      rc = pack_input(c, c->x32, batch, h, w);
-      double loss = 0.0;
-      if (rc == RTM_CNN_OK) rc = loss_grad_dev(c, c->t32, batch, h, w, &loss);
+      rc = pack_input(c, c->ds_x, batch, h, w, c->ds_order, b0, c->ds_t);
+      if (rc == RTM_CNN_OK)
+        rc = loss_grad_dev(c, c->t32, batch, h, w, c->ds_sq + (size_t)nb * SQ_BLOCKS);
       if (rc == RTM_CNN_OK) rc = adam_dev(c, lr, 0.9f, 0.999f, 1e-8f);
       if (rc != RTM_CNN_OK) return rc;
-      sum += loss;
       ++nb;
     }
+    // the batches' losses are read once an epoch
+    CNNCHK(c, hipMemcpyAsync(part.data(), c->ds_sq, (size_t)nb * SQ_BLOCKS * sizeof(double),
+                             hipMemcpyDeviceToHost, c->stream));
+    CNNCHK(c, hipStreamSynchronize(c->stream));
+    double sum = 0.0;
+    for (int i = 0; i < nb; ++i) sum += loss_of(part.data() + (size_t)i * SQ_BLOCKS, (long long)batch * h * w);
     if (loss_per_epoch) loss_per_epoch[ep] = nb ? sum / nb : 0.0;
   }
   CNNCHK(c, hipStreamSynchronize(c->stream));
