@@ -926,18 +926,14 @@ int rtm_set_model(rtm_ctx* c, const float* v, const float* r1, const float* w, c
     for (int k = 0; k < nvel; ++k) nfd = std::max(nfd, index[k + 1] - index[k] - 1);
   }
   if (nfd > c->p.nfdmax) return fail(c, RTM_E_ARG, "table operator length %d > nfdmax %d", nfd, c->p.nfdmax);
-  const int CS = ((2 + nfd) + 3) & ~3;
+  const int CS = ((1 + nfd) + 3) & ~3;  // CoefRow
   std::vector<float> tab((size_t)nrow * CS, 0.f);
-  const double h1 = 1.0 + (double)c->p.hzx2_1;
   for (int k = 0; k < nrow; ++k) {
     int top = ls ? index[k] : 0;
     int M = ls ? index[k + 1] - index[k] - 1 : c->p.nfdmax;
     if (M > nfd) return fail(c, RTM_E_ARG, "bin %d has M=%d > nfdmax=%d", k, M, nfd);
     if (ls && (top < 0 || index[k + 1] > nc)) return fail(c, RTM_E_ARG, "index[%d] outside c[%d]", k, nc);
-    double c0d = 0.0;
-    if (M >= 0) c0d = h1 * (double)coef[top];  // (1.0+hzx2_1)*Dc[M_top] (kernel.cu:58)
-    memcpy(&tab[(size_t)k * CS], &c0d, sizeof(double));
-    for (int l = 1; l <= M; ++l) tab[(size_t)k * CS + 1 + l] = coef[top + l];
+    for (int l = 0; l <= M; ++l) tab[(size_t)k * CS + l] = coef[top + l];
   }
   int rc = RTM_OK;
   if (!c->d_ctab || c->ctab_n < tab.size()) {
@@ -960,6 +956,7 @@ int rtm_set_model(rtm_ctx* c, const float* v, const float* r1, const float* w, c
   c->win_ref.assign(c->p.max_shots, 0);
   c->win_nx.assign(c->p.max_shots, 0);
   c->win_fp.assign(2 * (size_t)c->p.max_shots, 0);
+  m.h1 = 1.0 + (double)c->p.hzx2_1;  // (1.0+hzx2_1)*Dc[M_top] (kernel.cu:58)
   m.hzx2_1 = c->p.hzx2_1; m.tao2 = c->p.tao2; m.h2 = c->p.h2;
   m.taoh = c->p.taoh; m.taoh2 = c->p.taoh2;
   c->nfd = nfd;

@@ -93,9 +93,14 @@ __device__ __forceinline__ void bst1s(Rsrc r, unsigned vo, unsigned so, float v)
   __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), r, (int)(vo + so), 0, RTM_STREAM_POLICY);
 }
 
+// Coefficient row [c_0 .. c_NFD | zeros] of a cell, CS floats.  Gathering the
+// rows of a wave's cells is what its loads cost most (up to 64 cache lines an
+// instruction): with c_0 as the table's float, promoted here, a row of
+// half-length 3 is one 16-byte gather (two when the row held (1 + hzx2_1) c_0
+// in double), of 7 two, of 11 three.
 template <int NFD>
 struct CoefRow {
-  static constexpr int CS = ((2 + NFD) + 3) & ~3;
+  static constexpr int CS = ((1 + NFD) + 3) & ~3;
   static constexpr int NR = CS / 4;
   float4 r[NR];
   __device__ __forceinline__ void load(const float* ctab, unsigned byte_off) {
@@ -107,11 +112,10 @@ struct CoefRow {
 #pragma unroll
     for (int i = 0; i < NR; ++i) r[i] = bld4(t, byte_off + 16u * i, 0);
   }
-  __device__ __forceinline__ double c0d() const {
-    return __hiloint2double(__float_as_int(r[0].y), __float_as_int(r[0].x));
-  }
-  // tap coefficient c_l, l >= 1 (float index 1 + l in the row)
-  __device__ __forceinline__ float c(int l) const { return compr(r[(1 + l) >> 2], (1 + l) & 3); }
+  // centre coefficient (1.0 + hzx2_1) * c_0 of kernel.cu:58 in double
+  __device__ __forceinline__ double c0d(double h1) const { return h1 * (double)r[0].x; }
+  // tap coefficient c_l, l >= 1
+  __device__ __forceinline__ float c(int l) const { return compr(r[l >> 2], l & 3); }
 };
 
 // Final combine of the two-way update.

@@ -17,8 +17,7 @@ struct Grid {
   long long fstride;
 };
 
-// Model operands.  ctab rows are [c0' as double | c_1 .. c_NFD | zero pad],
-// c0' = (1.0 + hzx2_1) * c_0 in double (the promotion of kernel.cu:58).
+// Model operands.  ctab rows are [c_0 .. c_NFD | zero pad] (CoefRow).
 struct Model {
   long long mstride;   // 0: one model for all shots; fstride: windows ShotGeo::win apart
   const float* v;
@@ -36,6 +35,7 @@ struct Model {
   const float* tp;
   long long tpstride;
   int cs, nrow;
+  double h1;           // 1.0 + hzx2_1: the centre coefficient is h1 * c_0 in double (kernel.cu:58)
   float hzx2_1, tao2, h2, taoh, taoh2;
 };
 

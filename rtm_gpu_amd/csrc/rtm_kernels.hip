@@ -569,8 +569,8 @@ static inline unsigned blocks_for(long long n, int per = 256, unsigned cap = 409
 
 // Neighbour-tap planes: for cell (z, c) of the padded layout (c the storage
 // column) and l = 1..nfd, the tap-l coefficient of the rows of (z-l, c),
-// (z+l, c), (z, c-l), (z, c+l) -- 0 off the grid.  A row holds [c0' (double) |
-// c_1 .. c_NFD | zeros], so tap l sits at float 1 + l of the row.
+// (z+l, c), (z, c-l), (z, c+l) -- 0 off the grid.  Tap l
+// sits at float l of a row.
 __global__ void k_tap_planes(Grid g, const unsigned* ko, const float* ctab, int nfd, float* tp) {
   const long long n = (long long)g.nz * g.pitch;
   for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
@@ -582,7 +582,7 @@ __global__ void k_tap_planes(Grid g, const unsigned* ko, const float* ctab, int 
       for (int d = 0; d < 4; ++d) {
         float val = 0.0f;
         if (zz[d] >= 0 && zz[d] < g.nz && cc[d] >= 0 && cc[d] < g.pitch)
-          val = ctab[ko[(long long)zz[d] * g.pitch + cc[d]] / 4u + 1 + l];
+          val = ctab[ko[(long long)zz[d] * g.pitch + cc[d]] / 4u + l];
         tp[(long long)(4 * (l - 1) + d) * g.fstride + i] = val;
       }
     }

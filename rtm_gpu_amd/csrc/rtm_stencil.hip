@@ -276,7 +276,7 @@ __device__ __forceinline__ void interior_body(const IntArgs& a, const unsigned b
 #pragma unroll
       for (int jj = 0; jj < 4; ++jj) {
         const float u = compr(qc, jj);
-        float w1 = (float)(cr[jj].c0d() * (double)u);
+        float w1 = (float)(cr[jj].c0d(m.h1) * (double)u);
         if (T::adjt) {  // each tap with the neighbour's coefficient: (L^T mu)
 #pragma unroll
           for (int l = 1; l <= NFD; ++l) {
@@ -588,7 +588,7 @@ __device__ __forceinline__ void frame_body(const FrameArgs& a, const unsigned bi
       wave_lds_sync();
       // (4) pre-blend two-way value T of (tt, x) (Add / BKAdd, kernel.cu:46-80, 339-380)
       const CoefRow<NFD>& crc = cr[j % 2];
-      float w1 = (float)(crc.c0d() * (double)u);
+      float w1 = (float)(crc.c0d(m.h1) * (double)u);
 #pragma unroll
       for (int l = 1; l <= NFD; ++l) {
         float s = q[(j + NB - l + U) % U] + q[(j + NB + l) % U];
@@ -598,7 +598,7 @@ __device__ __forceinline__ void frame_body(const FrameArgs& a, const unsigned bi
       }
       if (MODE == FR_ADJ) {  // (L^T mu) on interior cells, each tap with the neighbour's row
         const bool inner = tt >= N2 && tt < NZ - N2 && x >= N2 && x < NX - N2;
-        float w1t = (float)(crc.c0d() * (double)u);
+        float w1t = (float)(crc.c0d(m.h1) * (double)u);
 #pragma unroll
         for (int l = 1; l <= NFD; ++l) {
           const unsigned rz = rowm(tt);
@@ -873,7 +873,7 @@ __device__ __forceinline__ void frame_tb4_body(const FrameArgs& a, const int4 re
       for (int jj = 0; jj < 4; ++jj) {
         const CoefRow<NFD>& crc = cr[j % 2][jj];
         const float u = compr(qc, jj);
-        float w1 = (float)(crc.c0d() * (double)u);
+        float w1 = (float)(crc.c0d(m.h1) * (double)u);
 #pragma unroll
         for (int l = 1; l <= NFD; ++l) {
           float s = compr(q[(j + NB - l + U) % U], jj) + compr(q[(j + NB + l) % U], jj);

@@ -233,7 +233,7 @@ __global__ __launch_bounds__(512) void k_tile(const TileArgs a) {
   // tap sum of the cell at LDS position c (Add / BKAdd, kernel.cu:46-80,
   // 339-380); v(l), l = -NFD .. NFD: its column
   const auto taps = [&](const float* s, int c, const CoefRow<NFD>& cf, auto v) {
-    float w1 = (float)(cf.c0d() * (double)v(0));
+    float w1 = (float)(cf.c0d(m.h1) * (double)v(0));
 #pragma unroll
     for (int l = 1; l <= NFD; ++l) {
       float t = v(-l) + v(l);
@@ -248,7 +248,7 @@ __global__ __launch_bounds__(512) void k_tile(const TileArgs a) {
   const auto taps_t = [&](const float* s, int c, const CoefRow<NFD>& cf, unsigned o, auto v) {
     const float* tp = m.tp + (long long)sg.win * m.tpstride;
     const unsigned fb = (unsigned)g.fstride * 4u;
-    float w1 = (float)(cf.c0d() * (double)v(0));
+    float w1 = (float)(cf.c0d(m.h1) * (double)v(0));
 #pragma unroll
     for (int l = 1; l <= NFD; ++l) {
       const unsigned p = o + (unsigned)(4 * (l - 1)) * fb;
