@@ -69,7 +69,8 @@ def build_hip(verbose=True, force=True):
     out = os.path.join(LIB, "librtm_hip.so")
     # the longest half-lengths take longest to compile: first
     units = [(f"rtm_{f}.hip", f"{f}_{n}.o", [f"-DRTM_NFD={n}"])
-             for n in range(12, 0, -1) for f in ("stencil", "tile")]
+             for n in range(12, 0, -1) for f in ("stencil", "tile", "two")
+             if f != "two" or n <= 5]  # TWO_MAX_NFD
     units += [(f, f + ".o", []) for f in ("rtm_kernels.hip", "rtm_capi.hip", "rtm_cnn.hip")]
     units = [(os.path.join(CSRC, f), os.path.join(obj_dir, o), d) for f, o, d in units]
     deps = [os.path.join(CSRC, "rtm_kernels.h"), os.path.join(CSRC, "rtm_device.h"),

@@ -47,8 +47,9 @@ struct rtm_ctx {
   float *d_v = nullptr, *d_r1 = nullptr, *d_ctab = nullptr, *d_w = nullptr, *d_pm = nullptr;
   unsigned* d_ko = nullptr;
   size_t ctab_n = 0;
-  float* F[3] = {nullptr, nullptr, nullptr};
-  float* Q[3] = {nullptr, nullptr, nullptr};
+  // the fourth buffers: only for two steps per launch
+  float* F[4] = {nullptr, nullptr, nullptr, nullptr};
+  float* Q[4] = {nullptr, nullptr, nullptr, nullptr};
   float *SU = nullptr, *SQ = nullptr, *I1 = nullptr, *I2 = nullptr;
   float *d_data = nullptr, *d_rec = nullptr;
   ShotGeo* d_geo = nullptr;    // per shot of the batch
@@ -74,8 +75,9 @@ struct rtm_ctx {
   // host-side state
   std::vector<float> wav;
   int nshot = 0;
-  int f0 = 0, f1 = 1, f2 = 2, q0 = 0, q1 = 1, q2 = 2;
+  int f0 = 0, f1 = 1, f2 = 2, f3 = 3, q0 = 0, q1 = 1, q2 = 2, q3 = 3;
   int kf = -1, kb = -2;  // next forward / backward step; -1/-2 = not begun
+  int rings_for = -1;    // the rings of F[f2], F[f3] hold strips rings_for, rings_for - 1
   int img_pend = 0;      // backward steps whose image terms are still to be applied (0..2)
   // least-squares migration operators
   bool born = false;     // the forward pass is a Born pass (records hold dU)
@@ -99,6 +101,12 @@ struct rtm_ctx {
   bool model_ok = false, wav_ok = false, shots_ok = false, data_ok = false, save_strips = true;
   int zs = 32, nxt = 1;
   long long cells = 0;     // grid cells of the batch
+  int two_tuned = -1;      // rtm_autotune's choice: 1 two steps per launch, 0 one
+  int zs2[5] = {0};        // rows per wave of two steps by kind (0: default)
+  bool quads = false;      // every four consecutive shots share width and model window
+  float* d_cp = nullptr;   // coefficient planes (TwoArgs::cp) of the model windows
+  size_t cp_cap = 0;
+  bool cp_ok = false;      // they match the current windows
   bool march_set = false;  // the caller chose something of the marching kernels
   int tile_tuned = -1;     // rtm_autotune's choice for the batch: 1 k_tile, 0 the marching kernels
   int zs_epi[16] = {0};  // rows per wave per interior kernel kind (0: zs)
@@ -106,7 +114,7 @@ struct rtm_ctx {
   bool graph_on = false;
   hipGraph_t graph = nullptr;
   hipGraphExec_t gexec = nullptr;
-  int g_f[3] = {0, 1, 2}, g_q[3] = {0, 1, 2}, g_kf = 0, g_kb = 0;
+  int g_f[4] = {0, 1, 2, 3}, g_q[4] = {0, 1, 2, 3}, g_kf = 0, g_kb = 0;
   // timing
   int timing = 0;  // bit set of kernel kinds
   std::vector<EventPair> pending;
@@ -254,10 +262,20 @@ void fill_frame_args(rtm_ctx* c, FrameArgs& a) {
   a.data = c->d_data;
   a.st = c->st;
   a.save_strips = 0;
-  a.rf = nullptr;
-  a.rbps = 0;
+  a.rf[0] = a.rf[1] = nullptr;
+  a.rk[0] = a.rk[1] = 0;
+  a.nrf = a.rbps = 0;
   a.ua = a.ub = a.uc = nullptr;
   a.adjt = 0;
+}
+
+// Have a receiver or adjoint frame launch restore the strips of slot k into the
+// rings of field f as well.
+void carry_restore(rtm_ctx* c, FrameArgs& a, float* f, int k) {
+  a.rf[a.nrf] = f;
+  a.rk[a.nrf] = k;
+  a.nrf += 1;
+  a.rbps = strip_restore_blocks(c->g);
 }
 
 // ---- finite-value watch -------------------------------------------------------
@@ -307,11 +325,29 @@ int watch_read(rtm_ctx* c, const char* pass) {
 // frame runs, fuse_frame, frame_split) gets them, unless rtm_autotune has timed
 // the two for the batch's migration.
 constexpr long long kTileWork = 50000000;
+
+// Two steps per launch (k_two) for the forward and backward passes of a
+// migration: half-lengths up to 5, every four consecutive shots on one model
+// window.  Measured (k_two / marching / k_tile, migration of 351 x 1701 shots,
+// ms per 100 steps, not tuned): 8.7 M cells 16.6 / 17.0 / 15.3, 11.6 M 18.5 /
+// 20.6 / 19.3, 17.4 M 23.2 / 25.6 / 28.8, 34.7 M 41.6 / 46.2 / 56.4; of 200 x
+// 400 shots, 6.8 M cells 16.4 / 16.3 / 15.8, 10.1 M 17.6 / 20.1 / 24.1.
+constexpr long long kTwoCells = 10000000;
+bool two_possible(const rtm_ctx* c) {
+  return c->F[3] && c->Q[3] && c->nfd <= TWO_MAX_NFD && c->nshot >= TWO_SHOTS && c->quads &&
+         !c->p.fuse_frame && c->cp_ok;
+}
+bool use_two(const rtm_ctx* c) {
+  if (!two_possible(c) || c->tile_tuned == 1) return false;
+  if (c->two_tuned >= 0) return c->two_tuned != 0;
+  return !c->march_set && c->cells >= kTwoCells;
+}
+
 bool use_tile(const rtm_ctx* c, int pass) {
   if (c->march_set) return false;
-  const bool two = pass == TILE_BORN || pass == TILE_ADJ;
-  if (!two && c->tile_tuned >= 0) return c->tile_tuned != 0;
-  return c->cells * c->nfd <= (two ? 2 : 1) * kTileWork;
+  const bool both = pass == TILE_BORN || pass == TILE_ADJ;
+  if (!both && c->tile_tuned >= 0) return c->tile_tuned != 0;
+  return (both || !use_two(c)) && c->cells * c->nfd <= (both ? 2 : 1) * kTileWork;
 }
 hipError_t tile_step(rtm_ctx* c, int pass, const TileArgs& a) {
   return launch_tile(pass, c->nfd, a, c->nshot, c->cells, c->stream);
@@ -356,12 +392,111 @@ hipError_t launch_frame_split(rtm_ctx* c, int mode, FrameArgs f) {
   return launch_frame(mode, c->nfd, f, c->nshot, c->ntiles, c->stream);
 }
 
+// Rows per wave of k_two where the autotuner has not chosen: the height whose
+// blocks, two to a CU at a time, take the fewest rounds times iterations
+// (rows + 2 NFD).
+int zs2_for(const rtm_ctx* c, int kind) {
+  if (c->zs2[kind] > 0) return c->zs2[kind];
+  const int ql = 2 * c->nfd + 3, cols = 256 - 2 * ((c->nfd + 3) & ~3);
+  const long long per = (long long)((c->g.mnx + cols - 1) / cols) * ((c->nshot + TWO_SHOTS - 1) / TWO_SHOTS);
+  int best = 0;
+  long long cost = 0;
+  for (int m : {11, 8, 6, 4, 3, 2}) {
+    const int rows = m * ql - 2 * c->nfd;
+    const long long blocks = per * ((c->g.mnz + rows - 1) / rows);
+    const long long v = (blocks + 511) / 512 * (m * ql);
+    if (best == 0 || v < cost) { best = rows; cost = v; }
+  }
+  return best;
+}
+
+void fill_two_args(rtm_ctx* c, TwoArgs& a, int kind) {
+  a = TwoArgs{};
+  a.g = c->g;
+  a.m = c->m;
+  a.r = c->r;
+  a.geo = c->d_geo;
+  a.cp = c->d_cp;
+  a.cpstride = c->m.mstride ? (long long)(c->nfd + 2) * c->g.fstride : 0;
+  a.nt = c->p.nt;
+  a.zs = zs2_for(c, kind);
+  a.data = c->d_data;
+  a.su = c->SU; a.sq = c->SQ; a.i1 = c->I1; a.i2 = c->I2;
+  a.icompen = c->p.icompen;
+}
+
+// The coefficient planes of the batch's model windows, where two steps per
+// launch may use them.  Allocates: not inside a stream capture.
+int ensure_planes(rtm_ctx* c) {
+  c->quads = true;
+  for (int s = 0; s < c->nshot; ++s) {
+    const ShotGeo &a = c->geo[s / TWO_SHOTS * TWO_SHOTS], &b = c->geo[s];
+    c->quads = c->quads && a.nx == b.nx && a.win == b.win;
+  }
+  if (c->cp_ok || !c->F[3] || !c->Q[3] || c->nfd > TWO_MAX_NFD || !c->quads || c->nshot < TWO_SHOTS ||
+      c->capturing)
+    return RTM_OK;
+  int nwin = 1;
+  if (c->m.mstride)
+    for (int s = 0; s < c->nshot; ++s) nwin = std::max(nwin, c->geo[s].win + 1);
+  const size_t per = (size_t)(c->nfd + 2) * c->g.fstride;
+  if (c->cp_cap < per * nwin) {
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    dfree_t(c, &c->d_cp, c->cp_cap);
+    c->cp_cap = 0;
+    if (dalloc_t(c, &c->d_cp, per * nwin) != RTM_OK) return RTM_OK;  // one step per launch
+    c->cp_cap = per * nwin;
+  }
+  for (int w = 0; w < nwin; ++w)
+    if (!c->m.mstride || c->win_ref[w] > 0)
+      HIPCHK(c, launch_coef_planes(c->g, c->m.ko + (size_t)w * c->m.mstride,
+                                   c->m.pm + (size_t)w * c->m.mstride, c->m.ctab, c->nfd,
+                                   c->d_cp + (size_t)w * per, c->stream));
+  c->cp_ok = true;
+  return RTM_OK;
+}
+
+// The quantisation of the strips of step k - 1 (reduced-precision storage),
+// ahead of step k.
+int forward_before(rtm_ctx* c, int k) {
+  if (c->save_strips && c->st.fmt != RTM_STRIP_F32 && k >= 3)
+    HIPCHK(c, launch_strip_finish(c->g, c->st, c->d_geo, k - 1, c->nshot, c->stream));
+  return RTM_OK;
+}
+// The frame of forward step k (Add + Hybrid1/2/3, kernel.cu:46-208) from fields
+// u1, u0 into u2.
+FrameArgs forward_frame(rtm_ctx* c, int k, float wav, const float* u1, const float* u0, float* u2) {
+  FrameArgs f;
+  fill_frame_args(c, f);
+  f.u1 = u1; f.u0 = u0; f.u2 = u2;
+  f.wav = wav; f.k = k;
+  f.save_strips = c->save_strips ? 1 : 0;
+  return f;
+}
+// What follows forward step k once u(k) is complete in field u.
+int forward_after(rtm_ctx* c, int k, const float* u, bool record) {
+  if (c->save_strips && c->st.fmt != RTM_STRIP_F32 && k == c->p.nt - 1)
+    HIPCHK(c, launch_strip_finish(c->g, c->st, c->d_geo, k, c->nshot, c->stream));
+  if (c->save_strips && c->snap_slot[k] >= 0)  // checkpoint snapshot of u(k)
+    HIPCHK(c, launch_snap_save(c->g, u, c->sn, c->d_geo, c->snap_slot[k], c->nshot, c->stream));
+  if (record)  // receiver recording of u(k)
+    HIPCHK(c, launch_record(c->g, c->r, c->d_geo, u, c->d_rec, k, c->p.nt, c->nshot, c->stream));
+  if (watch_due(c, k, c->p.nt - 1)) return watch(c, u, k);
+  return RTM_OK;
+}
+float forward_wav(const rtm_ctx* c, int k) {  // kernel.cu:812-813
+  return (k < c->p.nt2) ? c->wav[k - 1] : 0.0f;
+}
+float backward_wav(const rtm_ctx* c, int k) {  // kernel.cu:889-890
+  return (k < c->p.nt2) ? c->wav[k + 1] : 0.0f;
+}
+
 // born: the caller runs a Born pass (born_step), whose scattered field a tile
 // launch advances together with the background.
 int forward_step(rtm_ctx* c, int k, bool born = false) {
-  const float wv = (k < c->p.nt2) ? c->wav[k - 1] : 0.0f;  // kernel.cu:812-813
-  const bool quant = c->save_strips && c->st.fmt != RTM_STRIP_F32;
-  if (quant && k >= 3) HIPCHK(c, launch_strip_finish(c->g, c->st, c->d_geo, k - 1, c->nshot, c->stream));
+  const float wv = forward_wav(c, k);
+  int rc = forward_before(c, k);
+  if (rc != RTM_OK) return rc;
   const bool tile = use_tile(c, born ? TILE_BORN : TILE_FWD);
   if (tile) {
     TileArgs a;
@@ -372,18 +507,14 @@ int forward_step(rtm_ctx* c, int k, bool born = false) {
     HIPCHK(c, tile_step(c, born ? TILE_BORN : TILE_FWD, a));
   } else {
     // Add (FP32 combine) or Add_Con (FP64 combine) (kernel.cu:46-114) on the
-    // interior, Add + Hybrid1/2/3 on the frame (kernel.cu:116-208)
+    // interior, the frame beside it
     const int epi = c->p.ilste ? EPI_FWD64 : EPI_FWD;
     IntArgs a;
     fill_int_args(c, a);
     a.u1 = c->F[c->f1]; a.u0 = c->F[c->f0]; a.u2 = c->F[c->f2];
     a.wav = wv; a.k = k;
     a.zs = zs_for(c, epi);
-    FrameArgs f;
-    fill_frame_args(c, f);
-    f.u1 = c->F[c->f1]; f.u0 = c->F[c->f0]; f.u2 = c->F[c->f2];
-    f.wav = wv; f.k = k;
-    f.save_strips = c->save_strips ? 1 : 0;
+    const FrameArgs f = forward_frame(c, k, wv, c->F[c->f1], c->F[c->f0], c->F[c->f2]);
     if (fused(c, epi, FR_FWD)) {
       Timed t(c, RTM_K_FWD_INTERIOR);  // the fused launch counts as the interior kind
       HIPCHK(c, launch_step(epi, FR_FWD, c->nfd, a, f, c->nshot, c->ntiles, c->stream));
@@ -396,17 +527,43 @@ int forward_step(rtm_ctx* c, int k, bool born = false) {
       HIPCHK(c, launch_frame_split(c, FR_FWD, f));
     }
   }
-  if (quant && k == c->p.nt - 1) HIPCHK(c, launch_strip_finish(c->g, c->st, c->d_geo, k, c->nshot, c->stream));
-  if (c->save_strips && c->snap_slot[k] >= 0)  // checkpoint snapshot of u(k)
-    HIPCHK(c, launch_snap_save(c->g, c->F[c->f2], c->sn, c->d_geo, c->snap_slot[k], c->nshot, c->stream));
-  if (c->p.record && !c->born && !tile)  // receiver recording of u(k)
-    HIPCHK(c, launch_record(c->g, c->r, c->d_geo, c->F[c->f2], c->d_rec, k, c->p.nt, c->nshot, c->stream));
-  if (watch_due(c, k, c->p.nt - 1)) {
-    int rc = watch(c, c->F[c->f2], k);
-    if (rc != RTM_OK) return rc;
-  }
+  rc = forward_after(c, k, c->F[c->f2], c->p.record && !c->born && !tile);
   int t = c->f0; c->f0 = c->f1; c->f1 = c->f2; c->f2 = t;  // Deliver (kernel.cu:820)
-  return RTM_OK;
+  return rc;
+}
+
+// Forward steps k and k + 1: the frame of u(k), the interiors of both, the
+// frame of u(k+1).
+int forward_two(rtm_ctx* c, int k) {
+  float *u1 = c->F[c->f1], *u0 = c->F[c->f0], *ua = c->F[c->f2], *ub = c->F[c->f3];
+  const float wa = forward_wav(c, k), wb = forward_wav(c, k + 1);
+  int rc = forward_before(c, k);
+  if (rc != RTM_OK) return rc;
+  {
+    Timed t(c, RTM_K_FWD_FRAME);
+    HIPCHK(c, launch_frame_split(c, FR_FWD, forward_frame(c, k, wa, u1, u0, ua)));
+  }
+  {
+    const int kind = c->p.ilste ? TWO_FWD64 : TWO_FWD;
+    TwoArgs a;
+    fill_two_args(c, a, kind);
+    a.u1 = u1; a.u0 = u0; a.ua = ua; a.ub = ub;
+    a.wa = wa; a.wb = wb; a.k = k;
+    Timed t(c, RTM_K_FWD_INTERIOR);  // both steps
+    HIPCHK(c, launch_two(kind, c->nfd, a, c->nshot, c->stream));
+  }
+  rc = forward_before(c, k + 1);
+  if (rc != RTM_OK) return rc;
+  {
+    Timed t(c, RTM_K_FWD_FRAME);
+    HIPCHK(c, launch_frame_split(c, FR_FWD, forward_frame(c, k + 1, wb, ua, u1, ub)));
+  }
+  const bool record = c->p.record && !c->born;
+  rc = forward_after(c, k, ua, record);
+  if (rc == RTM_OK) rc = forward_after(c, k + 1, ub, record);
+  const int o0 = c->f0, o1 = c->f1;
+  c->f0 = c->f2; c->f1 = c->f3; c->f2 = o1; c->f3 = o0;
+  return rc;
 }
 
 // The end of backward step k: the finite-value watch and the rotation of the
@@ -422,6 +579,15 @@ int backward_done(rtm_ctx* c, int k, bool image) {
   return RTM_OK;
 }
 
+// The frame of receiver step k (BKAdd + BKHybrid1/2, kernel.cu:339-487).
+FrameArgs receiver_frame(rtm_ctx* c, int k, const float* u1, const float* u0, float* u2) {
+  FrameArgs f;
+  fill_frame_args(c, f);
+  f.u1 = u1; f.u0 = u0; f.u2 = u2;
+  f.wav = 0.f; f.k = k;
+  return f;
+}
+
 // Backward step k.  The image terms of a step (Rel_*, kernel.cu:489-517) are
 // applied by the receiver step of every third step for the three steps at once
 // (k_interior<EPI_RCV>): the rotating buffers still hold u(k+2), u(k+1), u(k)
@@ -429,8 +595,8 @@ int backward_done(rtm_ctx* c, int k, bool image) {
 // u(k) is in its buffer by then too.  flush: the caller may look at the images
 // after this step, so the terms of every step so far are applied.
 int backward_step(rtm_ctx* c, int k, bool flush) {
-  const float wv = (k < c->p.nt2) ? c->wav[k + 1] : 0.0f;  // kernel.cu:889-890
-  const bool image = flush || c->img_pend == 2;
+  const float wv = backward_wav(c, k);
+  const bool image = flush || c->img_pend >= 2;
   const int ercv = image ? EPI_RCV : EPI_RCV0;
   if (use_tile(c, TILE_MIG) && c->snap_slot[k] < 0) {
     TileArgs a;
@@ -462,6 +628,7 @@ int backward_step(rtm_ctx* c, int k, bool flush) {
   if (c->snap_slot[k] >= 0)  // checkpoint: the reconstructed u(k) is replaced by its snapshot
     HIPCHK(c, launch_snap_restore(c->g, c->F[c->f2], c->sn, c->d_geo, c->snap_slot[k], c->nshot, c->stream));
   { int t = c->f0; c->f0 = c->f1; c->f1 = c->f2; c->f2 = t; }  // Deliver_EFF (kernel.cu:903)
+  c->rings_for = -1;
   {  // BKAdd (kernel.cu:913) + Rel_* (kernel.cu:923-930) on the interior, BKAdd
      // on the frame + BKHybrid1/2 (kernel.cu:913-920)
     IntArgs a;
@@ -471,14 +638,8 @@ int backward_step(rtm_ctx* c, int k, bool flush) {
     a.nimg = c->img_pend + 1;
     a.wav = 0.f; a.k = k;
     a.zs = zs_for(c, ercv);
-    FrameArgs f;
-    fill_frame_args(c, f);
-    f.u1 = c->Q[c->q1]; f.u0 = c->Q[c->q0]; f.u2 = c->Q[c->q2];
-    f.wav = 0.f; f.k = k;
-    if (restore_in_frame) {  // u(k) is F[f1] after the rotation
-      f.rf = c->F[c->f1];
-      f.rbps = strip_restore_blocks(c->g);
-    }
+    FrameArgs f = receiver_frame(c, k, c->Q[c->q1], c->Q[c->q0], c->Q[c->q2]);
+    if (restore_in_frame) carry_restore(c, f, c->F[c->f1], k);  // u(k) after the rotation
     const int kind = image ? RTM_K_RCVI_INTERIOR : RTM_K_RCV_INTERIOR;
     if (fused(c, ercv, FR_RCV)) {
       Timed t(c, kind);  // the fused launch counts as the interior kind
@@ -493,6 +654,77 @@ int backward_step(rtm_ctx* c, int k, bool flush) {
     }
   }
   return backward_done(c, k, image);
+}
+
+// Backward steps k and k - 1 in one launch per field, neither a checkpoint (a
+// snapshot would replace u(k) before its next use): left >= 2 steps of the call
+// from step k on.
+bool backward_two_ok(const rtm_ctx* c, int k, int left) {
+  return left >= 2 && k >= 1 && use_two(c) && c->snap_slot[k] < 0 && c->snap_slot[k - 1] < 0;
+}
+
+// The strips of both steps are in the rings of the buffers that receive u(k) and
+// u(k-1) before the reconstruction; the last frame launch of the steps before
+// carried them where it knew of these (rings_for), into rings that nothing read
+// any more.  The receiver frame of step k comes before the two interiors, that
+// of step k-1 after.  Image terms as in backward_step, up to four steps at once:
+// the buffers hold u(k+2) .. u(k-1), and q(k+2), q(k+1) are the receiver
+// launch's own operands.
+int backward_two(rtm_ctx* c, int k, bool flush, int left) {
+  float *ua = c->F[c->f2], *ub = c->F[c->f3];
+  if (c->rings_for != k) {
+    Timed t(c, RTM_K_STRIP_RESTORE);
+    HIPCHK(c, launch_strip_restore(c->g, ua, c->st, c->d_geo, k, c->nshot, c->stream));
+    HIPCHK(c, launch_strip_restore(c->g, ub, c->st, c->d_geo, k - 1, c->nshot, c->stream));
+  }
+  {
+    TwoArgs a;
+    fill_two_args(c, a, TWO_SRC);
+    a.u1 = c->F[c->f1]; a.u0 = c->F[c->f0]; a.ua = ua; a.ub = ub;
+    a.wa = backward_wav(c, k); a.wb = backward_wav(c, k - 1); a.k = k;
+    Timed t(c, RTM_K_SRC_INTERIOR);  // both steps
+    HIPCHK(c, launch_two(TWO_SRC, c->nfd, a, c->nshot, c->stream));
+  }
+  float *q1 = c->Q[c->q1], *q0 = c->Q[c->q0], *qa = c->Q[c->q2], *qb = c->Q[c->q3];
+  {
+    Timed t(c, RTM_K_RCV_FRAME);
+    HIPCHK(c, launch_frame_split(c, FR_RCV, receiver_frame(c, k, q1, q0, qa)));
+  }
+  const bool image = flush || c->img_pend >= 1;
+  {
+    const int kind = image ? TWO_RCV : TWO_RCV0;
+    TwoArgs a;
+    fill_two_args(c, a, kind);
+    a.u1 = q1; a.u0 = q0; a.ua = qa; a.ub = qb;
+    a.k = k;
+    a.us[0] = c->F[c->f0]; a.us[1] = c->F[c->f1]; a.us[2] = ua; a.us[3] = ub;
+    a.nimg = c->img_pend + 2;
+    Timed t(c, image ? RTM_K_RCVI_INTERIOR : RTM_K_RCV_INTERIOR);  // both steps
+    HIPCHK(c, launch_two(kind, c->nfd, a, c->nshot, c->stream));
+  }
+  // u(k-1), u(k), u(k+1), u(k+2) from newest to oldest, and q alike
+  const int o0 = c->f0, o1 = c->f1, p0 = c->q0, p1 = c->q1;
+  c->f0 = c->f2; c->f1 = c->f3; c->f2 = o1; c->f3 = o0;
+  {
+    FrameArgs f = receiver_frame(c, k - 1, qa, q1, qb);
+    c->rings_for = -1;
+    if (backward_two_ok(c, k - 2, left - 2)) {
+      carry_restore(c, f, c->F[c->f2], k - 2);
+      carry_restore(c, f, c->F[c->f3], k - 3);
+      c->rings_for = k - 2;
+    }
+    Timed t(c, RTM_K_RCV_FRAME);
+    HIPCHK(c, launch_frame_split(c, FR_RCV, f));
+  }
+  c->q0 = c->q2; c->q1 = c->q3; c->q2 = p1; c->q3 = p0;
+  c->img_pend = image ? 0 : c->img_pend + 2;
+  for (int i = 0; i < 2; ++i) {  // u and q of steps k, k-1
+    if (!watch_due(c, k - i, 0)) continue;
+    int rc = watch(c, i ? ub : ua, k - i);
+    if (rc == RTM_OK) rc = watch(c, i ? qb : qa, k - i);
+    if (rc != RTM_OK) return rc;
+  }
+  return RTM_OK;
 }
 
 // Born step k: the background step, then the scattered field from dU(k-1),
@@ -566,8 +798,7 @@ int adjoint_update(rtm_ctx* c, int k, bool image, float* restore = nullptr) {
     a.wav = 0.f; a.k = k;
     a.adjt = c->p.ilste == 0;
     if (restore) {
-      a.rf = restore;
-      a.rbps = strip_restore_blocks(c->g);
+      carry_restore(c, a, restore, k);
     }
     Timed t(c, RTM_K_ADJ_FRAME);
     HIPCHK(c, launch_frame(FR_ADJ, c->nfd, a, c->nshot, c->ntiles, c->stream));
@@ -578,7 +809,7 @@ int adjoint_update(rtm_ctx* c, int k, bool image, float* restore = nullptr) {
 // Adjoint step k: the background u(k) reconstructed as in backward_step,
 // then the adjoint update with imaging.
 int adjoint_step(rtm_ctx* c, int k) {
-  const float wv = (k < c->p.nt2) ? c->wav[k + 1] : 0.0f;
+  const float wv = backward_wav(c, k);
   if (use_tile(c, TILE_ADJ) && c->snap_slot[k] < 0) {
     TileArgs a;
     fill_tile_args(c, a, wv, k);
@@ -666,7 +897,7 @@ int upload_geometry(rtm_ctx* c) {
   HIPCHK(c, hipMemcpyAsync(c->d_geo, c->geo.data(), ns * sizeof(ShotGeo), hipMemcpyHostToDevice, c->stream));
   int rc = upload_frame_records(c);
   if (rc != RTM_OK) return rc;
-  if (ns != c->nshot) c->tile_tuned = -1;  // tuned for another batch
+  if (ns != c->nshot) c->tile_tuned = c->two_tuned = -1;  // tuned for another batch
   c->cells = 0;
   for (const ShotGeo& q : c->geo) c->cells += (long long)c->g.nz * q.nx;
   c->nshot = ns;
@@ -873,10 +1104,25 @@ int rtm_create(const rtm_params* p, rtm_ctx** out) {
     rtm_destroy(c);
     return code;
   }
+  // The fourth buffers of two steps per launch, last, and only where they leave
+  // an eighth of the card for what is allocated later: without them every
+  // launch takes one step.
+  size_t mem_free = 0, mem_all = 0;
+  if ((long long)p->max_shots * g.nz * g.nx >= kTwoCells && p->max_shots >= TWO_SHOTS &&
+      hipMemGetInfo(&mem_free, &mem_all) == hipSuccess &&
+      mem_free >= 2 * fb * sizeof(float) + mem_all / 8) {
+    if (dalloc_t(c, &c->F[3], fb) == RTM_OK && dalloc_t(c, &c->Q[3], fb) != RTM_OK)
+      dfree_t(c, &c->F[3], fb);
+    c->err.clear();
+  }
   // Zero everything once so guard columns hold finite values.
   for (int i = 0; i < 3; ++i) {
     HIPCHK(c, launch_fill(c->F[i], (long long)fb, 0.f, c->stream));
     HIPCHK(c, launch_fill(c->Q[i], (long long)fb, 0.f, c->stream));
+  }
+  if (c->F[3]) {
+    HIPCHK(c, launch_fill(c->F[3], (long long)fb, 0.f, c->stream));
+    HIPCHK(c, launch_fill(c->Q[3], (long long)fb, 0.f, c->stream));
   }
   HIPCHK(c, launch_fill(c->SU, (long long)fb, 0.f, c->stream));
   HIPCHK(c, launch_fill(c->SQ, (long long)fb, 0.f, c->stream));
@@ -960,7 +1206,7 @@ int rtm_set_model(rtm_ctx* c, const float* v, const float* r1, const float* w, c
   m.hzx2_1 = c->p.hzx2_1; m.tao2 = c->p.tao2; m.h2 = c->p.h2;
   m.taoh = c->p.taoh; m.taoh2 = c->p.taoh2;
   c->nfd = nfd;
-  c->tp_ok = false;
+  c->tp_ok = c->cp_ok = false;
   drop_graph(c);
   c->model_ok = true;
   return RTM_OK;
@@ -1015,7 +1261,7 @@ int rtm_set_shot_geometry(rtm_ctx* c, int nshot, const rtm_shot_geom* sg) {
   c->win_ref.assign(c->p.max_shots, 0);
   c->win_nx.assign(c->p.max_shots, 0);
   c->win_fp.assign(2 * (size_t)c->p.max_shots, 0);
-  c->tp_ok = false;
+  c->tp_ok = c->cp_ok = false;
   return upload_geometry(c);
 }
 
@@ -1075,7 +1321,7 @@ int rtm_set_shot_model(rtm_ctx* c, int shot, const float* v, const float* r1) {
     c->win_nx[w] = nx;
     c->win_fp[2 * w] = fp[0];
     c->win_fp[2 * w + 1] = fp[1];
-    c->tp_ok = false;
+    c->tp_ok = c->cp_ok = false;
     }
   c->win_ref[w] += 1;
   c->geo[shot].win = w;
@@ -1129,7 +1375,9 @@ int rtm_forward_begin(rtm_ctx* c, int save_strips) {
   if (c->m.mstride != 0)
     for (int s = 0; s < c->nshot; ++s)
       if (!c->shot_model[s]) return fail(c, RTM_E_STATE, "shot %d has no model window", s);
-  c->f0 = 0; c->f1 = 1; c->f2 = 2;
+  int prc = ensure_planes(c);
+  if (prc != RTM_OK) return prc;
+  c->f0 = 0; c->f1 = 1; c->f2 = 2; c->f3 = 3;
   c->save_strips = save_strips != 0;
   c->born = false;
   const float spike = (float)((double)c->wav[0] / 2.0);  // f(0.0,f0)/2.0 (kernel.cu:803)
@@ -1158,9 +1406,12 @@ int rtm_forward_begin(rtm_ctx* c, int save_strips) {
 int rtm_forward_advance(rtm_ctx* c, int nsteps) {
   if (!c) return RTM_E_ARG;
   if (c->kf < 2) return fail(c, RTM_E_STATE, "rtm_forward_begin first");
-  for (int i = 0; i < nsteps && c->kf < c->p.nt; ++i, ++c->kf) {
-    int rc = forward_step(c, c->kf);
+  for (int left = std::min(nsteps, c->p.nt - c->kf); left > 0;) {
+    const int n = left >= 2 && use_two(c) ? 2 : 1;
+    int rc = n == 2 ? forward_two(c, c->kf) : forward_step(c, c->kf);
     if (rc != RTM_OK) return rc;
+    c->kf += n;
+    left -= n;
   }
   return watch_read(c, "forward");
 }
@@ -1172,7 +1423,7 @@ int rtm_backward_begin(rtm_ctx* c) {
   if (!c->data_ok) return fail(c, RTM_E_STATE, "rtm_set_gathers first");
   // DBW1 = u(NT-2), DBW0 = u(NT-1) (kernel.cu:822-825): swap roles of f0/f1.
   std::swap(c->f0, c->f1);
-  c->q0 = 0; c->q1 = 1; c->q2 = 2;
+  c->q0 = 0; c->q1 = 1; c->q2 = 2; c->q3 = 3;
   c->adj = false;
   const float spike = (float)((double)c->wav[0] / 2.0);
   int wrc = watch_reset(c);
@@ -1183,15 +1434,19 @@ int rtm_backward_begin(rtm_ctx* c) {
   HIPCHK(c, launch_strip_restore(c->g, c->F[c->f1], c->st, c->d_geo, c->p.nt - 2, c->nshot, c->stream));
   c->kb = c->p.nt - 3;
   c->img_pend = 0;
+  c->rings_for = -1;
   return RTM_OK;
 }
 
 int rtm_backward_advance(rtm_ctx* c, int nsteps) {
   if (!c) return RTM_E_ARG;
   if (c->kb < -1) return fail(c, RTM_E_STATE, "rtm_backward_begin first");
-  for (int i = 0; i < nsteps && c->kb >= 0; ++i, --c->kb) {
-    int rc = backward_step(c, c->kb, i == nsteps - 1 || c->kb == 0);
+  for (int left = std::min(nsteps, c->kb + 1); left > 0;) {
+    const int n = backward_two_ok(c, c->kb, left) ? 2 : 1;
+    int rc = n == 2 ? backward_two(c, c->kb, left == 2, left) : backward_step(c, c->kb, left == 1);
     if (rc != RTM_OK) return rc;
+    c->kb -= n;
+    left -= n;
   }
   return watch_read(c, "backward");
 }
@@ -1495,6 +1750,8 @@ int rtm_migrate(rtm_ctx* c) {
   if (!c->model_ok || !c->wav_ok || !c->shots_ok || !c->data_ok)
     return fail(c, RTM_E_STATE, "model, wavelet, shots and gathers must be set");
   if (!c->gexec) {
+    int prc = ensure_planes(c);
+    if (prc != RTM_OK) return prc;
     // Capture the whole launch sequence once; the host-side buffer rotation
     // is deterministic, so the replay leaves the same state as the capture.
     const int saved_timing = c->timing;
@@ -1517,14 +1774,14 @@ int rtm_migrate(rtm_ctx* c) {
       drop_graph(c);
       return fail(c, RTM_E_HIP, "hipGraphInstantiate: %s", hipGetErrorString(e));
     }
-    c->g_f[0] = c->f0; c->g_f[1] = c->f1; c->g_f[2] = c->f2;
-    c->g_q[0] = c->q0; c->g_q[1] = c->q1; c->g_q[2] = c->q2;
+    c->g_f[0] = c->f0; c->g_f[1] = c->f1; c->g_f[2] = c->f2; c->g_f[3] = c->f3;
+    c->g_q[0] = c->q0; c->g_q[1] = c->q1; c->g_q[2] = c->q2; c->g_q[3] = c->q3;
     c->g_kf = c->kf;
     c->g_kb = c->kb;
   }
   HIPCHK(c, hipGraphLaunch(c->gexec, c->stream));
-  c->f0 = c->g_f[0]; c->f1 = c->g_f[1]; c->f2 = c->g_f[2];
-  c->q0 = c->g_q[0]; c->q1 = c->g_q[1]; c->q2 = c->g_q[2];
+  c->f0 = c->g_f[0]; c->f1 = c->g_f[1]; c->f2 = c->g_f[2]; c->f3 = c->g_f[3];
+  c->q0 = c->g_q[0]; c->q1 = c->g_q[1]; c->q2 = c->g_q[2]; c->q3 = c->g_q[3];
   c->kf = c->g_kf;
   c->kb = c->g_kb;
   c->save_strips = true;
@@ -1607,6 +1864,7 @@ int rtm_autotune(rtm_ctx* c, int nsteps, int* zseg) {
     if (c->zs_epi[kinds[ki]] <= 0) c->zs_epi[kinds[ki]] = 32;
   const int nt = c->p.nt;
   int kf = 2, kb = nt - 3;
+  int two_choice = 0;  // two steps per launch
   auto pairs = [&](int n) -> int {
     for (int i = 0; i < n; ++i) {
       int r = forward_step(c, kf);
@@ -1662,6 +1920,67 @@ int rtm_autotune(rtm_ctx* c, int nsteps, int* zseg) {
       c->zs_epi[kinds[ki]] = kMult[bi] * interior_queue_rows(kinds[ki], c->nfd);
     }
   }
+  auto fours = [&](bool on) -> int {  // four steps each way, one imaging cycle of k_two
+    c->two_tuned = on ? 1 : 0;
+    if (kf + 3 >= nt) kf = 2;
+    if (kb < 4) kb = nt - 3;
+    if (on) c->img_pend = 0;
+    int r = RTM_OK;
+    for (int i = 0; i < 4 && r == RTM_OK; i += on ? 2 : 1) {
+      r = on ? forward_two(c, kf + i) : forward_step(c, kf + i);
+      if (r != RTM_OK) return r;
+      if (!on) r = backward_step(c, kb - i, false);
+      else if (backward_two_ok(c, kb - i, 2)) r = backward_two(c, kb - i, false, 2);
+    }
+    kf += 4;
+    kb -= 4;
+    return r;
+  };
+  // Two steps per launch: their heights, then against one step per launch, on
+  // the time of the interiors of four steps each way.
+  c->two_tuned = 0;
+  if (rc == RTM_OK && two_possible(c) && nt >= 12) {
+    static const int kMult2[] = {3, 4, 6, 8, 11};
+    constexpr int kN2 = 5;
+    const int tk[4] = {RTM_K_FWD_INTERIOR, RTM_K_SRC_INTERIOR, RTM_K_RCV_INTERIOR, RTM_K_RCVI_INTERIOR};
+    const int zk[4] = {c->p.ilste ? TWO_FWD64 : TWO_FWD, TWO_SRC, TWO_RCV0, TWO_RCV};
+    unsigned mask = 0;
+    for (int k : tk) mask |= 1u << k;
+    const int ql = 2 * c->nfd + 3;
+    double tot[kN2][4] = {}, one = 0.0;
+    for (int round = 0; round < kRounds && rc == RTM_OK; ++round)
+      for (int i = 0; i <= kN2 && rc == RTM_OK; ++i) {
+        const int ci = (round & 1) ? kN2 - i : i;  // kN2: one step per launch
+        const bool on = ci < kN2;
+        if (on)
+          for (int k : zk) c->zs2[k] = kMult2[ci] * ql - 2 * c->nfd;
+        c->timing = 0;
+        rc = fours(on);
+        c->timing = (int)mask;
+        for (int k : tk) { c->t_ms[k] = 0.0; c->t_n[k] = 0; }
+        if (rc == RTM_OK) rc = fours(on);
+        if (rc == RTM_OK && !on) rc = fours(on);
+        if (rc == RTM_OK && !on) rc = fours(on);
+        if (rc == RTM_OK) rc = drain_timing(c);
+        for (int w = 0; w < 4; ++w) {
+          if (on) tot[ci][w] += c->t_ms[tk[w]];
+          else one += c->t_ms[tk[w]] / 3.0;  // three cycles of four: whole imaging cycles of three
+        }
+      }
+    double best = 0.0;
+    for (int w = 0; w < 4; ++w) {
+      int bi = 0;
+      for (int i = 1; i < kN2; ++i)
+        if (tot[i][w] < tot[bi][w]) bi = i;
+      c->zs2[zk[w]] = kMult2[bi] * ql - 2 * c->nfd;
+      best += tot[bi][w];
+    }
+    c->two_tuned = 0;
+    c->img_pend = 0;
+    if (rc == RTM_OK && best < one) two_choice = 1;
+    if (kf >= nt) kf = 2;
+    if (kb < 0) kb = nt - 3;
+  }
   // Frame record runs, timed on both frame kernels of the step pair: the top
   // and bottom bands in runs of n2, n2/2 or n2/3 rows (with float4 records:
   // their k_frame ends), then the side bands in runs of the default, half or a
@@ -1710,31 +2029,36 @@ int rtm_autotune(rtm_ctx* c, int nsteps, int* zseg) {
       c->p.frame_split = tot[1] < tot[0] ? 1 : 0;
     }
   }
-  // The tuned marching kernels against whole steps by k_tile, on the time of
-  // everything a step pair launches over whole imaging cycles.
-  // Batches far from the line between them (use_tile) are not timed.
-  const long long work = c->cells * c->nfd;
-  if (rc == RTM_OK && !c->p.fuse_frame && work <= 4 * kTileWork) {
+  // The tuned kernels against whole steps by k_tile, on the time of everything
+  // that twelve steps each way launch (whole imaging cycles).  Batches far from
+  // the line between them (use_tile) are not timed.
+  int tile_choice = 0;
+  if (rc == RTM_OK && !c->p.fuse_frame && c->cells * c->nfd <= 4 * kTileWork) {
     double tot[2] = {0.0, 0.0};
     for (int round = 0; round < kRounds && rc == RTM_OK; ++round)
       for (int i = 0; i < 2 && rc == RTM_OK; ++i) {
         const int on = (round & 1) ? 1 - i : i;
+        const bool two = !on && two_choice;
         c->tile_tuned = on;
         c->timing = 0;
-        rc = pairs(3);
+        rc = two ? fours(true) : pairs(3);
         c->timing = -1;
         for (int k = 0; k < RTM_K_NKINDS; ++k) { c->t_ms[k] = 0.0; c->t_n[k] = 0; }
-        if (rc == RTM_OK) rc = pairs(3 * ((per + 2) / 3));
+        for (int n = 0; n < 3 && rc == RTM_OK; ++n) rc = two ? fours(true) : pairs(4);
         if (rc == RTM_OK) rc = drain_timing(c);
         for (int k = 0; k < RTM_K_NKINDS; ++k) tot[on] += c->t_ms[k];
+        c->two_tuned = 0;
       }
-    c->tile_tuned = tot[1] < tot[0] ? 1 : 0;
+    tile_choice = tot[1] < tot[0] ? 1 : 0;
   }
+  c->tile_tuned = tile_choice;
   c->timing = saved_timing;
   c->check_every = saved_check;
   for (int i = 0; i < RTM_K_NKINDS; ++i) { c->t_ms[i] = 0.0; c->t_n[i] = 0; }
   c->zs_epi[EPI_BORN] = c->zs_epi[EPI_BORN64] = c->zs_epi[EPI_ADJ] = c->zs_epi[EPI_RCV];
   c->zs = c->zs_epi[fwd];
+  c->two_tuned = two_choice;
+  c->rings_for = -1;
   c->kf = -1;
   c->kb = -2;
   drop_graph(c);

@@ -129,12 +129,54 @@ struct FrameArgs {
   int save_strips;
   const float *ua, *ub, *uc;  // Born background fields (as in IntArgs)
   int adjt;            // adjoint with per-cell rows: interior cells take the transposed stencil
-  // receiver and adjoint frames only: rbps > 0 appends rbps blocks per shot
-  // that restore the strips of slot k into the rings of field rf
-  // (k_strip_restore's work)
-  float* rf;
-  int rbps;
+  // receiver and adjoint frames only: rbps > 0 appends rbps blocks per shot and
+  // field that restore the strips of slot rk[i] into the rings of field rf[i],
+  // i < nrf (k_strip_restore's work)
+  float* rf[2];
+  int rk[2];
+  int nrf, rbps;
 };
+
+// Two time steps of the interior in one launch (rtm_two.hip): the forward
+// field (FP32 / FP64 combine), the reconstruction, the receiver field without
+// and with imaging.
+enum { TWO_FWD = 0, TWO_FWD64 = 1, TWO_SRC = 2, TWO_RCV0 = 3, TWO_RCV = 4 };
+#define TWO_MAX_NFD 5  // longest half-length with these kernels
+constexpr int TWO_SHOTS = 4;  // shots of a block, on one model window
+
+struct TwoArgs {
+  Grid g;
+  Model m;
+  Rcv r;
+  const ShotGeo* geo;
+  // coefficient planes of a model window: c_0 .. c_NFD, P; fstride apart, a
+  // window's nfd + 2 planes cpstride apart (0: one window)
+  const float* cp;
+  long long cpstride;
+  const float *u1, *u0;  // newer and older field
+  float *ua, *ub;        // first and second step; frame cells of ua are read
+  float wa, wb;          // source amplitudes of the two steps
+  int k, nt;             // TWO_RCV*: steps k and k - 1
+  int nxt, zs, nshot;    // column tiles, rows per wave, shots
+  const float* data;     // [shot][nt][n]
+  // TWO_RCV: source field of steps k+2 .. k-1, sums and images
+  const float* us[4];
+  float *su, *sq, *i1, *i2;
+  int icompen;
+  int nimg;              // steps k+nimg-2 .. k-1 imaged (2..4)
+};
+template <int NFD>
+struct TwoOps {
+  static hipError_t two(int kind, dim3 grid, const TwoArgs& a, hipStream_t s);
+};
+// Rows per wave nearest to the request (rows + 2 nfd iterations, a multiple of
+// the register queue).
+int two_rows(int nfd, int rows);
+hipError_t launch_two(int kind, int nfd_inst, TwoArgs a, int nshot, hipStream_t s);
+// Coefficient planes (TwoArgs::cp) of one window from its coefficient offsets
+// and P.
+hipError_t launch_coef_planes(const Grid& g, const unsigned* ko, const float* pm, const float* ctab,
+                              int nfd, float* cp, hipStream_t s);
 
 // A whole time step in one launch, one cell per thread (rtm_tile.hip).
 enum { TILE_FWD = 0, TILE_MIG = 1, TILE_BORN = 2, TILE_ADJ = 3 };

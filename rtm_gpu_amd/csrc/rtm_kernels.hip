@@ -423,6 +423,39 @@ hipError_t launch_interior(int epi, int nfd, IntArgs a, int nshot, hipStream_t s
 #undef CASE
 }
 
+int two_rows(int nfd, int rows) {
+  const int ql = 2 * nfd + 3;
+  return std::max(1, (rows + 2 * nfd + ql / 2) / ql) * ql - 2 * nfd;
+}
+
+hipError_t launch_two(int kind, int nfd, TwoArgs a, int nshot, hipStream_t s) {
+  const int cols = 256 - 2 * ((nfd + 3) & ~3);  // columns written by a wave
+  a.zs = two_rows(nfd, a.zs);
+  a.nxt = (a.g.mnx + cols - 1) / cols;
+  a.nshot = nshot;
+  const int nseg = (a.g.mnz + a.zs - 1) / a.zs;
+  const dim3 grid(a.nxt * nseg * ((nshot + TWO_SHOTS - 1) / TWO_SHOTS));
+  switch (nfd) {
+    case 1: return TwoOps<1>::two(kind, grid, a, s);
+    case 2: return TwoOps<2>::two(kind, grid, a, s);
+    case 3: return TwoOps<3>::two(kind, grid, a, s);
+    case 4: return TwoOps<4>::two(kind, grid, a, s);
+    case 5: return TwoOps<5>::two(kind, grid, a, s);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+// A thread per cell of the padded layout.
+__global__ void k_coef_planes(long long n, long long fstride, const unsigned* ko, const float* pm,
+                              const float* ctab, int nfd, float* cp) {
+  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
+       i += (long long)gridDim.x * blockDim.x) {
+    const float* row = ctab + ko[i] / 4u;
+    for (int l = 0; l <= nfd; ++l) cp[(long long)l * fstride + i] = row[l];
+    cp[(long long)(nfd + 1) * fstride + i] = pm[i];
+  }
+}
+
 int frame_segment_rows(int nfd) {
   const int nb = nfd > 2 ? nfd : 2;
   return 2 * (nb + nfd + 1 + 2) - 2;  // two register-queue cycles per side run
@@ -501,7 +534,7 @@ hipError_t launch_frame(int mode, int nfd, FrameArgs a, int nshot, int nrec, hip
   a.nrec = nrec;
   if (mode != FR_RCV && mode != FR_ADJ) a.rbps = 0;
   // one wave per (region run, shot) record, then the restore blocks
-  dim3 grid((nrec + 3) / 4 + (a.rbps > 0 ? a.rbps * nshot : 0));
+  dim3 grid((nrec + 3) / 4 + (a.rbps > 0 ? a.rbps * nshot * a.nrf : 0));
 #define CASE(N) case N: return StencilOps<N>::frame(mode, grid, a, s);
   switch (nfd) {
     RTM_NFD_CASES(CASE)
@@ -592,6 +625,12 @@ hipError_t launch_tap_planes(const Grid& g, const unsigned* ko, const float* cta
                              float* tp, hipStream_t s) {
   hipLaunchKernelGGL(k_tap_planes, dim3(blocks_for((long long)g.nz * g.pitch, 256, 2048)),
                      dim3(256), 0, s, g, ko, ctab, nfd, tp);
+  return hipGetLastError();
+}
+hipError_t launch_coef_planes(const Grid& g, const unsigned* ko, const float* pm, const float* ctab,
+                              int nfd, float* cp, hipStream_t s) {
+  hipLaunchKernelGGL(k_coef_planes, dim3(blocks_for(g.fstride, 256, 2048)), dim3(256), 0, s, g.fstride,
+                     g.fstride, ko, pm, ctab, nfd, cp);
   return hipGetLastError();
 }
 hipError_t launch_flag_reset(unsigned* flag, hipStream_t s) {

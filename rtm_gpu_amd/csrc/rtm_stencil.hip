@@ -967,7 +967,10 @@ __global__ __launch_bounds__(256) void k_frame(const FrameArgs a) {
   if ((MODE == FR_RCV || MODE == FR_ADJ) && a.rbps > 0) {
     const unsigned nfb = ((unsigned)a.nrec + 3u) >> 2;
     if (blockIdx.x >= nfb) {
-      strip_restore_body(a.g, a.rf, a.st, a.geo, a.k, blockIdx.x - nfb, (unsigned)a.rbps);
+      const unsigned b = blockIdx.x - nfb, per = (unsigned)(a.rbps * a.nshot);
+      const bool second = b >= per;  // of two fields
+      strip_restore_body(a.g, second ? a.rf[1] : a.rf[0], a.st, a.geo, second ? a.rk[1] : a.rk[0],
+                         second ? b - per : b, (unsigned)a.rbps);
       return;
     }
   }

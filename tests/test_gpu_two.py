@@ -1,0 +1,93 @@
+"""Two time steps per launch (the kernel of large batches) against one step per
+launch, bit for bit.  The marching kernels it is compared with equal the oracle
+in test_gpu_parity.py."""
+import numpy as np
+import pytest
+
+from cases import build_case, hip_context
+
+pytestmark = pytest.mark.gpu
+
+# 41 shots (one past a block's four) of 440 x 618 cells: the batches of 10 M
+# cells and more that take two steps per launch by default
+SHOTS, NZ, NX, N2 = 41, 400, 578, 20
+
+
+def passes(ctx, seis, calls):
+    """Forward and backward pass in calls of the given lengths, with the fields
+    after some of them."""
+    from rtm_gpu_amd import hip
+    nt, last = ctx.p.nt, ctx.nshot - 1
+    ctx.set_gathers(seis)
+    got = []
+    ctx.forward_begin()
+    for n in (*calls, nt):
+        ctx.forward_advance(n)
+        got += [ctx.field(w, shot=last) for w in (hip.FIELD_U, hip.FIELD_U_PREV)]
+    got += [ctx.strip(s, nt // 2) for s in (0, last)]
+    ctx.backward_begin()
+    for n in (*calls, nt):
+        ctx.backward_advance(n)
+        got += [ctx.field(w, shot=last) for w in (hip.FIELD_Q, hip.FIELD_I1)]
+        # the reconstructed field is the interior and the strip rings around it
+        got.append(ctx.field(hip.FIELD_U, shot=last)[N2:-N2, N2:-N2])
+    got += [ctx.field(w, shot=s) for s in (0, 3, last)
+            for w in (hip.FIELD_I1, hip.FIELD_I2, hip.FIELD_Q)]
+    if ctx.p.record:
+        got.append(ctx.records())
+    return got
+
+
+@pytest.mark.parametrize("nfd,ilste,icompen,snap_every,strips", [
+    (1, 1, 1, 0, 0), (2, 1, 0, 0, 0), (3, 1, 1, 0, 1), (4, 1, 1, 9, 0), (4, 0, 1, 0, 2),
+    (5, 1, 1, 0, 0)])
+def test_two_steps_per_launch(nfd, ilste, icompen, snap_every, strips):
+    case = build_case(name="two", mod_nz=NZ, mod_nx=NX, n2=N2, nfdmax=nfd, nfdmin=min(2, nfd),
+                      ilste=ilste, icompen=icompen, nt=44, nshot=SHOTS, depth_step=7.0, src_x1=90,
+                      tao=0.0008, ds=3)
+    rng = np.random.default_rng(nfd)
+    seis = (0.01 * rng.standard_normal((SHOTS, case["cfg"]["n"], case["cfg"]["nt"]))).astype(np.float32)
+    out = []
+    for zseg in (0, 16):  # 16 rows per wave: one step per launch
+        ctx = hip_context(case, nshot=SHOTS, record=1, zseg=zseg, snap_every=snap_every,
+                          strip_format=strips)
+        # calls of 1, 5, 2 and 7 steps: single steps between pairs, one to four
+        # pending image terms at their ends
+        out.append(passes(ctx, seis, (1, 5, 2, 7)))
+        ctx.close()
+    for i, (a, b) in enumerate(zip(*out)):
+        assert np.array_equal(a, b), i
+
+
+@pytest.mark.parametrize("group", [4, 2])
+def test_two_steps_with_shared_windows(group):
+    """A ragged batch on two model windows of different widths, given to runs of
+    four shots (a block's shots share their window) and of two (they do not, and
+    the batch takes one step per launch)."""
+    from rtm_gpu_amd import hip
+    case = build_case(name="twowin", mod_nz=NZ, mod_nx=NX, n2=N2, nt=30, nshot=1)
+    cfg, m = case["cfg"], case["model"]
+    keys = ("nz", "nx", "n2", "nfdmax", "nt", "nt2", "ilste", "icompen", "s_l", "s_r", "s_z",
+            "ds", "n", "tao2", "h2", "taoh", "taoh2", "hzx2_1")
+    n, widths = 44, (cfg["nx"], cfg["nx"] - 37)
+    geoms = []
+    for s in range(n):
+        nx = widths[s // group % 2]
+        w = nx - 2 * N2
+        geoms.append(dict(nx=nx, r_u=N2 + s, r_x=N2 + 10 * s % w, s_l=N2, s_r=N2 + w - 1, n=w, x_img=0))
+    rng = np.random.default_rng(3)
+    seis = (0.01 * rng.standard_normal((n, cfg["n"], cfg["nt"]))).astype(np.float32)
+    out = []
+    for zseg in (0, 16):
+        ctx = hip.Context(**{k: cfg[k] for k in keys}, max_shots=n, zseg=zseg)
+        ctx.set_model(m["v"], m["r1"], m["w"], m["c"], m["index"], m["nvel"], m["vmin"], m["dv"])
+        ctx.set_wavelet(m["wav"])
+        ctx.set_shot_geometry(geoms)
+        for s, g in enumerate(geoms):
+            v = np.ascontiguousarray(m["v"][:, :g["nx"]] if s // group % 2 == 0 else m["v"][:, -g["nx"]:])
+            r1 = np.ascontiguousarray(m["r1"][:, :g["nx"]] if s // group % 2 == 0 else m["r1"][:, -g["nx"]:])
+            ctx.set_shot_model(s, v, r1)
+        out.append(passes(ctx, seis, (3, 8)))
+        ctx.close()
+    for i, (a, b) in enumerate(zip(*out)):
+        assert np.array_equal(a, b), i
