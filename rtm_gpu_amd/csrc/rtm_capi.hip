@@ -397,7 +397,7 @@ hipError_t launch_frame_split(rtm_ctx* c, int mode, FrameArgs f) {
 // (rows + 2 NFD).
 int zs2_for(const rtm_ctx* c, int kind) {
   if (c->zs2[kind] > 0) return c->zs2[kind];
-  const int ql = 2 * c->nfd + 3, cols = 256 - 2 * ((c->nfd + 3) & ~3);
+  const int ql = 2 * c->nfd + 3, cols = two_cols(c->g, c->nfd, c->nshot);
   const long long per = (long long)((c->g.mnx + cols - 1) / cols) * ((c->nshot + TWO_SHOTS - 1) / TWO_SHOTS);
   int best = 0;
   long long cost = 0;

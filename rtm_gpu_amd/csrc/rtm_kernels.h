@@ -157,7 +157,8 @@ struct TwoArgs {
   float *ua, *ub;        // first and second step; frame cells of ua are read
   float wa, wb;          // source amplitudes of the two steps
   int k, nt;             // TWO_RCV*: steps k and k - 1
-  int nxt, zs, nshot;    // column tiles, rows per wave, shots
+  int cols, nxt, zs;     // columns written by a wave, column tiles, rows per wave
+  int nshot;             // shots
   const float* data;     // [shot][nt][n]
   // TWO_RCV: source field of steps k+2 .. k-1, sums and images
   const float* us[4];
@@ -169,6 +170,9 @@ template <int NFD>
 struct TwoOps {
   static hipError_t two(int kind, dim3 grid, const TwoArgs& a, hipStream_t s);
 };
+// Columns written by a wave: 224, whole 128-byte lines, or all that the halo
+// leaves.
+int two_cols(const Grid& g, int nfd, int nshot);
 // Rows per wave nearest to the request (rows + 2 nfd iterations, a multiple of
 // the register queue).
 int two_rows(int nfd, int rows);

@@ -423,15 +423,27 @@ hipError_t launch_interior(int epi, int nfd, IntArgs a, int nshot, hipStream_t s
 #undef CASE
 }
 
+// Interior rows start on a 128-byte line.  Tiles of 224 columns write whole
+// lines; others write the lines at their sides in two parts, from two blocks,
+// and each part is a masked write to memory.  Where the four buffers of a field
+// exceed the 256 MB last-level cache that costs more than the tiles it saves:
+// two forward steps of 128 shots of 351 x 1701 302 us (224 columns), 306 (240),
+// 336 (248), with the images of four 1143, 1209, 1307; 32 shots forward 87, 90,
+// 97; but 16 shots 57, 58, 51.
+int two_cols(const Grid& g, int nfd, int nshot) {
+  const long long bytes = 4ll * nshot * g.fstride * (long long)sizeof(float);
+  return bytes > (256ll << 20) ? 224 : 256 - 2 * ((nfd + 3) & ~3);
+}
+
 int two_rows(int nfd, int rows) {
   const int ql = 2 * nfd + 3;
   return std::max(1, (rows + 2 * nfd + ql / 2) / ql) * ql - 2 * nfd;
 }
 
 hipError_t launch_two(int kind, int nfd, TwoArgs a, int nshot, hipStream_t s) {
-  const int cols = 256 - 2 * ((nfd + 3) & ~3);  // columns written by a wave
   a.zs = two_rows(nfd, a.zs);
-  a.nxt = (a.g.mnx + cols - 1) / cols;
+  a.cols = two_cols(a.g, nfd, nshot);
+  a.nxt = (a.g.mnx + a.cols - 1) / a.cols;
   a.nshot = nshot;
   const int nseg = (a.g.mnz + a.zs - 1) / a.zs;
   const dim3 grid(a.nxt * nseg * ((nshot + TWO_SHOTS - 1) / TWO_SHOTS));

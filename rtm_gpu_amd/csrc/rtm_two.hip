@@ -8,7 +8,7 @@
 // t+1 first, the reconstruction restores its strips first.
 //
 // A wave marches 256 columns of one shot, computes u(t+1) on all of them and
-// u(t+2) on the 256 - 2H in the middle, NFD rows behind: row z of u(t+1) comes
+// u(t+2) on the a.cols <= 256 - 2H in the middle, NFD rows behind: row z of u(t+1) comes
 // from a register queue of u(t) rows and goes to a second queue, row z - NFD of
 // u(t+2) comes from that one, with the oldest row of the first queue as its
 // older operand.  A segment of zs rows takes zs + 2 NFD iterations.
@@ -21,10 +21,10 @@
 // wave and step, the L1 is what such a kernel waits for: two steps took 401 us
 // at half-length 3 (128 reverse-VSP shots), one step per launch 2 x 212.
 // Measured on 128 shots of 351 x 1701, us for two steps (two launches of
-// k_interior): forward 318 (424) at half-length 3, 328 (478) at 4, 353 (532) at
-// 5; the receiver field, four steps with their images, 1632 (1790).  318 us are 4.3 TB/s of the pass's reads and writes
-// (halo rows and columns included), against 5.4 TB/s of a streaming kernel: the
-// four waves wait for each other at every row.  At half-length 6 the 256
+// k_interior): forward 298 (424) at half-length 3, 354 (532) at 5; the receiver
+// field, four steps with their images, 1434 (1790).  298 us are 4.5 TB/s of the
+// pass's reads and writes (halo rows and columns included), against 5.4 TB/s of
+// a streaming kernel: the four waves wait for each other at every row.  At half-length 6 the 256
 // registers of two waves per SIMD spill (469 against 510 us; 137 against 106 on
 // 24 shots): not built.
 //
@@ -58,6 +58,7 @@ __global__ __launch_bounds__(256, 2) void k_two(const TwoArgs a) {
 
   const Grid& g = a.g;
   const Model& m = a.m;
+  const int WC = a.cols, M = (256 - WC) / 2;  // M >= H, a multiple of 4
   const int lane = threadIdx.x & 63;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   // blocks shot group fastest, as k_interior's
@@ -71,10 +72,10 @@ __global__ __launch_bounds__(256, 2) void k_two(const TwoArgs a) {
   const int n2 = g.n2, zhi = g.nz - n2, zlast = g.nz - 1;
   const int zs = n2 + zseg * a.zs, ze = min(zs + a.zs, zhi);  // rows written
   const int cend = sg.nx - n2;
-  const int cb = n2 + xt * (256 - 2 * H);  // first column written
+  const int cb = n2 + xt * WC;  // first column written
   if (zs >= zhi || cb >= cend) return;     // the same for the block's shots
-  const int cw = min(cb + 256 - 2 * H, cend);  // first column not written
-  const int c0 = cb - H + lane * 4;
+  const int cw = min(cb + WC, cend);  // first column not written
+  const int c0 = cb - M + lane * 4;
   const int clast = sg.nx - ((sg.nx - n2) & 3);
   const unsigned vcol = (unsigned)(g.x0 + min(c0, clast)) * 4u;
   bool colok[4], wr[4], full = live, any_out = false;
@@ -85,14 +86,14 @@ __global__ __launch_bounds__(256, 2) void k_two(const TwoArgs a) {
     full = full && wr[jj];
     any_out = any_out || !colok[jj];
   }
-  const bool edge_tile = cend < cb + 256 - 2 * H;  // the wave holds the interior's right edge
+  const bool edge_tile = cend < cb + WC;  // the wave holds the interior's right edge
   const unsigned vst = (unsigned)(g.x0 + c0) * 4u, vst4 = full ? vst : kDrop;
   const unsigned vout = any_out ? vcol : kDrop;  // lanes with cells of u(t+1) off the interior
   unsigned vhal = kDrop;
   int hpos = H / 4 + lane;
-  if (lane < H / 4) { vhal = (unsigned)max(g.x0 + cb - 2 * H + 4 * lane, 0) * 4u; hpos = lane; }
+  if (lane < H / 4) { vhal = (unsigned)max(g.x0 + cb - M - H + 4 * lane, 0) * 4u; hpos = lane; }
   else if (lane < 2 * (H / 4)) {
-    vhal = (unsigned)(g.x0 + min(cb - H + 256 + 4 * (lane - H / 4), clast)) * 4u;
+    vhal = (unsigned)(g.x0 + min(cb - M + 256 + 4 * (lane - H / 4), clast)) * 4u;
     hpos = 64 + lane;
   }
 
