@@ -44,7 +44,7 @@ struct rtm_ctx {
   size_t bytes = 0;
   std::vector<void*> allocs;
   // device buffers
-  float *d_v = nullptr, *d_r1 = nullptr, *d_ctab = nullptr, *d_w = nullptr, *d_pm = nullptr;
+  float *d_v = nullptr, *d_r1 = nullptr, *d_ctab = nullptr, *d_w = nullptr, *d_pm = nullptr, *d_fs = nullptr;
   unsigned* d_ko = nullptr;
   size_t ctab_n = 0;
   // the fourth buffers: only for two steps per launch
@@ -58,11 +58,13 @@ struct rtm_ctx {
   int4* d_tiles = nullptr;     // frame (tile, shot) records of the batch
   int ntiles = 0, tile_cap = 0;  // FRAME_ALL records; capacity of d_tiles
   int nsplit = 0, nvec = 0;      // FRAME_SCALAR and FRAME_VEC records after them
+  int qrows = 0;  // rows per block of k_frame_quad; 0: quad_rows
   int fseg_tb = 0, fseg_side = 0;  // rows per frame record: top/bottom bands, side bands
   // model windows of a ragged batch (allocated on first use): slot w holds
   // one distinct window; shots whose windows are equal share a slot
   float *d_mv = nullptr, *d_mr1 = nullptr, *d_mpm = nullptr;
   unsigned* d_mko = nullptr;
+  float* d_mfs = nullptr;
   std::vector<char> shot_model;
   std::vector<int> win_ref;                 // shots using each slot
   std::vector<int> win_nx;                  // width of each slot's window
@@ -375,12 +377,39 @@ static bool fused(const rtm_ctx* c, int epi, int mode) {
   return c->p.fuse_frame != 0 && step_fusable(epi, mode);
 }
 
-// The frame of a forward or receiver step: split between k_frame (the band
+long long plane_stride(const rtm_ctx* c) {
+  return c->m.mstride ? (long long)two_planes(c->nfd) * c->g.fstride : 0;
+}
+
+// Rows per block of k_frame_quad where the autotuner has not chosen: of the
+// band's whole height, half and a third of it the one whose blocks, two to a
+// CU at a time, take the fewest rounds times iterations (rows + 2).
+int quad_rows(const rtm_ctx* c) {
+  if (c->qrows > 0) return c->qrows;
+  const int n2 = c->g.n2, per = 2 * frame4_windows(c->g, c->g.nx) * ((c->nshot + TWO_SHOTS - 1) / TWO_SHOTS);
+  int best = n2, cost = 0;
+  for (int m = 1; m <= 3; ++m) {
+    const int rows = (n2 + m - 1) / m, v = (per * ((n2 + rows - 1) / rows) + 511) / 512 * (rows + 2);
+    if (m == 1 || v < cost) { best = rows; cost = v; }
+  }
+  return best;
+}
+
+// The frame of a forward or receiver step of a batch that takes two steps per
+// launch: one launch of k_frame_quad.  Of others: split between k_frame (the band
 // ends at the corners, the side bands) and k_frame4 (the edge cells of the top
 // and bottom bands) when rtm_params.frame_split asks for it and the batch has
 // float4 records, else k_frame on the FRAME_ALL records.  The two launches
 // write disjoint cells.
 hipError_t launch_frame_split(rtm_ctx* c, int mode, FrameArgs f) {
+  if (use_two(c) && c->nvec > 0) {
+    f.recs = c->d_tiles + c->ntiles;
+    f.cp = c->d_cp;
+    f.cpstride = plane_stride(c);
+    f.qwin = frame4_windows(c->g, c->g.nx);
+    f.qrows = quad_rows(c);
+    return launch_frame_quad(mode, c->nfd, f, c->nshot, c->nsplit, c->stream);
+  }
   if (c->p.frame_split && c->nvec > 0 && frame4_supported(c->nfd)) {
     FrameArgs fs = f;
     fs.recs = c->d_tiles + c->ntiles;
@@ -417,7 +446,7 @@ void fill_two_args(rtm_ctx* c, TwoArgs& a, int kind) {
   a.r = c->r;
   a.geo = c->d_geo;
   a.cp = c->d_cp;
-  a.cpstride = c->m.mstride ? (long long)(c->nfd + 2) * c->g.fstride : 0;
+  a.cpstride = plane_stride(c);
   a.nt = c->p.nt;
   a.zs = zs2_for(c, kind);
   a.data = c->d_data;
@@ -439,7 +468,7 @@ int ensure_planes(rtm_ctx* c) {
   int nwin = 1;
   if (c->m.mstride)
     for (int s = 0; s < c->nshot; ++s) nwin = std::max(nwin, c->geo[s].win + 1);
-  const size_t per = (size_t)(c->nfd + 2) * c->g.fstride;
+  const size_t per = (size_t)two_planes(c->nfd) * c->g.fstride;
   if (c->cp_cap < per * nwin) {
     HIPCHK(c, hipStreamSynchronize(c->stream));
     dfree_t(c, &c->d_cp, c->cp_cap);
@@ -449,9 +478,7 @@ int ensure_planes(rtm_ctx* c) {
   }
   for (int w = 0; w < nwin; ++w)
     if (!c->m.mstride || c->win_ref[w] > 0)
-      HIPCHK(c, launch_coef_planes(c->g, c->m.ko + (size_t)w * c->m.mstride,
-                                   c->m.pm + (size_t)w * c->m.mstride, c->m.ctab, c->nfd,
-                                   c->d_cp + (size_t)w * per, c->stream));
+      HIPCHK(c, launch_coef_planes(c->g, c->m, w, c->nfd, c->d_cp + (size_t)w * per, c->stream));
   c->cp_ok = true;
   return RTM_OK;
 }
@@ -870,9 +897,12 @@ int upload_frame_records(rtm_ctx* c) {
   int count[3] = {0, 0, 0};
   for (int kind = FRAME_ALL; kind <= FRAME_VEC; ++kind) {
     std::vector<std::vector<int4>> per(ns);
+    // beside float4 records only the corners are left of the bands: few waves,
+    // in runs short enough not to outlast the others
+    const int seg_tb = kind == FRAME_SCALAR ? std::min(c->fseg_tb, (c->g.n2 + 2) / 3) : c->fseg_tb;
     size_t most = 0;
     for (int s = 0; s < ns; ++s) {
-      build_tiles(c->g, c->geo[s].nx, s, c->fseg_tb, c->fseg_side, kind, per[s]);
+      build_tiles(c->g, c->geo[s].nx, s, seg_tb, c->fseg_side, kind, per[s]);
       most = std::max(most, per[s].size());
     }
     const size_t at = rec.size();
@@ -915,7 +945,7 @@ int upload_geometry(rtm_ctx* c) {
 // velocity bin's coefficient row (kernel.cu:55-56: FP32 quotient, double +
 // 0.5, truncation, clamped to the table).  Guard columns repeat the edge.
 int upload_model_window(rtm_ctx* c, int nx, const float* v, const float* r1, float* dv_, float* dr_,
-                        float* dp_, unsigned* dk_) {
+                        float* dp_, unsigned* dk_, float* df_) {
   const Grid& g = c->g;
   std::vector<float> pv((size_t)g.fstride, 0.f), pr((size_t)g.fstride, 0.f), pp((size_t)g.fstride);
   std::vector<unsigned> pk((size_t)g.fstride);
@@ -941,6 +971,7 @@ int upload_model_window(rtm_ctx* c, int nx, const float* v, const float* r1, flo
   HIPCHK(c, hipMemcpyAsync(dr_, pr.data(), b, hipMemcpyHostToDevice, c->stream));
   HIPCHK(c, hipMemcpyAsync(dp_, pp.data(), b, hipMemcpyHostToDevice, c->stream));
   HIPCHK(c, hipMemcpyAsync(dk_, pk.data(), b, hipMemcpyHostToDevice, c->stream));
+  HIPCHK(c, launch_frame_lat(g, nx, dv_, c->p.taoh2, df_, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   return RTM_OK;
 }
@@ -1030,6 +1061,7 @@ int rtm_create(const rtm_params* p, rtm_ctx** out) {
   if (rc == RTM_OK) rc = dalloc_t(c, &c->I2, fb);
   if (rc == RTM_OK) rc = dalloc_t(c, &c->d_v, (size_t)g.fstride);
   if (rc == RTM_OK) rc = dalloc_t(c, &c->d_r1, (size_t)g.fstride);
+  if (rc == RTM_OK) rc = dalloc_t(c, &c->d_fs, (size_t)g.fstride);
   if (rc == RTM_OK) rc = dalloc_t(c, &c->d_pm, (size_t)g.fstride);
   if (rc == RTM_OK) rc = dalloc_t(c, &c->d_ko, (size_t)g.fstride);
   if (rc == RTM_OK) rc = dalloc_t(c, &c->d_w, (size_t)g.n2 + 1);
@@ -1081,11 +1113,15 @@ int rtm_create(const rtm_params* p, rtm_ctx** out) {
   }
   {
     c->fseg_tb = g.n2;
-    c->fseg_side = frame_segment_rows(g.nfd);
+    const int seg0 = frame_segment_rows(g.nfd);
+    // 100 steps each way of 48 Taylor shots (half-length 10): 19.4 ms in side
+    // runs of 44 rows, 18.1 of 16, 18.4 of 8; 128 reverse-VSP shots 84.5, 83.3,
+    // 83.5
+    c->fseg_side = std::min(seg0, 16);
     // the most records one shot of any width takes at the shortest runs the
     // autotuner tries, over the three lists (a narrower shot may take more
     // than the widest: its side bands may not pack into one wave)
-    const int min_tb = std::max(1, (g.n2 + 2) / 3), min_side = std::max(1, c->fseg_side / 4);
+    const int min_tb = std::max(1, (g.n2 + 2) / 3), min_side = std::max(1, seg0 / 4);
     int most = 0;
     for (int nx = 1; nx <= g.nx; ++nx) {
       int tot = 0;
@@ -1189,13 +1225,13 @@ int rtm_set_model(rtm_ctx* c, const float* v, const float* r1, const float* w, c
   }
   HIPCHK(c, hipMemcpyAsync(c->d_ctab, tab.data(), tab.size() * sizeof(float), hipMemcpyHostToDevice, c->stream));
   c->tab_vmin = vmin; c->tab_dv = dv; c->tab_nrow = nrow; c->tab_cs = CS; c->tab_ls = ls;
-  rc = upload_model_window(c, g.nx, v, r1, c->d_v, c->d_r1, c->d_pm, c->d_ko);
+  rc = upload_model_window(c, g.nx, v, r1, c->d_v, c->d_r1, c->d_pm, c->d_ko, c->d_fs);
   if (rc != RTM_OK) return rc;
   HIPCHK(c, hipMemcpyAsync(c->d_w, w, (g.n2 + 1) * sizeof(float), hipMemcpyHostToDevice, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   Model& m = c->m;
   m.mstride = 0;  // one model for every shot until rtm_set_shot_model
-  m.v = c->d_v; m.r1 = c->d_r1; m.ctab = c->d_ctab; m.w = c->d_w;
+  m.v = c->d_v; m.r1 = c->d_r1; m.fs = c->d_fs; m.ctab = c->d_ctab; m.w = c->d_w;
   m.pm = c->d_pm; m.ko = c->d_ko;
   m.cs = CS; m.nrow = nrow;
   c->shot_model.assign(c->p.max_shots, 0);
@@ -1293,6 +1329,7 @@ int rtm_set_shot_model(rtm_ctx* c, int shot, const float* v, const float* r1) {
     if (rc == RTM_OK) rc = dalloc_t(c, &c->d_mr1, n);
     if (rc == RTM_OK) rc = dalloc_t(c, &c->d_mpm, n);
     if (rc == RTM_OK) rc = dalloc_t(c, &c->d_mko, n);
+    if (rc == RTM_OK) rc = dalloc_t(c, &c->d_mfs, n);
     if (rc != RTM_OK) return rc;
   }
   if (c->win_ref.size() != (size_t)c->p.max_shots) {
@@ -1313,7 +1350,7 @@ int rtm_set_shot_model(rtm_ctx* c, int shot, const float* v, const float* r1) {
       if (c->win_ref[i] == 0) w = i;
     if (w < 0) return fail(c, RTM_E_STATE, "no free model window slot");
     const size_t o = (size_t)w * g.fstride;
-    int rc = upload_model_window(c, nx, v, r1, c->d_mv + o, c->d_mr1 + o, c->d_mpm + o, c->d_mko + o);
+    int rc = upload_model_window(c, nx, v, r1, c->d_mv + o, c->d_mr1 + o, c->d_mpm + o, c->d_mko + o, c->d_mfs + o);
     if (rc != RTM_OK) {
       c->shot_model[shot] = 0;
       return rc;
@@ -1329,7 +1366,7 @@ int rtm_set_shot_model(rtm_ctx* c, int shot, const float* v, const float* r1) {
   HIPCHK(c, hipStreamSynchronize(c->stream));
   Model& m = c->m;
   m.mstride = g.fstride;
-  m.v = c->d_mv; m.r1 = c->d_mr1; m.pm = c->d_mpm; m.ko = c->d_mko;
+  m.v = c->d_mv; m.r1 = c->d_mr1; m.fs = c->d_mfs; m.pm = c->d_mpm; m.ko = c->d_mko;
   c->shot_model[shot] = 1;
   drop_graph(c);
   return RTM_OK;
@@ -1981,10 +2018,11 @@ int rtm_autotune(rtm_ctx* c, int nsteps, int* zseg) {
     if (kf >= nt) kf = 2;
     if (kb < 0) kb = nt - 3;
   }
-  // Frame record runs, timed on both frame kernels of the step pair: the top
-  // and bottom bands in runs of n2, n2/2 or n2/3 rows (with float4 records:
-  // their k_frame ends), then the side bands in runs of the default, half or a
-  // quarter of it.  Shorter runs put more waves in flight at the cost of
+  // Frame record runs, timed on both frame kernels of the step pair (of four
+  // steps each way where those take two per launch): the top and bottom bands in
+  // runs of n2, n2/2 or n2/3 rows (with float4 records: their k_frame ends; the
+  // blocks of k_frame_quad), then the side bands in runs of the default, half or
+  // a quarter of it.  Shorter runs put more waves in flight at the cost of
   // recomputing two pre-blend rows per run.
   if (rc == RTM_OK) {
     const Grid& g = c->g;
@@ -1996,6 +2034,18 @@ int rtm_autotune(rtm_ctx* c, int nsteps, int* zseg) {
     const unsigned fmask =
         (fused(c, fwd, FR_FWD) ? 1u << RTM_K_FWD_INTERIOR : 1u << RTM_K_FWD_FRAME) |
         (fused(c, EPI_RCV0, FR_RCV) ? 1u << RTM_K_RCV_INTERIOR : 1u << RTM_K_RCV_FRAME);
+    const bool quad = two_choice && c->nvec > 0;
+    auto measure_frames = [&](double* ms) -> int {
+      if (!quad) return measure(fmask, ms);
+      c->timing = 0;
+      int r = fours(true);
+      c->timing = (int)fmask;
+      for (int k = 0; k < RTM_K_NKINDS; ++k) { c->t_ms[k] = 0.0; c->t_n[k] = 0; }
+      if (r == RTM_OK) r = fours(true);
+      if (r == RTM_OK) r = drain_timing(c);
+      *ms = c->t_ms[RTM_K_FWD_FRAME] + c->t_ms[RTM_K_RCV_FRAME];
+      return r;
+    };
     for (int which = 0; which < 2 && rc == RTM_OK; ++which) {
       int& run = which == 0 ? c->fseg_tb : c->fseg_side;
       double tot[3] = {0.0, 0.0, 0.0};
@@ -2003,20 +2053,28 @@ int rtm_autotune(rtm_ctx* c, int nsteps, int* zseg) {
         for (int i = 0; i < 3 && rc == RTM_OK; ++i) {
           const int ci = (round & 1) ? 2 - i : i;
           run = cand[which][ci];
+          if (which == 0) c->qrows = run;
           rc = upload_frame_records(c);
           double ms = 0.0;
-          if (rc == RTM_OK) rc = measure(fmask, &ms);
+          if (rc == RTM_OK) rc = measure_frames(&ms);
           tot[ci] += ms;
         }
       int bi = 0;
       for (int i = 1; i < 3; ++i)
         if (tot[i] < tot[bi]) bi = i;
       run = cand[which][bi];
+      if (which == 0) c->qrows = run;
     }
     if (rc == RTM_OK) rc = upload_frame_records(c);
+    c->two_tuned = 0;
+    if (quad) {
+      c->img_pend = 0;
+      if (kf >= nt) kf = 2;
+      if (kb < 0) kb = nt - 3;
+    }
     // the frame split on and off (the four-column launch pays only when the
     // batch fills the GPU with frame waves)
-    if (rc == RTM_OK && c->nvec > 0 && frame4_supported(c->nfd) && !fused(c, fwd, FR_FWD)) {
+    if (rc == RTM_OK && c->nvec > 0 && frame4_supported(c->nfd) && !fused(c, fwd, FR_FWD) && !quad) {
       double tot[2] = {0.0, 0.0};
       for (int round = 0; round < kRounds && rc == RTM_OK; ++round)
         for (int i = 0; i < 2 && rc == RTM_OK; ++i) {

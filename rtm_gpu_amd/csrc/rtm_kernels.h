@@ -22,6 +22,9 @@ struct Model {
   long long mstride;   // 0: one model for all shots; fstride: windows ShotGeo::win apart
   const float* v;
   const float* r1;
+  // (taoh2*vq)*vq of the frame cell's one-way update, vq the velocity that the
+  // reference reads there (launch_frame_lat), padded layout
+  const float* fs;
   const float* pm;     // v*v*tao2*h2 per cell (FP32, left to right), padded layout
   const unsigned* ko;  // byte offset of the cell's coefficient row in ctab, padded layout
   const float* ctab;
@@ -135,6 +138,11 @@ struct FrameArgs {
   float* rf[2];
   int rk[2];
   int nrf, rbps;
+  // k_frame_quad: planes (TwoArgs::cp), float4 windows and rows per block,
+  // blocks of the part
+  const float* cp;
+  long long cpstride;
+  int qwin, qrows, nquad;
 };
 
 // Two time steps of the interior in one launch (rtm_two.hip): the forward
@@ -149,8 +157,10 @@ struct TwoArgs {
   Model m;
   Rcv r;
   const ShotGeo* geo;
-  // coefficient planes of a model window: c_0 .. c_NFD, P; fstride apart, a
-  // window's nfd + 2 planes cpstride apart (0: one window)
+  // planes of a model window, fstride apart: c_0 .. c_NFD, P, and the one-way
+  // operands of a top or bottom edge cell (kernel.cu:122-133): taoh v,
+  // 1 / (taoh v + 1), taoh2 vq vq.  A window's two_planes(nfd) planes are
+  // cpstride apart (0: one window)
   const float* cp;
   long long cpstride;
   const float *u1, *u0;  // newer and older field
@@ -177,10 +187,11 @@ int two_cols(const Grid& g, int nfd, int nshot);
 // the register queue).
 int two_rows(int nfd, int rows);
 hipError_t launch_two(int kind, int nfd_inst, TwoArgs a, int nshot, hipStream_t s);
-// Coefficient planes (TwoArgs::cp) of one window from its coefficient offsets
-// and P.
-hipError_t launch_coef_planes(const Grid& g, const unsigned* ko, const float* pm, const float* ctab,
-                              int nfd, float* cp, hipStream_t s);
+// Model::fs of a window nx columns wide from its velocities.
+hipError_t launch_frame_lat(const Grid& g, int nx, const float* v, float taoh2, float* fs, hipStream_t s);
+// Planes (TwoArgs::cp) of window win.
+constexpr int two_planes(int nfd) { return nfd + 5; }
+hipError_t launch_coef_planes(const Grid& g, const Model& m, int win, int nfd, float* cp, hipStream_t s);
 
 // A whole time step in one launch, one cell per thread (rtm_tile.hip).
 enum { TILE_FWD = 0, TILE_MIG = 1, TILE_BORN = 2, TILE_ADJ = 3 };
@@ -227,6 +238,7 @@ struct StencilOps {
   static hipError_t interior(int epi, dim3 grid, const IntArgs& a, hipStream_t s);
   static hipError_t frame(int mode, dim3 grid, const FrameArgs& a, hipStream_t s);
   static hipError_t frame4(int mode, dim3 grid, const FrameArgs& a, hipStream_t s);
+  static hipError_t frame_quad(int mode, dim3 grid, const FrameArgs& a, hipStream_t s);
   static hipError_t step(int epi, dim3 grid, const IntArgs& ia, const FrameArgs& fa, unsigned nint,
                          unsigned nfr, hipStream_t s);
 };
@@ -259,6 +271,14 @@ void frame_records(const Grid& g, int nx, int shot, int seg_tb, int seg, int kin
 // The float4 top/bottom frame kernel (forward and receiver fields) exists for
 // these compile-time stencil half-lengths.
 bool frame4_supported(int nfd_inst);
+// The float4 windows of a band of a shot nx columns wide (k_frame4,
+// k_frame_quad) write the columns n2+4 .. frame4_end-1, 248 each.
+__host__ __device__ inline int frame4_end(int n2, int nx) { return n2 + ((nx - 2 * n2 - 1) & ~3); }
+constexpr int QUAD_MAX_ROWS = 60;  // rows of a k_frame_quad block: one lane each, with two around them
+int frame4_windows(const Grid& g, int nx);
+// The whole frame of a forward or receiver step of a batch that k_two may
+// take: nrec FRAME_SCALAR records and a.qwin windows in runs of a.qrows rows.
+hipError_t launch_frame_quad(int mode, int nfd_inst, FrameArgs a, int nshot, int nrec, hipStream_t s);
 hipError_t launch_frame4(int mode, int nfd_inst, FrameArgs a, int nshot, int nrecords,
                          hipStream_t s);
 int frame_segment_rows(int nfd);

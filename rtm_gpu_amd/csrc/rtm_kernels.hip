@@ -457,14 +457,37 @@ hipError_t launch_two(int kind, int nfd, TwoArgs a, int nshot, hipStream_t s) {
   }
 }
 
-// A thread per cell of the padded layout.
-__global__ void k_coef_planes(long long n, long long fstride, const unsigned* ko, const float* pm,
-                              const float* ctab, int nfd, float* cp) {
+// The velocity of a frame cell's lateral term: its own on the top edge; Dv[(N2-x)*NX+y],
+// the mirrored top-band cell, on the bottom edge (kernel.cu:132); Dv[(N2-y)*NX+x], a
+// top-band cell, on the sides (kernel.cu:128, 136), where z may pass a row's end.
+// Read by every step from here: a wave of side cells reading the velocities
+// themselves touches a cache line per lane.
+__global__ void k_frame_lat(const Grid g, int nx, const float* v, float taoh2, float* fs) {
+  const long long n = (long long)g.nz * nx;
   for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (long long)gridDim.x * blockDim.x) {
-    const float* row = ctab + ko[i] / 4u;
-    for (int l = 0; l <= nfd; ++l) cp[(long long)l * fstride + i] = row[l];
-    cp[(long long)(nfd + 1) * fstride + i] = pm[i];
+    const int z = (int)(i / nx), x = (int)(i % nx);
+    const int ar = min(min(z, x), min(g.nz - 1 - z, nx - 1 - x));
+    const bool top = z == ar, bot = !top && z == g.nz - 1 - ar;
+    const int zq = top ? z : (bot ? ar : min(ar + z / nx, g.nz - 1));
+    const int xq = (top || bot) ? x : z % nx;
+    const float vq = v[(long long)zq * g.pitch + g.x0 + xq];
+    fs[(long long)z * g.pitch + g.x0 + x] = (taoh2 * vq) * vq;
+  }
+}
+
+// A thread per cell of the padded layout.
+__global__ void k_coef_planes(const Grid g, const Model m, long long wo, int nfd, float* cp) {
+  const long long fs = g.fstride, n = (long long)g.nz * g.pitch;
+  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
+       i += (long long)gridDim.x * blockDim.x) {
+    const float* row = m.ctab + m.ko[wo + i] / 4u;
+    for (int l = 0; l <= nfd; ++l) cp[l * fs + i] = row[l];
+    cp[(nfd + 1) * fs + i] = m.pm[wo + i];
+    const float tv = m.taoh * m.v[wo + i];
+    cp[(nfd + 2) * fs + i] = tv;
+    cp[(nfd + 3) * fs + i] = 1.0f / (tv + 1.0f);
+    cp[(nfd + 4) * fs + i] = m.fs[wo + i];
   }
 }
 
@@ -472,13 +495,13 @@ int frame_segment_rows(int nfd) {
   const int nb = nfd > 2 ? nfd : 2;
   return 2 * (nb + nfd + 1 + 2) - 2;  // two register-queue cycles per side run
 }
-// Float4 windows of the top and bottom bands (k_frame4): first column n2,
-// 252 apart, writing [cs+1, min(cs+253, nx-n2-1)).  None when the band's edge
-// cells do not reach one window or n2 leaves no room for the column halo.
-static int tb4_windows(const Grid& g, int nx) {
-  const int wend = nx - g.n2 - 1;
-  if (g.n2 < 12 || wend <= g.n2 + 1) return 0;
-  return (wend - (g.n2 + 1) + 251) / 252;
+// Float4 windows of the top and bottom bands: first column n2, 248 apart,
+// writing [cs+4, min(cs+252, frame4_end)).  None when the band's edge cells do
+// not reach one window or n2 leaves no room for the column halo.
+int frame4_windows(const Grid& g, int nx) {
+  const int wend = frame4_end(g.n2, nx);
+  if (g.n2 < 12 || nx < 2 * g.n2 || wend <= g.n2 + 4) return 0;
+  return (wend - (g.n2 + 4) + 247) / 248;
 }
 
 void frame_records(const Grid& g, int nx, int shot, int seg_tb, int seg, int kind, int4* out,
@@ -488,9 +511,9 @@ void frame_records(const Grid& g, int nx, int shot, int seg_tb, int seg, int kin
     if (out) out[n] = make_int4(z0, cx0, band | (rows << 4) | (ncol << 20), shot);
     ++n;
   };
-  const int nw = kind == FRAME_ALL ? 0 : tb4_windows(g, nx);
+  const int nw = kind == FRAME_ALL ? 0 : frame4_windows(g, nx);
   // top band, bottom band, in runs of seg_tb rows (the float4 records: one
-  // run of the whole band, each wave writing 252 columns)
+  // run of the whole band, each wave writing 248 columns)
   const int run = kind == FRAME_VEC ? g.n2 : seg_tb;
   for (int b = 0; b < 2; ++b) {
     const int zb = b == 0 ? 0 : g.nz - g.n2, ze = b == 0 ? g.n2 : g.nz;
@@ -500,10 +523,10 @@ void frame_records(const Grid& g, int nx, int shot, int seg_tb, int seg, int kin
         if (kind != FRAME_VEC)
           for (int cx0 = -1; cx0 + 1 < nx; cx0 += 62) put(z0, cx0, b, rows, 0);
       } else if (kind == FRAME_VEC) {
-        for (int w = 0; w < nw; ++w) put(z0, g.n2 + 252 * w, b, rows, 0);
-      } else {  // the columns left to the scalar kernel: [0, n2+1) and [nx-n2-1, nx)
-        for (int c = 0; c < g.n2 + 1; c += 62) put(z0, c - 1, b, rows, std::min(62, g.n2 + 1 - c));
-        for (int c = nx - g.n2 - 1; c < nx; c += 62) put(z0, c - 1, b, rows, std::min(62, nx - c));
+        for (int w = 0; w < nw; ++w) put(z0, g.n2 + 248 * w, b, rows, 0);
+      } else {  // the columns left to the scalar kernel
+        for (int c = 0; c < g.n2 + 4; c += 62) put(z0, c - 1, b, rows, std::min(62, g.n2 + 4 - c));
+        for (int c = frame4_end(g.n2, nx); c < nx; c += 62) put(z0, c - 1, b, rows, std::min(62, nx - c));
       }
     }
   }
@@ -539,6 +562,23 @@ hipError_t launch_frame4(int mode, int nfd, FrameArgs a, int nshot, int nrec, hi
     default: return hipErrorInvalidValue;
   }
 #undef CASE
+}
+
+hipError_t launch_frame_quad(int mode, int nfd, FrameArgs a, int nshot, int nrec, hipStream_t s) {
+  a.nshot = nshot;
+  a.nrec = nrec;
+  if (mode != FR_RCV) a.rbps = 0;
+  a.qrows = std::min(a.qrows, QUAD_MAX_ROWS);
+  a.nquad = 2 * a.qwin * ((a.g.n2 + a.qrows - 1) / a.qrows) * ((nshot + TWO_SHOTS - 1) / TWO_SHOTS);
+  const dim3 grid(a.nquad + (nrec + 3) / 4 + (a.rbps > 0 ? a.rbps * nshot * a.nrf : 0));
+  switch (nfd) {
+    case 1: return StencilOps<1>::frame_quad(mode, grid, a, s);
+    case 2: return StencilOps<2>::frame_quad(mode, grid, a, s);
+    case 3: return StencilOps<3>::frame_quad(mode, grid, a, s);
+    case 4: return StencilOps<4>::frame_quad(mode, grid, a, s);
+    case 5: return StencilOps<5>::frame_quad(mode, grid, a, s);
+    default: return hipErrorInvalidValue;
+  }
 }
 
 hipError_t launch_frame(int mode, int nfd, FrameArgs a, int nshot, int nrec, hipStream_t s) {
@@ -639,10 +679,14 @@ hipError_t launch_tap_planes(const Grid& g, const unsigned* ko, const float* cta
                      dim3(256), 0, s, g, ko, ctab, nfd, tp);
   return hipGetLastError();
 }
-hipError_t launch_coef_planes(const Grid& g, const unsigned* ko, const float* pm, const float* ctab,
-                              int nfd, float* cp, hipStream_t s) {
-  hipLaunchKernelGGL(k_coef_planes, dim3(blocks_for(g.fstride, 256, 2048)), dim3(256), 0, s, g.fstride,
-                     g.fstride, ko, pm, ctab, nfd, cp);
+hipError_t launch_frame_lat(const Grid& g, int nx, const float* v, float taoh2, float* fs, hipStream_t s) {
+  hipLaunchKernelGGL(k_frame_lat, dim3(blocks_for((long long)g.nz * nx, 256, 2048)), dim3(256), 0, s, g,
+                     nx, v, taoh2, fs);
+  return hipGetLastError();
+}
+hipError_t launch_coef_planes(const Grid& g, const Model& m, int win, int nfd, float* cp, hipStream_t s) {
+  hipLaunchKernelGGL(k_coef_planes, dim3(blocks_for(g.fstride, 256, 2048)), dim3(256), 0, s, g, m,
+                     (long long)win * m.mstride, nfd, cp);
   return hipGetLastError();
 }
 hipError_t launch_flag_reset(unsigned* flag, hipStream_t s) {

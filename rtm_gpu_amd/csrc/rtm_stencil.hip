@@ -384,8 +384,17 @@ __device__ __forceinline__ void interior_body(const IntArgs& a, const unsigned b
 // row earlier), row operands arrive PD rows ahead and the one-way operands two
 // rows ahead, and each row waits only on loads issued a row or more before.
 // No block-level barrier: the four waves of a block are independent.
-template <int NFD, int MODE>
-__device__ __forceinline__ void frame_body(const FrameArgs& a, const unsigned bid) {
+//
+// SIDE (forward and receiver): a record of the side bands, whose written cells
+// are all side cells of Hybrid1/Hybrid2 (kernel.cu:126-137), the corner rows'
+// innermost ones aside.  Their inner neighbour is one column away in a
+// direction that is the lane's own, so two cross-lane reads a row replace ten,
+// and the ring and blend weight of a lane are its own.  The side bands are bound
+// by instruction issue and by the L1: 128 shots of 351 x 1701 took 44 us a step
+// (half-length 3), 36 with this body and the lateral factors of Model::fs (a
+// side cell's velocity lies in another row for every lane).
+template <int NFD, int MODE, bool SIDE>
+__device__ __forceinline__ void frame_body(const FrameArgs& a, const int4 rec) {
   constexpr int PD = 2;                   // rows of prefetch
   constexpr int NB = NFD > 2 ? NFD : 2;   // queue rows kept behind the T row
   // The row loop is unrolled by U, a multiple of 12 that holds the u1 rows
@@ -400,9 +409,6 @@ __device__ __forceinline__ void frame_body(const FrameArgs& a, const unsigned bi
   const Model& m = a.m;
   const int lane = threadIdx.x & 63;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int ri = (int)bid * 4 + wv;
-  if (ri >= a.nrec) return;
-  const int4 rec = a.recs[ri];
   const int z0 = rec.x, cx0 = rec.y, band = rec.z & 15, nrows = (rec.z >> 4) & 0xffff, shot = rec.w;
   const int ncol = (rec.z >> 20) & 0xff;  // top/bottom: written lanes 1..ncol (0: 1..62)
   const ShotGeo sg = a.geo[shot];
@@ -411,7 +417,7 @@ __device__ __forceinline__ void frame_body(const FrameArgs& a, const unsigned bi
   // lanes 0..31 hold columns -1..30 (the left band and its inner
   // neighbour), lanes 32..63 columns nx-31..nx; lanes 1..30 and 33..62
   // write.  The +-1 lane shuffles of the one-way update stay inside a half.
-  const bool packed = band == 4;
+  const bool packed = (SIDE || MODE == FR_BORN || MODE == FR_ADJ) && band == 4;
   const bool rhalf = packed && lane >= 32;
   const int x = packed ? (rhalf ? NX - 63 + lane : lane - 1) : cx0 + lane;
   const int xm = mirror_idx(x, NX);
@@ -435,13 +441,13 @@ __device__ __forceinline__ void frame_body(const FrameArgs& a, const unsigned bi
   const Rsrc R1 = rsrc(a.u1 + so, fb), R0 = rsrc(a.u0 + so, fb), R2 = rsrc(a.u2 + so, fb);
   const long long mo = (long long)sg.win * m.mstride;
   const Rsrc RP = rsrc(m.pm + mo, fb), RK = rsrc(m.ko + mo, fb);
-  const Rsrc RV = rsrc(m.v + mo, fb), RR = rsrc(m.r1 + mo, fb);
+  const Rsrc RV = rsrc(m.v + mo, fb), RR = rsrc(m.r1 + mo, fb), RQ = rsrc(m.fs + mo, fb);
   const Rsrc RC = rsrc(m.ctab, (unsigned)(m.nrow * m.cs) * 4u);
   const Rsrc RW = rsrc(m.w, (unsigned)(N2 + 1) * 4u);
   const unsigned P4 = (unsigned)g.pitch * 4u;
-  auto rowm = [&](int z) -> unsigned { return (unsigned)mirror_idx(z, NZ) * P4; };
-  auto colb = [&](int c) -> unsigned { return (unsigned)(g.x0 + c) * 4u; };
-  const unsigned vcol = colb(xm);
+  auto rowm = [=](int z) __attribute__((always_inline)) -> unsigned { return (unsigned)mirror_idx(z, NZ) * P4; };
+  auto colb = [&](int c) __attribute__((always_inline)) -> unsigned { return (unsigned)(g.x0 + c) * 4u; };
+  const unsigned vcol = colb(xm), vst = outcol ? vcol : kDrop;
 
   // halo columns of the LDS row: lanes 0..NFD-1 the left ones, NFD..2NFD-1
   // the right ones (packed: the left half's two halos, then lanes
@@ -466,12 +472,12 @@ __device__ __forceinline__ void frame_body(const FrameArgs& a, const unsigned bi
   rr.s_r = sg.s_r;
   int rs = 0;
   const bool isrcv = (MODE == FR_RCV || MODE == FR_ADJ) && is_receiver(x, rr, &rs);
-  Rsrc RD;
+  float ev = 0.f;
   if (MODE == FR_RCV || MODE == FR_ADJ) {
     const int kd = MODE == FR_RCV ? a.k + 1 : a.k;
-    RD = rsrc(a.data + ((long long)shot * a.nt + kd) * a.r.n, (unsigned)a.r.n * 4u);
+    const Rsrc RD = rsrc(a.data + ((long long)shot * a.nt + kd) * a.r.n, (unsigned)a.r.n * 4u);
+    ev = bld1(RD, isrcv ? (unsigned)rs * 4u : kDrop, 0u);
   }
-  const unsigned vrcv = isrcv ? (unsigned)rs * 4u : kDrop;
   // strip slot of this step (FP32) or its FP32 staging (FP16 / BF16)
   Rsrc RS;
   if (MODE == FR_FWD) {
@@ -481,6 +487,24 @@ __device__ __forceinline__ void frame_body(const FrameArgs& a, const unsigned bi
         : a.st.stage + ((long long)shot * 2 + (a.k & 1)) * ss;
     RS = rsrc(sb, a.save_strips ? (unsigned)ss * 4u : 0u);
   }
+  // strip element of (z, x) (strip_elem): the lane's part, and the row's in the loop
+  unsigned vstrip = kDrop;
+  if (MODE == FR_FWD) {
+    if (SIDE) {
+      if (x >= N2 - g.nfd && x < N2) vstrip = (unsigned)(N2 - 1 - x) * 4u;
+      else if (x >= NX - N2 && x < NX - N2 + g.nfd) vstrip = (unsigned)(g.mnz * g.nfd + x - (NX - N2)) * 4u;
+    } else if (x >= N2 && x < NX - N2) {
+      vstrip = (unsigned)(2 * g.mnz * g.nfd + x - N2) * 4u;
+    }
+    if (!outcol) vstrip = kDrop;
+  }
+  const int sd = g.nfd, smnx = sg.mnx;
+  auto strip_put_row = [=](int z, unsigned drop, float val) __attribute__((always_inline)) {
+    const bool up = z >= N2 - sd && z < N2, dn = z >= NZ - N2 && z < NZ - N2 + sd;
+    const int e = SIDE ? (z - N2) * sd : (up ? (N2 - 1 - z) * smnx : (sd + z - (NZ - N2)) * smnx);
+    const bool on = SIDE ? z >= N2 && z < NZ - N2 : up || dn;
+    bst1s(RS, (vstrip + (on ? (unsigned)e * 4u : 0u)) | drop | (on ? 0u : kDrop), 0u, val);
+  };
   // adjoint with per-cell rows: the interior cells of the march (the rows and
   // columns next to the frame, whose pre-blend values the one-way update
   // reads) take the transposed stencil of the interior kernel
@@ -494,27 +518,20 @@ __device__ __forceinline__ void frame_body(const FrameArgs& a, const unsigned bi
   }
   constexpr int NE = MODE == FR_BORN ? 4 : 1;  // extra operands of a T row
 
-  // one-way operands of row zr (velocity, r1, the Q1 velocity, blend weight)
-  auto abc_ops = [&](int zr, float& vp, float& r1v, float& vq, float& wv_) {
-    const int ar = min(min(zr, x), min(NZ - 1 - zr, NX - 1 - x));
-    // row zr as a linear index of the model: row zr / NX, column zr % NX (uniform)
-    const int zdiv = zr / NX, zmod = zr - zdiv * NX;
-    const bool topc = zr == ar, botc = !topc && zr == NZ - 1 - ar;
-    // top: the cell itself; bottom: Dv[(N2-x)*NX+y] (kernel.cu:132); sides:
-    // Dv[(N2-y)*NX+x] (kernel.cu:128,136), a top-band cell
-    int zq = topc ? zr : (botc ? ar : ar + zdiv);
-    int xq = (topc || botc) ? x : zmod;
-    zq = min(max(zq, 0), NZ - 1);
-    xq = min(max(xq, 0), NX - 1);
+  // one-way operands of row zr (velocity, r1, lateral factor, blend weight; SIDE:
+  // the weight is the lane's, r1 that of the corner rows)
+  auto abc_ops = [&](int zr, float& vp, float& r1v, float& sqv, float& wv_) __attribute__((always_inline)) {
     vp = bld1(RV, vcol, rowm(zr));
-    r1v = bld1(RR, vcol, rowm(zr));
-    vq = bld1(RV, colb(xq) + (unsigned)zq * P4, 0u);
-    wv_ = bld1(RW, (unsigned)min(max(N2 - ar, 0), N2) * 4u, 0u);
+    sqv = bld1(RQ, vcol, rowm(zr));
+    if (!SIDE) {
+      const int ar = min(min(zr, x), min(NZ - 1 - zr, NX - 1 - x));
+      r1v = bld1(RR, vcol, rowm(zr));
+      wv_ = bld1(RW, (unsigned)min(max(N2 - ar, 0), N2) * 4u, 0u);
+    }
   };
-  // extra operands of T row zr: the data sample, or the Born source terms
-  auto t_ops = [&](int zr, float* e) {
-    if (MODE == FR_RCV || MODE == FR_ADJ) e[0] = bld1(RD, zr == a.r.s_z ? vrcv : kDrop, 0u);
-    else if (MODE == FR_BORN) {
+  // extra operands of T row zr: the Born source terms
+  auto t_ops = [&](int zr, float* e) __attribute__((always_inline)) {
+    if (MODE == FR_BORN) {
       const unsigned rz = rowm(zr);
       e[0] = bld1(RBX, vcol, rz); e[1] = bld1(RBA, vcol, rz);
       e[2] = bld1(RBB, vcol, rz); e[3] = bld1(RBC, vcol, rz);
@@ -522,6 +539,17 @@ __device__ __forceinline__ void frame_body(const FrameArgs& a, const unsigned bi
       e[0] = 0.f;
     }
   };
+  float r1top = 0.f, r1bot = 0.f, wside = 0.f;
+  const bool inr = x < N2;  // SIDE: inner neighbour to the right
+  const bool clane = x == N2 - 1 || x == NX - N2;
+  const int inl = (inr ? lane + 1 : lane - 1) * 4;
+  if (SIDE) {
+    r1top = bld1(RR, vcol, rowm(N2));
+    r1bot = bld1(RR, vcol, rowm(NZ - N2 - 1));
+    wside = bld1(RW, (unsigned)min(max(N2 - min(x, NX - 1 - x), 0), N2) * 4u, 0u);
+  }
+  float TS[3] = {0.f, 0.f, 0.f};  // SIDE: T rows it-2 .. it at the inner neighbour
+  float US[2] = {0.f, 0.f};       // SIDE: u1 rows it-1, it there
 
   // Circular buffers, indexed by the iteration number it (T row t0 + it):
   //   q[U]     u1 rows (row t0 - NB + i in slot i % U)
@@ -626,14 +654,38 @@ __device__ __forceinline__ void frame_body(const FrameArgs& a, const unsigned bi
         Tn = inner ? __builtin_fmaf(ex[0], d2u, Tn) : Tn;
       } else if (MODE == FR_ADJ) {   // adjoint field: P * r(k) added at the receivers
         Tn = combine_p(u, u0, pmv, w1, false);
-        Tn = (isrcv && tt == a.r.s_z) ? Tn + pmv * ex[0] : Tn;
+        Tn = (isrcv && tt == a.r.s_z) ? Tn + pmv * ev : Tn;
       } else {                       // receiver field: data replace where non-zero
         Tn = combine_p(u, u0, pmv, w1, false);
-        Tn = (isrcv && tt == a.r.s_z && ex[0] != 0.0f) ? ex[0] : Tn;
+        Tn = (tt == a.r.s_z && ev != 0.0f) ? ev : Tn;  // 0 without a receiver
       }
       T[j % 3] = Tn;
       // (5) one-way value and blend of row z = tt - 1 (written from the third row on)
-      if (pure_tb) {  // top edge (inner row z+1) or bottom edge (inner row z-1) (kernel.cu:122-125,130-133)
+      if (SIDE) {  // left edge (inner column x+1) or right edge (x-1) (kernel.cu:126-129,134-137)
+        const int z = tt - 1;
+        TS[j % 3] = __int_as_float(__builtin_amdgcn_ds_bpermute(inl, __float_as_int(Tn)));
+        const float Ti = TS[(j + 2) % 3], Tip = TS[j % 3], Tim = TS[(j + 1) % 3];
+        const float U0z = u0b[(j + 1) % 6], U0p = u0b[(j + 2) % 6], U0m = u0b[j % 6];
+        const float U0i = __int_as_float(__builtin_amdgcn_ds_bpermute(inl, __float_as_int(U0z)));
+        const float U1z = q[(j + NB - 1) % U], U1i = US[(j + 1) % 2];
+        US[j % 2] = inr ? hr[0] : hl[0];
+        const int ab = j % 3;
+        const float tv = m.taoh * vpb[ab];
+        const float t1 = tv * ((Ti - U0i) + U0z);
+        const float t2 = ((((-2.0f * U1z) + U0z) + Ti) - 2.0f * U1i) + U0i;
+        const float lap = ((((Tip - 2.0f * Ti) + Tim) + U0p) - 2.0f * U0z) + U0m;
+        const float t3 = vqb[ab] * lap;
+        // the corner cells of the first and last row (kernel.cu:138-155)
+        const bool corner = clane && (z == N2 || z == NZ - N2 - 1);
+        const float r1v = z == N2 ? r1top : r1bot;
+        const float num_c = U1z + r1v * (Ti + (z == N2 ? T[j % 3] : T[(j + 1) % 3]));
+        const float den = corner ? 2.0f * r1v + 1.0f : tv + 1.0f;
+        const float O = (1.0f / den) * (corner ? num_c : (t1 - t2) + t3);
+        const float val = (1.0f - wside) * T[(j + 2) % 3] + wside * O;
+        const unsigned rd = it >= 2 && z < z0 + nrows ? 0u : kDrop;
+        bst1s(R2, vst | rd, rowm(z), val);
+        if (MODE == FR_FWD) strip_put_row(z, rd, val);  // Hybrid3 (kernel.cu:184-208)
+      } else if (pure_tb) {  // top edge (inner row z+1) or bottom edge (inner row z-1) (kernel.cu:122-125,130-133)
         const int z = tt - 1;
         const bool tp = band == 0;
         const float T0 = T[(j + 2) % 3];
@@ -645,20 +697,17 @@ __device__ __forceinline__ void frame_body(const FrameArgs& a, const unsigned bi
         const float Til = __shfl_up(Tin, 1), Tir = __shfl_down(Tin, 1);
         const float U0l = __shfl_up(U0z, 1), U0r = __shfl_down(U0z, 1);
         const int ab = j % 3;
-        const float vp = vpb[ab], vq = vqb[ab], wgt = wb[ab];
+        const float vp = vpb[ab], wgt = wb[ab];
         const float tv = m.taoh * vp;
         const float t1 = tv * ((Tin - U0i) + U0z);
         const float t2 = ((((-2.0f * U1z) + U0z) + Tin) - 2.0f * U1i) + U0i;
         const float lap = ((((Tir - 2.0f * Tin) + Til) + U0r) - 2.0f * U0z) + U0l;
-        const float t3 = ((m.taoh2 * vq) * vq) * lap;
+        const float t3 = vqb[ab] * lap;
         const float O = (1.0f / (tv + 1.0f)) * ((t1 - t2) + t3);
         const float val = (1.0f - wgt) * T0 + wgt * O;
-        const bool out = outcol && it >= 2 && z < z0 + nrows;
-        bst1s(R2, out ? vcol : kDrop, rowm(z), val);
-        if (MODE == FR_FWD) {  // Hybrid3 (kernel.cu:184-208)
-          const int e = strip_elem(g, NX, sg.mnx, z, x);
-          bst1s(RS, (out && e >= 0) ? (unsigned)e * 4u : kDrop, 0u, val);
-        }
+        const unsigned rd = it >= 2 && z < z0 + nrows ? 0u : kDrop;
+        bst1s(R2, vst | rd, rowm(z), val);
+        if (MODE == FR_FWD) strip_put_row(z, rd, val);  // Hybrid3 (kernel.cu:184-208)
       } else {
         const int z = tt - 1;
         const float Tm = T[(j + 1) % 3], T0 = T[(j + 2) % 3], Tp = T[j % 3];
@@ -677,7 +726,7 @@ __device__ __forceinline__ void frame_body(const FrameArgs& a, const unsigned bi
         const bool top = z == ar, bot = !top && z == br, side = !top && !bot;
         const bool inr = x == ar;  // side cell with its inner neighbour to the right
         const int ab = j % 3;      // one-way operands of row z
-        const float vp = vpb[ab], r1v = r1b[ab], vq = vqb[ab], wgt = wb[ab];
+        const float vp = vpb[ab], r1v = r1b[ab], wgt = wb[ab];
         // corner cells (kernel.cu:138-155)
         const float Tx = (x - ar <= 1) ? T0r : T0l;
         const float Tz = (z - ar <= 1) ? Tp : Tm;
@@ -694,17 +743,14 @@ __device__ __forceinline__ void frame_body(const FrameArgs& a, const unsigned bi
         const float t1 = tv * ((Ti - U0i) + U0z);
         const float t2 = ((((-2.0f * U1z) + U0z) + Ti) - 2.0f * U1i) + U0i;
         const float lap = ((((Tip - 2.0f * Ti) + Tim) + U0pp) - 2.0f * U0z) + U0pm;
-        const float t3 = ((m.taoh2 * vq) * vq) * lap;
+        const float t3 = vqb[ab] * lap;
         const float num_s = (t1 - t2) + t3;
         const float den_s = tv + 1.0f;
         const float O = (1.0f / (corner ? den_c : den_s)) * (corner ? num_c : num_s);
         const float val = (1.0f - wgt) * T0 + wgt * O;
-        const bool out = outcol && it >= 2 && z < z0 + nrows;
-        bst1s(R2, out ? vcol : kDrop, rowm(z), val);
-        if (MODE == FR_FWD) {  // Hybrid3 (kernel.cu:184-208)
-          const int e = strip_elem(g, NX, sg.mnx, z, x);
-          bst1s(RS, (out && e >= 0) ? (unsigned)e * 4u : kDrop, 0u, val);
-        }
+        const unsigned rd = it >= 2 && z < z0 + nrows ? 0u : kDrop;
+        bst1s(R2, vst | rd, rowm(z), val);
+        if (MODE == FR_FWD) strip_put_row(z, rd, val);  // Hybrid3 (kernel.cu:184-208)
       }
     }
   }
@@ -714,11 +760,11 @@ __device__ __forceinline__ void frame_body(const FrameArgs& a, const unsigned bi
 // Top and bottom bands away from the corners, four columns per lane.  A record
 // (z0, cs, band | rows << 4, shot) covers the 256 columns cs .. cs+255 (cs ==
 // n2 mod 4, so each lane's float4 is aligned like the interior kernel's) and
-// writes the columns cs+1 .. cs+252 left of nx-n2-1.  Every written cell is a
+// writes the columns cs+4 .. cs+251 left of frame4_end.  Every written cell is a
 // top-edge (bottom-edge) cell of Hybrid1/Hybrid2 (kernel.cu:122-125, 130-133):
 // its one-way update reads the inner row and the lateral neighbours x-1, x+1
-// of the same row, so lane 0's first column and lane 63's last three only
-// supply neighbours.  The row march, the look-ahead of the operands and the
+// of the same row, so lanes 0 and 63 only supply neighbours, and a lane writes
+// all of its float4 or nothing.  The row march, the look-ahead of the operands and the
 // arithmetic are those of frame_body's top/bottom path, operation for
 // operation, so both give the same bits; per cell this one spends a quarter of
 // the row addressing, masks and buffer instructions.  FR_FWD and FR_RCV only.
@@ -739,18 +785,12 @@ __device__ __forceinline__ void frame_tb4_body(const FrameArgs& a, const int4 re
   const int z0 = rec.x, cs = rec.y, nrows = (rec.z >> 4) & 0xffff, shot = rec.w;
   const ShotGeo sg = a.geo[shot];
   const int NX = sg.nx, NZ = g.nz, N2 = g.n2;
-  const int wend = NX - N2 - 1;  // first column past the edge cells
+  const int wend = frame4_end(N2, NX);
   const int c0 = cs + 4 * lane;
   const int clast = NX - ((NX - N2) & 3);  // largest c == n2 (mod 4) with c <= nx
   const unsigned vcol = (unsigned)(g.x0 + min(c0, clast)) * 4u;
-  bool wr[4];
-  bool full = true;
-#pragma unroll
-  for (int jj = 0; jj < 4; ++jj) {
-    wr[jj] = c0 + jj > cs && c0 + jj <= cs + 252 && c0 + jj < wend;
-    full = full && wr[jj];
-  }
-  const unsigned vst = (unsigned)(g.x0 + c0) * 4u;
+  const bool out = lane >= 1 && lane <= 62 && c0 < wend;
+  const unsigned vst = out ? (unsigned)(g.x0 + c0) * 4u : kDrop;
   // halo float4s of the LDS row: lanes 0 .. H/4-1 left, H/4 .. 2H/4-1 right
   // (columns past the shot's width only feed unwritten columns)
   unsigned vhal = kDrop;
@@ -766,11 +806,11 @@ __device__ __forceinline__ void frame_tb4_body(const FrameArgs& a, const int4 re
   const Rsrc R1 = rsrc(a.u1 + so, fb), R0 = rsrc(a.u0 + so, fb), R2 = rsrc(a.u2 + so, fb);
   const long long mo = (long long)sg.win * m.mstride;
   const Rsrc RP = rsrc(m.pm + mo, fb), RK = rsrc(m.ko + mo, fb), RV = rsrc(m.v + mo, fb);
+  const Rsrc RQ = rsrc(m.fs + mo, fb);
   const Rsrc RC = rsrc(m.ctab, (unsigned)(m.nrow * m.cs) * 4u);
   const Rsrc RW = rsrc(m.w, (unsigned)(N2 + 1) * 4u);
   const unsigned P4 = (unsigned)g.pitch * 4u;
   auto rowm = [&](int z) -> unsigned { return (unsigned)mirror_idx(z, NZ) * P4; };
-  auto rowc = [&](int z) -> unsigned { return (unsigned)min(max(z, 0), NZ - 1) * P4; };
   // ring of row zr: zr (top edge), nz-1-zr (bottom edge)
   auto ring = [&](int zr) -> int { return BOT ? NZ - 1 - zr : zr; };
 
@@ -827,7 +867,7 @@ __device__ __forceinline__ void frame_tb4_body(const FrameArgs& a, const int4 re
   cr[0][3].load(RC, kb[0].w);
   const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
   float4 T[3] = {z4, z4, z4};
-  float4 vpb[3] = {z4, z4, z4}, vqb[3] = {z4, z4, z4};  // slot (it + 1) % 3 holds row t0 + it
+  float4 vpb[3] = {z4, z4, z4}, sqb[3] = {z4, z4, z4};  // slot (it + 1) % 3 holds row t0 + it
   float wb[3] = {0.f, 0.f, 0.f};
 
   for (int base = 0; base < niter; base += U) {
@@ -850,11 +890,10 @@ __device__ __forceinline__ void frame_tb4_body(const FrameArgs& a, const int4 re
       pmb[(j + PD) % 3] = bld4(RP, vcol, rowm(tt + PD));
       halb[(j + PD) % 3] = bld4(R1, vhal, rowm(tt + PD));
       u0b[(j + 2 + PD) % 6] = bld4s(R0, vcol, rowm(tt + PD));
-      // one-way operands of row tt+1: velocity, the Q1 velocity (the cell
-      // itself on the top edge; Dv[(N2-x)*NX+y], the mirrored top-band cell,
-      // on the bottom edge, kernel.cu:132) and the blend weight of its ring
+      // one-way operands of row tt+1: velocity, on the bottom edge the lateral
+      // factor (on the top edge the velocity's own), the blend weight of its ring
       vpb[(j + 2) % 3] = bld4(RV, vcol, rowm(tt + 1));
-      if (BOT) vqb[(j + 2) % 3] = bld4(RV, vcol, rowc(NZ - 1 - (tt + 1)));
+      if (BOT) sqb[(j + 2) % 3] = bld4(RQ, vcol, rowm(tt + 1));
       wb[(j + 2) % 3] = bld1(RW, (unsigned)min(max(N2 - ring(tt + 1), 0), N2) * 4u, 0u);
       __builtin_amdgcn_sched_barrier(0);
       // (3) horizontal neighbours of row tt through LDS
@@ -905,7 +944,7 @@ __device__ __forceinline__ void frame_tb4_body(const FrameArgs& a, const int4 re
       const float Ul = __shfl_up(U0zv.w, 1), Ur = __shfl_down(U0zv.x, 1);
       const int ab = j % 3;
       const float4 vpv = vpb[ab];
-      const float4 vqv = BOT ? vqb[ab] : vpb[ab];
+      const float4 sqv = sqb[ab];
       const float wgt = wb[ab];
       float val[4];
 #pragma unroll
@@ -917,28 +956,25 @@ __device__ __forceinline__ void frame_tb4_body(const FrameArgs& a, const int4 re
         const float Tir = jj == 3 ? Tr : compr(Tinv, jj + 1);
         const float U0l = jj == 0 ? Ul : compr(U0zv, jj - 1);
         const float U0r = jj == 3 ? Ur : compr(U0zv, jj + 1);
-        const float vp = compr(vpv, jj), vq = compr(vqv, jj);
+        const float vp = compr(vpv, jj);
         const float tv = m.taoh * vp;
         const float t1 = tv * ((Tin - U0i) + U0z);
         const float t2 = ((((-2.0f * U1z) + U0z) + Tin) - 2.0f * U1i) + U0i;
         const float lap = ((((Tir - 2.0f * Tin) + Til) + U0r) - 2.0f * U0z) + U0l;
-        const float t3 = ((m.taoh2 * vq) * vq) * lap;
+        const float t3 = (BOT ? compr(sqv, jj) : (m.taoh2 * vp) * vp) * lap;
         const float O = (1.0f / (tv + 1.0f)) * ((t1 - t2) + t3);
         val[jj] = (1.0f - wgt) * T0 + wgt * O;
       }
       const bool rowout = it >= 2 && z < z0 + nrows;
       const unsigned rz = rowm(z);
-      bst4s(R2, (rowout && full) ? vst : kDrop, rz, val[0], val[1], val[2], val[3]);
-#pragma unroll
-      for (int jj = 0; jj < 4; ++jj)
-        bst1s_(R2, (rowout && !full && wr[jj]) ? vst + 4u * jj : kDrop, rz, val[jj]);
+      bst4s(R2, vst | (rowout ? 0u : kDrop), rz, val[0], val[1], val[2], val[3]);
       if (MODE == FR_FWD) {  // Hybrid3 (kernel.cu:184-208)
         const bool srow = BOT ? (z >= NZ - N2 && z < NZ - N2 + g.nfd) : (z >= N2 - g.nfd && z < N2);
-        const int sbase = BOT ? 2 * sa + sbb + (z - (NZ - N2)) * sg.mnx - N2
-                              : 2 * sa + (N2 - 1 - z) * sg.mnx - N2;
-#pragma unroll
-        for (int jj = 0; jj < 4; ++jj)
-          bst1s(RS, (rowout && srow && wr[jj]) ? (unsigned)(sbase + c0 + jj) * 4u : kDrop, 0u, val[jj]);
+        if (rowout && srow) {
+          const int sbase = BOT ? 2 * sa + sbb + (z - (NZ - N2)) * sg.mnx - N2
+                                : 2 * sa + (N2 - 1 - z) * sg.mnx - N2;
+          bst4s(RS, out ? (unsigned)(sbase + c0) * 4u : kDrop, 0u, val[0], val[1], val[2], val[3]);
+        }
       }
     }
   }
@@ -963,19 +999,271 @@ __global__ __launch_bounds__(256) void k_frame4(const FrameArgs a) {
 // reconstructed field (FrameArgs::rf): its blocks follow the record blocks and
 // fill the wave slots the frame's few long waves leave free.
 template <int NFD, int MODE>
-__global__ __launch_bounds__(256) void k_frame(const FrameArgs a) {
+__device__ __forceinline__ void frame_records_body(const FrameArgs& a, const unsigned bid) {
   if ((MODE == FR_RCV || MODE == FR_ADJ) && a.rbps > 0) {
     const unsigned nfb = ((unsigned)a.nrec + 3u) >> 2;
-    if (blockIdx.x >= nfb) {
-      const unsigned b = blockIdx.x - nfb, per = (unsigned)(a.rbps * a.nshot);
+    if (bid >= nfb) {
+      const unsigned b = bid - nfb, per = (unsigned)(a.rbps * a.nshot);
       const bool second = b >= per;  // of two fields
       strip_restore_body(a.g, second ? a.rf[1] : a.rf[0], a.st, a.geo, second ? a.rk[1] : a.rk[0],
                          second ? b - per : b, (unsigned)a.rbps);
       return;
     }
   }
-  frame_body<NFD, MODE>(a, blockIdx.x);
+  const int ri = (int)bid * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (ri >= a.nrec) return;
+  const int4 rec = a.recs[ri];
+  if ((MODE == FR_FWD || MODE == FR_RCV) && (rec.z & 15) >= 2) frame_body<NFD, MODE, true>(a, rec);
+  else frame_body<NFD, MODE, false>(a, rec);
 }
+
+template <int NFD, int MODE>
+__global__ __launch_bounds__(256) void k_frame(const FrameArgs a) {
+  frame_records_body<NFD, MODE>(a, blockIdx.x);
+}
+
+#if RTM_NFD <= 5  // TWO_MAX_NFD
+// The same cells for batches whose blocks of four shots share a model window
+// (k_two's): the four waves of a block march the band of four shots row by row
+// together, and the window's coefficient planes, P and the three one-way
+// operands (TwoArgs::cp) go through LDS, each plane loaded by one wave.  Seven
+// buffer instructions a row instead of eleven and no division; 155 registers
+// instead of 217 at half-length 3, three waves per SIMD.
+template <int NFD, int MODE, bool BOT>
+__device__ __forceinline__ void frame_quad_body(const FrameArgs& a, const int z0, const int nrows,
+                                                const int cs, const int s4,
+                                                float4 (*cf)[NFD + 5][64], float4 (*lds)[64 + 2 * ((NFD + 3) / 4)],
+                                                float4* dat) {
+  static_assert(MODE == FR_FWD || MODE == FR_RCV, "forward and receiver frames only");
+  constexpr int PD = 2;                   // rows of prefetch
+  constexpr int NB = NFD > 2 ? NFD : 2;   // queue rows kept behind the T row
+  constexpr int U = (NB + NFD + 1 + PD + 11) / 12 * 12;
+  constexpr int H = (NFD + 3) & ~3;
+  constexpr int NWIN = 1 + 2 * (H / 4);
+  constexpr int NPL = NFD + 5, NL = (NPL + 3) / 4;
+  const Grid& g = a.g;
+  const Model& m = a.m;
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const bool live = s4 + wv < a.nshot;  // a wave past the batch only loads planes
+  const int shot = live ? s4 + wv : a.nshot - 1;
+  const ShotGeo sg = a.geo[shot];
+  const int NX = sg.nx, NZ = g.nz, N2 = g.n2;
+  const int wend = frame4_end(N2, NX);
+  if (cs + 4 >= wend) return;  // the same for the block's shots
+  const int c0 = cs + 4 * lane;
+  const int clast = NX - ((NX - N2) & 3);  // largest c == n2 (mod 4) with c <= nx
+  const unsigned vcol = (unsigned)(g.x0 + min(c0, clast)) * 4u;
+  const bool out = live && lane >= 1 && lane <= 62 && c0 < wend;
+  const unsigned vst = out ? (unsigned)(g.x0 + c0) * 4u : kDrop;
+  unsigned vhal = kDrop;
+  int hpos = H / 4 + lane;
+  if (lane < H / 4) { vhal = (unsigned)(g.x0 + cs - H + 4 * lane) * 4u; hpos = lane; }
+  else if (lane < 2 * (H / 4)) {
+    vhal = (unsigned)(g.x0 + min(cs + 256 + 4 * (lane - H / 4), clast)) * 4u;
+    hpos = 64 + lane;
+  }
+
+  const long long so = (long long)shot * g.fstride;
+  const unsigned fb = (unsigned)g.fstride * 4u;
+  const Rsrc R1 = rsrc(a.u1 + so, fb), R0 = rsrc(a.u0 + so, fb), R2 = rsrc(a.u2 + so, fb);
+  const Rsrc RW = rsrc(m.w, (unsigned)(N2 + 1) * 4u);
+  // the wave's planes: wv, wv + 4, ..; the one-way operands lag a row
+  const float* cp = a.cp + (long long)sg.win * a.cpstride;
+  Rsrc RPL[NL];
+  int lag[NL];
+#pragma unroll
+  for (int i = 0; i < NL; ++i) {
+    const int pl = wv + 4 * i;
+    RPL[i] = rsrc(cp + (long long)min(pl, NPL - 1) * g.fstride, pl < NPL ? fb : 0u);
+    lag[i] = pl >= NFD + 2 ? 1 : 0;
+  }
+  const unsigned P4 = (unsigned)g.pitch * 4u;
+  auto rowm = [=](int z) -> unsigned { return (unsigned)mirror_idx(z, NZ) * P4; };
+
+  if (MODE == FR_RCV) {  // this step's data samples, as in frame_tb4_body
+    float ev[4];
+    Rcv rr = a.r;
+    rr.s_l = sg.s_l;
+    rr.s_r = sg.s_r;
+    const Rsrc RD = rsrc(a.data + ((long long)shot * a.nt + a.k + 1) * a.r.n, (unsigned)a.r.n * 4u);
+#pragma unroll
+    for (int jj = 0; jj < 4; ++jj) {
+      int rs = 0;
+      const bool isr = is_receiver(c0 + jj, rr, &rs);
+      ev[jj] = bld1(RD, isr ? (unsigned)rs * 4u : kDrop, 0u);
+    }
+    dat[threadIdx.x] = make_float4(ev[0], ev[1], ev[2], ev[3]);
+  }
+  Rsrc RS;  // strip rows, as in frame_tb4_body
+  if (MODE == FR_FWD) {
+    const long long ss = a.st.ss;
+    const float* sb = a.st.fmt == 0
+        ? (const float*)a.st.base + ((long long)shot * a.st.nslot + a.k % a.st.nslot) * ss
+        : a.st.stage + ((long long)shot * 2 + (a.k & 1)) * ss;
+    RS = rsrc(sb, a.save_strips ? (unsigned)ss * 4u : 0u);
+  }
+  const int sa = g.mnz * g.nfd, sbb = g.nfd * sg.mnx;
+  const float hzx2_1 = m.hzx2_1;
+  const double h1 = m.h1;
+  const int srow = MODE == FR_FWD ? sg.r_u : a.r.s_z;
+  const bool f64comb = MODE == FR_FWD && a.f64comb != 0;
+
+  const int t0 = z0 - 1;          // T row of the first iteration
+  const int niter = nrows + 2;    // T rows z0-1 .. z0+nrows
+  float4 q[U];
+  float4 pl[NL];                  // planes of iteration it + 1
+#pragma unroll
+  for (int i = 0; i < NL; ++i) {
+    const float4 p0 = bld4(RPL[i], vcol, rowm(t0 - lag[i]));
+    pl[i] = bld4(RPL[i], vcol, rowm(t0 + 1 - lag[i]));
+    if (wv + 4 * i < NPL) cf[0][wv + 4 * i][lane] = p0;
+  }
+#pragma unroll
+  for (int s = 0; s < NB + NFD + PD; ++s) q[s] = bld4(R1, vcol, rowm(t0 - NB + s));
+  float4 halb[3], u0b[6];
+#pragma unroll
+  for (int d = 0; d < PD; ++d) {
+    halb[d] = bld4(R1, vhal, rowm(t0 + d));
+    u0b[2 + d] = bld4s(R0, vcol, rowm(t0 + d));   // slot (it + 2) % 6 holds row t0 + it
+  }
+  u0b[0] = bld4s(R0, vcol, rowm(t0 - 2));
+  u0b[1] = bld4s(R0, vcol, rowm(t0 - 1));
+  const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
+  float4 T[3] = {z4, z4, z4};
+  // blend weight of row t0 + lane (QUAD_MAX_ROWS keeps a run's rows in the lanes)
+  const int ringl = BOT ? NZ - 1 - (t0 + lane) : t0 + lane;
+  const int wlane = __float_as_int(bld1(RW, (unsigned)min(max(N2 - ringl, 0), N2) * 4u, 0u));
+  block_lds_sync();
+
+  for (int base = 0; base < niter; base += U) {
+#pragma unroll
+    for (int j = 0; j < U; ++j) {
+      const int it = base + j;   // base is a multiple of U, so it % L == j % L for L | 12
+      if (it >= niter) break;    // the same for the whole block
+      const int tt = t0 + it;
+      // planes of the next row to LDS, of the row after it from memory
+#pragma unroll
+      for (int i = 0; i < NL; ++i)
+        if (wv + 4 * i < NPL) cf[(j + 1) & 1][wv + 4 * i][lane] = pl[i];
+#pragma unroll
+      for (int i = 0; i < NL; ++i) pl[i] = bld4(RPL[i], vcol, rowm(tt + 2 - lag[i]));
+      q[(j + NB + NFD + PD) % U] = bld4(R1, vcol, rowm(tt + NFD + PD));
+      halb[(j + PD) % 3] = bld4(R1, vhal, rowm(tt + PD));
+      u0b[(j + 2 + PD) % 6] = bld4s(R0, vcol, rowm(tt + PD));
+      __builtin_amdgcn_sched_barrier(0);
+      // horizontal neighbours of row tt through LDS
+      const float4 qc = q[(j + NB) % U];
+      lds[wv][hpos] = halb[j % 3];
+      lds[wv][H / 4 + lane] = qc;
+      wave_lds_sync();
+      float4 win[NWIN];
+#pragma unroll
+      for (int t = 0; t < NWIN; ++t) win[t] = lds[wv][lane + t];
+      wave_lds_sync();
+      // pre-blend two-way values T of row tt (Add / BKAdd, kernel.cu:46-80, 339-380)
+      const float4 (*cr)[64] = cf[j & 1];
+      const float4 u0v = u0b[(j + 2) % 6], k0 = cr[0][lane], pv = cr[NFD + 1][lane];
+      float w1[4], tn[4];
+#pragma unroll
+      for (int jj = 0; jj < 4; ++jj)
+        w1[jj] = (float)((h1 * (double)compr(k0, jj)) * (double)compr(qc, jj));
+#pragma unroll
+      for (int l = 1; l <= NFD; ++l) {
+        const float4 kl = cr[l][lane];
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj) {
+          float s = compr(q[(j + NB - l + U) % U], jj) + compr(q[(j + NB + l) % U], jj);
+          s = __builtin_fmaf(s, hzx2_1, compr(win[(H + jj - l) >> 2], (H + jj - l) & 3));
+          s = s + compr(win[(H + jj + l) >> 2], (H + jj + l) & 3);
+          w1[jj] = __builtin_fmaf(compr(kl, jj), s, w1[jj]);
+        }
+      }
+#pragma unroll
+      for (int jj = 0; jj < 4; ++jj) {
+        float Tn = combine_p(compr(qc, jj), compr(u0v, jj), compr(pv, jj), w1[jj], f64comb);
+        if (MODE == FR_FWD) Tn = (tt == srow && c0 + jj == sg.r_x) ? Tn + a.wav : Tn;
+        tn[jj] = Tn;
+      }
+      if (MODE == FR_RCV && tt == srow) {
+        const float4 ev = dat[threadIdx.x];
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj) tn[jj] = compr(ev, jj) != 0.0f ? compr(ev, jj) : tn[jj];
+      }
+      T[j % 3] = make_float4(tn[0], tn[1], tn[2], tn[3]);
+      __builtin_amdgcn_sched_barrier(0);
+      // one-way value and blend of row z = tt - 1 (written from the third row on)
+      const int z = tt - 1;
+      const float4 T0v = T[(j + 2) % 3];
+      const float4 Tinv = BOT ? T[(j + 1) % 3] : T[j % 3];
+      const float4 U1zv = q[(j + NB - 1) % U];
+      const float4 U1iv = BOT ? q[(j + NB - 2) % U] : q[(j + NB) % U];
+      const float4 U0zv = u0b[(j + 1) % 6];
+      const float4 U0iv = BOT ? u0b[j % 6] : u0b[(j + 2) % 6];
+      const float Tl = __shfl_up(Tinv.w, 1), Tr = __shfl_down(Tinv.x, 1);
+      const float Ul = __shfl_up(U0zv.w, 1), Ur = __shfl_down(U0zv.x, 1);
+      const float wgt = __int_as_float(__builtin_amdgcn_readlane(wlane, max(it - 1, 0)));
+      const float4 tvv = cr[NFD + 2][lane], div = cr[NFD + 3][lane], sqv = cr[NFD + 4][lane];
+      float val[4];
+#pragma unroll
+      for (int jj = 0; jj < 4; ++jj) {
+        const float T0 = compr(T0v, jj), Tin = compr(Tinv, jj);
+        const float U1z = compr(U1zv, jj), U1i = compr(U1iv, jj);
+        const float U0z = compr(U0zv, jj), U0i = compr(U0iv, jj);
+        const float Til = jj == 0 ? Tl : compr(Tinv, jj - 1);
+        const float Tir = jj == 3 ? Tr : compr(Tinv, jj + 1);
+        const float U0l = jj == 0 ? Ul : compr(U0zv, jj - 1);
+        const float U0r = jj == 3 ? Ur : compr(U0zv, jj + 1);
+        const float t1 = compr(tvv, jj) * ((Tin - U0i) + U0z);
+        const float t2 = ((((-2.0f * U1z) + U0z) + Tin) - 2.0f * U1i) + U0i;
+        const float lap = ((((Tir - 2.0f * Tin) + Til) + U0r) - 2.0f * U0z) + U0l;
+        const float t3 = compr(sqv, jj) * lap;
+        const float O = compr(div, jj) * ((t1 - t2) + t3);
+        val[jj] = (1.0f - wgt) * T0 + wgt * O;
+      }
+      const bool rowout = it >= 2 && z < z0 + nrows;
+      const unsigned rz = rowm(z);
+      bst4s(R2, vst | (rowout ? 0u : kDrop), rz, val[0], val[1], val[2], val[3]);
+      if (MODE == FR_FWD) {  // Hybrid3 (kernel.cu:184-208)
+        const bool strow = BOT ? (z >= NZ - N2 && z < NZ - N2 + g.nfd) : (z >= N2 - g.nfd && z < N2);
+        if (rowout && strow) {
+          const int sbase = BOT ? 2 * sa + sbb + (z - (NZ - N2)) * sg.mnx - N2
+                                : 2 * sa + (N2 - 1 - z) * sg.mnx - N2;
+          bst4s(RS, out ? (unsigned)(sbase + c0) * 4u : kDrop, 0u, val[0], val[1], val[2], val[3]);
+        }
+      }
+      block_lds_sync();
+    }
+  }
+}
+
+// The whole frame of a forward or receiver step of such a batch in one launch:
+// the blocks of frame_quad_body, shot group fastest, then those of k_frame.
+// Against one launch of k_frame on every cell or, for large batches, one each of
+// k_frame and k_frame4 (whichever the autotuner had chosen), half-length 3, us a
+// step: 128 shots of 351 x 1701 forward 112 -> 77, receiver field (half of the
+// launches with the restore of two strip sets) 106 -> 86; 32 shots 50 -> 28; 16
+// shots 24 -> 21.  77 us move 140 MB, 26 us at the rate of a large copy: waves
+// march 30 rows at about 1 us a row.
+template <int NFD, int MODE>
+__global__ __launch_bounds__(256, NFD <= 3 ? 3 : 2) void k_frame_quad(const FrameArgs a) {
+  __shared__ float4 cf[2][NFD + 5][64];
+  __shared__ float4 lds[4][64 + 2 * ((NFD + 3) / 4)];
+  __shared__ float4 dat[MODE == FR_RCV ? 256 : 1];
+  unsigned b = blockIdx.x;
+  if (b < (unsigned)a.nquad) {
+    const unsigned nsg = ((unsigned)a.nshot + 3u) >> 2;
+    const int s4 = (int)(b % nsg) * 4;
+    const unsigned t = b / nsg;
+    const int w = (int)(t % (unsigned)a.qwin), r = (int)(t / (unsigned)a.qwin);
+    const int zr = (r >> 1) * a.qrows, rows = min(a.qrows, a.g.n2 - zr), cs = a.g.n2 + 248 * w;
+    if (r & 1) frame_quad_body<NFD, MODE, true>(a, a.g.nz - a.g.n2 + zr, rows, cs, s4, cf, lds, dat);
+    else frame_quad_body<NFD, MODE, false>(a, zr, rows, cs, s4, cf, lds, dat);
+    return;
+  }
+  frame_records_body<NFD, MODE>(a, b - (unsigned)a.nquad);
+}
+#endif
 
 // One time step's interior and frame work in one launch.  The two write
 // disjoint cells of u(k+1) and only read u(k), u(k-1) and the model, so they
@@ -994,7 +1282,7 @@ __global__ __launch_bounds__(256) void k_step(const IntArgs ia, const FrameArgs 
   const unsigned before = min(nfu, (u + R - 1u) / R);  // frame units ahead of unit u
   if (u % R == 0u && u / R < nfu) {
     const unsigned b = (u / R) * 8u + s8;
-    if (b < nfr) frame_body<NFD, MODE>(fa, b);
+    if (b < nfr) frame_records_body<NFD, MODE>(fa, b);
   } else {
     const unsigned b = (u - before) * 8u + s8;
     if (b < nint) interior_body<NFD, EPI>(ia, b);
@@ -1037,6 +1325,20 @@ hipError_t StencilOps<RTM_NFD>::frame4(int mode, dim3 grid, const FrameArgs& a, 
   const dim3 block(256);
   if (mode == FR_FWD) hipLaunchKernelGGL((k_frame4<N, FR_FWD>), grid, block, 0, s, a);
   else if (mode == FR_RCV) hipLaunchKernelGGL((k_frame4<N, FR_RCV>), grid, block, 0, s, a);
+  else return hipErrorInvalidValue;
+  return hipGetLastError();
+#else
+  return hipErrorInvalidValue;
+#endif
+}
+
+template <>
+hipError_t StencilOps<RTM_NFD>::frame_quad(int mode, dim3 grid, const FrameArgs& a, hipStream_t s) {
+#if RTM_NFD <= 5
+  constexpr int N = RTM_NFD;
+  const dim3 block(256);
+  if (mode == FR_FWD) hipLaunchKernelGGL((k_frame_quad<N, FR_FWD>), grid, block, 0, s, a);
+  else if (mode == FR_RCV) hipLaunchKernelGGL((k_frame_quad<N, FR_RCV>), grid, block, 0, s, a);
   else return hipErrorInvalidValue;
   return hipGetLastError();
 #else

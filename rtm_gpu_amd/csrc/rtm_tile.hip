@@ -189,22 +189,15 @@ __global__ __launch_bounds__(512) void k_tile(const TileArgs a) {
     }
   }
   // one-way operands of the frame cells (kernel.cu:116-183) and their strips
-  float vp[CPT] = {}, vq[CPT] = {}, r1v[CPT] = {}, wgt[CPT] = {}, ring[CPT] = {};
+  float vp[CPT] = {}, fsv[CPT] = {}, r1v[CPT] = {}, wgt[CPT] = {}, ring[CPT] = {};
   int se[CPT];
 #pragma unroll
   for (int j = 0; j < CPT; ++j) {
     se[j] = -1;
     if (!edge || !cell[j] || inner[j]) continue;
-    // the Q1 velocity: the cell itself on the top edge; Dv[(N2-x)*NX+y] on the
-    // bottom and Dv[(N2-y)*NX+x] on the sides (kernel.cu:128,132,136): row z of
-    // the model as a linear index is row z / NX, column z % NX
     const int z = zw + j, ar = min(min(z, x), min(NZ - 1 - z, NX - 1 - x));
-    const bool topc = z == ar, botc = !topc && z == NZ - 1 - ar;
-    const int zdiv = z / NX, zmod = z - zdiv * NX;
-    const int zq = min(max(topc ? z : (botc ? ar : ar + zdiv), 0), NZ - 1);
-    const int xq = min(max(topc || botc ? x : zmod, 0), NX - 1);
     vp[j] = ldg(m.v + mo, own[j]);
-    vq[j] = ldg(m.v + mo, at(zq, xq));
+    fsv[j] = ldg(m.fs + mo, own[j]);
     r1v[j] = ldg(m.r1 + mo, own[j]);
     wgt[j] = m.w[min(max(N2 - ar, 0), N2)];
     se[j] = strip_elem(g, NX, sg.mnx, z, x);
@@ -335,7 +328,7 @@ __global__ __launch_bounds__(512) void k_tile(const TileArgs a) {
         const float t2 = ((((-2.0f * U1z) + U0z) + Ti) - 2.0f * U1i) + U0i;
         const float lap = ((((T[ri + lat] - 2.0f * Ti) + T[ri - lat]) + s0[rc + lat]) - 2.0f * U0z) +
                           s0[rc - lat];
-        const float t3 = ((m.taoh2 * vq[j]) * vq[j]) * lap;
+        const float t3 = fsv[j] * lap;
         const float num_s = (t1 - t2) + t3;
         const float den_s = tv + 1.0f;
         const float O = (1.0f / (corner ? den_c : den_s)) * (corner ? num_c : num_s);

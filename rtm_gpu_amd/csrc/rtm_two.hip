@@ -35,13 +35,6 @@
 
 namespace rtm {
 
-// Barrier of the block for LDS data alone: loads from memory stay in flight.
-__device__ __forceinline__ void block_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 template <int NFD, int KIND>
 __global__ __launch_bounds__(256, 2) void k_two(const TwoArgs a) {
   constexpr bool RCV = KIND == TWO_RCV0 || KIND == TWO_RCV, IMG = KIND == TWO_RCV;

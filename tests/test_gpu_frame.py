@@ -1,0 +1,69 @@
+"""The frame kernels where their shapes change: bands that pack into one wave
+and bands that do not, runs longer than a wave's lanes, against the oracle; the
+whole frame in one launch (large batches) against the marching frame kernel."""
+import numpy as np
+import pytest
+
+from cases import build_case, hip_context, oracle_engine, synth_gather
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("mod_nz,mod_nx,n2,nfdmax,ilste", [
+    (30, 37, 10, 3, 1),    # both side bands in one wave
+    (45, 60, 30, 5, 0),    # the widest that pack
+    (37, 70, 31, 4, 1),    # one wave per side
+    (20, 300, 66, 10, 1)])  # two waves per side, more bands than interior
+@pytest.mark.parametrize("frame_split", [0, 1])
+def test_marched_frame_equals_oracle(mod_nz, mod_nx, n2, nfdmax, ilste, frame_split):
+    from rtm_gpu_amd import hip
+    case = build_case(name="frame", mod_nz=mod_nz, mod_nx=mod_nx, n2=n2, nfdmax=nfdmax, ilste=ilste,
+                      nt=120, tao=0.0008, src_x1=9)
+    nt, inner = case["cfg"]["nt"], (slice(n2, -n2), slice(n2, -n2))
+    seis = synth_gather(case)
+    e = oracle_engine(case)
+    ctx = hip_context(case, nshot=1, zseg=16, frame_split=frame_split)
+    ctx.set_gathers(seis[None])
+    e.forward_begin()
+    ctx.forward_begin()
+    for n in (3, nt):
+        e.forward_advance(n)
+        ctx.forward_advance(n)
+        assert np.array_equal(ctx.field(hip.FIELD_U), e.field(0)), n
+    e.backward_begin(seis)
+    ctx.backward_begin()
+    for n in (3, nt):
+        e.backward_advance(n)
+        ctx.backward_advance(n)
+        assert np.array_equal(ctx.field(hip.FIELD_Q), e.field(2)), n
+        assert np.array_equal(ctx.field(hip.FIELD_I1)[inner], e.field(3)[inner]), n
+    ctx.close()
+
+
+@pytest.mark.parametrize("nz,nx,n2,nfdmax,ilste", [
+    (400, 578, 12, 3, 1),   # the narrowest frame with windows of four columns
+    (370, 601, 31, 5, 1),   # one wave per side
+    (300, 497, 64, 4, 0)])  # more rows than a block takes, two corner records
+def test_whole_frame_launch(nz, nx, n2, nfdmax, ilste):
+    from rtm_gpu_amd import hip
+    shots = -(-10_000_000 // ((nz + 2 * n2) * (nx + 2 * n2)))
+    shots += (2 - shots) % 4  # two of a block's four past the batch
+    case = build_case(name="quad", mod_nz=nz, mod_nx=nx, n2=n2, nfdmax=nfdmax, ilste=ilste, nt=41,
+                      nshot=shots, depth_step=6.0, src_x1=50, tao=0.0008)
+    rng = np.random.default_rng(n2)
+    seis = (0.01 * rng.standard_normal((shots, case["cfg"]["n"], 41))).astype(np.float32)
+    out = []
+    for zseg in (0, 16):  # 16 rows per wave: one step per launch
+        ctx = hip_context(case, nshot=shots, zseg=zseg)
+        ctx.set_gathers(seis)
+        ctx.forward_begin()
+        ctx.forward_advance(41)
+        got = [ctx.field(w, shot=s) for s in (0, shots - 1) for w in (hip.FIELD_U, hip.FIELD_U_PREV)]
+        got += [ctx.strip(shots - 1, k) for k in (20, 39)]
+        ctx.backward_begin()
+        ctx.backward_advance(41)
+        got += [ctx.field(w, shot=s) for s in (0, shots - 1) for w in (hip.FIELD_Q, hip.FIELD_I1)]
+        out.append(got)
+        ctx.close()
+    for i, (a, b) in enumerate(zip(*out)):
+        assert np.array_equal(a, b), i
