@@ -422,18 +422,21 @@ hipError_t launch_frame_split(rtm_ctx* c, int mode, FrameArgs f) {
 }
 
 // Rows per wave of k_two where the autotuner has not chosen: the height whose
-// blocks, two to a CU at a time, take the fewest rounds times iterations
-// (rows + 2 NFD).
+// blocks, two to a CU at a time (three where the kernel's registers allow),
+// take the fewest rounds times iterations (rows + 2 NFD).  32 shots forward
+// 87 us for three, 91 for two.
 int zs2_for(const rtm_ctx* c, int kind) {
   if (c->zs2[kind] > 0) return c->zs2[kind];
   const int ql = 2 * c->nfd + 3, cols = two_cols(c->g, c->nfd, c->nshot);
   const long long per = (long long)((c->g.mnx + cols - 1) / cols) * ((c->nshot + TWO_SHOTS - 1) / TWO_SHOTS);
+  const bool three = c->nfd <= 3 && (kind == TWO_FWD || kind == TWO_RCV0);  // 168 registers
+  const long long res = three ? 768 : 512;
   int best = 0;
   long long cost = 0;
   for (int m : {11, 8, 6, 4, 3, 2}) {
     const int rows = m * ql - 2 * c->nfd;
     const long long blocks = per * ((c->g.mnz + rows - 1) / rows);
-    const long long v = (blocks + 511) / 512 * (m * ql);
+    const long long v = (blocks + res - 1) / res * (m * ql);
     if (best == 0 || v < cost) { best = rows; cost = v; }
   }
   return best;
