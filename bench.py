@@ -206,17 +206,22 @@ def run_apertures(a):
     print(json.dumps(out), flush=True)
 
 
-def algorithmic_bytes(kind, d, n2, nfd, nshot, n):
+def algorithmic_bytes(kind, d, n2, nfd, nshot, n, two=False):
     """Minimum HBM bytes one launch of each kernel must move.  Per interior
     cell and shot: forward / source reconstruction read u1, u0 and write u2
-    (12 B), and so does the receiver step; every third one also images.  The
-    velocity model is shared by
-    the shots of a launch (4 B per cell per launch)."""
+    (12 B), and so does the receiver step; every third one also images.  A
+    launch of two steps (two) reads two fields and writes two (16 B), and every
+    second one of the receiver field images four steps.  The velocity model is
+    shared by the shots of a launch (4 B per cell per launch)."""
     from rtm_gpu_amd import hip
     nz, nx = d.nz, d.nx
     nI = (nz - 2 * n2) * (nx - 2 * n2)
     nF = nz * nx - nI
     ss = 2 * nfd * ((nz - 2 * n2) + (nx - 2 * n2))
+    if two and kind in (hip.K_FWD_INTERIOR, hip.K_SRC_INTERIOR, hip.K_RCV_INTERIOR):
+        return nshot * nI * 16 + nI * 4
+    if two and kind == hip.K_RCVI_INTERIOR:  # and u(k+2) .. u(k-1), q(k+2), the sums and images
+        return nshot * (nI * 68 + 2 * n * 4) + nI * 4
     if kind == hip.K_FWD_INTERIOR or kind == hip.K_SRC_INTERIOR:
         return nshot * nI * 12 + nI * 4
     if kind == hip.K_FWD_FRAME:
@@ -853,6 +858,11 @@ def main():
         hip.K_FWD_INTERIOR: (hip.K_FWD_FRAME, "k_step<EPI_FWD+FR_FWD>"),
         hip.K_RCV_INTERIOR: (hip.K_RCV_FRAME, "k_step<EPI_RCV0+FR_RCV>"),
         hip.K_RCVI_INTERIOR: (hip.K_RCV_FRAME, "k_step<EPI_RCV+FR_RCV>")}
+    # A batch that takes two steps per launch runs two frame launches to one of
+    # the interior (k_two).
+    interior_kinds = (hip.K_FWD_INTERIOR, hip.K_SRC_INTERIOR, hip.K_RCV_INTERIOR,
+                      hip.K_RCVI_INTERIOR)
+    two = ctx.kernel_time(hip.K_FWD_FRAME)[1] > 1.5 * ctx.kernel_time(hip.K_FWD_INTERIOR)[1]
     # Without a checkpoint snapshot (none here) and with separate launches, the
     # receiver frame launch of every backward step also restores the strips of
     # the reconstructed field (k_strip_restore's work and bytes).
@@ -863,7 +873,9 @@ def main():
         except hip.RtmError:  # a kind this build of the library does not time
             continue
         if n:
-            b = algorithmic_bytes(k, d, cfg.n2, cfg.nfdmax, a.shots, cfg.n)
+            b = algorithmic_bytes(k, d, cfg.n2, cfg.nfdmax, a.shots, cfg.n, two)
+            if two and k in interior_kinds:
+                name = name.replace("k_interior<EPI_", "k_two<TWO_")
             if k in fusedk and ctx.kernel_time(fusedk[k][0])[1] == 0:
                 b += algorithmic_bytes(fusedk[k][0], d, cfg.n2, cfg.nfdmax, a.shots, cfg.n)
                 name = fusedk[k][1]

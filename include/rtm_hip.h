@@ -53,7 +53,8 @@ enum {
 
 /* Kernel kinds for rtm_kernel_time().  Small batches run a whole step in one
  * launch, which counts under the interior kind of its pass (the receiver kinds
- * for a backward step).  Otherwise a frame kind times the frame launches
+ * for a backward step).  Large batches run two steps of a field's interior in
+ * one launch, then counted once.  Otherwise a frame kind times the frame launches
  * of one step together; on migration and adjoint steps without a checkpoint
  * snapshot (and with separate launches) RTM_K_RCV_FRAME / RTM_K_ADJ_FRAME
  * include the strip restore of the reconstructed field, which
@@ -62,8 +63,8 @@ enum {
   RTM_K_FWD_INTERIOR = 0, RTM_K_FWD_FRAME = 1, RTM_K_SRC_INTERIOR = 2, RTM_K_STRIP_RESTORE = 3,
   RTM_K_RCV_INTERIOR = 4, RTM_K_RCV_FRAME = 5, RTM_K_BORN_INTERIOR = 6, RTM_K_BORN_FRAME = 7,
   RTM_K_ADJ_INTERIOR = 8, RTM_K_ADJ_FRAME = 9,
-  /* RTM_K_RCVI_INTERIOR: the receiver steps that apply image terms (of up to
-   * three steps at once); RTM_K_RCV_INTERIOR: those that do not.
+  /* RTM_K_RCVI_INTERIOR: the receiver launches that apply image terms (of up to
+   * three steps at once, four where a launch takes two steps); RTM_K_RCV_INTERIOR: those that do not.
    * RTM_K_SRCI_INTERIOR is no longer launched. */
   RTM_K_SRCI_INTERIOR = 10, RTM_K_RCVI_INTERIOR = 11, RTM_K_NKINDS = 12
 };
@@ -109,7 +110,9 @@ typedef struct rtm_params {
                             the whole frame in the one-column kernel.  Results are the
                             same bit for bit; the split pays only on large batches (its
                             launch takes about as long for one shot as for 128), so
-                            rtm_autotune times both and keeps the faster. */
+                            rtm_autotune times both and keeps the faster.  Batches that
+                            take two steps per launch run the whole frame in a kernel of
+                            their own instead. */
 } rtm_params;
 
 /* One shot of a ragged batch (uneven apertures; not in the reference, whose
@@ -291,7 +294,8 @@ int rtm_data_dot_noalloc(const float* x, const float* y, long long n, long long 
  * frame kernels' row runs (rtm_set_frame_runs) are timed the same way, top and
  * bottom bands first, on the sum of both frame kernels' times, and last the
  * frame split (rtm_params.frame_split) on and off, and the tuned kernels
- * against whole steps in one launch. */
+ * against whole steps in one launch.  Large batches also time two steps per
+ * launch, with heights of their own, against one. */
 int rtm_autotune(rtm_ctx* ctx, int nsteps, int* zseg);
 /* The autotuner's three choices set by hand: rows per wave of the forward,
  * the source-reconstruction and the receiver-step kernels (Born and the

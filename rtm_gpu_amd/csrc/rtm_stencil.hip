@@ -1243,8 +1243,9 @@ __device__ __forceinline__ void frame_quad_body(const FrameArgs& a, const int z0
 // k_frame and k_frame4 (whichever the autotuner had chosen), half-length 3, us a
 // step: 128 shots of 351 x 1701 forward 112 -> 77, receiver field (half of the
 // launches with the restore of two strip sets) 106 -> 86; 32 shots 50 -> 28; 16
-// shots 24 -> 21.  77 us move 140 MB, 26 us at the rate of a large copy: waves
-// march 30 rows at about 1 us a row.
+// shots 24 -> 21.  Counters of 128 shots: 0.34 GB a step, 140 MB of it results
+// and their operands, at 4 TB/s: halo rows of the runs, and side bands that take
+// a part of every line they touch.
 template <int NFD, int MODE>
 __global__ __launch_bounds__(256, NFD <= 3 ? 3 : 2) void k_frame_quad(const FrameArgs a) {
   __shared__ float4 cf[2][NFD + 5][64];

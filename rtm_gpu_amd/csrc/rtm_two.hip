@@ -22,11 +22,12 @@
 // at half-length 3 (128 reverse-VSP shots), one step per launch 2 x 212.
 // Measured on 128 shots of 351 x 1701, us for two steps (two launches of
 // k_interior): forward 298 (424) at half-length 3, 354 (532) at 5; the receiver
-// field, four steps with their images, 1434 (1790).  298 us are 4.5 TB/s of the
-// pass's reads and writes (halo rows and columns included), against 5.4 TB/s of
-// a streaming kernel: the four waves wait for each other at every row.  At half-length 6 the 256
-// registers of two waves per SIMD spill (469 against 510 us; 137 against 106 on
-// 24 shots): not built.
+// field, four steps with their images, 1434 (1790).  Counters at half-length 4:
+// 1.59 GB for two forward steps (1.22 are the fields, the rest halo rows and
+// columns) and 6.10 GB with the images of four, 5.2-5.3 TB/s, the rate of a
+// streaming kernel (5.3).  Imaging operands loaded a row ahead (253 registers)
+// changed nothing.  At half-length 6 the 256 registers of two waves per SIMD
+// spill (469 against 510 us; 137 against 106 on 24 shots): not built.
 //
 // Every cell takes the operations of k_interior in their order: same bits.
 #include <hip/hip_runtime.h>
