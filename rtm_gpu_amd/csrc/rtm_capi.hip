@@ -330,11 +330,13 @@ constexpr long long kTileWork = 50000000;
 
 // Two steps per launch (k_two) for the forward and backward passes of a
 // migration: half-lengths up to 5, every four consecutive shots on one model
-// window.  Measured (k_two / marching / k_tile, migration of 351 x 1701 shots,
-// ms per 100 steps, not tuned): 8.7 M cells 16.6 / 17.0 / 15.3, 11.6 M 18.5 /
-// 20.6 / 19.3, 17.4 M 23.2 / 25.6 / 28.8, 34.7 M 41.6 / 46.2 / 56.4; of 200 x
-// 400 shots, 6.8 M cells 16.4 / 16.3 / 15.8, 10.1 M 17.6 / 20.1 / 24.1.
-constexpr long long kTwoCells = 10000000;
+// window.  k_two marches and needs a batch that fills the GPU, k_tile's work per
+// cell grows with the half-length.  Measured (k_two / k_tile, migration of 351 x
+// 1701 shots, ms per 100 steps, not tuned): half-length 2, 4.3 M cells 8.1 / 7.4,
+// 5.8 M 8.8 / 9.0, 8.7 M 11.2 / 14.5; 3, 5.8 M 10.2 / 9.3, 7.2 M 12.6 / 12.6,
+// 8.7 M 13.2 / 15.2; 5, 7.2 M 17.9 / 13.7, 8.7 M 18.4 / 16.4, 10.1 M 18.8 / 18.8.
+// Against k_interior: 11.6 M cells 18.5 / 20.6, 34.7 M 41.6 / 46.2.
+constexpr long long two_cells(int nfd) { return 3000000 + 1400000ll * nfd; }
 bool two_possible(const rtm_ctx* c) {
   return c->F[3] && c->Q[3] && c->nfd <= TWO_MAX_NFD && c->nshot >= TWO_SHOTS && c->quads &&
          !c->p.fuse_frame && c->cp_ok;
@@ -342,7 +344,7 @@ bool two_possible(const rtm_ctx* c) {
 bool use_two(const rtm_ctx* c) {
   if (!two_possible(c) || c->tile_tuned == 1) return false;
   if (c->two_tuned >= 0) return c->two_tuned != 0;
-  return !c->march_set && c->cells >= kTwoCells;
+  return !c->march_set && c->cells >= two_cells(c->nfd);
 }
 
 bool use_tile(const rtm_ctx* c, int pass) {
@@ -1147,7 +1149,7 @@ int rtm_create(const rtm_params* p, rtm_ctx** out) {
   // an eighth of the card for what is allocated later: without them every
   // launch takes one step.
   size_t mem_free = 0, mem_all = 0;
-  if ((long long)p->max_shots * g.nz * g.nx >= kTwoCells && p->max_shots >= TWO_SHOTS &&
+  if ((long long)p->max_shots * g.nz * g.nx >= two_cells(1) && p->max_shots >= TWO_SHOTS &&
       hipMemGetInfo(&mem_free, &mem_all) == hipSuccess &&
       mem_free >= 2 * fb * sizeof(float) + mem_all / 8) {
     if (dalloc_t(c, &c->F[3], fb) == RTM_OK && dalloc_t(c, &c->Q[3], fb) != RTM_OK)
