@@ -58,6 +58,7 @@ struct rtm_ctx {
   int4* d_tiles = nullptr;     // frame (tile, shot) records of the batch
   int ntiles = 0, tile_cap = 0;  // FRAME_ALL records; capacity of d_tiles
   int nsplit = 0, nvec = 0;      // FRAME_SCALAR and FRAME_VEC records after them
+  size_t fs_cap = 0;  // planes of d_fs
   int qrows = 0;  // rows per block of k_frame_quad; 0: quad_rows
   int fseg_tb = 0, fseg_side = 0;  // rows per frame record: top/bottom bands, side bands
   // model windows of a ragged batch (allocated on first use): slot w holds
@@ -888,6 +889,38 @@ void build_tiles(const Grid& g, int nx, int shot, int seg_tb, int seg, int kind,
 }
 
 int choose_zs(rtm_ctx* c, int nshot);
+// With one model for all shots: a plane of Model::fs per width of the batch
+// (the side and bottom cells' factors depend on it), the widest shot's first.
+// Windows of their own bring theirs (rtm_set_shot_model).
+int lateral_planes(rtm_ctx* c) {
+  if (!c->model_ok || c->m.mstride != 0) return RTM_OK;
+  const Grid& g = c->g;
+  std::vector<int> widths{g.nx};
+  for (ShotGeo& q : c->geo) {
+    size_t i = 0;
+    while (i < widths.size() && widths[i] != q.nx) ++i;
+    if (i == widths.size()) widths.push_back(q.nx);
+    q.fw = (int)i;
+  }
+  if (widths.size() > c->fs_cap) {
+    float* p = nullptr;
+    const int rc = dalloc_t(c, &p, widths.size() * g.fstride);
+    if (rc != RTM_OK) return rc;
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    dfree_t(c, &c->d_fs, c->fs_cap * g.fstride);
+    c->d_fs = p;
+    c->fs_cap = widths.size();
+  }
+  for (size_t i = 0; i < widths.size(); ++i)
+    HIPCHK(c, launch_frame_lat(g, widths[i], c->d_v, c->p.taoh2, c->d_fs + i * g.fstride, c->stream));
+  c->m.fs = c->d_fs;
+  if (!c->geo.empty()) {
+    HIPCHK(c, hipMemcpyAsync(c->d_geo, c->geo.data(), c->geo.size() * sizeof(ShotGeo), hipMemcpyHostToDevice, c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+  }
+  return RTM_OK;
+}
+
 void drop_graph(rtm_ctx* c);
 
 // The batch's frame records for the context's run lengths, three lists one
@@ -930,7 +963,9 @@ int upload_frame_records(rtm_ctx* c) {
 int upload_geometry(rtm_ctx* c) {
   const int ns = (int)c->geo.size();
   HIPCHK(c, hipMemcpyAsync(c->d_geo, c->geo.data(), ns * sizeof(ShotGeo), hipMemcpyHostToDevice, c->stream));
-  int rc = upload_frame_records(c);
+  int rc = lateral_planes(c);
+  if (rc != RTM_OK) return rc;
+  rc = upload_frame_records(c);
   if (rc != RTM_OK) return rc;
   if (ns != c->nshot) c->tile_tuned = c->two_tuned = -1;  // tuned for another batch
   c->cells = 0;
@@ -950,7 +985,7 @@ int upload_geometry(rtm_ctx* c) {
 // velocity bin's coefficient row (kernel.cu:55-56: FP32 quotient, double +
 // 0.5, truncation, clamped to the table).  Guard columns repeat the edge.
 int upload_model_window(rtm_ctx* c, int nx, const float* v, const float* r1, float* dv_, float* dr_,
-                        float* dp_, unsigned* dk_, float* df_) {
+                        float* dp_, unsigned* dk_) {
   const Grid& g = c->g;
   std::vector<float> pv((size_t)g.fstride, 0.f), pr((size_t)g.fstride, 0.f), pp((size_t)g.fstride);
   std::vector<unsigned> pk((size_t)g.fstride);
@@ -976,7 +1011,6 @@ int upload_model_window(rtm_ctx* c, int nx, const float* v, const float* r1, flo
   HIPCHK(c, hipMemcpyAsync(dr_, pr.data(), b, hipMemcpyHostToDevice, c->stream));
   HIPCHK(c, hipMemcpyAsync(dp_, pp.data(), b, hipMemcpyHostToDevice, c->stream));
   HIPCHK(c, hipMemcpyAsync(dk_, pk.data(), b, hipMemcpyHostToDevice, c->stream));
-  HIPCHK(c, launch_frame_lat(g, nx, dv_, c->p.taoh2, df_, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   return RTM_OK;
 }
@@ -1067,6 +1101,7 @@ int rtm_create(const rtm_params* p, rtm_ctx** out) {
   if (rc == RTM_OK) rc = dalloc_t(c, &c->d_v, (size_t)g.fstride);
   if (rc == RTM_OK) rc = dalloc_t(c, &c->d_r1, (size_t)g.fstride);
   if (rc == RTM_OK) rc = dalloc_t(c, &c->d_fs, (size_t)g.fstride);
+  c->fs_cap = 1;
   if (rc == RTM_OK) rc = dalloc_t(c, &c->d_pm, (size_t)g.fstride);
   if (rc == RTM_OK) rc = dalloc_t(c, &c->d_ko, (size_t)g.fstride);
   if (rc == RTM_OK) rc = dalloc_t(c, &c->d_w, (size_t)g.n2 + 1);
@@ -1230,7 +1265,7 @@ int rtm_set_model(rtm_ctx* c, const float* v, const float* r1, const float* w, c
   }
   HIPCHK(c, hipMemcpyAsync(c->d_ctab, tab.data(), tab.size() * sizeof(float), hipMemcpyHostToDevice, c->stream));
   c->tab_vmin = vmin; c->tab_dv = dv; c->tab_nrow = nrow; c->tab_cs = CS; c->tab_ls = ls;
-  rc = upload_model_window(c, g.nx, v, r1, c->d_v, c->d_r1, c->d_pm, c->d_ko, c->d_fs);
+  rc = upload_model_window(c, g.nx, v, r1, c->d_v, c->d_r1, c->d_pm, c->d_ko);
   if (rc != RTM_OK) return rc;
   HIPCHK(c, hipMemcpyAsync(c->d_w, w, (g.n2 + 1) * sizeof(float), hipMemcpyHostToDevice, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -1250,7 +1285,7 @@ int rtm_set_model(rtm_ctx* c, const float* v, const float* r1, const float* w, c
   c->tp_ok = c->cp_ok = false;
   drop_graph(c);
   c->model_ok = true;
-  return RTM_OK;
+  return lateral_planes(c);
 }
 
 int rtm_set_wavelet(rtm_ctx* c, const float* wav) {
@@ -1355,7 +1390,9 @@ int rtm_set_shot_model(rtm_ctx* c, int shot, const float* v, const float* r1) {
       if (c->win_ref[i] == 0) w = i;
     if (w < 0) return fail(c, RTM_E_STATE, "no free model window slot");
     const size_t o = (size_t)w * g.fstride;
-    int rc = upload_model_window(c, nx, v, r1, c->d_mv + o, c->d_mr1 + o, c->d_mpm + o, c->d_mko + o, c->d_mfs + o);
+    int rc = upload_model_window(c, nx, v, r1, c->d_mv + o, c->d_mr1 + o, c->d_mpm + o, c->d_mko + o);
+    if (rc == RTM_OK && launch_frame_lat(g, nx, c->d_mv + o, c->p.taoh2, c->d_mfs + o, c->stream) != hipSuccess)
+      rc = fail(c, RTM_E_HIP, "lateral factors of shot %d", shot);
     if (rc != RTM_OK) {
       c->shot_model[shot] = 0;
       return rc;
@@ -1367,6 +1404,7 @@ int rtm_set_shot_model(rtm_ctx* c, int shot, const float* v, const float* r1) {
     }
   c->win_ref[w] += 1;
   c->geo[shot].win = w;
+  c->geo[shot].fw = w;
   HIPCHK(c, hipMemcpyAsync(c->d_geo + shot, &c->geo[shot], sizeof(ShotGeo), hipMemcpyHostToDevice, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   Model& m = c->m;

@@ -23,7 +23,8 @@ struct Model {
   const float* v;
   const float* r1;
   // (taoh2*vq)*vq of the frame cell's one-way update, vq the velocity that the
-  // reference reads there (launch_frame_lat), padded layout
+  // reference reads there (launch_frame_lat), padded layout, fstride per plane
+  // ShotGeo::fw
   const float* fs;
   const float* pm;     // v*v*tao2*h2 per cell (FP32, left to right), padded layout
   const unsigned* ko;  // byte offset of the cell's coefficient row in ctab, padded layout
@@ -56,6 +57,7 @@ struct ShotGeo {
   int r_u, r_x;        // source
   int x_img;           // image column of interior column 0
   int win;             // model window of the shot (Model::mstride apart; 0 with one model)
+  int fw;              // its plane of Model::fs: the window's, or with one model its width's
 };
 
 // Strip storage: fp32, or fp16/bf16 with a per-(shot, slot) scale.
@@ -157,9 +159,9 @@ struct TwoArgs {
   Model m;
   Rcv r;
   const ShotGeo* geo;
-  // planes of a model window, fstride apart: c_0 .. c_NFD, P, and the one-way
-  // operands of a top or bottom edge cell (kernel.cu:122-133): taoh v,
-  // 1 / (taoh v + 1), taoh2 vq vq.  A window's two_planes(nfd) planes are
+  // planes of a model window, fstride apart: c_0 .. c_NFD, P, and for the one-way
+  // update of a top or bottom edge cell (kernel.cu:122-133) taoh v and
+  // 1 / (taoh v + 1).  A window's two_planes(nfd) planes are
   // cpstride apart (0: one window)
   const float* cp;
   long long cpstride;
@@ -190,7 +192,7 @@ hipError_t launch_two(int kind, int nfd_inst, TwoArgs a, int nshot, hipStream_t 
 // Model::fs of a window nx columns wide from its velocities.
 hipError_t launch_frame_lat(const Grid& g, int nx, const float* v, float taoh2, float* fs, hipStream_t s);
 // Planes (TwoArgs::cp) of window win.
-constexpr int two_planes(int nfd) { return nfd + 5; }
+constexpr int two_planes(int nfd) { return nfd + 4; }
 hipError_t launch_coef_planes(const Grid& g, const Model& m, int win, int nfd, float* cp, hipStream_t s);
 
 // A whole time step in one launch, one cell per thread (rtm_tile.hip).

@@ -487,7 +487,6 @@ __global__ void k_coef_planes(const Grid g, const Model m, long long wo, int nfd
     const float tv = m.taoh * m.v[wo + i];
     cp[(nfd + 2) * fs + i] = tv;
     cp[(nfd + 3) * fs + i] = 1.0f / (tv + 1.0f);
-    cp[(nfd + 4) * fs + i] = m.fs[wo + i];
   }
 }
 

@@ -441,7 +441,7 @@ __device__ __forceinline__ void frame_body(const FrameArgs& a, const int4 rec) {
   const Rsrc R1 = rsrc(a.u1 + so, fb), R0 = rsrc(a.u0 + so, fb), R2 = rsrc(a.u2 + so, fb);
   const long long mo = (long long)sg.win * m.mstride;
   const Rsrc RP = rsrc(m.pm + mo, fb), RK = rsrc(m.ko + mo, fb);
-  const Rsrc RV = rsrc(m.v + mo, fb), RR = rsrc(m.r1 + mo, fb), RQ = rsrc(m.fs + mo, fb);
+  const Rsrc RV = rsrc(m.v + mo, fb), RR = rsrc(m.r1 + mo, fb), RQ = rsrc(m.fs + sg.fw * g.fstride, fb);
   const Rsrc RC = rsrc(m.ctab, (unsigned)(m.nrow * m.cs) * 4u);
   const Rsrc RW = rsrc(m.w, (unsigned)(N2 + 1) * 4u);
   const unsigned P4 = (unsigned)g.pitch * 4u;
@@ -806,7 +806,7 @@ __device__ __forceinline__ void frame_tb4_body(const FrameArgs& a, const int4 re
   const Rsrc R1 = rsrc(a.u1 + so, fb), R0 = rsrc(a.u0 + so, fb), R2 = rsrc(a.u2 + so, fb);
   const long long mo = (long long)sg.win * m.mstride;
   const Rsrc RP = rsrc(m.pm + mo, fb), RK = rsrc(m.ko + mo, fb), RV = rsrc(m.v + mo, fb);
-  const Rsrc RQ = rsrc(m.fs + mo, fb);
+  const Rsrc RQ = rsrc(m.fs + sg.fw * g.fstride, fb);
   const Rsrc RC = rsrc(m.ctab, (unsigned)(m.nrow * m.cs) * 4u);
   const Rsrc RW = rsrc(m.w, (unsigned)(N2 + 1) * 4u);
   const unsigned P4 = (unsigned)g.pitch * 4u;
@@ -1026,7 +1026,8 @@ __global__ __launch_bounds__(256) void k_frame(const FrameArgs a) {
 // The same cells for batches whose blocks of four shots share a model window
 // (k_two's): the four waves of a block march the band of four shots row by row
 // together, and the window's coefficient planes, P and the three one-way
-// operands (TwoArgs::cp) go through LDS, each plane loaded by one wave.  Seven
+// operands (TwoArgs::cp, Model::fs) go through LDS, each plane loaded by one
+// wave.  Seven
 // buffer instructions a row instead of eleven and no division; 155 registers
 // instead of 217 at half-length 3, three waves per SIMD.
 template <int NFD, int MODE, bool BOT>
@@ -1075,7 +1076,8 @@ __device__ __forceinline__ void frame_quad_body(const FrameArgs& a, const int z0
 #pragma unroll
   for (int i = 0; i < NL; ++i) {
     const int pl = wv + 4 * i;
-    RPL[i] = rsrc(cp + (long long)min(pl, NPL - 1) * g.fstride, pl < NPL ? fb : 0u);
+    const float* p = pl < NPL - 1 ? cp + pl * g.fstride : m.fs + sg.fw * g.fstride;
+    RPL[i] = rsrc(p, pl < NPL ? fb : 0u);
     lag[i] = pl >= NFD + 2 ? 1 : 0;
   }
   const unsigned P4 = (unsigned)g.pitch * 4u;

@@ -197,7 +197,7 @@ __global__ __launch_bounds__(512) void k_tile(const TileArgs a) {
     if (!edge || !cell[j] || inner[j]) continue;
     const int z = zw + j, ar = min(min(z, x), min(NZ - 1 - z, NX - 1 - x));
     vp[j] = ldg(m.v + mo, own[j]);
-    fsv[j] = ldg(m.fs + mo, own[j]);
+    fsv[j] = ldg(m.fs + sg.fw * g.fstride, own[j]);
     r1v[j] = ldg(m.r1 + mo, own[j]);
     wgt[j] = m.w[min(max(N2 - ar, 0), N2)];
     se[j] = strip_elem(g, NX, sg.mnx, z, x);

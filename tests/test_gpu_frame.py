@@ -67,3 +67,43 @@ def test_whole_frame_launch(nz, nx, n2, nfdmax, ilste):
         ctx.close()
     for i, (a, b) in enumerate(zip(*out)):
         assert np.array_equal(a, b), i
+
+
+@pytest.mark.parametrize("nshot,zseg,frame_split", [
+    (3, 0, 0), (3, 16, 0), (3, 16, 1), (44, 0, 0)])  # whole steps by tiles, marching, two steps
+def test_widths_on_one_model(nshot, zseg, frame_split):
+    """Shots of several widths on the context's one model equal shots with the
+    model's first columns as windows of their own."""
+    from rtm_gpu_amd import hip
+    nz, nx, n2 = (60, 150, 14) if nshot == 3 else (400, 578, 20)
+    case = build_case(name="widths", mod_nz=nz, mod_nx=nx, n2=n2, nt=50, nshot=1, tao=0.0008)
+    cfg, m = case["cfg"], case["model"]
+    keys = ("nz", "nx", "n2", "nfdmax", "nt", "nt2", "ilste", "icompen", "s_l", "s_r", "s_z",
+            "ds", "n", "tao2", "h2", "taoh", "taoh2", "hzx2_1")
+    geoms = []
+    for s in range(nshot):
+        w = cfg["nx"] - 2 * n2 - 29 * (s % 3 if nshot == 3 else s // 4 % 2)
+        geoms.append(dict(nx=w + 2 * n2, r_u=n2 + s % 40, r_x=n2 + 5, s_l=n2, s_r=n2 + w - 1, n=w, x_img=0))
+    rng = np.random.default_rng(1)
+    seis = (0.01 * rng.standard_normal((nshot, cfg["n"], cfg["nt"]))).astype(np.float32)
+    v, r1 = (np.asarray(a).reshape(cfg["nz"], cfg["nx"]) for a in (m["v"], m["r1"]))
+    out = []
+    for windows in (False, True):
+        ctx = hip.Context(max_shots=nshot, zseg=zseg, frame_split=frame_split, **{k: cfg[k] for k in keys})
+        ctx.set_model(v, r1, m["w"], m["c"], m["index"], m["nvel"], m["vmin"], m["dv"])
+        ctx.set_wavelet(m["wav"])
+        ctx.set_shot_geometry(geoms)
+        if windows:
+            for s, q in enumerate(geoms):
+                ctx.set_shot_model(s, np.ascontiguousarray(v[:, :q["nx"]]), np.ascontiguousarray(r1[:, :q["nx"]]))
+        ctx.set_gathers(seis)
+        ctx.forward_begin()
+        ctx.forward_advance(cfg["nt"])
+        got = [ctx.field(hip.FIELD_U, shot=s) for s in range(nshot)]
+        ctx.backward_begin()
+        ctx.backward_advance(cfg["nt"])
+        got += [ctx.field(w, shot=s) for s in range(nshot) for w in (hip.FIELD_Q, hip.FIELD_I1)]
+        out.append(got)
+        ctx.close()
+    for i, (a, b) in enumerate(zip(*out)):
+        assert np.array_equal(a, b), i
