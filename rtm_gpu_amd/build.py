@@ -73,8 +73,8 @@ def build_hip(verbose=True, force=True):
              if f != "two" or n <= 5]  # TWO_MAX_NFD
     units += [(f, f + ".o", []) for f in ("rtm_kernels.hip", "rtm_capi.hip", "rtm_cnn.hip")]
     units = [(os.path.join(CSRC, f), os.path.join(obj_dir, o), d) for f, o, d in units]
-    deps = [os.path.join(CSRC, "rtm_kernels.h"), os.path.join(CSRC, "rtm_device.h"),
-            os.path.join(ROOT, "include", "rtm_hip.h"), os.path.join(ROOT, "include", "rtm_cnn.h")]
+    deps = [os.path.join(CSRC, f) for f in ("rtm_kernels.h", "rtm_device.h", "rtm_plan.h")]
+    deps += [os.path.join(ROOT, "include", f) for f in ("rtm_hip.h", "rtm_cnn.h")]
     todo = [(s, o, d) for s, o, d in units if force or _stale(o, s, deps)]
     from concurrent.futures import ThreadPoolExecutor
     jobs = int(os.environ.get("MAX_JOBS", 0)) or min(16, os.cpu_count() or 1)

@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "rtm_plan.h"
+
 namespace rtm {
 
 // Padded-grid geometry in device memory.  Cell (z, x) of shot s in a field

@@ -46,7 +46,7 @@ __global__ __launch_bounds__(512) void k_tile(const TileArgs a) {
   constexpr bool MIG = PASS == TILE_MIG, BORN = PASS == TILE_BORN, ADJ = PASS == TILE_ADJ;
   constexpr bool TWO = PASS != TILE_FWD;                       // q on the whole grid
   constexpr int NT = 512, TH = 8 * CPT;
-  constexpr int R = NFD + 1, LW = 64 + 2 * R, LH = TH + 2 * R, NL = (LH * LW + NT - 1) / NT;
+  constexpr int R = tile_halo(NFD), LW = 64 + 2 * R, LH = TH + 2 * R, NL = (LH * LW + NT - 1) / NT;
   constexpr int RW = 66, RH = TH + 2, NR = (RH * RW + NT - 1) / NT;  // cells with a T value
   __shared__ float su1[LH * LW], sq1[TWO ? LH * LW : 1];
   __shared__ float tu[FWD ? RH * RW : 1], tu0[FWD ? RH * RW : 1];
@@ -66,7 +66,8 @@ __global__ __launch_bounds__(512) void k_tile(const TileArgs a) {
     return zz >= N2 && zz < NZ - N2 && xx >= N2 && xx < NX - N2;
   };
   // uniform: tiles with frame cells, tiles with interior cells
-  const bool edge = z0 < N2 || z0 + TH > NZ - N2 || x0 < N2 || x0 + 64 > NX - N2;
+  const bool edge = tile_edge(z0, x0, TH, N2, NZ, NX);
+  const bool direct = tile_direct(z0, x0, TH, NFD, N2, NZ, NX);
   const bool has_inner = z0 + TH > N2 && z0 < NZ - N2 && x0 + 64 > N2 && x0 < NX - N2;
 
   const long long so = (long long)shot * g.fstride, mo = (long long)sg.win * m.mstride;
@@ -103,7 +104,7 @@ __global__ __launch_bounds__(512) void k_tile(const TileArgs a) {
     for (int j = 0; j < CPT; ++j) ko[j] = __float_as_uint(ldg(mk, own[j]));
   }
   float lu[NL], lq[TWO ? NL : 1];
-  if (edge) {  // the outer mirror (kernel.cu:65-68)
+  if (!direct) {  // the outer mirror (kernel.cu:65-68)
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
       const int e = tid + i * NT, r = e / LW;
@@ -111,7 +112,7 @@ __global__ __launch_bounds__(512) void k_tile(const TileArgs a) {
       lu[i] = need_u ? ldg(u1, o) : 0.f;
       if (TWO) lq[i] = ldg(q1, o);
     }
-  } else {  // every access inside the grid: NFD <= n2
+  } else {  // every access inside the grid
     const int r = tid / LW;
     int c = tid - r * LW;
     unsigned o = at(z0 - R + r, x0 - R + c);

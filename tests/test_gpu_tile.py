@@ -69,3 +69,11 @@ def test_tile_passes_equal_marching(nshot, mod_nz, mod_nx, ilste, strip_format):
         ctx.close()
     for i, (a, b) in enumerate(zip(*out)):
         assert np.array_equal(a, b), i
+
+
+@pytest.mark.parametrize("mod_nz,mod_nx,n", [
+    (120, 170, 8),    # tiles without frame cells that start at row n2 and that end at nz - n2
+    (91, 150, 5),     # rows up to nz - n2 = 96
+    (92, 150, 12)])   # ... 104, the longest operator
+def test_tile_steps_with_a_frame_as_deep_as_the_operator(mod_nz, mod_nx, n):
+    test_tile_steps_equal_oracle(mod_nz, mod_nx, n, n, 1, 1)

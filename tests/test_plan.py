@@ -1,0 +1,71 @@
+"""Index rules of the launches (rtm_gpu_amd/csrc/rtm_plan.h), enumerated on the
+CPU: the header compiled by itself."""
+import ctypes as C
+import os
+import subprocess
+
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "rtm_gpu_amd", "csrc")
+
+SHIM = r"""
+#include "rtm_plan.h"
+using namespace rtm;
+// Tiles of an nz x nx grid that load without clamps and whose staged cells
+// leave it.  rule 0: the kernel's; 1: every tile without frame cells.
+extern "C" int tiles_outside(int nz, int nx, int n2, int nfd, int th, int rule) {
+  int bad = 0;
+  const int r = tile_halo(nfd);
+  for (int z0 = 0; z0 < nz; z0 += th)
+    for (int x0 = 0; x0 < nx; x0 += 64) {
+      const bool direct = rule == 0 ? tile_direct(z0, x0, th, nfd, n2, nz, nx)
+                                    : !tile_edge(z0, x0, th, n2, nz, nx);
+      if (!direct) continue;
+      const int zl = z0 - r, zh = z0 + th + r - 1, xl = x0 - r, xh = x0 + 64 + r - 1;
+      bad += zl < 0 || zh >= nz || xl < 0 || xh >= nx;
+    }
+  return bad;
+}
+// Tiles without frame cells that load through the mirror.
+extern "C" int tiles_clamped(int nz, int nx, int n2, int nfd, int th) {
+  int n = 0;
+  for (int z0 = 0; z0 < nz; z0 += th)
+    for (int x0 = 0; x0 < nx; x0 += 64)
+      n += !tile_edge(z0, x0, th, n2, nz, nx) && !tile_direct(z0, x0, th, nfd, n2, nz, nx);
+  return n;
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def plan(tmp_path_factory):
+    d = tmp_path_factory.mktemp("plan")
+    src, so = d / "plan.cpp", d / "plan.so"
+    src.write_text(SHIM)
+    subprocess.run(["g++", "-O1", "-std=c++17", "-Wall", "-Werror", "-shared", "-fPIC", "-I", CSRC,
+                    str(src), "-o", str(so)], check=True)
+    return C.CDLL(str(so))
+
+
+@pytest.mark.parametrize("nfd", range(1, 13))
+def test_tiles_stage_cells_of_the_grid_only(plan, nfd):
+    heights = range(2, 140)
+    widths = [w for m in (64, 128, 192) for w in range(m - 3, m + 4)] + [16]
+    for n2 in (nfd, nfd + 1, nfd + 5, 32):
+        for th in (8, 16):
+            for h in heights:
+                for w in widths:
+                    nz, nx = h + 2 * n2, w + 2 * n2
+                    assert plan.tiles_outside(nz, nx, n2, nfd, th, 0) == 0, (nz, nx, n2, th)
+                    if n2 > nfd:  # no tile is clamped that need not be
+                        assert plan.tiles_clamped(nz, nx, n2, nfd, th) == 0, (nz, nx, n2, th)
+
+
+def test_a_frame_as_deep_as_the_operator_needs_the_clamp(plan):
+    """Row -1 (a tile that starts at n2 == nfd) and row nz (one that ends at
+    nz - n2) are what a tile without frame cells would load there."""
+    assert plan.tiles_outside(136, 186, 8, 8, 8, 1) > 0
+    for nfd in range(1, 13):
+        nz = 96 + nfd  # nz - n2 = 96
+        assert plan.tiles_outside(nz, 186, nfd, nfd, 8, 1) > 0, nfd
+        assert plan.tiles_outside(nz, 186, nfd, nfd, 16, 1) > 0, nfd
