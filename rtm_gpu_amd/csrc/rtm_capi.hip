@@ -2012,8 +2012,8 @@ int rtm_autotune(rtm_ctx* c, int nsteps, int* zseg) {
       if (!on) r = backward_step(c, kb - i, false);
       else if (backward_two_ok(c, kb - i, 2)) r = backward_two(c, kb - i, false, 2);
     }
-    kf += 4;
-    kb -= 4;
+    kf = kf + 4 < nt ? kf + 4 : 2;  // the steps that pairs() takes next
+    kb = kb >= 4 ? kb - 4 : nt - 3;
     return r;
   };
   // Two steps per launch: their heights, then against one step per launch, on
@@ -2058,8 +2058,6 @@ int rtm_autotune(rtm_ctx* c, int nsteps, int* zseg) {
     c->two_tuned = 0;
     c->img_pend = 0;
     if (rc == RTM_OK && best < one) two_choice = 1;
-    if (kf >= nt) kf = 2;
-    if (kb < 0) kb = nt - 3;
   }
   // Frame record runs, timed on both frame kernels of the step pair (of four
   // steps each way where those take two per launch): the top and bottom bands in
@@ -2110,11 +2108,7 @@ int rtm_autotune(rtm_ctx* c, int nsteps, int* zseg) {
     }
     if (rc == RTM_OK) rc = upload_frame_records(c);
     c->two_tuned = 0;
-    if (quad) {
-      c->img_pend = 0;
-      if (kf >= nt) kf = 2;
-      if (kb < 0) kb = nt - 3;
-    }
+    if (quad) c->img_pend = 0;
     // the frame split on and off (the four-column launch pays only when the
     // batch fills the GPU with frame waves)
     if (rc == RTM_OK && c->nvec > 0 && frame4_supported(c->nfd) && !fused(c, fwd, FR_FWD) && !quad) {

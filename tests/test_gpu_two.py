@@ -91,3 +91,22 @@ def test_two_steps_with_shared_windows(group):
         ctx.close()
     for i, (a, b) in enumerate(zip(*out)):
         assert np.array_equal(a, b), i
+
+
+def test_autotuned_batch():
+    """rtm_autotune on such a batch times two steps per launch, one step and
+    whole steps; the migration and its records are those of the fixed kernels.
+    At 75 time samples a cycle of four steps ends at the last one."""
+    case = build_case(name="two", mod_nz=NZ, mod_nx=NX, n2=N2, nfdmax=3, ilste=1, nt=75, nshot=SHOTS,
+                      depth_step=7.0, src_x1=90, tao=0.0008, ds=3)
+    rng = np.random.default_rng(9)
+    seis = (0.01 * rng.standard_normal((SHOTS, case["cfg"]["n"], case["cfg"]["nt"]))).astype(np.float32)
+    out = []
+    for tuned in (True, False):
+        ctx = hip_context(case, nshot=SHOTS, record=1, zseg=0 if tuned else 16)
+        if tuned:
+            ctx.autotune(8)
+        out.append(passes(ctx, seis, (11,)))
+        ctx.close()
+    for i, (a, b) in enumerate(zip(*out)):
+        assert np.array_equal(a, b), i
