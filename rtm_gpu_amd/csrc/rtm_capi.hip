@@ -1401,8 +1401,9 @@ int rtm_set_shot_model(rtm_ctx* c, int shot, const float* v, const float* r1) {
     c->win_fp[2 * w] = fp[0];
     c->win_fp[2 * w + 1] = fp[1];
     c->tp_ok = c->cp_ok = false;
-    }
+  }
   c->win_ref[w] += 1;
+  if (c->geo[shot].win != w) c->quads = false;  // until the next pass looks again
   c->geo[shot].win = w;
   c->geo[shot].fw = w;
   HIPCHK(c, hipMemcpyAsync(c->d_geo + shot, &c->geo[shot], sizeof(ShotGeo), hipMemcpyHostToDevice, c->stream));

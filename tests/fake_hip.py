@@ -85,3 +85,16 @@ def set_model(ctx, nz, nx, n2, nfd, v=1500.0):
 
 def shots(ctx, n):
     ctx.set_shots([ctx.n2] * n, [ctx.n2 + 1] * n)
+
+
+def ragged(ctx, n, widths=None):
+    """A ragged batch of n shots (widths: of each, default the grid's)."""
+    n2 = ctx.n2
+    ctx.set_shot_geometry([dict(nx=w, r_u=n2, r_x=n2 + 1, s_l=n2, s_r=w - n2 - 1, n=w - 2 * n2, x_img=0)
+                           for w in widths or [ctx.nx] * n])
+
+
+def window(ctx, shot, v, nx=None):
+    import numpy as np
+    a = np.full((ctx.nz, nx or ctx.nx), v, np.float32)
+    ctx.set_shot_model(shot, a, a * 0)

@@ -110,3 +110,38 @@ def test_autotuned_batch():
         ctx.close()
     for i, (a, b) in enumerate(zip(*out)):
         assert np.array_equal(a, b), i
+
+
+def test_window_changed_between_the_passes():
+    """Shot 0 takes the other window of the batch for the backward pass: its
+    block's four shots no longer share one."""
+    from rtm_gpu_amd import hip
+    case = build_case(name="twochg", mod_nz=NZ, mod_nx=NX, n2=N2, nt=30, nshot=1)
+    cfg, m = case["cfg"], case["model"]
+    keys = ("nz", "nx", "n2", "nfdmax", "nt", "nt2", "ilste", "icompen", "s_l", "s_r", "s_z",
+            "ds", "n", "tao2", "h2", "taoh", "taoh2", "hzx2_1")
+    n, nt = 40, cfg["nt"]
+    rng = np.random.default_rng(5)
+    seis = (0.01 * rng.standard_normal((n, cfg["n"], nt))).astype(np.float32)
+    v = np.ascontiguousarray(m["v"]).reshape(cfg["nz"], cfg["nx"])
+    r1 = np.ascontiguousarray(m["r1"]).reshape(v.shape)
+    wins = [(v, r1), (v[:, ::-1], r1[:, ::-1])]
+    out = []
+    for zseg in (0, 16):
+        ctx = hip.Context(**{k: cfg[k] for k in keys}, max_shots=n, zseg=zseg)
+        ctx.set_model(m["v"], m["r1"], m["w"], m["c"], m["index"], m["nvel"], m["vmin"], m["dv"])
+        ctx.set_wavelet(m["wav"])
+        ctx.set_shot_geometry([dict(nx=cfg["nx"], r_u=N2 + s, r_x=N2 + 90, s_l=cfg["s_l"], s_r=cfg["s_r"],
+                                    n=cfg["n"], x_img=0) for s in range(n)])
+        for s in range(n):
+            ctx.set_shot_model(s, *wins[s >= 20])
+        ctx.set_gathers(seis)
+        ctx.forward_begin()
+        ctx.forward_advance(nt)
+        ctx.set_shot_model(0, *wins[1])
+        ctx.backward_begin()
+        ctx.backward_advance(nt)
+        out.append([ctx.field(w, shot=s) for s in (0, 1, 4, 39) for w in (hip.FIELD_I1, hip.FIELD_I2, hip.FIELD_Q)])
+        ctx.close()
+    for i, (a, b) in enumerate(zip(*out)):
+        assert np.array_equal(a, b), i

@@ -27,3 +27,29 @@ for nt in list(range(12, 150)) + [184, 366, 420, 428, 482]:
 out(bad)
 """)
     assert bad == []
+
+
+def test_window_changed_between_the_passes():
+    """A shot that moves to another shot's window after the forward pass no
+    longer shares the window of its block's four: one step per launch from there."""
+    got = run("""
+ctx = context(check_every=-1)
+ragged(ctx, 40)
+for s in range(40):
+    window(ctx, s, 1500.0 if s < 20 else 1600.0)
+import numpy as np
+ctx.set_gathers(np.zeros((40, ctx.p.n, ctx.p.nt), np.float32))
+res = []
+for change in (False, True):
+    ctx.forward_begin()
+    ctx.forward_advance(60)
+    log()
+    if change:
+        window(ctx, 0, 1600.0)
+    ctx.backward_begin()
+    ctx.backward_advance(60)
+    res.append(sorted({r["kernel"] for r in log() if r["kernel"] in ("k_two", "k_interior", "k_tile")}))
+out(res)
+""")
+    assert got[0] == ["k_two"]
+    assert "k_two" not in got[1]
