@@ -58,14 +58,15 @@ struct rtm_ctx {
   int4* d_tiles = nullptr;     // frame (tile, shot) records of the batch
   int ntiles = 0, tile_cap = 0;  // FRAME_ALL records; capacity of d_tiles
   int nsplit = 0, nvec = 0;      // FRAME_SCALAR and FRAME_VEC records after them
-  size_t fs_cap = 0;  // planes of d_fs
+  size_t fs_cap = 0;        // planes of d_fs
+  std::vector<int> fs_nx;   // widths whose planes match the current model
+  bool fs_ok = false;       // the batch's shots have theirs (ShotGeo::fw)
   int qrows = 0;  // rows per block of k_frame_quad; 0: quad_rows
   int fseg_tb = 0, fseg_side = 0;  // rows per frame record: top/bottom bands, side bands
   // model windows of a ragged batch (allocated on first use): slot w holds
   // one distinct window; shots whose windows are equal share a slot
   float *d_mv = nullptr, *d_mr1 = nullptr, *d_mpm = nullptr;
   unsigned* d_mko = nullptr;
-  float* d_mfs = nullptr;
   std::vector<char> shot_model;
   std::vector<int> win_ref;                 // shots using each slot
   std::vector<int> win_nx;                  // width of each slot's window
@@ -489,6 +490,42 @@ int ensure_planes(rtm_ctx* c) {
   return RTM_OK;
 }
 
+// With one model for all shots: a plane of Model::fs per width of the batch (the
+// side cells' factors depend on it).  Windows of their own bring theirs
+// (rtm_set_shot_model), and may still be to come when the geometry is set, so
+// the planes are made where a pass is about to read them.  Allocates: not inside
+// a stream capture.
+int ensure_lateral(rtm_ctx* c) {
+  if (c->fs_ok || c->m.mstride != 0) return RTM_OK;
+  const Grid& g = c->g;
+  std::vector<int> need;
+  for (const ShotGeo& q : c->geo)
+    if (std::find(need.begin(), need.end(), q.nx) == need.end()) need.push_back(q.nx);
+  bool have = true;
+  for (int nx : need) have = have && std::find(c->fs_nx.begin(), c->fs_nx.end(), nx) != c->fs_nx.end();
+  if (!have) {
+    c->fs_nx.clear();
+    if (need.size() > c->fs_cap) {
+      HIPCHK(c, hipStreamSynchronize(c->stream));
+      dfree_t(c, &c->d_fs, c->fs_cap * g.fstride);
+      c->fs_cap = 0;
+      const int rc = dalloc_t(c, &c->d_fs, need.size() * g.fstride);
+      if (rc != RTM_OK) return rc;
+      c->fs_cap = need.size();
+    }
+    for (size_t i = 0; i < need.size(); ++i)
+      HIPCHK(c, launch_frame_lat(g, need[i], c->d_v, c->p.taoh2, false, c->d_fs + i * g.fstride, c->stream));
+    c->fs_nx = need;
+  }
+  c->m.fs = c->d_fs;
+  for (ShotGeo& q : c->geo)
+    q.fw = (int)(std::find(c->fs_nx.begin(), c->fs_nx.end(), q.nx) - c->fs_nx.begin());
+  HIPCHK(c, hipMemcpyAsync(c->d_geo, c->geo.data(), c->geo.size() * sizeof(ShotGeo), hipMemcpyHostToDevice, c->stream));
+  HIPCHK(c, hipStreamSynchronize(c->stream));
+  c->fs_ok = true;
+  return RTM_OK;
+}
+
 // The quantisation of the strips of step k - 1 (reduced-precision storage),
 // ahead of step k.
 int forward_before(rtm_ctx* c, int k) {
@@ -889,38 +926,6 @@ void build_tiles(const Grid& g, int nx, int shot, int seg_tb, int seg, int kind,
 }
 
 int choose_zs(rtm_ctx* c, int nshot);
-// With one model for all shots: a plane of Model::fs per width of the batch
-// (the side and bottom cells' factors depend on it), the widest shot's first.
-// Windows of their own bring theirs (rtm_set_shot_model).
-int lateral_planes(rtm_ctx* c) {
-  if (!c->model_ok || c->m.mstride != 0) return RTM_OK;
-  const Grid& g = c->g;
-  std::vector<int> widths{g.nx};
-  for (ShotGeo& q : c->geo) {
-    size_t i = 0;
-    while (i < widths.size() && widths[i] != q.nx) ++i;
-    if (i == widths.size()) widths.push_back(q.nx);
-    q.fw = (int)i;
-  }
-  if (widths.size() > c->fs_cap) {
-    float* p = nullptr;
-    const int rc = dalloc_t(c, &p, widths.size() * g.fstride);
-    if (rc != RTM_OK) return rc;
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    dfree_t(c, &c->d_fs, c->fs_cap * g.fstride);
-    c->d_fs = p;
-    c->fs_cap = widths.size();
-  }
-  for (size_t i = 0; i < widths.size(); ++i)
-    HIPCHK(c, launch_frame_lat(g, widths[i], c->d_v, c->p.taoh2, c->d_fs + i * g.fstride, c->stream));
-  c->m.fs = c->d_fs;
-  if (!c->geo.empty()) {
-    HIPCHK(c, hipMemcpyAsync(c->d_geo, c->geo.data(), c->geo.size() * sizeof(ShotGeo), hipMemcpyHostToDevice, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-  }
-  return RTM_OK;
-}
-
 void drop_graph(rtm_ctx* c);
 
 // The batch's frame records for the context's run lengths, three lists one
@@ -963,9 +968,8 @@ int upload_frame_records(rtm_ctx* c) {
 int upload_geometry(rtm_ctx* c) {
   const int ns = (int)c->geo.size();
   HIPCHK(c, hipMemcpyAsync(c->d_geo, c->geo.data(), ns * sizeof(ShotGeo), hipMemcpyHostToDevice, c->stream));
-  int rc = lateral_planes(c);
-  if (rc != RTM_OK) return rc;
-  rc = upload_frame_records(c);
+  c->fs_ok = false;
+  int rc = upload_frame_records(c);
   if (rc != RTM_OK) return rc;
   if (ns != c->nshot) c->tile_tuned = c->two_tuned = -1;  // tuned for another batch
   c->cells = 0;
@@ -1271,7 +1275,7 @@ int rtm_set_model(rtm_ctx* c, const float* v, const float* r1, const float* w, c
   HIPCHK(c, hipStreamSynchronize(c->stream));
   Model& m = c->m;
   m.mstride = 0;  // one model for every shot until rtm_set_shot_model
-  m.v = c->d_v; m.r1 = c->d_r1; m.fs = c->d_fs; m.ctab = c->d_ctab; m.w = c->d_w;
+  m.v = c->d_v; m.r1 = c->d_r1; m.ctab = c->d_ctab; m.w = c->d_w;
   m.pm = c->d_pm; m.ko = c->d_ko;
   m.cs = CS; m.nrow = nrow;
   c->shot_model.assign(c->p.max_shots, 0);
@@ -1284,8 +1288,10 @@ int rtm_set_model(rtm_ctx* c, const float* v, const float* r1, const float* w, c
   c->nfd = nfd;
   c->tp_ok = c->cp_ok = false;
   drop_graph(c);
+  c->fs_nx.clear();
+  c->fs_ok = false;
   c->model_ok = true;
-  return lateral_planes(c);
+  return RTM_OK;
 }
 
 int rtm_set_wavelet(rtm_ctx* c, const float* wav) {
@@ -1369,7 +1375,6 @@ int rtm_set_shot_model(rtm_ctx* c, int shot, const float* v, const float* r1) {
     if (rc == RTM_OK) rc = dalloc_t(c, &c->d_mr1, n);
     if (rc == RTM_OK) rc = dalloc_t(c, &c->d_mpm, n);
     if (rc == RTM_OK) rc = dalloc_t(c, &c->d_mko, n);
-    if (rc == RTM_OK) rc = dalloc_t(c, &c->d_mfs, n);
     if (rc != RTM_OK) return rc;
   }
   if (c->win_ref.size() != (size_t)c->p.max_shots) {
@@ -1391,7 +1396,9 @@ int rtm_set_shot_model(rtm_ctx* c, int shot, const float* v, const float* r1) {
     if (w < 0) return fail(c, RTM_E_STATE, "no free model window slot");
     const size_t o = (size_t)w * g.fstride;
     int rc = upload_model_window(c, nx, v, r1, c->d_mv + o, c->d_mr1 + o, c->d_mpm + o, c->d_mko + o);
-    if (rc == RTM_OK && launch_frame_lat(g, nx, c->d_mv + o, c->p.taoh2, c->d_mfs + o, c->stream) != hipSuccess)
+    // r1 is read at the corner cells only, the lateral factors at the other
+    // frame cells: one plane holds both
+    if (rc == RTM_OK && launch_frame_lat(g, nx, c->d_mv + o, c->p.taoh2, true, c->d_mr1 + o, c->stream) != hipSuccess)
       rc = fail(c, RTM_E_HIP, "lateral factors of shot %d", shot);
     if (rc != RTM_OK) {
       c->shot_model[shot] = 0;
@@ -1410,7 +1417,7 @@ int rtm_set_shot_model(rtm_ctx* c, int shot, const float* v, const float* r1) {
   HIPCHK(c, hipStreamSynchronize(c->stream));
   Model& m = c->m;
   m.mstride = g.fstride;
-  m.v = c->d_mv; m.r1 = c->d_mr1; m.fs = c->d_mfs; m.pm = c->d_mpm; m.ko = c->d_mko;
+  m.v = c->d_mv; m.r1 = m.fs = c->d_mr1; m.pm = c->d_mpm; m.ko = c->d_mko;
   c->shot_model[shot] = 1;
   drop_graph(c);
   return RTM_OK;
@@ -1487,6 +1494,8 @@ int rtm_forward_begin(rtm_ctx* c, int save_strips) {
 int rtm_forward_advance(rtm_ctx* c, int nsteps) {
   if (!c) return RTM_E_ARG;
   if (c->kf < 2) return fail(c, RTM_E_STATE, "rtm_forward_begin first");
+  const int lrc = ensure_lateral(c);
+  if (lrc != RTM_OK) return lrc;
   for (int left = std::min(nsteps, c->p.nt - c->kf); left > 0;) {
     const int n = left >= 2 && use_two(c) ? 2 : 1;
     int rc = n == 2 ? forward_two(c, c->kf) : forward_step(c, c->kf);
@@ -1522,6 +1531,8 @@ int rtm_backward_begin(rtm_ctx* c) {
 int rtm_backward_advance(rtm_ctx* c, int nsteps) {
   if (!c) return RTM_E_ARG;
   if (c->kb < -1) return fail(c, RTM_E_STATE, "rtm_backward_begin first");
+  const int lrc = ensure_lateral(c);
+  if (lrc != RTM_OK) return lrc;
   for (int left = std::min(nsteps, c->kb + 1); left > 0;) {
     const int n = backward_two_ok(c, c->kb, left) ? 2 : 1;
     int rc = n == 2 ? backward_two(c, c->kb, left == 2, left) : backward_step(c, c->kb, left == 1);
@@ -1583,6 +1594,8 @@ int rtm_born_begin(rtm_ctx* c) {
 int rtm_born_advance(rtm_ctx* c, int nsteps) {
   if (!c) return RTM_E_ARG;
   if (!c->born || c->kf < 2) return fail(c, RTM_E_STATE, "rtm_born_begin first");
+  const int lrc = ensure_lateral(c);
+  if (lrc != RTM_OK) return lrc;
   for (int i = 0; i < nsteps && c->kf < c->p.nt; ++i, ++c->kf) {
     int rc = born_step(c, c->kf);
     if (rc != RTM_OK) return rc;
@@ -1595,6 +1608,8 @@ int rtm_adjoint_begin(rtm_ctx* c) {
   if (c->kf != c->p.nt) return fail(c, RTM_E_STATE, "forward pass incomplete (k=%d of %d)", c->kf, c->p.nt);
   if (!c->save_strips) return fail(c, RTM_E_STATE, "forward pass ran without strips");
   if (!c->data_ok) return fail(c, RTM_E_STATE, "rtm_set_gathers first (residuals)");
+  const int lrc = ensure_lateral(c);
+  if (lrc != RTM_OK) return lrc;
   if (c->p.ilste == 0 && !c->tp_ok) {  // neighbour-tap planes of the current model windows
     const Grid& g = c->g;
     int nwin = 1;  // slots 0 .. nwin-1 (one model: slot 0)
@@ -1641,6 +1656,8 @@ int rtm_adjoint_begin(rtm_ctx* c) {
 int rtm_adjoint_advance(rtm_ctx* c, int nsteps) {
   if (!c) return RTM_E_ARG;
   if (!c->adj || c->kb < -1) return fail(c, RTM_E_STATE, "rtm_adjoint_begin first");
+  const int lrc = ensure_lateral(c);
+  if (lrc != RTM_OK) return lrc;
   for (int i = 0; i < nsteps && c->kb >= 0; ++i, --c->kb) {
     int rc = adjoint_step(c, c->kb);
     if (rc != RTM_OK) return rc;
@@ -1832,6 +1849,7 @@ int rtm_migrate(rtm_ctx* c) {
     return fail(c, RTM_E_STATE, "model, wavelet, shots and gathers must be set");
   if (!c->gexec) {
     int prc = ensure_planes(c);
+    if (prc == RTM_OK) prc = ensure_lateral(c);
     if (prc != RTM_OK) return prc;
     // Capture the whole launch sequence once; the host-side buffer rotation
     // is deterministic, so the replay leaves the same state as the capture.
@@ -1933,6 +1951,7 @@ int rtm_autotune(rtm_ctx* c, int nsteps, int* zseg) {
   c->tile_tuned = 0;
   c->march_set = c->p.fuse_frame != 0;
   int rc = rtm_forward_begin(c, 1);
+  if (rc == RTM_OK) rc = ensure_lateral(c);
   if (rc == RTM_OK && !c->data_ok)
     rc = launch_fill(c->d_data, (long long)c->nshot * c->p.nt * c->p.n, 0.f, c->stream) == hipSuccess
              ? RTM_OK : fail(c, RTM_E_HIP, "autotune: fill");

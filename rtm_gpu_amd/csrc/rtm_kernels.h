@@ -26,7 +26,8 @@ struct Model {
   const float* r1;
   // (taoh2*vq)*vq of the frame cell's one-way update, vq the velocity that the
   // reference reads there (launch_frame_lat), padded layout, fstride per plane
-  // ShotGeo::fw
+  // ShotGeo::fw; windows of their own keep it in the plane of r1, beside the
+  // corner cells' values
   const float* fs;
   const float* pm;     // v*v*tao2*h2 per cell (FP32, left to right), padded layout
   const unsigned* ko;  // byte offset of the cell's coefficient row in ctab, padded layout
@@ -191,8 +192,10 @@ int two_cols(const Grid& g, int nfd, int nshot);
 // the register queue).
 int two_rows(int nfd, int rows);
 hipError_t launch_two(int kind, int nfd_inst, TwoArgs a, int nshot, hipStream_t s);
-// Model::fs of a window nx columns wide from its velocities.
-hipError_t launch_frame_lat(const Grid& g, int nx, const float* v, float taoh2, float* fs, hipStream_t s);
+// Model::fs of a window nx columns wide from its velocities.  keep_corners: the
+// corner cells, whose update reads r1 instead, keep what fs holds there.
+hipError_t launch_frame_lat(const Grid& g, int nx, const float* v, float taoh2, bool keep_corners,
+                            float* fs, hipStream_t s);
 // Planes (TwoArgs::cp) of window win.
 constexpr int two_planes(int nfd) { return nfd + 4; }
 hipError_t launch_coef_planes(const Grid& g, const Model& m, int win, int nfd, float* cp, hipStream_t s);

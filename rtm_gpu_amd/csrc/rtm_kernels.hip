@@ -462,13 +462,16 @@ hipError_t launch_two(int kind, int nfd, TwoArgs a, int nshot, hipStream_t s) {
 // top-band cell, on the sides (kernel.cu:128, 136), where z may pass a row's end.
 // Read by every step from here: a wave of side cells reading the velocities
 // themselves touches a cache line per lane.
-__global__ void k_frame_lat(const Grid g, int nx, const float* v, float taoh2, float* fs) {
+__global__ void k_frame_lat(const Grid g, int nx, const float* v, float taoh2, bool keep_corners,
+                            float* fs) {
   const long long n = (long long)g.nz * nx;
   for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (long long)gridDim.x * blockDim.x) {
     const int z = (int)(i / nx), x = (int)(i % nx);
     const int ar = min(min(z, x), min(g.nz - 1 - z, nx - 1 - x));
     const bool top = z == ar, bot = !top && z == g.nz - 1 - ar;
+    if (keep_corners && (z - ar <= 1 || g.nz - 1 - ar - z <= 1) && (x - ar <= 1 || nx - 1 - ar - x <= 1))
+      continue;
     const int zq = top ? z : (bot ? ar : min(ar + z / nx, g.nz - 1));
     const int xq = (top || bot) ? x : z % nx;
     const float vq = v[(long long)zq * g.pitch + g.x0 + xq];
@@ -678,9 +681,10 @@ hipError_t launch_tap_planes(const Grid& g, const unsigned* ko, const float* cta
                      dim3(256), 0, s, g, ko, ctab, nfd, tp);
   return hipGetLastError();
 }
-hipError_t launch_frame_lat(const Grid& g, int nx, const float* v, float taoh2, float* fs, hipStream_t s) {
+hipError_t launch_frame_lat(const Grid& g, int nx, const float* v, float taoh2, bool keep_corners,
+                            float* fs, hipStream_t s) {
   hipLaunchKernelGGL(k_frame_lat, dim3(blocks_for((long long)g.nz * nx, 256, 2048)), dim3(256), 0, s, g,
-                     nx, v, taoh2, fs);
+                     nx, v, taoh2, keep_corners, fs);
   return hipGetLastError();
 }
 hipError_t launch_coef_planes(const Grid& g, const Model& m, int win, int nfd, float* cp, hipStream_t s) {

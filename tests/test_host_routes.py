@@ -53,3 +53,73 @@ out(res)
 """)
     assert got[0] == ["k_two"]
     assert "k_two" not in got[1]
+
+
+def test_lateral_factors_take_no_memory_that_nothing_reads():
+    """Setting a ragged geometry allocates nothing: shots may still bring windows,
+    whose factors share the plane of r1.  With one model, a plane per width is
+    made when a pass needs it."""
+    got = run("""
+n = 12
+widths = [300 + 10 * s for s in range(n)]
+ctx = context(nz=120, nx=420, shots=n, check_every=-1)
+b0 = ctx.device_bytes()
+ragged(ctx, n, widths)
+b1 = ctx.device_bytes()
+for s, w in enumerate(widths):
+    window(ctx, s, 1500.0 + s, w)
+ctx.forward_begin(); ctx.forward_advance(60)
+b2 = ctx.device_bytes()
+one = context(nz=120, nx=420, shots=n, check_every=-1)
+ragged(one, n, widths)
+c0 = one.device_bytes()
+one.forward_begin(); one.forward_advance(60)
+c1 = one.device_bytes()
+ragged(one, n, widths[::-1])          # the same widths: nothing new
+log()
+one.forward_begin(); one.forward_advance(60)
+again = sum("frame_lat" in r["kernel"] for r in log())
+pitch = (12 + 420 + 4 + 63) // 64 * 64  # 12 guard columns on the left with n2 = 20
+out([b1 - b0, (b2 - b1) / (4 * 120 * pitch), (c1 - c0) / (4 * 120 * pitch), again, one.device_bytes() - c1])
+""")
+    assert got == [0, 4 * 12, 12 - 1, 0, 0]
+
+
+def test_a_batch_that_finds_no_memory_leaves_the_context_usable():
+    got = run("""
+ctx = context(nz=120, nx=420, shots=12, check_every=-1)
+shots(ctx, 12)
+ctx.forward_begin(); ctx.forward_advance(60)
+from rtm_gpu_amd import hip
+fake.fake_limit(fake.fake_used() + 1000)
+ragged(ctx, 3, [300, 310, 320])
+ctx.forward_begin()
+try:
+    ctx.forward_advance(60)
+    raised = False
+except hip.RtmError as e:
+    raised = "hipMalloc" in str(e)
+shots(ctx, 12)
+log()
+ctx.forward_begin(); ctx.forward_advance(60)
+rows = log()
+out([raised, any(r["dead"] for r in rows), sum(r["kernel"] == "k_tile" for r in rows)])
+""")
+    assert got == [True, False, 58]
+
+
+def test_model_set_between_the_passes():
+    """A model set after the forward pass is the one the backward pass takes,
+    its lateral factors included."""
+    got = run("""
+import numpy as np
+ctx = context(nz=120, nx=420, shots=3, check_every=-1)
+shots(ctx, 3)
+ctx.set_gathers(np.zeros((3, ctx.p.n, ctx.p.nt), np.float32))
+ctx.forward_begin(); ctx.forward_advance(60)
+log()
+set_model(ctx, 120, 420, 20, 3, v=1600.0)
+ctx.backward_begin(); ctx.backward_advance(60)
+out([r["kernel"] for r in log() if "frame_lat" in r["kernel"] or "k_tile" in r["kernel"]][:2])
+""")
+    assert "frame_lat" in got[0] and got[1] == "k_tile"
