@@ -147,12 +147,23 @@ int fail(rtm_ctx* c, int code, const char* fmt, ...) {
                   __FILE__, __LINE__);                                                      \
   } while (0)
 
-int dalloc(rtm_ctx* c, void** p, size_t n) {
+void drop_graph(rtm_ctx* c);
+void release_two(rtm_ctx* c);
+
+// optional: memory that the call can do without; what is held of that kind is
+// given back before a required allocation fails.
+int dalloc(rtm_ctx* c, void** p, size_t n, bool optional = false) {
   *p = nullptr;
   if (n == 0) n = 16;
   hipError_t e = hipMalloc(p, n);
+  if (e != hipSuccess && !optional && c->F[3]) {
+    (void)hipGetLastError();
+    release_two(c);
+    e = hipMalloc(p, n);
+  }
   if (e != hipSuccess) {
     (void)hipGetLastError();
+    if (optional) return RTM_E_NOMEM;
     return fail(c, RTM_E_NOMEM, "hipMalloc(%zu bytes) failed: %s", n, hipGetErrorString(e));
   }
   c->allocs.push_back(*p);
@@ -160,8 +171,8 @@ int dalloc(rtm_ctx* c, void** p, size_t n) {
   return RTM_OK;
 }
 template <typename T>
-int dalloc_t(rtm_ctx* c, T** p, size_t count) {
-  return dalloc(c, reinterpret_cast<void**>(p), count * sizeof(T));
+int dalloc_t(rtm_ctx* c, T** p, size_t count, bool optional = false) {
+  return dalloc(c, reinterpret_cast<void**>(p), count * sizeof(T), optional);
 }
 // Release one allocation made by dalloc before the context is destroyed.
 template <typename T>
@@ -461,17 +472,56 @@ void fill_two_args(rtm_ctx* c, TwoArgs& a, int kind) {
   a.icompen = c->p.icompen;
 }
 
-// The coefficient planes of the batch's model windows, where two steps per
-// launch may use them.  Allocates: not inside a stream capture.
-int ensure_planes(rtm_ctx* c) {
+// Give back what only two steps per launch use.  The fields of a pass may lie in
+// the fourth buffers: the one of each four that holds none becomes the fourth.
+void release_two(rtm_ctx* c) {
+  (void)hipStreamSynchronize(c->stream);
+  drop_graph(c);
+  const size_t fb = (size_t)c->p.max_shots * c->g.fstride;
+  const auto spare = [](float** b, int& i0, int& i1, int& i2, int& i3) {
+    std::swap(b[3], b[i3]);
+    for (int* i : {&i0, &i1, &i2})
+      if (*i == 3) *i = i3;
+    i3 = 3;
+  };
+  spare(c->F, c->f0, c->f1, c->f2, c->f3);
+  spare(c->Q, c->q0, c->q1, c->q2, c->q3);
+  dfree_t(c, &c->F[3], fb);
+  dfree_t(c, &c->Q[3], fb);
+  dfree_t(c, &c->d_cp, c->cp_cap);
+  c->cp_cap = 0;
+  c->cp_ok = false;
+  c->rings_for = -1;
+}
+
+// What two steps per launch need where the batch may take them: the fourth
+// buffers, only if they leave an eighth of the card for what is allocated later,
+// and the coefficient planes of the batch's model windows.  Without them every
+// launch takes one step.  Allocates: not inside a stream capture.
+int ensure_two(rtm_ctx* c) {
   c->quads = true;
   for (int s = 0; s < c->nshot; ++s) {
     const ShotGeo &a = c->geo[s / TWO_SHOTS * TWO_SHOTS], &b = c->geo[s];
     c->quads = c->quads && a.nx == b.nx && a.win == b.win;
   }
-  if (c->cp_ok || !c->F[3] || !c->Q[3] || c->nfd > TWO_MAX_NFD || !c->quads || c->nshot < TWO_SHOTS ||
-      c->capturing)
+  if (c->capturing || !c->quads || c->nshot < TWO_SHOTS || c->nfd > TWO_MAX_NFD || c->march_set ||
+      c->cells < two_cells(1))
     return RTM_OK;
+  if (!c->F[3]) {
+    const size_t fb = (size_t)c->p.max_shots * c->g.fstride;
+    size_t mem_free = 0, mem_all = 0;
+    if (hipMemGetInfo(&mem_free, &mem_all) != hipSuccess ||
+        mem_free < 2 * fb * sizeof(float) + mem_all / 8)
+      return RTM_OK;
+    if (dalloc_t(c, &c->F[3], fb, true) != RTM_OK) return RTM_OK;
+    if (dalloc_t(c, &c->Q[3], fb, true) != RTM_OK) {
+      dfree_t(c, &c->F[3], fb);
+      return RTM_OK;
+    }
+    HIPCHK(c, launch_fill(c->F[3], (long long)fb, 0.f, c->stream));
+    HIPCHK(c, launch_fill(c->Q[3], (long long)fb, 0.f, c->stream));
+  }
+  if (c->cp_ok) return RTM_OK;
   int nwin = 1;
   if (c->m.mstride)
     for (int s = 0; s < c->nshot; ++s) nwin = std::max(nwin, c->geo[s].win + 1);
@@ -480,7 +530,10 @@ int ensure_planes(rtm_ctx* c) {
     HIPCHK(c, hipStreamSynchronize(c->stream));
     dfree_t(c, &c->d_cp, c->cp_cap);
     c->cp_cap = 0;
-    if (dalloc_t(c, &c->d_cp, per * nwin) != RTM_OK) return RTM_OK;  // one step per launch
+    if (dalloc_t(c, &c->d_cp, per * nwin, true) != RTM_OK) {
+      release_two(c);
+      return RTM_OK;
+    }
     c->cp_cap = per * nwin;
   }
   for (int w = 0; w < nwin; ++w)
@@ -926,8 +979,6 @@ void build_tiles(const Grid& g, int nx, int shot, int seg_tb, int seg, int kind,
 }
 
 int choose_zs(rtm_ctx* c, int nshot);
-void drop_graph(rtm_ctx* c);
-
 // The batch's frame records for the context's run lengths, three lists one
 // after the other: every frame cell for k_frame (FRAME_ALL: the Born and
 // adjoint frames, the one-launch step), then the split frame of the forward
@@ -1184,25 +1235,10 @@ int rtm_create(const rtm_params* p, rtm_ctx** out) {
     rtm_destroy(c);
     return code;
   }
-  // The fourth buffers of two steps per launch, last, and only where they leave
-  // an eighth of the card for what is allocated later: without them every
-  // launch takes one step.
-  size_t mem_free = 0, mem_all = 0;
-  if ((long long)p->max_shots * g.nz * g.nx >= two_cells(1) && p->max_shots >= TWO_SHOTS &&
-      hipMemGetInfo(&mem_free, &mem_all) == hipSuccess &&
-      mem_free >= 2 * fb * sizeof(float) + mem_all / 8) {
-    if (dalloc_t(c, &c->F[3], fb) == RTM_OK && dalloc_t(c, &c->Q[3], fb) != RTM_OK)
-      dfree_t(c, &c->F[3], fb);
-    c->err.clear();
-  }
   // Zero everything once so guard columns hold finite values.
   for (int i = 0; i < 3; ++i) {
     HIPCHK(c, launch_fill(c->F[i], (long long)fb, 0.f, c->stream));
     HIPCHK(c, launch_fill(c->Q[i], (long long)fb, 0.f, c->stream));
-  }
-  if (c->F[3]) {
-    HIPCHK(c, launch_fill(c->F[3], (long long)fb, 0.f, c->stream));
-    HIPCHK(c, launch_fill(c->Q[3], (long long)fb, 0.f, c->stream));
   }
   HIPCHK(c, launch_fill(c->SU, (long long)fb, 0.f, c->stream));
   HIPCHK(c, launch_fill(c->SQ, (long long)fb, 0.f, c->stream));
@@ -1463,7 +1499,7 @@ int rtm_forward_begin(rtm_ctx* c, int save_strips) {
   if (c->m.mstride != 0)
     for (int s = 0; s < c->nshot; ++s)
       if (!c->shot_model[s]) return fail(c, RTM_E_STATE, "shot %d has no model window", s);
-  int prc = ensure_planes(c);
+  int prc = ensure_two(c);
   if (prc != RTM_OK) return prc;
   c->f0 = 0; c->f1 = 1; c->f2 = 2; c->f3 = 3;
   c->save_strips = save_strips != 0;
@@ -1586,7 +1622,7 @@ int rtm_born_begin(rtm_ctx* c) {
   const long long fb = (long long)c->nshot * g.fstride;
   for (int i = 0; i < 3; ++i) HIPCHK(c, launch_fill(c->Q[i], fb, 0.f, c->stream));
   HIPCHK(c, launch_fill(c->d_rec, (long long)c->nshot * c->p.nt * c->p.n, 0.f, c->stream));
-  c->q0 = 0; c->q1 = 1; c->q2 = 2;
+  c->q0 = 0; c->q1 = 1; c->q2 = 2; c->q3 = 3;
   c->born = true;
   return RTM_OK;
 }
@@ -1641,7 +1677,7 @@ int rtm_adjoint_begin(rtm_ctx* c) {
   for (int i = 0; i < 3; ++i) HIPCHK(c, launch_fill(c->Q[i], fb, 0.f, c->stream));
   HIPCHK(c, launch_fill(c->I1, fb, 0.f, c->stream));
   HIPCHK(c, launch_strip_restore(c->g, c->F[c->f1], c->st, c->d_geo, c->p.nt - 2, c->nshot, c->stream));
-  c->q0 = 0; c->q1 = 1; c->q2 = 2;
+  c->q0 = 0; c->q1 = 1; c->q2 = 2; c->q3 = 3;
   c->adj = true;
   c->kb = -2;
   c->kf = -1;  // the reconstruction consumes the forward end state
@@ -1848,7 +1884,7 @@ int rtm_migrate(rtm_ctx* c) {
   if (!c->model_ok || !c->wav_ok || !c->shots_ok || !c->data_ok)
     return fail(c, RTM_E_STATE, "model, wavelet, shots and gathers must be set");
   if (!c->gexec) {
-    int prc = ensure_planes(c);
+    int prc = ensure_two(c);
     if (prc == RTM_OK) prc = ensure_lateral(c);
     if (prc != RTM_OK) return prc;
     // Capture the whole launch sequence once; the host-side buffer rotation

@@ -92,12 +92,14 @@ hipError_t hipLaunchKernel(const void* f, dim3, dim3, void** a, size_t, hipStrea
     l.t = "k_two";
     tmpl(n, "k_two", l);
     l.num("k", t.k).num("nt", t.nt).num("zs", t.zs).num("nimg", t.nimg);
+    l.num("u1", (long long)t.u1).num("u0", (long long)t.u0).num("ua", (long long)t.ua).num("ub", (long long)t.ub);
     l.field(t.u1).field(t.u0).field(t.ua).field(t.ub).field(t.cp);
   } else if (has(n, "k_interiorI")) {
     const IntArgs& t = *(IntArgs*)a[0];
     l.t = "k_interior";
     tmpl(n, "k_interior", l);
     l.num("k", t.k).num("nt", t.nt).num("zs", t.zs);
+    l.num("u1", (long long)t.u1).num("u0", (long long)t.u0).num("u2", (long long)t.u2);
     l.field(t.u1).field(t.u0).field(t.u2).field(t.uk).field(t.ua).field(t.ub);
   } else if (has(n, "k_frame")  && !has(n, "k_frame_lat")) {
     const FrameArgs& t = *(FrameArgs*)a[0];

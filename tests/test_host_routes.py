@@ -123,3 +123,71 @@ ctx.backward_begin(); ctx.backward_advance(60)
 out([r["kernel"] for r in log() if "frame_lat" in r["kernel"] or "k_tile" in r["kernel"]][:2])
 """)
     assert "frame_lat" in got[0] and got[1] == "k_tile"
+
+
+def test_buffers_of_two_steps_per_launch_are_held_by_batches_that_take_them():
+    got = run("""
+import numpy as np
+fb = 4 * 41 * 440 * 640
+res = []
+for kind in ("two", "fixed heights", "own windows", "small"):
+    ctx = context(zseg=16 if kind == "fixed heights" else 0, check_every=-1)
+    b = [ctx.device_bytes()]
+    n = 4 if kind == "small" else 40
+    if kind == "own windows":
+        ragged(ctx, n)
+        for s in range(n):
+            window(ctx, s, 1500.0 + s)
+        b[0] += 4 * fb
+    else:
+        shots(ctx, n)
+    log()
+    ctx.forward_begin(); ctx.forward_advance(60)
+    rows = log()
+    res.append([round((ctx.device_bytes() - b[0]) / fb, 1), any(r["kernel"] == "k_two" for r in rows),
+                any(r["dead"] for r in rows)])
+    ctx.close()
+out(res)
+""")
+    assert got == [[2.2, True, False], [0.0, False, False], [0.0, False, False], [0.0, False, False]]
+
+
+@pytest.mark.parametrize("steps", [0, 1, 2, 3, 5, 6])
+@pytest.mark.parametrize("backward", [False, True])
+def test_required_memory_takes_the_place_of_those_buffers(steps, backward):
+    """An allocation that fails beside them succeeds in their place, wherever the
+    rotation has put the fields of the running pass; the pass goes on, one step per
+    launch, from the two fields written last."""
+    got = run(f"""
+import numpy as np
+backward, steps = {backward}, {steps}
+kinds = dict(k_two=2, k_interior=1) if backward else dict(k_two=1, k_interior=3)  # TWO_*, EPI_*
+
+def launches():  # of the forward or the reconstructed field
+    rows = log()
+    assert not any(r["dead"] for r in rows)
+    return [r for r in rows if r["kernel"] in kinds and r["kind"] == kinds[r["kernel"]]]
+
+ctx = context(nt=61, nfd=5, check_every=-1)
+shots(ctx, 40)
+ctx.forward_begin()
+if backward:
+    ctx.set_gathers(np.zeros((40, ctx.p.n, ctx.p.nt), np.float32))
+    ctx.forward_advance(61)
+    ctx.backward_begin()
+advance = ctx.backward_advance if backward else ctx.forward_advance
+log()
+for n in [1] * (steps % 2) + [2] * (steps // 2):
+    advance(n)
+last = launches()[-1:]
+held = ctx.device_bytes()
+fake.fake_limit(fake.fake_used() + 1000)
+ctx.set_reflectivity(np.zeros((400, 578), np.float32))
+freed = held - ctx.device_bytes()
+advance(3)
+one = launches()
+newest = [(r["ub"], r["ua"]) if r["kernel"] == "k_two" else (r["u2"], r["u1"]) for r in last]
+out([freed > 2 * 4 * 41 * 440 * 640, [r["kernel"] for r in one], len({{r["u2"] for r in one}}),
+     newest in ([], [(one[0]["u1"], one[0]["u0"])])])
+""")
+    assert got == [True, ["k_interior"] * 3, 3, True]
