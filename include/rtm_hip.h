@@ -295,11 +295,15 @@ int rtm_data_dot_noalloc(const float* x, const float* y, long long n, long long 
  * bottom bands first, on the sum of both frame kernels' times, and last the
  * frame split (rtm_params.frame_split) on and off, and the tuned kernels
  * against whole steps in one launch.  Large batches also time two steps per
- * launch, with heights of their own, against one. */
+ * launch, with heights of their own, against one; the context then runs what was
+ * fastest, and zseg[3] describes the marching kernels also where that is another. */
 int rtm_autotune(rtm_ctx* ctx, int nsteps, int* zseg);
 /* The autotuner's three choices set by hand: rows per wave of the forward,
  * the source-reconstruction and the receiver-step kernels (Born and the
- * adjoint take the receiver step's). */
+ * adjoint take the receiver step's).  These are the marching kernels of one step
+ * per launch: setting their heights or their frame runs selects them for the
+ * context, also where whole steps in one launch or two steps per launch would
+ * be taken, until rtm_autotune is called (again). */
 int rtm_set_zseg(rtm_ctx* ctx, const int* zseg);
 /* Rows per frame-kernel wave: the top and bottom bands run in pieces of
  * rows_tb rows (ceil(n2/3)..n2; where the four-column kernel takes the middle

@@ -337,8 +337,8 @@ int watch_read(rtm_ctx* c, const char* pass) {
 // steps), so the line is twice as high there.
 //
 // A caller who sets anything that belongs to the marching kernels (zseg,
-// frame runs, fuse_frame, frame_split) gets them, unless rtm_autotune has timed
-// the two for the batch's migration.
+// frame runs, fuse_frame, frame_split) gets them, one step per launch, until
+// rtm_autotune times them against the others for the batch's migration.
 constexpr long long kTileWork = 50000000;
 
 // Two steps per launch (k_two) for the forward and backward passes of a
@@ -355,9 +355,9 @@ bool two_possible(const rtm_ctx* c) {
          !c->p.fuse_frame && c->cp_ok;
 }
 bool use_two(const rtm_ctx* c) {
-  if (!two_possible(c) || c->tile_tuned == 1) return false;
+  if (c->march_set || !two_possible(c) || c->tile_tuned == 1) return false;
   if (c->two_tuned >= 0) return c->two_tuned != 0;
-  return !c->march_set && c->cells >= two_cells(c->nfd);
+  return c->cells >= two_cells(c->nfd);
 }
 
 bool use_tile(const rtm_ctx* c, int pass) {

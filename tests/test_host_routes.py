@@ -191,3 +191,33 @@ out([freed > 2 * 4 * 41 * 440 * 640, [r["kernel"] for r in one], len({{r["u2"] f
      newest in ([], [(one[0]["u1"], one[0]["u0"])])])
 """)
     assert got == [True, ["k_interior"] * 3, 3, True]
+
+
+@pytest.mark.parametrize("nshot", [40, 12])  # two steps per launch; whole steps
+def test_heights_set_after_the_autotuner_are_used(nshot):
+    """The later of rtm_autotune and rtm_set_zseg / rtm_set_frame_runs decides."""
+    got = run(f"""
+def kernels():
+    log()
+    ctx.forward_begin(); ctx.forward_advance(60)
+    return sorted({{r["kernel"] for r in log() if r["kernel"] in ("k_two", "k_tile", "k_interior")}})
+res = []
+for which in ("zseg", "runs"):
+    ctx = context(check_every=-1)
+    fake.fake_cost(b"k_two", 0.5)
+    fake.fake_cost(b"k_tile", {9.0 if nshot == 40 else 0.5})
+    shots(ctx, {nshot})
+    ctx.autotune(8)
+    res.append(kernels())
+    if which == "zseg":
+        ctx.set_zseg(14, 14, 14)
+    else:
+        ctx.set_frame_runs(10, 16)
+    res.append(kernels())
+    ctx.autotune(8)
+    res.append(kernels())
+    ctx.close()
+out(res)
+""")
+    tuned = ["k_two"] if nshot == 40 else ["k_tile"]
+    assert got == [tuned, ["k_interior"], tuned] * 2
