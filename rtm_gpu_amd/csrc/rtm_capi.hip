@@ -105,6 +105,7 @@ struct rtm_ctx {
   bool model_ok = false, wav_ok = false, shots_ok = false, data_ok = false, save_strips = true;
   int zs = 32, nxt = 1;
   long long cells = 0;     // grid cells of the batch
+  long long tuned_cells = 0;  // of the batch that rtm_autotune timed
   int two_tuned = -1;      // rtm_autotune's choice: 1 two steps per launch, 0 one
   int zs2[5] = {0};        // rows per wave of two steps by kind (0: default)
   bool quads = false;      // every four consecutive shots share width and model window
@@ -1015,6 +1016,14 @@ int upload_frame_records(rtm_ctx* c) {
   return RTM_OK;
 }
 
+// The autotuner's choice between the kernels and what it tuned for two steps per
+// launch belong to batches like the one it timed.
+void forget_choice(rtm_ctx* c) {
+  c->tile_tuned = c->two_tuned = -1;
+  std::fill(std::begin(c->zs2), std::end(c->zs2), 0);
+  c->qrows = 0;
+}
+
 // Upload the batch geometry and its frame records.
 int upload_geometry(rtm_ctx* c) {
   const int ns = (int)c->geo.size();
@@ -1022,9 +1031,12 @@ int upload_geometry(rtm_ctx* c) {
   c->fs_ok = false;
   int rc = upload_frame_records(c);
   if (rc != RTM_OK) return rc;
-  if (ns != c->nshot) c->tile_tuned = c->two_tuned = -1;  // tuned for another batch
   c->cells = 0;
   for (const ShotGeo& q : c->geo) c->cells += (long long)c->g.nz * q.nx;
+  // The batches of a survey differ a little in their widths; within a third of
+  // the cells the kernels keep their order (kTileWork, two_cells).
+  if (ns != c->nshot || 4 * c->cells < 3 * c->tuned_cells || 3 * c->cells > 4 * c->tuned_cells)
+    forget_choice(c);
   c->nshot = ns;
   choose_zs(c, ns);
   drop_graph(c);
@@ -1321,6 +1333,7 @@ int rtm_set_model(rtm_ctx* c, const float* v, const float* r1, const float* w, c
   m.h1 = 1.0 + (double)c->p.hzx2_1;  // (1.0+hzx2_1)*Dc[M_top] (kernel.cu:58)
   m.hzx2_1 = c->p.hzx2_1; m.tao2 = c->p.tao2; m.h2 = c->p.h2;
   m.taoh = c->p.taoh; m.taoh2 = c->p.taoh2;
+  if (nfd != c->nfd) forget_choice(c);
   c->nfd = nfd;
   c->tp_ok = c->cp_ok = false;
   drop_graph(c);
@@ -2209,6 +2222,7 @@ int rtm_autotune(rtm_ctx* c, int nsteps, int* zseg) {
   c->zs_epi[EPI_BORN] = c->zs_epi[EPI_BORN64] = c->zs_epi[EPI_ADJ] = c->zs_epi[EPI_RCV];
   c->zs = c->zs_epi[fwd];
   c->two_tuned = two_choice;
+  c->tuned_cells = c->cells;
   c->rings_for = -1;
   c->kf = -1;
   c->kb = -2;

@@ -221,3 +221,53 @@ out(res)
 """)
     tuned = ["k_two"] if nshot == 40 else ["k_tile"]
     assert got == [tuned, ["k_interior"], tuned] * 2
+
+
+def test_a_choice_of_the_autotuner_is_for_batches_like_its_own():
+    """Whole steps chosen on narrow shots are not taken for a batch of the same
+    count that is much larger; a batch of about the same size keeps them."""
+    got = run("""
+def kernels():
+    log()
+    ctx.forward_begin(); ctx.forward_advance(60)
+    return sorted({r["kernel"] for r in log() if r["kernel"] in ("k_two", "k_tile", "k_interior")})
+fake.fake_cost(b"k_tile", 0.1)
+ctx = context(nx=2400, nfd=5, shots=30, check_every=-1)
+res = []
+for width in (900, 860, 2400, 900):
+    ragged(ctx, 30, [width] * 30)
+    if not res:
+        ctx.autotune(8)
+    res.append(kernels())
+out(res)
+""")
+    assert got == [["k_tile"], ["k_tile"], ["k_two"], ["k_two"]]
+
+
+def test_a_longer_operator_drops_the_choice():
+    got = run("""
+import numpy as np
+from rtm_gpu_amd import hip
+def kernels():
+    log()
+    ctx.forward_begin(); ctx.forward_advance(60)
+    return sorted({r["kernel"] for r in log() if r["kernel"] in ("k_two", "k_tile", "k_interior")})
+# least-squares rows: the operator is as long as the table's longest row
+nz, nx, n2, n, nt = 440, 618, 20, 578, 60
+ctx = hip.Context(nz=nz, nx=nx, n2=n2, nfdmax=12, nt=nt, nt2=nt, ilste=0, icompen=1, s_l=n2,
+                  s_r=nx - n2 - 1, s_z=n2, ds=1, n=n, tao2=1e-6, h2=1e-2, taoh=1e-4, taoh2=1e-8,
+                  hzx2_1=1.0, max_shots=41, check_every=-1)
+ctx.set_wavelet(np.zeros(nt + 1, np.float32))
+z = np.full((nz, nx), 1500.0, np.float32)
+def model(nfd):
+    ctx.set_model(z, z * 0, np.zeros(n2 + 1), np.ones(nfd + 1), np.array([0, nfd + 1], np.int32), 1, 1500.0, 1.0)
+fake.fake_cost(b"k_tile", 0.1)
+model(2)
+shots(ctx, 41)
+ctx.autotune(8)
+res = [kernels()]
+model(12)
+res.append(kernels())
+out(res)
+""")
+    assert got == [["k_tile"], ["k_interior"]]
