@@ -2073,13 +2073,27 @@ int rtm_autotune(rtm_ctx* c, int nsteps, int* zseg) {
     c->two_tuned = on ? 1 : 0;
     if (kf + 3 >= nt) kf = 2;
     if (kb < 4) kb = nt - 3;
+    // away from checkpoints, where those leave four steps between them: a
+    // checkpoint's step is launched by itself
+    const auto free4 = [&](int k) {
+      return c->snap_slot[k] < 0 && c->snap_slot[k - 1] < 0 && c->snap_slot[k - 2] < 0 && c->snap_slot[k - 3] < 0;
+    };
+    int b = kb;
+    while (b >= 4 && !free4(b)) --b;
+    if (b < 4)
+      for (b = nt - 3; b >= 4 && !free4(b);) --b;
+    if (b >= 4) kb = b;
     if (on) c->img_pend = 0;
     int r = RTM_OK;
     for (int i = 0; i < 4 && r == RTM_OK; i += on ? 2 : 1) {
       r = on ? forward_two(c, kf + i) : forward_step(c, kf + i);
       if (r != RTM_OK) return r;
-      if (!on) r = backward_step(c, kb - i, false);
-      else if (backward_two_ok(c, kb - i, 2)) r = backward_two(c, kb - i, false, 2);
+      if (on && backward_two_ok(c, kb - i, 2)) {
+        r = backward_two(c, kb - i, false, 2);
+      } else {
+        r = backward_step(c, kb - i, false);
+        if (on && r == RTM_OK) r = backward_step(c, kb - i - 1, false);
+      }
     }
     kf = kf + 4 < nt ? kf + 4 : 2;  // the steps that pairs() takes next
     kb = kb >= 4 ? kb - 4 : nt - 3;

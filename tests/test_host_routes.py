@@ -271,3 +271,43 @@ res.append(kernels())
 out(res)
 """)
     assert got == [["k_tile"], ["k_interior"]]
+
+
+@pytest.mark.parametrize("snap_every", [0, 20, 50, 4])
+def test_two_steps_are_timed_on_whole_cycles(snap_every):
+    """A cycle that rtm_autotune times takes four steps each way, checkpoint or
+    not: as many of the reconstruction as of the forward field, and of the
+    receiver field; away from checkpoints where they leave room."""
+    got = run(f"""
+ctx = context(nt=150, shots=41, snap_every={snap_every}, check_every=-1)
+shots(ctx, 41)
+fake.fake_cost(b"k_two", 0.5)
+fake.fake_cost(b"k_tile", 9.0)
+log()
+ctx.autotune(8)
+steps = dict(fwd=0, src=0, rcv=0)
+pairs = 0
+for r in log():
+    if r["kernel"] == "k_two":
+        steps[("fwd", "fwd", "src", "rcv", "rcv")[r["kind"]]] += 2
+        pairs += r["kind"] == 2
+    elif r["kernel"] == "k_interior":
+        name = {{0: "fwd", 3: "fwd", 1: "src", 2: "rcv", 7: "rcv"}}.get(r["kind"])
+        steps[name] += 1
+    elif r["kernel"] == "k_tile":
+        for name in (["fwd"], ["src", "rcv"])[r["kind"]]:
+            steps[name] += 1
+out([steps["fwd"] - steps["src"], steps["src"] - steps["rcv"], pairs])
+""")
+    full = run(f"""
+ctx = context(nt=150, shots=41, check_every=-1)
+shots(ctx, 41)
+fake.fake_cost(b"k_two", 0.5)
+fake.fake_cost(b"k_tile", 9.0)
+log()
+ctx.autotune(8)
+out(sum(r["kernel"] == "k_two" and r["kind"] == 2 for r in log()))
+""")
+    assert got[:2] == [0, 0]
+    if snap_every != 4:  # checkpoints at steps 4, 5, 8, 9, ...: every cycle meets some
+        assert got[2] == full
