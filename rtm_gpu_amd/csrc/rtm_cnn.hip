@@ -689,7 +689,7 @@ struct rtm_cnn {
   // device-resident training set
   float *ds_x = nullptr, *ds_t = nullptr;
   int* ds_order = nullptr;
-  double* ds_sq = nullptr;  // loss partial sums of the batches of an epoch
+  double* ds_sq = nullptr;  // loss partial sums of up to LOSS_BATCHES batches
   int ds_nb = 0;
   long long ds_cap = 0;
   int ds_n = 0;
@@ -834,6 +834,7 @@ int pack_input(rtm_cnn* c, const float* x_dev, int n, int h, int w, const int* o
 }
 
 constexpr int SQ_BLOCKS = 256;  // partial sums of a batch's loss
+constexpr int LOSS_BATCHES = 1024;  // losses that rtm_cnn_fit reads back at a time (2 MB)
 // The loss of a batch of npix pixels from its partial sums.
 double loss_of(const double* part, long long npix) {
   double s = 0.0;
@@ -1072,16 +1073,16 @@ int rtm_cnn_fit(rtm_cnn* c, const float* x, const float* t, int n, int h, int w,
     c->ds_cap = (long long)need;
     c->ds_n = n;
   }
-  const int batches = n / batch;
-  if (batches > c->ds_nb) {
+  const int batches = n / batch, keep = std::min(batches, LOSS_BATCHES);
+  if (keep > c->ds_nb) {
     CNNCHK(c, hipStreamSynchronize(c->stream));
     cfree_dev(c, &c->ds_sq);
     c->ds_nb = 0;
-    rc = calloc_dev(c, &c->ds_sq, (size_t)batches * SQ_BLOCKS);
+    rc = calloc_dev(c, &c->ds_sq, (size_t)keep * SQ_BLOCKS);
     if (rc != RTM_CNN_OK) return rc;
-    c->ds_nb = batches;
+    c->ds_nb = keep;
   }
-  std::vector<double> part((size_t)batches * SQ_BLOCKS);
+  std::vector<double> part((size_t)keep * SQ_BLOCKS);
   CNNCHK(c, hipMemcpyAsync(c->ds_x, x, need * c->c[0] * sizeof(float), hipMemcpyHostToDevice, c->stream));
   CNNCHK(c, hipMemcpyAsync(c->ds_t, t, need * sizeof(float), hipMemcpyHostToDevice, c->stream));
   std::vector<int> order(n);
@@ -1098,22 +1099,23 @@ int rtm_cnn_fit(rtm_cnn* c, const float* x, const float* t, int n, int h, int w,
     }
     // the previous epoch ended with a stream synchronisation (the loss read-back)
     CNNCHK(c, hipMemcpyAsync(c->ds_order, order.data(), n * sizeof(int), hipMemcpyHostToDevice, c->stream));
-    int nb = 0;
-    for (int b0 = 0; b0 + batch <= n; b0 += batch) {
-      rc = pack_input(c, c->ds_x, batch, h, w, c->ds_order, b0, c->ds_t);
+    double sum = 0.0;
+    for (int nb = 0; nb < batches; ++nb) {
+      const int slot = nb % keep;
+      rc = pack_input(c, c->ds_x, batch, h, w, c->ds_order, nb * batch, c->ds_t);
       if (rc == RTM_CNN_OK)
-        rc = loss_grad_dev(c, c->t32, batch, h, w, c->ds_sq + (size_t)nb * SQ_BLOCKS);
+        rc = loss_grad_dev(c, c->t32, batch, h, w, c->ds_sq + (size_t)slot * SQ_BLOCKS);
       if (rc == RTM_CNN_OK) rc = adam_dev(c, lr, 0.9f, 0.999f, 1e-8f);
       if (rc != RTM_CNN_OK) return rc;
-      ++nb;
+      if (slot + 1 < keep && nb + 1 < batches) continue;
+      // the losses are read once an epoch, or when the room for them is full
+      CNNCHK(c, hipMemcpyAsync(part.data(), c->ds_sq, (size_t)(slot + 1) * SQ_BLOCKS * sizeof(double),
+                               hipMemcpyDeviceToHost, c->stream));
+      CNNCHK(c, hipStreamSynchronize(c->stream));
+      for (int i = 0; i <= slot; ++i)
+        sum += loss_of(part.data() + (size_t)i * SQ_BLOCKS, (long long)batch * h * w);
     }
-    // the batches' losses are read once an epoch
-    CNNCHK(c, hipMemcpyAsync(part.data(), c->ds_sq, (size_t)nb * SQ_BLOCKS * sizeof(double),
-                             hipMemcpyDeviceToHost, c->stream));
-    CNNCHK(c, hipStreamSynchronize(c->stream));
-    double sum = 0.0;
-    for (int i = 0; i < nb; ++i) sum += loss_of(part.data() + (size_t)i * SQ_BLOCKS, (long long)batch * h * w);
-    if (loss_per_epoch) loss_per_epoch[ep] = nb ? sum / nb : 0.0;
+    if (loss_per_epoch) loss_per_epoch[ep] = sum / batches;
   }
   CNNCHK(c, hipStreamSynchronize(c->stream));
   return RTM_CNN_OK;

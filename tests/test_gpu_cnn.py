@@ -206,3 +206,19 @@ def test_fit_learns_a_deconvolution():
     assert hist[-1] < 0.3 * ident
     y = net.forward(x[:8])
     assert float(np.mean((y - t[:8]) ** 2)) < 0.4 * ident
+
+
+def test_epoch_loss_over_more_batches_than_are_kept():
+    """1100 batches of one image with a zero learning rate: the epoch's loss is
+    the mean over the set, which one batch of all of it gives."""
+    from rtm_gpu_amd import cnn
+    rng = np.random.default_rng(6)
+    n = 1100
+    x = rng.standard_normal((n, 1, 4, 4)).astype(np.float32)
+    t = rng.standard_normal((n, 4, 4)).astype(np.float32)
+    net = cnn.Deblur([1, 8, 1], n * 16, n * 4)
+    net.init_params(seed=2, last_zero=False)
+    loss, _ = net.loss_grad(x, t)
+    hist = net.fit(x, t, epochs=2, batch=1, lr=0.0, seed=3)
+    # FP64 sums of the same FP32 differences in another order
+    assert np.abs(hist - loss).max() <= 1e-12 * loss

@@ -311,3 +311,25 @@ out(sum(r["kernel"] == "k_two" and r["kind"] == 2 for r in log()))
     assert got[:2] == [0, 0]
     if snap_every != 4:  # checkpoints at steps 4, 5, 8, 9, ...: every cycle meets some
         assert got[2] == full
+
+
+def test_fit_keeps_the_losses_of_a_bounded_number_of_batches():
+    """Training on many small batches holds no more device memory for their
+    losses than on a thousand of them."""
+    got = run("""
+import numpy as np
+from rtm_gpu_amd import cnn
+used = []
+for n in (1024, 3000):
+    net = cnn.Deblur([1, 4, 1], 64, 8)
+    x = np.zeros((n, 1, 2, 2), np.float32)
+    log()
+    b = fake.fake_used()
+    net.fit(x, x[:, 0], 2, 1, 1e-3)
+    used.append(fake.fake_used() - b - n * (4 + 4 + 1) * 4)
+    steps = sum("k_adam" in r["kernel"] for r in log())
+    net.close()
+    used.append(steps)
+out(used)
+""")
+    assert got == [1024 * 256 * 8, 2048, 1024 * 256 * 8, 6000]
