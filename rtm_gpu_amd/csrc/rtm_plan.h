@@ -15,19 +15,13 @@ namespace rtm {
 // where it holds frame cells, of the ring of cells whose pre-blend values they
 // read.
 RTM_HD constexpr int tile_halo(int nfd) { return nfd + 1; }
-// The tile holds cells of the frame (n2 deep on an nz x nx grid).
-RTM_HD inline bool tile_edge(int z0, int x0, int th, int n2, int nz, int nx) {
-  return z0 < n2 || z0 + th > nz - n2 || x0 < n2 || x0 + 64 > nx - n2;
-}
-// All that the tile stages lies on the grid.  A tile without frame cells reaches
-// a cell past it where n2 == nfd: the outermost ring, of which it uses nothing.
-RTM_HD inline bool tile_inside(int z0, int x0, int th, int nfd, int nz, int nx) {
-  const int r = tile_halo(nfd);
-  return z0 >= r && z0 + th + r <= nz && x0 >= r && x0 + 64 + r <= nx;
-}
-// Such a tile loads without clamps, every other one through the outer mirror.
-RTM_HD inline bool tile_direct(int z0, int x0, int th, int nfd, int n2, int nz, int nx) {
-  return !tile_edge(z0, x0, th, n2, nz, nx) && tile_inside(z0, x0, th, nfd, nz, nx);
+// The tile takes the path of tiles with frame cells (n2 deep on an nz x nx grid):
+// clamped loads.  The others load without clamps, so what they stage has to lie
+// on the grid: where n2 == nfd a tile beside the frame reaches a cell past it and
+// takes the clamped path as well.
+RTM_HD inline bool tile_edge(int z0, int x0, int th, int nfd, int n2, int nz, int nx) {
+  const int e = n2 > tile_halo(nfd) ? n2 : tile_halo(nfd);
+  return z0 < e || z0 + th > nz - e || x0 < e || x0 + 64 > nx - e;
 }
 
 }  // namespace rtm

@@ -66,8 +66,7 @@ __global__ __launch_bounds__(512) void k_tile(const TileArgs a) {
     return zz >= N2 && zz < NZ - N2 && xx >= N2 && xx < NX - N2;
   };
   // uniform: tiles with frame cells, tiles with interior cells
-  const bool edge = tile_edge(z0, x0, TH, N2, NZ, NX);
-  const bool direct = tile_direct(z0, x0, TH, NFD, N2, NZ, NX);
+  const bool edge = tile_edge(z0, x0, TH, NFD, N2, NZ, NX);
   const bool has_inner = z0 + TH > N2 && z0 < NZ - N2 && x0 + 64 > N2 && x0 < NX - N2;
 
   const long long so = (long long)shot * g.fstride, mo = (long long)sg.win * m.mstride;
@@ -104,7 +103,7 @@ __global__ __launch_bounds__(512) void k_tile(const TileArgs a) {
     for (int j = 0; j < CPT; ++j) ko[j] = __float_as_uint(ldg(mk, own[j]));
   }
   float lu[NL], lq[TWO ? NL : 1];
-  if (!direct) {  // the outer mirror (kernel.cu:65-68)
+  if (edge) {  // the outer mirror (kernel.cu:65-68)
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
       const int e = tid + i * NT, r = e / LW;

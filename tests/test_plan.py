@@ -12,27 +12,19 @@ SHIM = r"""
 #include "rtm_plan.h"
 using namespace rtm;
 // Tiles of an nz x nx grid that load without clamps and whose staged cells
-// leave it.  rule 0: the kernel's; 1: every tile without frame cells.
-extern "C" int tiles_outside(int nz, int nx, int n2, int nfd, int th, int rule) {
+// leave it.  e: the depth up to which a tile counts as one of the frame (0: the
+// kernel's rule).
+extern "C" int tiles_outside(int nz, int nx, int n2, int nfd, int th, int e) {
   int bad = 0;
   const int r = tile_halo(nfd);
   for (int z0 = 0; z0 < nz; z0 += th)
     for (int x0 = 0; x0 < nx; x0 += 64) {
-      const bool direct = rule == 0 ? tile_direct(z0, x0, th, nfd, n2, nz, nx)
-                                    : !tile_edge(z0, x0, th, n2, nz, nx);
-      if (!direct) continue;
+      if (e ? z0 < e || z0 + th > nz - e || x0 < e || x0 + 64 > nx - e
+            : tile_edge(z0, x0, th, nfd, n2, nz, nx)) continue;
       const int zl = z0 - r, zh = z0 + th + r - 1, xl = x0 - r, xh = x0 + 64 + r - 1;
       bad += zl < 0 || zh >= nz || xl < 0 || xh >= nx;
     }
   return bad;
-}
-// Tiles without frame cells that load through the mirror.
-extern "C" int tiles_clamped(int nz, int nx, int n2, int nfd, int th) {
-  int n = 0;
-  for (int z0 = 0; z0 < nz; z0 += th)
-    for (int x0 = 0; x0 < nx; x0 += 64)
-      n += !tile_edge(z0, x0, th, n2, nz, nx) && !tile_direct(z0, x0, th, nfd, n2, nz, nx);
-  return n;
 }
 """
 
@@ -57,15 +49,13 @@ def test_tiles_stage_cells_of_the_grid_only(plan, nfd):
                 for w in widths:
                     nz, nx = h + 2 * n2, w + 2 * n2
                     assert plan.tiles_outside(nz, nx, n2, nfd, th, 0) == 0, (nz, nx, n2, th)
-                    if n2 > nfd:  # no tile is clamped that need not be
-                        assert plan.tiles_clamped(nz, nx, n2, nfd, th) == 0, (nz, nx, n2, th)
 
 
 def test_a_frame_as_deep_as_the_operator_needs_the_clamp(plan):
     """Row -1 (a tile that starts at n2 == nfd) and row nz (one that ends at
     nz - n2) are what a tile without frame cells would load there."""
-    assert plan.tiles_outside(136, 186, 8, 8, 8, 1) > 0
+    assert plan.tiles_outside(136, 186, 8, 8, 8, 8) > 0
     for nfd in range(1, 13):
         nz = 96 + nfd  # nz - n2 = 96
-        assert plan.tiles_outside(nz, 186, nfd, nfd, 8, 1) > 0, nfd
-        assert plan.tiles_outside(nz, 186, nfd, nfd, 16, 1) > 0, nfd
+        assert plan.tiles_outside(nz, 186, nfd, nfd, 8, nfd) > 0, nfd
+        assert plan.tiles_outside(nz, 186, nfd, nfd, 16, nfd) > 0, nfd
