@@ -105,6 +105,8 @@ struct rtm_ctx {
   bool model_ok = false, wav_ok = false, shots_ok = false, data_ok = false, save_strips = true;
   int zs = 32, nxt = 1;
   long long cells = 0;     // grid cells of the batch
+  mutable BatchWork work;  // of the batch, made on first use
+  mutable bool work_ok = false;
   long long tuned_cells = 0;  // of the batch that rtm_autotune timed
   int two_tuned = -1;      // rtm_autotune's choice: 1 two steps per launch, 0 one
   int zs2[5] = {0};        // rows per wave of two steps by kind (0: default)
@@ -323,34 +325,41 @@ int watch_read(rtm_ctx* c, const char* pass) {
   return RTM_OK;
 }
 
-// Whole steps by k_tile instead of the marching kernels.
-//
-// A marching wave spends 0.5 to 1 us on each of its 20 to 30 rows whatever the
-// batch, so a small batch costs the same as one that fills the GPU; k_tile is
-// two memory accesses deep, but it is bound by instruction issue where the
-// marching kernels run at the memory's rate.  Its work per cell grows with the
-// half-length, so the line is drawn on cells times half-length.  Measured
-// (k_tile against marching, forward + backward, ms per 100 steps): half-length
-// 3, 1.4 M cells 3.6 / 10.6, 12 M 19 / 22, 23 M 40 / 35; half-length 10, 0.6 M
-// cells 3.1 / 14.1, 2.5 M 8.9 / 14.9, 5 M 15.8 / 15.6, 10 M 31 / 22.  A Born
-// or adjoint step takes both fields through one launch and shares the
-// coefficient rows: at half-length 4, 11 M cells 29 / 34, 22 M 143 / 164 (250
-// steps), so the line is twice as high there.
+// Which kernels a batch takes: whole steps in one launch (k_tile), two steps of
+// the interior per launch (k_two; half-lengths up to 5, every four consecutive
+// shots on one model window), or the marching kernels of one step, whichever the
+// costs of rtm_plan.h are lowest for.
 //
 // A caller who sets anything that belongs to the marching kernels (zseg,
 // frame runs, fuse_frame, frame_split) gets them, one step per launch, until
 // rtm_autotune times them against the others for the batch's migration.
-constexpr long long kTileWork = 50000000;
+const BatchWork& batch_work(const rtm_ctx* c) {
+  if (c->work_ok) return c->work;
+  const Grid& g = c->g;
+  BatchWork w;
+  const int cols = two_cols(g, std::min(c->nfd, TWO_MAX_NFD), c->nshot);
+  double cells = 0.0;
+  for (const ShotGeo& q : c->geo) {
+    w.add(g.nz, q.nx, g.n2, cols);
+    cells += 1e-6 * g.nz * q.nx;
+  }
+  const double ns = std::max<double>(1.0, (double)c->geo.size());
+  w.quad = ((c->nshot + TWO_SHOTS - 1) / TWO_SHOTS) * TWO_SHOTS / ns;
+  if (c->m.mstride) {
+    int n = 0;
+    for (int r : c->win_ref) n += r > 0;
+    w.windows = cells * n / ns;
+  }
+  c->work = w;
+  c->work_ok = true;
+  return c->work;
+}
+double cost_tile(const rtm_ctx* c, bool both) { return cost::tile(batch_work(c), c->nfd, both, c->tab_ls); }
+double cost_march(const rtm_ctx* c, bool both) { return cost::march(batch_work(c), c->nfd, both, c->tab_ls); }
+double cost_two(const rtm_ctx* c) {
+  return c->nfd <= TWO_MAX_NFD ? cost::two(batch_work(c), c->nfd) : HUGE_VAL;
+}
 
-// Two steps per launch (k_two) for the forward and backward passes of a
-// migration: half-lengths up to 5, every four consecutive shots on one model
-// window.  k_two marches and needs a batch that fills the GPU, k_tile's work per
-// cell grows with the half-length.  Measured (k_two / k_tile, migration of 351 x
-// 1701 shots, ms per 100 steps, not tuned): half-length 2, 4.3 M cells 8.1 / 7.4,
-// 5.8 M 8.8 / 9.0, 8.7 M 11.2 / 14.5; 3, 5.8 M 10.2 / 9.3, 7.2 M 12.6 / 12.6,
-// 8.7 M 13.2 / 15.2; 5, 7.2 M 17.9 / 13.7, 8.7 M 18.4 / 16.4, 10.1 M 18.8 / 18.8.
-// Against k_interior: 11.6 M cells 18.5 / 20.6, 34.7 M 41.6 / 46.2.
-constexpr long long two_cells(int nfd) { return 3000000 + 1400000ll * nfd; }
 bool two_possible(const rtm_ctx* c) {
   return c->F[3] && c->Q[3] && c->nfd <= TWO_MAX_NFD && c->nshot >= TWO_SHOTS && c->quads &&
          !c->p.fuse_frame && c->cp_ok;
@@ -358,14 +367,14 @@ bool two_possible(const rtm_ctx* c) {
 bool use_two(const rtm_ctx* c) {
   if (c->march_set || !two_possible(c) || c->tile_tuned == 1) return false;
   if (c->two_tuned >= 0) return c->two_tuned != 0;
-  return c->cells >= two_cells(c->nfd);
+  return cost_two(c) < std::min(cost_tile(c, false), cost_march(c, false));
 }
 
 bool use_tile(const rtm_ctx* c, int pass) {
   if (c->march_set) return false;
   const bool both = pass == TILE_BORN || pass == TILE_ADJ;
   if (!both && c->tile_tuned >= 0) return c->tile_tuned != 0;
-  return (both || !use_two(c)) && c->cells * c->nfd <= (both ? 2 : 1) * kTileWork;
+  return (both || !use_two(c)) && cost_tile(c, both) <= cost_march(c, both);
 }
 hipError_t tile_step(rtm_ctx* c, int pass, const TileArgs& a) {
   return launch_tile(pass, c->nfd, a, c->nshot, c->cells, c->stream);
@@ -495,8 +504,8 @@ void release_two(rtm_ctx* c) {
   c->rings_for = -1;
 }
 
-// What two steps per launch need where the batch may take them: the fourth
-// buffers, only if they leave an eighth of the card for what is allocated later,
+// What two steps per launch need where the batch may take them, by their cost or
+// by what the autotuner finds (costs are within 20%): the fourth buffers, only if they leave an eighth of the card for what is allocated later,
 // and the coefficient planes of the batch's model windows.  Without them every
 // launch takes one step.  Allocates: not inside a stream capture.
 int ensure_two(rtm_ctx* c) {
@@ -506,7 +515,7 @@ int ensure_two(rtm_ctx* c) {
     c->quads = c->quads && a.nx == b.nx && a.win == b.win;
   }
   if (c->capturing || !c->quads || c->nshot < TWO_SHOTS || c->nfd > TWO_MAX_NFD || c->march_set ||
-      c->cells < two_cells(1))
+      c->p.fuse_frame || cost_two(c) > 1.25 * std::min(cost_tile(c, false), cost_march(c, false)))
     return RTM_OK;
   if (!c->F[3]) {
     const size_t fb = (size_t)c->p.max_shots * c->g.fstride;
@@ -1031,10 +1040,11 @@ int upload_geometry(rtm_ctx* c) {
   c->fs_ok = false;
   int rc = upload_frame_records(c);
   if (rc != RTM_OK) return rc;
+  c->work_ok = false;
   c->cells = 0;
   for (const ShotGeo& q : c->geo) c->cells += (long long)c->g.nz * q.nx;
   // The batches of a survey differ a little in their widths; within a third of
-  // the cells the kernels keep their order (kTileWork, two_cells).
+  // the cells the choice is kept.
   if (ns != c->nshot || 4 * c->cells < 3 * c->tuned_cells || 3 * c->cells > 4 * c->tuned_cells)
     forget_choice(c);
   c->nshot = ns;
@@ -1334,6 +1344,7 @@ int rtm_set_model(rtm_ctx* c, const float* v, const float* r1, const float* w, c
   m.hzx2_1 = c->p.hzx2_1; m.tao2 = c->p.tao2; m.h2 = c->p.h2;
   m.taoh = c->p.taoh; m.taoh2 = c->p.taoh2;
   if (nfd != c->nfd) forget_choice(c);
+  c->work_ok = false;
   c->nfd = nfd;
   c->tp_ok = c->cp_ok = false;
   drop_graph(c);
@@ -1459,6 +1470,7 @@ int rtm_set_shot_model(rtm_ctx* c, int shot, const float* v, const float* r1) {
     c->tp_ok = c->cp_ok = false;
   }
   c->win_ref[w] += 1;
+  c->work_ok = false;
   if (c->geo[shot].win != w) c->quads = false;  // until the next pass looks again
   c->geo[shot].win = w;
   c->geo[shot].fw = w;
@@ -2208,10 +2220,10 @@ int rtm_autotune(rtm_ctx* c, int nsteps, int* zseg) {
     }
   }
   // The tuned kernels against whole steps by k_tile, on the time of everything
-  // that twelve steps each way launch (whole imaging cycles).  Batches far from
-  // the line between them (use_tile) are not timed.
+  // that twelve steps each way launch (whole imaging cycles), unless their costs
+  // are far apart.
   int tile_choice = 0;
-  if (rc == RTM_OK && !c->p.fuse_frame && c->cells * c->nfd <= 4 * kTileWork) {
+  if (rc == RTM_OK && !c->p.fuse_frame && cost_tile(c, false) <= 1.5 * std::min(cost_march(c, false), two_choice ? cost_two(c) : HUGE_VAL)) {
     double tot[2] = {0.0, 0.0};
     for (int round = 0; round < kRounds && rc == RTM_OK; ++round)
       for (int i = 0; i < 2 && rc == RTM_OK; ++i) {

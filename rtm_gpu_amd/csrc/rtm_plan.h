@@ -24,4 +24,82 @@ RTM_HD inline bool tile_edge(int z0, int x0, int th, int nfd, int n2, int nz, in
   return z0 < e || z0 + th > nz - e || x0 < e || x0 + 64 > nx - e;
 }
 
+// ---- which kernels a batch takes ----------------------------------------------
+// What the kernels work on in a step of a batch, in millions of cells, padding
+// included.
+struct BatchWork {
+  double tile_inner = 0, tile_edge = 0;  // k_tile: tiles without and with frame cells
+  double wave = 0, wave_two = 0;         // waves of k_interior (256 columns), of k_two
+  double inner = 0, frame = 0;           // cells of the interior, of the frame
+  double quad = 1;                       // shots of full blocks of four per shot
+  double windows = 0;                    // cells times distinct model windows per shot
+  // a shot of an nz x nx grid; two_cols: columns of a wave of k_two
+  void add(int nz, int nx, int n2, int two_cols) {
+    const int mnz = nz - 2 * n2, mnx = nx - 2 * n2;
+    const auto split = [n2](int n, int t, double* all, double* in) {  // tiles of t along n cells
+      *all = (n + t - 1) / t;
+      const int lo = (n2 + t - 1) / t, hi = (n - n2) / t;  // those from n2 to n - n2
+      *in = hi > lo ? hi - lo : 0;
+    };
+    double az, iz, ax, ix;
+    split(nz, 8, &az, &iz);
+    split(nx, 64, &ax, &ix);
+    tile_inner += iz * ix * 512e-6;
+    tile_edge += (az * ax - iz * ix) * 512e-6;
+    wave += (mnx + 255) / 256 * 256 * 1e-6 * mnz;
+    wave_two += (mnx + two_cols - 1) / two_cols * 256 * 1e-6 * mnz;
+    inner += 1e-6 * mnz * mnx;
+    frame += 1e-6 * nz * nx - 1e-6 * mnz * mnx;
+  }
+};
+
+// Microseconds of a forward and a backward step by half-length 1..12, fitted to
+// 880 timed batches: ten grids of 75 to 2400 columns, 2 to 60 M cells,
+// least-squares rows up to half-length 5, Taylor rows above.  A marching wave
+// spends 0.5 to 1 us on each of its 20 to 30 rows whatever the batch and pads
+// the interior to 256 columns; k_tile is two memory accesses deep but bound by
+// instruction issue, the more the longer the operator and the more of its tiles
+// hold frame cells; k_two takes two steps per pass over memory.  The sums are
+// within 20% of the times, and the kernel of the smallest one took on average
+// 0.6% longer than the fastest and at worst 1.24 times as long.  One line on the cells times the
+// half-length, which depends on none of the grid's shape, was 5.7% off on average
+// and up to twice as slow: 144 shots of 261 x 133 at half-length 8, 100 steps,
+// 22 ms by k_tile, 15 by the marching kernels.
+namespace cost {
+constexpr int kN = 12;
+constexpr double kTile[kN][3] = {  // per launch, tiles without, with frame cells
+    {3, 14.6, 18.3}, {1, 15.6, 19.4}, {1, 16.1, 20.4}, {1, 17.1, 21.7}, {1, 17.7, 22.6}, {4, 18.6, 23.0},
+    {4, 19.5, 26.7}, {6, 21.7, 30.8}, {7, 22.1, 31.8}, {8, 22.9, 33.6}, {9, 22.8, 33.8}, {10, 23.6, 34.0}};
+constexpr double kMarch[kN][4] = {  // per launch, waves, frame cells, interior cells
+    {37, 4.7, 16, 5.9}, {40, 4.7, 16, 5.8}, {40, 4.8, 16, 5.6}, {48, 4.9, 18, 7.6}, {48, 6.2, 15, 6.2},
+    {56, 6.8, 10, 4.7}, {62, 6.5, 11, 4.5}, {70, 6.9, 10, 4.2}, {79, 6.9, 11, 3.2}, {86, 6.6, 14, 2.3},
+    {97, 5.9, 13, 2.6}, {109, 5.7, 11, 1.0}};
+constexpr double kTwo[5][4] = {{30, 3.8, 14.4, 3.1}, {35, 4.3, 14.9, 2.6}, {46, 5.3, 14.0, 2.1},
+                               {52, 5.4, 18.0, 1.3}, {65, 7.5, 17.5, 0.5}};
+// the same of a Born and an adjoint step (half-lengths 7, 9, 11 between their
+// neighbours)
+constexpr double kTile2[kN][3] = {
+    {10, 17.4, 19.8}, {1, 20.7, 23.5}, {1, 21.4, 25.2}, {1, 24.8, 27.1}, {1, 27.9, 34.0}, {1, 25.4, 33.8},
+    {4, 25.6, 34.7}, {7, 25.9, 35.6}, {9, 31, 51}, {11, 35.7, 66}, {13, 36.6, 66}, {15, 37.5, 66}};
+constexpr double kMarch2[kN][4] = {
+    {17, 7.5, 33, 10.8}, {26, 8.3, 31, 11.2}, {46, 9.0, 29, 10.8}, {62, 9.8, 33, 13}, {95, 11.3, 25, 12.4},
+    {75, 9.9, 25, 7}, {90, 10.6, 25, 6.3}, {105, 11.4, 24, 5.5}, {119, 12, 27, 3}, {133, 12.5, 31, 0.3},
+    {147, 11.7, 31, 0.2}, {161, 10.8, 31, 0}};
+
+inline double tile(const BatchWork& w, int nfd, bool both, bool ls) {
+  const double* k = both ? kTile2[nfd - 1] : kTile[nfd - 1];
+  const double win = !both ? 2.0 : ls ? 2.3 + 1.9 * nfd : 2.5;  // a window's planes from memory
+  return k[0] + k[1] * w.tile_inner + k[2] * w.tile_edge + win * w.windows;
+}
+inline double march(const BatchWork& w, int nfd, bool both, bool ls) {
+  const double* k = both ? kMarch2[nfd - 1] : kMarch[nfd - 1];
+  const double win = !both ? 3.2 : ls ? 7 + 2.6 * nfd : 5.0;
+  return k[0] + k[1] * w.wave + k[2] * w.frame + k[3] * w.inner + win * w.windows;
+}
+inline double two(const BatchWork& w, int nfd) {  // windows: shared by four shots at least
+  const double* k = kTwo[nfd - 1];
+  return k[0] + k[1] * w.wave_two * w.quad + k[2] * w.frame * w.quad + k[3] * w.inner;
+}
+}  // namespace cost
+
 }  // namespace rtm

@@ -333,3 +333,46 @@ for n in (1024, 3000):
 out(used)
 """)
     assert got == [1024 * 256 * 8, 2048, 1024 * 256 * 8, 6000]
+
+
+# Batches timed on an MI355X, ms for 60 steps each way: marching kernels, two
+# steps per launch, whole steps in one launch (None: not timed or not built)
+TIMED = [
+    ("mig", 400, 140, 20, 8, 89, 8.3, None, 13.0), ("mig", 261, 133, 30, 7, 165, 9.1, None, 13.5),
+    ("mig", 400, 270, 20, 6, 62, 7.6, None, 10.8), ("mig", 400, 140, 20, 11, 65, 7.7, None, 10.6),
+    ("mig", 261, 133, 30, 5, 245, 12.3, 14.4, 16.8), ("mig", 400, 270, 20, 9, 41, 7.1, None, 9.5),
+    ("mig", 400, 140, 20, 3, 107, 8.2, 7.8, 10.3), ("mig", 400, 270, 20, 4, 79, 10.4, 9.7, 12.7),
+    ("mig", 400, 270, 20, 1, 37, 5.3, 3.9, 5.1), ("mig", 400, 140, 20, 12, 60, 8.0, None, 10.0),
+    ("mig", 411, 1761, 30, 3, 41, 22.9, 19.2, 30.7), ("mig", 411, 1761, 30, 3, 6, 6.9, 5.5, 4.4),
+    ("mig", 391, 700, 30, 3, 110, 23.8, 19.1, 32.6), ("mig", 261, 133, 30, 1, 115, 6.8, 5.5, 6.5),
+    ("pairs", 400, 270, 20, 10, 83, 19.0, None, 37.1), ("pairs", 400, 270, 20, 12, 69, 16.7, None, 31.5),
+    ("pairs", 400, 270, 20, 6, 139, 23.6, None, 34.4), ("pairs", 400, 270, 20, 8, 104, 20.3, None, 28.8),
+    ("pairs", 391, 700, 30, 2, 18, 10.4, None, 5.5), ("pairs", 391, 700, 30, 8, 20, 16.1, None, 9.5)]
+
+
+def test_a_batch_takes_the_kernel_that_was_fastest_on_it():
+    picks = run(f"""
+import numpy as np
+out_ = []
+for kind, nz, nx, n2, nfd, n in {[t[:6] for t in TIMED]}:
+    ctx = context(nz=nz, nx=nx, n2=n2, nfd=nfd, nt=20, shots=n, record=1, check_every=-1)
+    shots(ctx, n)
+    if kind == "pairs":
+        ctx.set_reflectivity(np.zeros((nz - 2 * n2, nx - 2 * n2), np.float32))
+        ctx.born_begin()
+    else:
+        ctx.forward_begin()
+    log()
+    (ctx.born_advance if kind == "pairs" else ctx.forward_advance)(20)
+    names = {{r["kernel"] for r in log()}}
+    out_.append([i for i, k in enumerate(("k_interior", "k_two", "k_tile")) if k in names][-1])
+    ctx.close()
+out(out_)
+""")
+    slow = []
+    for t, p in zip(TIMED, picks):
+        ms = t[6:]
+        best = min(m for m in ms if m)
+        if ms[p] > 1.15 * best:
+            slow.append((t, p))
+    assert slow == []

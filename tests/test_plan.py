@@ -26,6 +26,15 @@ extern "C" int tiles_outside(int nz, int nx, int n2, int nfd, int th, int e) {
     }
   return bad;
 }
+extern "C" int edge_tile(int z0, int x0, int th, int nfd, int n2, int nz, int nx) {
+  return tile_edge(z0, x0, th, nfd, n2, nz, nx);
+}
+extern "C" void tile_work(int nz, int nx, int n2, double* inner, double* edge) {
+  BatchWork w;
+  w.add(nz, nx, n2, 224);
+  *inner = w.tile_inner;
+  *edge = w.tile_edge;
+}
 """
 
 
@@ -59,3 +68,15 @@ def test_a_frame_as_deep_as_the_operator_needs_the_clamp(plan):
         nz = 96 + nfd  # nz - n2 = 96
         assert plan.tiles_outside(nz, 186, nfd, nfd, 8, nfd) > 0, nfd
         assert plan.tiles_outside(nz, 186, nfd, nfd, 16, nfd) > 0, nfd
+
+
+def test_tiles_with_and_without_frame_cells_are_counted(plan):
+    inner, edge = C.c_double(), C.c_double()
+    for n2 in (1, 8, 12, 20, 30, 66):
+        for nz, nx in ((2 * n2 + 2, 2 * n2 + 2), (261, 233), (411, 1761), (700, 175), (152, 192)):
+            plan.tile_work(nz, nx, n2, C.byref(inner), C.byref(edge))
+            n = [0, 0]
+            for z0 in range(0, nz, 8):
+                for x0 in range(0, nx, 64):
+                    n[plan.edge_tile(z0, x0, 8, n2 - 1, n2, nz, nx)] += 1
+            assert [round(inner.value / 512e-6), round(edge.value / 512e-6)] == n, (nz, nx, n2)
