@@ -4,6 +4,8 @@ engine on the same inputs.  The kernels evaluate the oracle's operation
 sequence, so records, fields, the accumulator G and the gradient G/P must be
 equal value for value.  Batches (uniform and ragged) must equal the shot-order
 sum of single-shot runs, and the pair must pass the dot-product test."""
+import functools
+
 import numpy as np
 import pytest
 
@@ -274,3 +276,26 @@ def test_cgls_on_the_gpu_follows_the_oracle():
     assert cases.rel_l2(m_gpu, m_ref) <= 1e-4
     rr = [h["rr"] for h in h_gpu]
     assert all(b < a for a, b in zip(rr, rr[1:]))
+
+
+@pytest.fixture
+def marching(monkeypatch):
+    """Contexts on the marching kernels: batches as small as these take whole
+    steps in one launch otherwise."""
+    one = functools.partial(hip_context, zseg=16)
+    monkeypatch.setitem(globals(), "hip_context", one)
+    monkeypatch.setattr(cases, "hip_context", one)
+
+
+@pytest.mark.parametrize("key", sorted(CASES))
+def test_marching_operators_match_the_oracle(marching, key):
+    test_born_matches_oracle(key)
+    test_adjoint_matches_oracle(key)
+
+
+def test_marching_batches(marching):
+    test_born_then_adjoint_reuses_the_background()
+    test_batch_equals_shot_order_sum()
+    test_ragged_batch_equals_single_shot_runs()
+    test_dot_product_fp32()
+    test_cgls_on_the_gpu_follows_the_oracle()

@@ -5,6 +5,8 @@ The bar: per-100-step wavefield relative L2 <= 1e-5 and final image relative
 L2 <= 1e-4 against the FP32 replica.  The kernels evaluate the same operation
 sequence as the replica, so these tests also report (and require) exact
 equality of the values; the FP64 oracle error is printed for information."""
+import functools
+
 import numpy as np
 import pytest
 
@@ -382,3 +384,24 @@ def test_autotune_keeps_results():
     for s in range(3):
         for which in (hip.FIELD_I1, hip.FIELD_I2):
             assert np.array_equal(ctx.field(which, shot=s), ref.field(which, shot=s))
+
+
+@pytest.fixture
+def marching(monkeypatch):
+    """This module's contexts run the marching kernels: batches as small as theirs
+    take whole steps in one launch otherwise."""
+    monkeypatch.setitem(globals(), "hip_context", functools.partial(hip_context, zseg=16))
+
+
+@pytest.mark.parametrize("key", list(CASES))
+def test_marching_kernels_equal_the_oracle(marching, key):
+    test_forward_wavefield_parity(key)
+    test_backward_and_images(key)
+    if key in ("ls_nfd4", "frame_src"):
+        test_receiver_records(key)
+
+
+def test_marching_batches(marching):
+    test_batched_shots_equal_single()
+    test_image_post_and_stack()
+    test_graph_replay_matches_eager()

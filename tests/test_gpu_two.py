@@ -1,6 +1,6 @@
 """Two time steps per launch (the kernel of large batches) against one step per
 launch, bit for bit.  The marching kernels it is compared with equal the oracle
-in test_gpu_parity.py."""
+in test_gpu_parity.py (test_marching_kernels_equal_the_oracle)."""
 import numpy as np
 import pytest
 
@@ -8,8 +8,8 @@ from cases import build_case, hip_context
 
 pytestmark = pytest.mark.gpu
 
-# 41 shots (one past a block's four) of 440 x 618 cells: the batches of 10 M
-# cells and more that take two steps per launch by default
+# 41 shots (one past a block's four) of 440 x 618 cells: batches that take two
+# steps per launch by default
 SHOTS, NZ, NX, N2 = 41, 400, 578, 20
 
 
@@ -142,6 +142,95 @@ def test_window_changed_between_the_passes():
         ctx.backward_begin()
         ctx.backward_advance(nt)
         out.append([ctx.field(w, shot=s) for s in (0, 1, 4, 39) for w in (hip.FIELD_I1, hip.FIELD_I2, hip.FIELD_Q)])
+        ctx.close()
+    for i, (a, b) in enumerate(zip(*out)):
+        assert np.array_equal(a, b), i
+
+
+def launches(ctx, seis, nt):
+    """Interior launches of a forward and of a backward pass."""
+    from rtm_gpu_amd import hip
+    ctx.set_gathers(seis)
+    ctx.set_timing(-1)
+    ctx.forward_begin()
+    ctx.forward_advance(nt)
+    ctx.backward_begin()
+    ctx.backward_advance(nt)
+    n = [ctx.kernel_time(k)[1] for k in (hip.K_FWD_INTERIOR, hip.K_SRC_INTERIOR, hip.K_RCV_INTERIOR,
+                                         hip.K_RCVI_INTERIOR, hip.K_FWD_FRAME)]
+    ctx.set_timing(0)
+    return n[0], n[1], n[2] + n[3], n[4]
+
+
+@pytest.mark.parametrize("nfd,ilste", [(1, 1), (2, 1), (3, 1), (4, 1), (4, 0), (5, 1)])
+def test_these_batches_take_two_steps_per_launch(nfd, ilste):
+    """The batches above do what their tests compare: 42 forward steps in 21
+    interior launches, and in 42 where the heights are set."""
+    case = build_case(name="two", mod_nz=NZ, mod_nx=NX, n2=N2, nfdmax=nfd, nfdmin=min(2, nfd),
+                      ilste=ilste, nt=44, nshot=SHOTS, depth_step=7.0, src_x1=90, tao=0.0008, ds=3)
+    seis = np.zeros((SHOTS, case["cfg"]["n"], 44), np.float32)
+    for zseg, want in ((0, (21, 21, 21, 42)), (16, (42, 42, 42, 42))):
+        ctx = hip_context(case, nshot=SHOTS, zseg=zseg)
+        assert launches(ctx, seis, 44) == want
+        ctx.close()
+
+
+def test_replayed_graph():
+    """A batch that takes two steps per launch as a captured graph, replayed with
+    eager work between the replays."""
+    from rtm_gpu_amd import hip
+    case = build_case(name="two", mod_nz=NZ, mod_nx=NX, n2=N2, nfdmax=3, nfdmin=2, ilste=1, nt=44,
+                      nshot=SHOTS, depth_step=7.0, src_x1=90, tao=0.0008, ds=3)
+    rng = np.random.default_rng(11)
+    sets = [(0.01 * rng.standard_normal((SHOTS, case["cfg"]["n"], 44))).astype(np.float32) for _ in range(2)]
+    fields = (hip.FIELD_U, hip.FIELD_Q, hip.FIELD_I1, hip.FIELD_I2)
+
+    def result(ctx):
+        got = [ctx.field(w, shot=s) for s in (0, SHOTS - 1) for w in fields]
+        return [got[0][N2:-N2, N2:-N2], *got[1:4], got[4][N2:-N2, N2:-N2], *got[5:]]
+
+    one = hip_context(case, nshot=SHOTS, record=1, zseg=16)
+    want = []
+    for d in sets:
+        one.set_gathers(d)
+        one.migrate()
+        want.append(result(one))
+    one.close()
+    ctx = hip_context(case, nshot=SHOTS, record=1)
+    ctx.set_graph(True)
+    for i in (0, 1, 0):
+        ctx.set_gathers(sets[i])
+        for again in range(2):
+            ctx.migrate()
+            for a, b in zip(result(ctx), want[i]):
+                assert np.array_equal(a, b), (i, again)
+        ctx.forward_begin()     # eager work on the same buffers
+        ctx.forward_advance(13)
+    ctx.close()
+
+
+def test_born_and_adjoint_beside_two_steps_per_launch():
+    """A batch whose migration takes two steps per launch and whose Born and
+    adjoint passes take one, their background frame in one launch."""
+    from rtm_gpu_amd import hip
+    n, nt = 103, 44
+    case = build_case(name="twoborn", mod_nz=260, mod_nx=217, n2=N2, nfdmax=3, nfdmin=3, ilste=0, nt=nt,
+                      nshot=n, depth_step=2.0, src_x1=90, tao=0.0008)
+    rng = np.random.default_rng(12)
+    refl = (0.1 * rng.standard_normal((260, 217))).astype(np.float32)
+    seis = (0.01 * rng.standard_normal((n, case["cfg"]["n"], nt))).astype(np.float32)
+    out = []
+    for zseg in (0, 16):
+        ctx = hip_context(case, nshot=n, record=1, zseg=zseg)
+        assert launches(ctx, seis, nt)[0] == (21 if zseg == 0 else 42)
+        ctx.set_reflectivity(refl)
+        ctx.set_timing(-1)
+        got = [ctx.born()]
+        assert ctx.kernel_time(hip.K_BORN_FRAME)[1] == nt - 2  # not whole steps in one launch
+        ctx.set_timing(0)
+        got += [ctx.field(hip.FIELD_Q, shot=s) for s in (0, n - 1)]
+        got.append(ctx.adjoint(seis))
+        out.append(got)
         ctx.close()
     for i, (a, b) in enumerate(zip(*out)):
         assert np.array_equal(a, b), i
