@@ -10,11 +10,6 @@ namespace rtm {
 
 // ---------------------------------------------------------------------------
 // helpers
-template <int I>
-__device__ __forceinline__ float comp(const float4& v) {
-  static_assert(I >= 0 && I < 4, "component");
-  return I == 0 ? v.x : (I == 1 ? v.y : (I == 2 ? v.z : v.w));
-}
 __device__ __forceinline__ float compr(const float4& v, int i) {
   return i == 0 ? v.x : (i == 1 ? v.y : (i == 2 ? v.z : v.w));
 }
@@ -87,9 +82,6 @@ __device__ __forceinline__ float bld1(Rsrc r, unsigned vo, unsigned so) {
 __device__ __forceinline__ unsigned bld1u(Rsrc r, unsigned vo, unsigned so) {
   return (unsigned)__builtin_amdgcn_raw_buffer_load_b32(r, (int)vo, (int)so, 0);
 }
-__device__ __forceinline__ void bst1(Rsrc r, unsigned vo, unsigned so, float v) {
-  __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), r, (int)(vo + so), 0, 0);
-}
 // streaming variants (u0 rows, u(k+1) and strip writes: touched once per step)
 __device__ __forceinline__ float bld1s(Rsrc r, unsigned vo, unsigned so) {
   return __uint_as_float((unsigned)__builtin_amdgcn_raw_buffer_load_b32(r, (int)vo, (int)so,
@@ -139,24 +131,6 @@ __device__ __forceinline__ bool is_receiver(int c, const Rcv& r, int* s) {
   *s = d / r.ds;
   return true;
 }
-
-// Row-major walk of a tile with `cols` columns by a 256-thread block: thread
-// t visits cells t, t+256, ... keeping (row, column) incrementally, so the
-// loop carries no integer division.
-struct TileWalk {
-  int i, j, di, dj, cols;
-  __device__ __forceinline__ explicit TileWalk(int c) : cols(c) {
-    i = (int)threadIdx.x / c;
-    j = (int)threadIdx.x - i * c;
-    di = 256 / c;
-    dj = 256 - di * c;
-  }
-  __device__ __forceinline__ void next() {
-    i += di;
-    j += dj;
-    if (j >= cols) { j -= cols; ++i; }
-  }
-};
 
 __device__ __forceinline__ int mirror_idx(int g, int n) {  // kernel.cu:65-68
   if (g < 0) g = -g;
@@ -211,23 +185,8 @@ __device__ __forceinline__ void strip_cell(const Grid& g, int nx, int mnx, unsig
     *x = g.n2 + (int)c;
   }
 }
-// Grid cell -> strip element index, or -1.
-__device__ __forceinline__ long long strip_index(const Grid& g, int nx, int mnx, int z, int x) {
-  const long long a = (long long)g.mnz * g.nfd, b = (long long)g.nfd * mnx;
-  const int n2 = g.n2, nfd = g.nfd;
-  if (z >= n2 && z < g.nz - n2) {
-    if (x >= n2 - nfd && x < n2) return (long long)(z - n2) * nfd + (n2 - 1 - x);
-    if (x >= nx - n2 && x < nx - n2 + nfd) return a + (long long)(z - n2) * nfd + (x - (nx - n2));
-    return -1;
-  }
-  if (x >= n2 && x < nx - n2) {
-    if (z >= n2 - nfd && z < n2) return 2 * a + (long long)(n2 - 1 - z) * mnx + (x - n2);
-    if (z >= g.nz - n2 && z < g.nz - n2 + nfd) return 2 * a + b + (long long)(z - (g.nz - n2)) * mnx + (x - n2);
-  }
-  return -1;
-}
-// Strip element of frame cell (z, x) of a shot nx wide, or -1 (strip_index
-// without branches, in 32 bits: a slot holds fewer than 2^31 elements).
+// Strip element of frame cell (z, x) of a shot nx wide, or -1; without branches,
+// in 32 bits (a slot holds fewer than 2^31 elements).
 __device__ __forceinline__ int strip_elem(const Grid& g, int nx, int mnx, int z, int x) {
   const int a = g.mnz * g.nfd, b = g.nfd * mnx, n2 = g.n2, nfd = g.nfd;
   const bool zin = z >= n2 && z < g.nz - n2, xin = x >= n2 && x < nx - n2;
