@@ -198,12 +198,12 @@ __global__ __launch_bounds__(256) void k_conv(const ConvArgs a) {
     }
     ConvOut<NCOB>::fetch(a, kg, t < tiles && x < a.w, row * (unsigned)a.w + (unsigned)x, e);
   };
-  unsigned t = blockIdx.x * 4u + (threadIdx.x >> 6);
+  unsigned t = blockIdx.x * 4u + (unsigned)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   b8 av[NK], nx[NK];
   typename ConvOut<NCOB>::Extra e{}, en{};
   fetch(t, av, e);
   for (; t < tiles; t += step) {
-    fetch(t + step, nx, en);
+    if (t + step < tiles) fetch(t + step, nx, en);
     f4 acc[NCOB];
 #pragma unroll
     for (int cb = 0; cb < NCOB; ++cb) acc[cb] = f4{0.f, 0.f, 0.f, 0.f};
