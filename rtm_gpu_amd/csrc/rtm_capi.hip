@@ -70,6 +70,7 @@ struct rtm_ctx {
   std::vector<char> shot_model;
   std::vector<int> win_ref;                 // shots using each slot
   std::vector<int> win_nx;                  // width of each slot's window
+  std::vector<float> win_lines;             // line_share of each
   std::vector<unsigned long long> win_fp;   // two 64-bit content fingerprints per slot
   float tab_vmin = 0.f, tab_dv = 1.f;  // bin parameters of the current table
   int tab_nrow = 1, tab_cs = 4;
@@ -107,6 +108,7 @@ struct rtm_ctx {
   long long cells = 0;     // grid cells of the batch
   mutable BatchWork work;  // of the batch, made on first use
   mutable bool work_ok = false;
+  float model_lines = 0.f;  // line_share of the context's model
   long long tuned_cells = 0;  // of the batch that rtm_autotune timed
   int two_tuned = -1;      // rtm_autotune's choice: 1 two steps per launch, 0 one
   int zs2[5] = {0};        // rows per wave of two steps by kind (0: default)
@@ -340,7 +342,7 @@ const BatchWork& batch_work(const rtm_ctx* c) {
   const int cols = two_cols(g, std::min(c->nfd, TWO_MAX_NFD), c->nshot);
   double cells = 0.0;
   for (const ShotGeo& q : c->geo) {
-    w.add(g.nz, q.nx, g.n2, cols);
+    w.add(g.nz, q.nx, g.n2, cols, c->m.mstride ? c->win_lines[q.win] : c->model_lines);
     cells += 1e-6 * g.nz * q.nx;
   }
   const double ns = std::max<double>(1.0, (double)c->geo.size());
@@ -1057,12 +1059,29 @@ int upload_geometry(rtm_ctx* c) {
   return RTM_OK;
 }
 
+// 128-byte lines of the coefficient table that a wave's 256 cells of a row touch,
+// per cell, over a sample of the rows (BatchWork::lines).
+float line_share(const rtm_ctx* c, int nx, const std::vector<unsigned>& ko) {
+  const Grid& g = c->g;
+  std::vector<int> seen((size_t)c->tab_nrow * c->tab_cs / 32 + 1, -1);
+  int chunk = 0;
+  long long lines = 0, cells = 0;
+  for (int z = 0; z < g.nz; z += std::max(1, g.nz / 16))
+    for (int x0 = 0; x0 < nx; x0 += 256, ++chunk)
+      for (int x = x0; x < std::min(nx, x0 + 256); ++x, ++cells) {
+        int& s = seen[ko[(size_t)z * g.pitch + g.x0 + x] >> 7];
+        lines += s != chunk;
+        s = chunk;
+      }
+  return (float)((double)lines / (double)cells);
+}
+
 // Pad a model window (v, r1 of nz x nx) into the padded layout and derive the
 // per-cell operands: p = v*v*tao2*h2 (kernel.cu:73) and the byte offset of the
 // velocity bin's coefficient row (kernel.cu:55-56: FP32 quotient, double +
 // 0.5, truncation, clamped to the table).  Guard columns repeat the edge.
 int upload_model_window(rtm_ctx* c, int nx, const float* v, const float* r1, float* dv_, float* dr_,
-                        float* dp_, unsigned* dk_) {
+                        float* dp_, unsigned* dk_, float* lines) {
   const Grid& g = c->g;
   std::vector<float> pv((size_t)g.fstride, 0.f), pr((size_t)g.fstride, 0.f), pp((size_t)g.fstride);
   std::vector<unsigned> pk((size_t)g.fstride);
@@ -1083,6 +1102,7 @@ int upload_model_window(rtm_ctx* c, int nx, const float* v, const float* r1, flo
     }
     pk[i] = (unsigned)kb * (unsigned)c->tab_cs * 4u;
   }
+  *lines = line_share(c, nx, pk);
   const size_t b = (size_t)g.fstride * sizeof(float);
   HIPCHK(c, hipMemcpyAsync(dv_, pv.data(), b, hipMemcpyHostToDevice, c->stream));
   HIPCHK(c, hipMemcpyAsync(dr_, pr.data(), b, hipMemcpyHostToDevice, c->stream));
@@ -1327,7 +1347,7 @@ int rtm_set_model(rtm_ctx* c, const float* v, const float* r1, const float* w, c
   }
   HIPCHK(c, hipMemcpyAsync(c->d_ctab, tab.data(), tab.size() * sizeof(float), hipMemcpyHostToDevice, c->stream));
   c->tab_vmin = vmin; c->tab_dv = dv; c->tab_nrow = nrow; c->tab_cs = CS; c->tab_ls = ls;
-  rc = upload_model_window(c, g.nx, v, r1, c->d_v, c->d_r1, c->d_pm, c->d_ko);
+  rc = upload_model_window(c, g.nx, v, r1, c->d_v, c->d_r1, c->d_pm, c->d_ko, &c->model_lines);
   if (rc != RTM_OK) return rc;
   HIPCHK(c, hipMemcpyAsync(c->d_w, w, (g.n2 + 1) * sizeof(float), hipMemcpyHostToDevice, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -1339,6 +1359,7 @@ int rtm_set_model(rtm_ctx* c, const float* v, const float* r1, const float* w, c
   c->shot_model.assign(c->p.max_shots, 0);
   c->win_ref.assign(c->p.max_shots, 0);
   c->win_nx.assign(c->p.max_shots, 0);
+  c->win_lines.assign(c->p.max_shots, 0.f);
   c->win_fp.assign(2 * (size_t)c->p.max_shots, 0);
   m.h1 = 1.0 + (double)c->p.hzx2_1;  // (1.0+hzx2_1)*Dc[M_top] (kernel.cu:58)
   m.hzx2_1 = c->p.hzx2_1; m.tao2 = c->p.tao2; m.h2 = c->p.h2;
@@ -1402,6 +1423,7 @@ int rtm_set_shot_geometry(rtm_ctx* c, int nshot, const rtm_shot_geom* sg) {
   std::fill(c->shot_model.begin(), c->shot_model.end(), 0);
   c->win_ref.assign(c->p.max_shots, 0);
   c->win_nx.assign(c->p.max_shots, 0);
+  c->win_lines.assign(c->p.max_shots, 0.f);
   c->win_fp.assign(2 * (size_t)c->p.max_shots, 0);
   c->tp_ok = c->cp_ok = false;
   return upload_geometry(c);
@@ -1440,6 +1462,7 @@ int rtm_set_shot_model(rtm_ctx* c, int shot, const float* v, const float* r1) {
   if (c->win_ref.size() != (size_t)c->p.max_shots) {
     c->win_ref.assign(c->p.max_shots, 0);
     c->win_nx.assign(c->p.max_shots, 0);
+    c->win_lines.assign(c->p.max_shots, 0.f);
     c->win_fp.assign(2 * (size_t)c->p.max_shots, 0);
   }
   const int nx = c->geo[shot].nx;
@@ -1455,7 +1478,7 @@ int rtm_set_shot_model(rtm_ctx* c, int shot, const float* v, const float* r1) {
       if (c->win_ref[i] == 0) w = i;
     if (w < 0) return fail(c, RTM_E_STATE, "no free model window slot");
     const size_t o = (size_t)w * g.fstride;
-    int rc = upload_model_window(c, nx, v, r1, c->d_mv + o, c->d_mr1 + o, c->d_mpm + o, c->d_mko + o);
+    int rc = upload_model_window(c, nx, v, r1, c->d_mv + o, c->d_mr1 + o, c->d_mpm + o, c->d_mko + o, &c->win_lines[w]);
     // r1 is read at the corner cells only, the lateral factors at the other
     // frame cells: one plane holds both
     if (rc == RTM_OK && launch_frame_lat(g, nx, c->d_mv + o, c->p.taoh2, true, c->d_mr1 + o, c->stream) != hipSuccess)

@@ -33,8 +33,10 @@ struct BatchWork {
   double inner = 0, frame = 0;           // cells of the interior, of the frame
   double quad = 1;                       // shots of full blocks of four per shot
   double windows = 0;                    // cells times distinct model windows per shot
-  // a shot of an nz x nx grid; two_cols: columns of a wave of k_two
-  void add(int nz, int nx, int n2, int two_cols) {
+  double lines = 0;                      // cells times coefficient lines per cell
+  // a shot of an nz x nx grid; two_cols: columns of a wave of k_two; line_share:
+  // 128-byte lines of the coefficient table that 256 cells of a row touch, per cell
+  void add(int nz, int nx, int n2, int two_cols, double line_share) {
     const int mnz = nz - 2 * n2, mnx = nx - 2 * n2;
     const auto split = [n2](int n, int t, double* all, double* in) {  // tiles of t along n cells
       *all = (n + t - 1) / t;
@@ -50,21 +52,25 @@ struct BatchWork {
     wave_two += (mnx + two_cols - 1) / two_cols * 256 * 1e-6 * mnz;
     inner += 1e-6 * mnz * mnx;
     frame += 1e-6 * nz * nx - 1e-6 * mnz * mnx;
+    lines += line_share * 1e-6 * nz * nx;
   }
 };
 
 // Microseconds of a forward and a backward step by half-length 1..12, fitted to
-// 880 timed batches: ten grids of 75 to 2400 columns, 2 to 60 M cells,
+// 1500 timed batches: ten grids of 75 to 2400 columns, 2 to 93 M cells,
 // least-squares rows up to half-length 5, Taylor rows above.  A marching wave
-// spends 0.5 to 1 us on each of its 20 to 30 rows whatever the batch and pads
-// the interior to 256 columns; k_tile is two memory accesses deep but bound by
-// instruction issue, the more the longer the operator and the more of its tiles
-// hold frame cells; k_two takes two steps per pass over memory.  The sums are
-// within 20% of the times, and the kernel of the smallest one took on average
-// 0.6% longer than the fastest and at worst 1.24 times as long.  One line on the cells times the
-// half-length, which depends on none of the grid's shape, was 5.7% off on average
-// and up to twice as slow: 144 shots of 261 x 133 at half-length 8, 100 steps,
-// 22 ms by k_tile, 15 by the marching kernels.
+// spends 0.5 to 1 us on each of its 20 to 30 rows whatever the batch, pads the
+// interior to 256 columns and gathers a coefficient row per cell, which costs by
+// the lines that its cells touch (a tenth of a line per cell in a smooth model,
+// 0.6 to 0.8 in a rough one: then it takes up to 1.7 times as long); k_tile is two
+// memory accesses deep but bound by instruction issue, the more the longer the
+// operator and the more of its tiles hold frame cells; k_two reads planes and takes
+// two steps per pass over memory.  The sums are within 25% of the times; the kernel
+// with the smallest one took on average 0.6% longer than the fastest, at worst 1.2
+// times as long.  One line on the cells times the half-length, which knows neither
+// the grid's shape nor the model, was 5% off on average and up to twice as slow: 171
+// shots of 261 x 133 at half-length 8, 60 steps each way, 16.7 ms by k_tile, 10.0 by
+// the marching kernels.
 namespace cost {
 constexpr int kN = 12;
 constexpr double kTile[kN][3] = {  // per launch, tiles without, with frame cells
@@ -86,15 +92,21 @@ constexpr double kMarch2[kN][4] = {
     {75, 9.9, 25, 7}, {90, 10.6, 25, 6.3}, {105, 11.4, 24, 5.5}, {119, 12, 27, 3}, {133, 12.5, 31, 0.3},
     {147, 11.7, 31, 0.2}, {161, 10.8, 31, 0}};
 
+// Coefficient lines beyond those of the fitted models, in millions.
+inline double more_lines(const BatchWork& w, int nfd) {
+  return w.lines - (nfd <= 5 ? 0.1 : 0.004) * (w.inner + w.frame);
+}
 inline double tile(const BatchWork& w, int nfd, bool both, bool ls) {
   const double* k = both ? kTile2[nfd - 1] : kTile[nfd - 1];
   const double win = !both ? 2.0 : ls ? 2.3 + 1.9 * nfd : 2.5;  // a window's planes from memory
-  return k[0] + k[1] * w.tile_inner + k[2] * w.tile_edge + win * w.windows;
+  return k[0] + k[1] * w.tile_inner + k[2] * w.tile_edge + win * w.windows +
+         (both ? 4.2 : 2.6) * more_lines(w, nfd);
 }
 inline double march(const BatchWork& w, int nfd, bool both, bool ls) {
   const double* k = both ? kMarch2[nfd - 1] : kMarch[nfd - 1];
   const double win = !both ? 3.2 : ls ? 7 + 2.6 * nfd : 5.0;
-  return k[0] + k[1] * w.wave + k[2] * w.frame + k[3] * w.inner + win * w.windows;
+  return k[0] + k[1] * w.wave + k[2] * w.frame + k[3] * w.inner + win * w.windows +
+         (both ? 16.0 : 12.7) * more_lines(w, nfd);
 }
 inline double two(const BatchWork& w, int nfd) {  // windows: shared by four shots at least
   const double* k = kTwo[nfd - 1];

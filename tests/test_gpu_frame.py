@@ -107,3 +107,48 @@ def test_widths_on_one_model(nshot, zseg, frame_split):
         ctx.close()
     for i, (a, b) in enumerate(zip(*out)):
         assert np.array_equal(a, b), i
+
+
+@pytest.mark.parametrize("nz,nx,n2,nfdmax", [
+    (400, 578, 12, 3),   # the narrowest frame with windows of four columns
+    (370, 601, 31, 5),   # one wave per side
+    (300, 497, 64, 4)])  # more rows than a block takes, two corner records
+def test_whole_frame_launch_on_a_rough_model(nz, nx, n2, nfdmax):
+    """A coefficient row of its own for almost every cell: such batches take two
+    steps per launch, and with them the frame in one launch."""
+    from rtm_gpu_amd import hip
+    shots = -(-12_000_000 // ((nz + 2 * n2) * (nx + 2 * n2)))
+    shots += (2 - shots) % 4  # two of a block's four past the batch
+    nt = 42
+    case = build_case(name="quadr", mod_nz=nz, mod_nx=nx, n2=n2, nfdmax=nfdmax, ilste=1, nt=nt,
+                      nshot=shots, depth_step=6.0, src_x1=50, tao=0.0008)
+    cfg, m = case["cfg"], case["model"]
+    z, x = np.mgrid[:cfg["nz"], :cfg["nx"]].astype(np.float32)
+    v = (3000 + 1300 * np.sin(x / 23 + 0.7 * np.sin(z / 31)) * np.cos(z / 19 + 0.5 * np.sin(x / 41))).astype(np.float32)
+    bins, row = 3000, np.asarray(m["c"], np.float32)[:nfdmax + 1]
+    table = (row[None, :] * (1 + 1e-3 * np.sin(np.arange(bins)))[:, None]).astype(np.float32)
+    keys = ("nz", "nx", "n2", "nfdmax", "nt", "nt2", "icompen", "s_l", "s_r", "s_z", "ds", "n",
+            "tao2", "h2", "taoh", "taoh2", "hzx2_1")
+    rng = np.random.default_rng(n2)
+    seis = (0.01 * rng.standard_normal((shots, cfg["n"], nt))).astype(np.float32)
+    out = []
+    for zseg in (0, 16):  # 16 rows per wave: one step per launch
+        ctx = hip.Context(**{k: cfg[k] for k in keys}, ilste=0, max_shots=shots, zseg=zseg)
+        ctx.set_model(v, np.full_like(v, 0.2), m["w"], table, np.arange(bins + 1) * (nfdmax + 1), bins, 1600.0, 1.0)
+        ctx.set_wavelet(m["wav"])
+        ctx.set_shots(case["r_u"], case["r_x"])
+        ctx.set_gathers(seis)
+        ctx.set_timing(-1)
+        ctx.forward_begin()
+        ctx.forward_advance(nt)
+        assert ctx.kernel_time(hip.K_FWD_INTERIOR)[1] == (nt - 2) // (2 if zseg == 0 else 1)
+        ctx.set_timing(0)
+        got = [ctx.field(w, shot=s) for s in (0, shots - 1) for w in (hip.FIELD_U, hip.FIELD_U_PREV)]
+        got += [ctx.strip(shots - 1, k) for k in (2, nt // 2, nt - 1)]
+        ctx.backward_begin()
+        ctx.backward_advance(nt)
+        got += [ctx.field(w, shot=s) for s in (0, shots - 1) for w in (hip.FIELD_Q, hip.FIELD_I1, hip.FIELD_I2)]
+        out.append(got)
+        ctx.close()
+    for i, (a, b) in enumerate(zip(*out)):
+        assert np.isfinite(a).all() and np.array_equal(a, b), i

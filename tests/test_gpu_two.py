@@ -162,7 +162,7 @@ def launches(ctx, seis, nt):
     return n[0], n[1], n[2] + n[3], n[4]
 
 
-@pytest.mark.parametrize("nfd,ilste", [(1, 1), (2, 1), (3, 1), (4, 1), (4, 0), (5, 1)])
+@pytest.mark.parametrize("nfd,ilste", [(1, 1), (2, 1), (3, 1), (4, 1), (4, 0)])
 def test_these_batches_take_two_steps_per_launch(nfd, ilste):
     """The batches above do what their tests compare: 42 forward steps in 21
     interior launches, and in 42 where the heights are set."""
@@ -231,6 +231,23 @@ def test_born_and_adjoint_beside_two_steps_per_launch():
         got += [ctx.field(hip.FIELD_Q, shot=s) for s in (0, n - 1)]
         got.append(ctx.adjoint(seis))
         out.append(got)
+        ctx.close()
+    for i, (a, b) in enumerate(zip(*out)):
+        assert np.array_equal(a, b), i
+
+
+def test_two_steps_per_launch_at_the_longest_half_length():
+    """Half-length 5 takes two steps per launch from larger batches on."""
+    n, nt = 93, 30
+    case = build_case(name="two", mod_nz=NZ, mod_nx=NX, n2=N2, nfdmax=5, ilste=1, nt=nt, nshot=n,
+                      depth_step=3.0, src_x1=90, tao=0.0008, ds=3)
+    rng = np.random.default_rng(13)
+    seis = (0.01 * rng.standard_normal((n, case["cfg"]["n"], nt))).astype(np.float32)
+    out = []
+    for zseg, want in ((0, (nt - 2) // 2), (16, nt - 2)):
+        ctx = hip_context(case, nshot=n, record=1, zseg=zseg)
+        assert launches(ctx, seis, nt)[:3] == (want,) * 3
+        out.append(passes(ctx, seis, (1, 6)))
         ctx.close()
     for i, (a, b) in enumerate(zip(*out)):
         assert np.array_equal(a, b), i

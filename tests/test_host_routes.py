@@ -241,7 +241,8 @@ for width in (900, 860, 2400, 900):
     res.append(kernels())
 out(res)
 """)
-    assert got == [["k_tile"], ["k_tile"], ["k_two"], ["k_two"]]
+    assert got[:2] == [["k_tile"], ["k_tile"]]
+    assert ["k_tile"] not in got[2:]
 
 
 def test_a_longer_operator_drops_the_choice():
@@ -376,3 +377,37 @@ out(out_)
         if ms[p] > 1.15 * best:
             slow.append((t, p))
     assert slow == []
+
+
+@pytest.mark.parametrize("nz,nx,n2,nfd,n,ms", [
+    (261, 300, 30, 4, 255, (28.1, 18.4, 31.1)), (261, 300, 30, 2, 511, (45.9, 29.6, 51.6)),
+    (440, 540, 20, 3, 42, (12.6, 10.0, 11.7)), (411, 1761, 30, 2, 14, (14.7, None, 12.1))])
+def test_a_rough_model_costs_the_kernels_that_gather(nz, nx, n2, nfd, n, ms):
+    """Cells whose coefficient rows lie in different lines: timed as above, on
+    shared windows or (None) a window per shot."""
+    pick = run(f"""
+import numpy as np
+from rtm_gpu_amd import hip
+nz, nx, n2, nfd, n, own = {nz}, {nx}, {n2}, {nfd}, {n}, {ms[1] is None}
+z, x = np.mgrid[:nz, :nx].astype(np.float32)
+v = (3000 + 1300 * np.sin(x / 23 + 0.7 * np.sin(z / 31)) * np.cos(z / 19 + 0.5 * np.sin(x / 41))).astype(np.float32)
+m, nt = nx - 2 * n2, 20
+ctx = hip.Context(nz=nz, nx=nx, n2=n2, nfdmax=nfd, nt=nt, nt2=nt, ilste=0, icompen=1, s_l=n2,
+                  s_r=nx - n2 - 1, s_z=n2, ds=1, n=m, tao2=1e-6, h2=1e-2, taoh=1e-4, taoh2=1e-8,
+                  hzx2_1=1.0, max_shots=n, check_every=-1)
+ctx.set_model(v, v * 0, np.zeros(n2 + 1), np.ones(3001 * (nfd + 1)),
+              (np.arange(3001) * (nfd + 1)).astype(np.int32), 3000, 1400.0, 1.0)
+ctx.set_wavelet(np.zeros(nt + 1, np.float32))
+if own:
+    ragged(ctx, n)
+    for s in range(n):
+        ctx.set_shot_model(s, v + np.float32(0.37 * s), v * 0)
+else:
+    shots(ctx, n)
+ctx.forward_begin()
+log()
+ctx.forward_advance(20)
+names = {{r["kernel"] for r in log()}}
+out([i for i, k in enumerate(("k_interior", "k_two", "k_tile")) if k in names][-1])
+""")
+    assert ms[pick] <= 1.15 * min(t for t in ms if t), pick

@@ -31,7 +31,7 @@ extern "C" int edge_tile(int z0, int x0, int th, int nfd, int n2, int nz, int nx
 }
 extern "C" void tile_work(int nz, int nx, int n2, double* inner, double* edge) {
   BatchWork w;
-  w.add(nz, nx, n2, 224);
+  w.add(nz, nx, n2, 224, 0.1);
   *inner = w.tile_inner;
   *edge = w.tile_edge;
 }
