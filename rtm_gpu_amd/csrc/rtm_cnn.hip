@@ -153,7 +153,9 @@ struct ConvOut {
 
 // Weight-stationary convolution of narrow inputs (8, 16 or 24 channels): a wave
 // holds its weights (all NK K-steps of NCOB blocks of 16 output channels) in
-// registers and walks 16-pixel row tiles, the next tile's inputs in flight.
+// registers and walks 16-pixel row tiles, the next tile's inputs in flight where
+// there is one (the addresses of one that is not there cost a wave with a single
+// tile: five layers of 16 channels at 32 x 64 x 64 0.195 ms a call, 0.183 without).
 // K-step ks covers k = 32 ks .. 32 ks + 31; lane group kg feeds k = 32 ks +
 // 8 kg .. +7, eight consecutive channels of one tap (cin_p is a multiple of 8).
 template <int NK, int NCOB>
